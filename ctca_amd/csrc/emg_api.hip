@@ -352,12 +352,15 @@ int emg_destroy(emg_ctx *c) {
   if (c->stream) (void)hipStreamSynchronize(c->stream);
   free_state64(c->s64);
   free_state64(c->t64);
-  free_state64(c->lam);
+  dfree(c->lam);
   for (int k = 0; k < kStateSlots; k++) free_state64(c->slot[k]);
   dfree(c->adj_e);
   dfree(c->adj_g);
   dfree(c->adj_q);
   dfree(c->adj_sum);
+  dfree(c->adj_bins.count);
+  dfree(c->adj_bins.start);
+  dfree(c->adj_bins.rec);
   FxBuckets &B = c->fx;
   for (int k = 0; k < 2; k++) {
     dfree(B.st[k].cell);
@@ -978,16 +981,14 @@ static int copy_state(const State64 &src, const State64 &dst, int64_t n, hipStre
 static int need_adjoint(emg_ctx *c) {
   int rc = need_fp64(c);
   if (rc) return rc;
-  if (c->lam.x) return EMG_OK;
-  if ((rc = alloc_state64(c->lam, c->cap_total)) ||
+  if (c->lam) return EMG_OK;
+  if ((rc = dalloc(&c->lam, 8 * (size_t)c->cap_total, "particle adjoints")) ||
       (rc = dalloc(&c->adj_e, 3 * c->ncell, "adjoint field")) ||
       (rc = dalloc(&c->adj_g, c->ncell, "adjoint density")) ||
       (rc = dalloc(&c->adj_q, EMG_MAX_SPECIES, "adjoint factors")) ||
-      (rc = dalloc(&c->adj_sum, 3 * EMG_MAX_SPECIES, "adjoint sums")))
+      (rc = dalloc(&c->adj_sum, (size_t)adj_vsum_need(), "adjoint sums")))
     return rc;
-  State64 &L = c->lam;
-  double *arr[6] = {L.x, L.y, L.z, L.vx, L.vy, L.vz};
-  for (double *p : arr) launch_zero(p, sizeof(double) * c->cap_total, c->stream);
+  launch_zero(c->lam, 8 * sizeof(double) * c->cap_total, c->stream);
   launch_zero(c->adj_e, sizeof(double) * 3 * c->ncell, c->stream);
   return hip_check(hipGetLastError(), "adjoint allocation");
 }
@@ -1022,9 +1023,7 @@ int emg_adj_reset(emg_ctx *c) {
   CTX_CHECK(c);
   int rc = need_adjoint(c);
   if (rc) return rc;
-  State64 &L = c->lam;
-  double *arr[6] = {L.x, L.y, L.z, L.vx, L.vy, L.vz};
-  for (double *p : arr) launch_zero(p, sizeof(double) * c->cap_total, c->stream);
+  launch_zero(c->lam, 8 * sizeof(double) * c->cap_total, c->stream);
   return hip_check(hipGetLastError(), "adjoint reset");
 }
 
@@ -1035,6 +1034,7 @@ int emg_adj_step(emg_ctx *c, int32_t ustep) {
   if (!rc) rc = need_fields(c);
   if (rc) return rc;
   if (ustep < 0) return set_error(EMG_ERR_ARG, "ustep must be >= 0");
+  if ((rc = adj_bins_alloc(c))) return rc;
   launch_adj_step64(c, ustep);
   return hip_check(hipGetLastError(), "adjoint step launch");
 }

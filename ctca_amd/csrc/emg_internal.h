@@ -161,6 +161,15 @@ constexpr int kRunSpan = 96;   // cells a block may span and stay whole
 constexpr int kRunCells = 64;  // cells per run of a cut block
 static_assert(kRunSpan >= kRunCells, "a cut block's runs span over kRunCells / 2 cells");
 
+// Workspace of the adjoint's transposed gather (k_adj.hip): counters and
+// cursors per tile, each tile's first record, the records of one pass.
+struct AdjBins {
+  int32_t *count;
+  int64_t *start;
+  void *rec;
+  int64_t len;  // records
+};
+
 // Upper-face accumulators of the charge.  The periodic accumulators add the
 // weight a particle puts on node n of an axis into node 0; the reference
 // keeps it apart until its border exchange and add_boundary_charge, which
@@ -253,11 +262,12 @@ struct emg_ctx {
   double *scratch;  // this device's static staging array (emg_get_rho_noalloc)
 
   // adjoint window (FP64 form)
-  emg::State64 lam;  // lambda_x in x, y, z; lambda_v in vx, vy, vz
+  double *lam;       // 8 per particle slot: lambda_x, lambda_v, 2 unused (one 64-byte line)
   double *adj_e;     // 3 x ncell: transposed gather of qmp * lambda_a
   double *adj_g;     // ncell: uploaded density adjoint
   double *adj_q;     // nspec: its factor per species
-  double *adj_sum;   // 3 x nspec: velocity adjoint sums
+  double *adj_sum;   // velocity adjoint sums, then their block partials
+  emg::AdjBins adj_bins;
   emg::State64 slot[emg::kStateSlots];  // saved particle states
   int64_t slot_cnt[emg::kStateSlots][EMG_MAX_SPECIES];
 
@@ -322,9 +332,11 @@ int sort64_commit(emg_ctx *c);
 int init_device(emg_ctx *c, const emg_device_species *spec, int nspec, uint64_t seed);
 
 // adjoint of the FP64 ES push (k_adj.hip)
-void launch_adj_step64(emg_ctx *c, int ustep);
+int adj_bins_alloc(emg_ctx *c);
+void launch_adj_step64(emg_ctx *c, int ustep);  // after adj_bins_alloc
 void launch_adj_density64(emg_ctx *c, const double *qfac_dev);
-void launch_adj_vsum(emg_ctx *c, double *out_dev);
+void launch_adj_vsum(emg_ctx *c, double *out_dev);  // out_dev: adj_vsum_need() doubles
+int64_t adj_vsum_need();
 
 // FP32 + fixed point (k_fx.hip)
 int fx_alloc(emg_ctx *c, int64_t ntotal);

@@ -12,11 +12,14 @@
 //   lambda_a = M^T w + w,   lambda_v <- M^T w  (M^T is the rotation by -b)
 //   lambda_x <- lambda_x + sum_c lambda_a_c * qmp * grad E_c(x_k)
 // and qmp * lambda_a is scattered with the same trilinear weights onto a
-// nodal adjoint field (the transpose of the gather), from which the host
+// nodal adjoint field (the transpose of the gather, binned by tiles: below),
+// from which the host
 // forms the adjoint of rho through the field solve; the contribution of
 // x_k to rho is then added by k_adj_density: lambda_x += q * grad g(x_k).
 // B enters as a constant (the electrostatic path keeps B static; the
 // gradient of a non-uniform B is not part of the step adjoint).
+#include <algorithm>
+
 #include "emg_internal.h"
 
 namespace emg {
@@ -77,64 +80,233 @@ __device__ __forceinline__ void rotate(double u[3], const double b[3]) {
   u[2] += bor * (tx * b[1] - ty * b[0]);
 }
 
-__global__ __launch_bounds__(kBlock) void k_adj_step64(State64 s, State64 lam, SpeciesTab sp,
-                                                      const double *__restrict__ node, Grid g,
-                                                      int ustep, double *__restrict__ adj_e) {
-  int is = blockIdx.y;
-  int64_t m = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (m >= sp.cnt[is]) return;
-  m += sp.off[is];
-  const double gustep = (double)ustep;
-  const double qmp = sp.qm[is] * gustep * 0.5;
-  Tri t = tri(s.x[m], s.y[m], s.z[m], g);
-  // nodal E/B at the eight corners
-  double e[8][3], bf[3] = {0.0, 0.0, 0.0};
-#pragma unroll
-  for (int q = 0; q < 8; q++) {
-    int a = q & 1, b = (q >> 1) & 1, c = q >> 2;
-    const double *p = node + 8 * nodal(g, t.i + a, t.j + b, t.k + c);
-    double w = t.wx[a] * t.wy[b] * t.wz[c];
-    e[q][0] = p[0];
-    e[q][1] = p[1];
-    e[q][2] = p[2];
-    bf[0] += w * p[3];
-    bf[1] += w * p[4];
-    bf[2] += w * p[5];
+// The particles of a window are in no spatial order (their order is that of
+// every saved state).  Stepped in that order, the kernel gathered 24 x 16 bytes
+// from random cells and sent one global FP64 atomic per particle, node and
+// component, at 22 G atomics/s: 9.28 ms for 8.8M particles on 64^3 cells, whose
+// state is 0.2 ms of traffic.  So a step bins the particles by tiles of
+// kAdjTile^3 cells first:
+//   k_adj_count   particles per tile (a block's counts in LDS, one atomic per
+//                 block and tile), then a scan;
+//   k_adj_bin     position and index of each particle, 32 bytes, to its tile's
+//                 range, a block's records of one tile in one run;
+//   k_adj_step64  one workgroup per tile: its nodes' E and B staged in LDS, the
+//                 reverse step of its particles (their adjoints are 64-byte
+//                 records, so an access at a random particle is one line), the
+//                 transposed gather summed in an LDS tile of FP64 nodes, each
+//                 of which reaches memory once.
+// At the same size: 0.08 + 0.26 + 0.50 ms, bound by the random 64-byte lines of
+// the adjoints.  (Binning only the scatter, with the gather in slot order, took
+// 0.08 + 2.22 + 0.18 ms.)  With more than kAdjLdsTiles tiles a
+// block's LDS counters would not fit, and each particle takes one global
+// atomic on its tile's counter.
+constexpr int kAdjTile = 8;
+constexpr int kAdjNode = kAdjTile + 1;        // nodes per axis of a tile
+constexpr int kAdjLdsTiles = 4096;            // 16 KB of LDS counters
+constexpr int64_t kAdjRecMax = int64_t(1) << 24;  // records per pass (512 MB)
+constexpr int kAdjBlock = 512;
+
+// position, and the particle's index | species << 56
+struct AdjRec {
+  double x, y, z;
+  int64_t ms;
+};
+static_assert(sizeof(AdjRec) == 32, "two 16-byte accesses");
+
+struct AdjTiles {
+  int ntx, nty, ntz, n;
+};
+
+__device__ __forceinline__ int adj_tile(const AdjTiles &a, int i, int j, int k) {
+  return ((k / kAdjTile) * a.nty + j / kAdjTile) * a.ntx + i / kAdjTile;
+}
+
+// The particles of a pass: [lo, hi) of each species, as indices of the state
+// arrays.  A block takes kBlock P of species blockIdx.y.
+struct AdjPass {
+  int64_t lo[EMG_MAX_SPECIES], hi[EMG_MAX_SPECIES];
+};
+
+template <int P>
+__global__ __launch_bounds__(kBlock) void k_adj_count(State64 s, AdjPass ps, AdjTiles at, Grid g,
+                                                      int32_t *count) {
+  extern __shared__ int32_t hist[];
+  const int is = blockIdx.y;
+  const int64_t beg = ps.lo[is] + (int64_t)blockIdx.x * (kBlock * P);
+  if (beg >= ps.hi[is]) return;  // uniform over the block
+  const bool lds = at.n <= kAdjLdsTiles;
+  if (lds) {
+    for (int t = threadIdx.x; t < at.n; t += kBlock) hist[t] = 0;
+    __syncthreads();
   }
-  double nb[3] = {-bf[0] * qmp, -bf[1] * qmp, -bf[2] * qmp};
-  double lx[3] = {lam.x[m], lam.y[m], lam.z[m]};
-  double w3[3] = {lam.vx[m] + gustep * lx[0], lam.vy[m] + gustep * lx[1],
-                  lam.vz[m] + gustep * lx[2]};
-  double mt[3] = {w3[0], w3[1], w3[2]};
-  rotate(mt, nb);
-  double la[3] = {mt[0] + w3[0], mt[1] + w3[1], mt[2] + w3[2]};
-  // lambda_x += qmp * grad (lambda_a . E)(x_k)
-  double sdot[8];
+#pragma unroll 4
+  for (int q = 0; q < P; q++) {
+    const int64_t m = beg + q * kBlock + threadIdx.x;
+    if (m < ps.hi[is]) {
+      const Tri t = tri(s.x[m], s.y[m], s.z[m], g);
+      const int tl = adj_tile(at, t.i, t.j, t.k);
+      if (lds) atomicAdd(&hist[tl], 1);
+      else atomicAdd(&count[tl], 1);
+    }
+  }
+  if (lds) {
+    __syncthreads();
+    for (int t = threadIdx.x; t < at.n; t += kBlock)
+      if (hist[t]) atomicAdd(&count[t], hist[t]);
+  }
+}
+
+template <int P>
+__global__ __launch_bounds__(kBlock) void k_adj_bin(State64 s, AdjPass ps, AdjTiles at, Grid g,
+                                                    const int64_t *__restrict__ start,
+                                                    int32_t *__restrict__ cursor,
+                                                    AdjRec *__restrict__ rec) {
+  // a tile's count, then its first record of this block; then each particle's
+  // tile and rank
+  extern __shared__ int32_t hist[];
+  static_assert(kAdjLdsTiles <= 1 << 16 && kBlock * P <= 1 << 16, "tile and rank in one word");
+  uint32_t *mine = reinterpret_cast<uint32_t *>(hist + at.n) + threadIdx.x;
+  const int is = blockIdx.y;
+  const int64_t beg = ps.lo[is] + (int64_t)blockIdx.x * (kBlock * P);
+  if (beg >= ps.hi[is]) return;  // uniform over the block
+  const bool lds = at.n <= kAdjLdsTiles;
+  if (lds) {
+    for (int t = threadIdx.x; t < at.n; t += kBlock) hist[t] = 0;
+    __syncthreads();
+#pragma unroll 4
+    for (int q = 0; q < P; q++) {
+      const int64_t m = beg + q * kBlock + threadIdx.x;
+      if (m < ps.hi[is]) {
+        const Tri t = tri(s.x[m], s.y[m], s.z[m], g);
+        const int tl = adj_tile(at, t.i, t.j, t.k);
+        mine[q * kBlock] = ((uint32_t)tl << 16) | (uint32_t)atomicAdd(&hist[tl], 1);
+      }
+    }
+    __syncthreads();
+    for (int t = threadIdx.x; t < at.n; t += kBlock)
+      if (hist[t]) hist[t] = (int32_t)start[t] + atomicAdd(&cursor[t], hist[t]);
+    __syncthreads();
+  }
+#pragma unroll 4
+  for (int q = 0; q < P; q++) {
+    const int64_t m = beg + q * kBlock + threadIdx.x;
+    if (m < ps.hi[is]) {
+      const double x = s.x[m], y = s.y[m], z = s.z[m];
+      int64_t d;
+      if (lds) {
+        const uint32_t tr = mine[q * kBlock];
+        d = hist[tr >> 16] + (int)(tr & 0xffffu);
+      } else {
+        const Tri t = tri(x, y, z, g);
+        const int tl = adj_tile(at, t.i, t.j, t.k);
+        d = start[tl] + atomicAdd(&cursor[tl], 1);
+      }
+      double2 *r = reinterpret_cast<double2 *>(rec + d);
+      r[0] = make_double2(x, y);
+      r[1] = make_double2(z, __longlong_as_double(m | ((int64_t)is << 56)));
+    }
+  }
+}
+
+// The reverse step of tile blockIdx.x's records (slice blockIdx.y of
+// gridDim.y).  A node strictly inside the tile belongs to this tile alone:
+// with one workgroup per tile it is added to adj_e without an atomic.
+__global__ __launch_bounds__(kAdjBlock) void k_adj_step64(double *__restrict__ lam, SpeciesTab sp,
+                                                         const double *__restrict__ node, Grid g,
+                                                         int ustep,
+                                                         const AdjRec *__restrict__ rec,
+                                                         const int64_t *__restrict__ start,
+                                                         AdjTiles at,
+                                                         double *__restrict__ adj_e) {
+  constexpr int N = kAdjNode, NN = N * N * N;
+  __shared__ double2 fs[3 * NN];  // E and B of the tile's nodes
+  __shared__ double acc[3 * NN];
+  const int tl = blockIdx.x;
+  const int64_t beg = start[tl], end = start[tl + 1];
+  const int64_t step = (int64_t)gridDim.y * kAdjBlock;
+  if (beg + (int64_t)blockIdx.y * kAdjBlock >= end) return;  // uniform over the block
+  const int ox = (tl % at.ntx) * kAdjTile, oy = (tl / at.ntx) % at.nty * kAdjTile,
+            oz = tl / (at.ntx * at.nty) * kAdjTile;
+  const int tx = min(kAdjTile, g.nx - ox), ty = min(kAdjTile, g.ny - oy),
+            tz = min(kAdjTile, g.nz - oz);
+  for (int q = threadIdx.x; q < 3 * NN; q += kAdjBlock) {
+    acc[q] = 0.0;
+    const int nq = q / 3, c = q - 3 * nq;
+    const int i = nq % N, j = (nq / N) % N, k = nq / (N * N);
+    if (i <= tx && j <= ty && k <= tz)
+      fs[q] = reinterpret_cast<const double2 *>(node + 8 * nodal(g, ox + i, oy + j, oz + k))[c];
+  }
+  __syncthreads();
+  const double gustep = (double)ustep;
+  int64_t m = beg + (int64_t)blockIdx.y * kAdjBlock + threadIdx.x;
+  double2 r0{}, r1{};
+  if (m < end) {
+    r0 = reinterpret_cast<const double2 *>(rec + m)[0];
+    r1 = reinterpret_cast<const double2 *>(rec + m)[1];
+  }
+  for (; m < end; m += step) {
+    const Tri t = tri(r0.x, r0.y, r1.x, g);
+    const int64_t ms = __double_as_longlong(r1.y);
+    double2 *lp = reinterpret_cast<double2 *>(lam + 8 * (ms & 0x00ffffffffffffffll));
+    const double2 l0 = lp[0], l1 = lp[1], l2 = lp[2];
+    if (m + step < end) {  // the next record, while this one's adjoints arrive
+      r0 = reinterpret_cast<const double2 *>(rec + m + step)[0];
+      r1 = reinterpret_cast<const double2 *>(rec + m + step)[1];
+    }
+    const double qmp = sp.qm[ms >> 56] * gustep * 0.5;
+    const int nc = ((t.k - oz) * N + (t.j - oy)) * N + (t.i - ox);
+    double bf[3] = {0.0, 0.0, 0.0};
 #pragma unroll
-  for (int q = 0; q < 8; q++) sdot[q] = la[0] * e[q][0] + la[1] * e[q][1] + la[2] * e[q][2];
-  double gr[3];
-  tri_grad(t, sdot, gr);
-  lam.x[m] = lx[0] + qmp * gr[0];
-  lam.y[m] = lx[1] + qmp * gr[1];
-  lam.z[m] = lx[2] + qmp * gr[2];
-  lam.vx[m] = mt[0];
-  lam.vy[m] = mt[1];
-  lam.vz[m] = mt[2];
-  // transpose of the gather: qmp * lambda_a onto the periodic nodes
+    for (int q = 0; q < 8; q++) {
+      const int a = q & 1, b = (q >> 1) & 1, c = q >> 2;
+      const double2 *f = fs + 3 * (nc + (c * N + b) * N + a);
+      const double w = t.wx[a] * t.wy[b] * t.wz[c];
+      bf[0] += w * f[1].y;
+      bf[1] += w * f[2].x;
+      bf[2] += w * f[2].y;
+    }
+    double nb[3] = {-bf[0] * qmp, -bf[1] * qmp, -bf[2] * qmp};
+    const double w3[3] = {l1.y + gustep * l0.x, l2.x + gustep * l0.y, l2.y + gustep * l1.x};
+    double mt[3] = {w3[0], w3[1], w3[2]};
+    rotate(mt, nb);
+    const double la[3] = {mt[0] + w3[0], mt[1] + w3[1], mt[2] + w3[2]};
+    // lambda_x += qmp * grad (lambda_a . E)(x_k), and qmp * lambda_a onto the nodes
+    double sdot[8];
 #pragma unroll
-  for (int q = 0; q < 8; q++) {
-    int a = q & 1, b = (q >> 1) & 1, c = q >> 2;
-    double w = qmp * t.wx[a] * t.wy[b] * t.wz[c];
-    double *d = adj_e + 3 * periodic(g, t.i + a, t.j + b, t.k + c);
-    atomicAdd(d + 0, w * la[0]);
-    atomicAdd(d + 1, w * la[1]);
-    atomicAdd(d + 2, w * la[2]);
+    for (int q = 0; q < 8; q++) {
+      const int a = q & 1, b = (q >> 1) & 1, c = q >> 2;
+      const int nq = nc + (c * N + b) * N + a;
+      const double2 *f = fs + 3 * nq;
+      sdot[q] = la[0] * f[0].x + la[1] * f[0].y + la[2] * f[1].x;
+      const double w = qmp * t.wx[a] * t.wy[b] * t.wz[c];
+      atomicAdd(&acc[nq], w * la[0]);
+      atomicAdd(&acc[nq + NN], w * la[1]);
+      atomicAdd(&acc[nq + 2 * NN], w * la[2]);
+    }
+    double gr[3];
+    tri_grad(t, sdot, gr);
+    lp[0] = make_double2(l0.x + qmp * gr[0], l0.y + qmp * gr[1]);
+    lp[1] = make_double2(l1.x + qmp * gr[2], mt[0]);
+    lp[2] = make_double2(mt[1], mt[2]);
+  }
+  __syncthreads();
+  for (int q = threadIdx.x; q < NN; q += kAdjBlock) {
+    const int i = q % N, j = (q / N) % N, k = q / (N * N);
+    if (i > tx || j > ty || k > tz) continue;
+    double *d = adj_e + 3 * periodic(g, ox + i, oy + j, oz + k);
+    const bool own = gridDim.y == 1 && i > 0 && i < tx && j > 0 && j < ty && k > 0 && k < tz;
+#pragma unroll
+    for (int c = 0; c < 3; c++) {
+      const double v = acc[c * NN + q];
+      if (own) d[c] += v;
+      else if (v != 0.0) atomicAdd(d + c, v);
+    }
   }
 }
 
 // lambda_x += qfac[is] * grad g(x) for the trilinear interpolant of the
 // periodic nodal scalar g (the adjoint of the particle's CIC charge)
-__global__ __launch_bounds__(kBlock) void k_adj_density64(State64 s, State64 lam, SpeciesTab sp,
+__global__ __launch_bounds__(kBlock) void k_adj_density64(State64 s, double *__restrict__ lam, SpeciesTab sp,
                                                          Grid g, const double *__restrict__ gn,
                                                          const double *__restrict__ qfac) {
   int is = blockIdx.y;
@@ -143,32 +315,38 @@ __global__ __launch_bounds__(kBlock) void k_adj_density64(State64 s, State64 lam
   int64_t m = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (m >= sp.cnt[is]) return;
   m += sp.off[is];
+  double *l = lam + 8 * m;
+  const double2 l0 = *reinterpret_cast<const double2 *>(l);
+  const double lz = l[2];
   Tri t = tri(s.x[m], s.y[m], s.z[m], g);
+  // the two nodes of each x edge in one 16-byte load (8-byte aligned); in the
+  // last cell the second one is node 0 of the row
   double v[8];
+  const int i0 = min(t.i, g.nx - 2);
+  const bool last = t.i != i0;
+  const int j1 = t.j + 1 == g.ny ? 0 : t.j + 1, k1 = t.k + 1 == g.nz ? 0 : t.k + 1;
 #pragma unroll
-  for (int q = 0; q < 8; q++) {
-    int a = q & 1, b = (q >> 1) & 1, c = q >> 2;
-    v[q] = gn[periodic(g, t.i + a, t.j + b, t.k + c)];
+  for (int q = 0; q < 4; q++) {
+    const double *row = gn + ((int64_t)(q >> 1 ? k1 : t.k) * g.ny + (q & 1 ? j1 : t.j)) * g.nx;
+    __builtin_memcpy(&v[2 * q], row + i0, 2 * sizeof(double));
+    if (last) {
+      v[2 * q] = v[2 * q + 1];
+      v[2 * q + 1] = row[0];
+    }
   }
   double gr[3];
   tri_grad(t, v, gr);
-  lam.x[m] += f * gr[0];
-  lam.y[m] += f * gr[1];
-  lam.z[m] += f * gr[2];
+  *reinterpret_cast<double2 *>(l) = make_double2(l0.x + f * gr[0], l0.y + f * gr[1]);
+  l[2] = lz + f * gr[2];
 }
 
-// per-species sums of lambda_v (block partials added atomically)
-__global__ __launch_bounds__(kBlock) void k_adj_vsum(State64 lam, SpeciesTab sp, double *out) {
+// per-species sums of lambda_v: kVsumBlocks block partials per species, then
+// one block adds them in block order: 0.11 ms at 8.8M particles.  (Three atomics
+// per block of 256 particles, on six addresses, took 0.79.)
+constexpr int kVsumBlocks = 512;
+
+__device__ __forceinline__ void vsum_block(double v[3], double *out) {
   __shared__ double red[3][kBlock];
-  int is = blockIdx.y;
-  int64_t m = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  double v[3] = {0.0, 0.0, 0.0};
-  if (m < sp.cnt[is]) {
-    m += sp.off[is];
-    v[0] = lam.vx[m];
-    v[1] = lam.vy[m];
-    v[2] = lam.vz[m];
-  }
   for (int d = 0; d < 3; d++) red[d][threadIdx.x] = v[d];
   __syncthreads();
   for (int o = kBlock / 2; o > 0; o >>= 1) {
@@ -176,7 +354,29 @@ __global__ __launch_bounds__(kBlock) void k_adj_vsum(State64 lam, SpeciesTab sp,
       for (int d = 0; d < 3; d++) red[d][threadIdx.x] += red[d][threadIdx.x + o];
     __syncthreads();
   }
-  if (threadIdx.x < 3) atomicAdd(&out[3 * is + threadIdx.x], red[threadIdx.x][0]);
+  if (threadIdx.x < 3) out[threadIdx.x] = red[threadIdx.x][0];
+}
+
+__global__ __launch_bounds__(kBlock) void k_adj_vsum(const double *__restrict__ lam, SpeciesTab sp,
+                                                    double *part) {
+  const int is = blockIdx.y;
+  double v[3] = {0.0, 0.0, 0.0};
+  for (int64_t m = (int64_t)blockIdx.x * kBlock + threadIdx.x; m < sp.cnt[is];
+       m += (int64_t)kVsumBlocks * kBlock) {
+    const double *l = lam + 8 * (sp.off[is] + m);
+    v[0] += l[3];
+    v[1] += l[4];
+    v[2] += l[5];
+  }
+  vsum_block(v, part + 3 * ((int64_t)is * kVsumBlocks + blockIdx.x));
+}
+
+__global__ __launch_bounds__(kBlock) void k_adj_vsum_final(const double *part, double *out) {
+  const int is = blockIdx.x;
+  double v[3] = {0.0, 0.0, 0.0};
+  for (int k = threadIdx.x; k < kVsumBlocks; k += kBlock)
+    for (int d = 0; d < 3; d++) v[d] += part[3 * ((int64_t)is * kVsumBlocks + k) + d];
+  vsum_block(v, out + 3 * is);
 }
 
 dim3 species_blocks(const SpeciesTab &sp) {
@@ -185,12 +385,98 @@ dim3 species_blocks(const SpeciesTab &sp) {
   return dim3((unsigned)((mx + kBlock - 1) / kBlock), sp.nspec);
 }
 
+AdjTiles adj_tiles(const Grid &g) {
+  AdjTiles a;
+  a.ntx = (g.nx + kAdjTile - 1) / kAdjTile;
+  a.nty = (g.ny + kAdjTile - 1) / kAdjTile;
+  a.ntz = (g.nz + kAdjTile - 1) / kAdjTile;
+  a.n = a.ntx * a.nty * a.ntz;
+  return a;
+}
+
 }  // namespace
+
+// the workspace of the binned transposed gather, kept with the context: the
+// tile counters and starts, and the records of one pass (halved until they
+// can be allocated: a step then takes more passes)
+int adj_bins_alloc(emg_ctx *c) {
+  AdjBins &B = c->adj_bins;
+  if (B.rec) return EMG_OK;
+  const int64_t n = adj_tiles(c->g).n;
+  if (!B.count && hipMalloc(&B.count, sizeof(int32_t) * 2 * n) != hipSuccess) {
+    B.count = nullptr;
+    return set_error(EMG_ERR_NOMEM, "adjoint tile counters");
+  }
+  if (!B.start && hipMalloc(&B.start, sizeof(int64_t) * (n + 1)) != hipSuccess) {
+    B.start = nullptr;
+    return set_error(EMG_ERR_NOMEM, "adjoint tile starts");
+  }
+  const int64_t need = scan_tmp_need(n);
+  if (need > c->scan_tmp_len) {
+    if (c->scan_tmp) (void)hipFree(c->scan_tmp);
+    c->scan_tmp_len = 0;
+    if (hipMalloc(&c->scan_tmp, sizeof(int64_t) * need) != hipSuccess) {
+      c->scan_tmp = nullptr;
+      return set_error(EMG_ERR_NOMEM, "scan scratch");
+    }
+    c->scan_tmp_len = need;
+  }
+  int64_t len = c->cap_total < 1 ? 1 : (c->cap_total < kAdjRecMax ? c->cap_total : kAdjRecMax);
+  while (hipMalloc(&B.rec, sizeof(AdjRec) * len) != hipSuccess) {
+    (void)hipGetLastError();
+    B.rec = nullptr;
+    if (len <= 65536) return set_error(EMG_ERR_NOMEM, "adjoint records");
+    len /= 2;
+  }
+  B.len = len;
+  return EMG_OK;
+}
+
+template <int P>
+static void adj_pass(emg_ctx *c, int ustep, const AdjPass &ps, int64_t most, int64_t total) {
+  const AdjBins &B = c->adj_bins;
+  const AdjTiles at = adj_tiles(c->g);
+  const dim3 grid((unsigned)((most + kBlock * P - 1) / (kBlock * P)), c->sp.nspec);
+  const bool counted = at.n <= kAdjLdsTiles;
+  const size_t lds = counted ? sizeof(int32_t) * at.n : 0;
+  launch_zero(B.count, sizeof(int32_t) * 2 * at.n, c->stream);
+  hipLaunchKernelGGL(k_adj_count<P>, grid, dim3(kBlock), lds, c->stream, c->s64, ps, at, c->g,
+                     B.count);
+  exclusive_scan_i32(B.count, B.start, at.n, c->scan_tmp, c->stream);
+  hipLaunchKernelGGL(k_adj_bin<P>, grid, dim3(kBlock),
+                     counted ? lds + sizeof(int32_t) * kBlock * P : 0, c->stream, c->s64, ps, at,
+                     c->g, B.start, B.count + at.n, static_cast<AdjRec *>(B.rec));
+  // about 512 workgroups or more (two per CU), of 16 rounds of records at least
+  int64_t split = (512 + at.n - 1) / at.n;
+  split = std::min<int64_t>(split, total / ((int64_t)at.n * kAdjBlock * 16) + 1);
+  hipLaunchKernelGGL(k_adj_step64, dim3(at.n, (unsigned)split), dim3(kAdjBlock), 0, c->stream,
+                     c->lam, c->sp, c->node64, c->g, ustep, static_cast<const AdjRec *>(B.rec),
+                     B.start, at, c->adj_e);
+}
 
 void launch_adj_step64(emg_ctx *c, int ustep) {
   launch_zero(c->adj_e, sizeof(double) * 3 * c->ncell, c->stream);
-  hipLaunchKernelGGL(k_adj_step64, species_blocks(c->sp), dim3(kBlock), 0, c->stream, c->s64,
-                     c->lam, c->sp, c->node64, c->g, ustep, c->adj_e);
+  int64_t done[EMG_MAX_SPECIES] = {};
+  for (;;) {  // passes of at most adj_bins.len particles
+    AdjPass ps{};
+    int64_t room = c->adj_bins.len, most = 0;
+    for (int s = 0; s < c->sp.nspec; s++) {
+      const int64_t k = std::min(room, c->sp.cnt[s] - done[s]);
+      ps.lo[s] = c->sp.off[s] + done[s];
+      ps.hi[s] = ps.lo[s] + k;
+      done[s] += k;
+      room -= k;
+      most = std::max(most, k);
+    }
+    if (most == 0) break;
+    const int64_t total = c->adj_bins.len - room;
+    // 16 particles per thread make a block's records of a tile a run of
+    // several; small populations need the blocks more
+    if (total >= (int64_t)kBlock * 16 * 512)
+      adj_pass<16>(c, ustep, ps, most, total);
+    else
+      adj_pass<4>(c, ustep, ps, most, total);
+  }
 }
 
 void launch_adj_density64(emg_ctx *c, const double *qfac_dev) {
@@ -199,9 +485,12 @@ void launch_adj_density64(emg_ctx *c, const double *qfac_dev) {
 }
 
 void launch_adj_vsum(emg_ctx *c, double *out_dev) {
-  launch_zero(out_dev, sizeof(double) * 3 * c->sp.nspec, c->stream);
-  hipLaunchKernelGGL(k_adj_vsum, species_blocks(c->sp), dim3(kBlock), 0, c->stream, c->lam, c->sp,
-                     out_dev);
+  hipLaunchKernelGGL(k_adj_vsum, dim3(kVsumBlocks, c->sp.nspec), dim3(kBlock), 0, c->stream, c->lam,
+                     c->sp, out_dev + 3 * EMG_MAX_SPECIES);
+  hipLaunchKernelGGL(k_adj_vsum_final, dim3(c->sp.nspec), dim3(kBlock), 0, c->stream,
+                     out_dev + 3 * EMG_MAX_SPECIES, out_dev);
 }
+
+int64_t adj_vsum_need() { return 3 * EMG_MAX_SPECIES * (1 + kVsumBlocks); }
 
 }  // namespace emg
