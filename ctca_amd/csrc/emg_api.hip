@@ -383,7 +383,10 @@ int emg_destroy(emg_ctx *c) {
   dfree(B.extra);
   dfree(B.hist);
   dfree(B.cursor);
-  dfree(B.shist);
+  dfree(B.shist[0]);
+  dfree(B.shist[1]);
+  dfree(B.plan_word);
+  dfree(B.plan_ticket);
   dfree(B.scur);
   dfree(B.spre);
   dfree(B.spl);

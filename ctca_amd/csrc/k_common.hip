@@ -41,46 +41,32 @@ __device__ int64_t block_excl_scan(int64_t v, int64_t *total) {
   return incl - v;
 }
 
-// With a second input in2, each term is in + 2^32 in2: one pass scans both
-// (the first sum must stay below 2^32), and k_scan_final splits the result.
 // A thread's kScanPer terms, all loaded before any is used (a full run as
-// four 16-byte loads per input: base is a multiple of kScanPer and the
-// inputs are allocation bases, so they are aligned), zero past n.
-__device__ __forceinline__ void scan_load(const int32_t *in, const int32_t *in2, int64_t n,
-                                          int64_t base, int64_t t[kScanPer]) {
+// four 16-byte loads: base is a multiple of kScanPer and the input is an
+// allocation's base, so they are aligned), zero past n.
+__device__ __forceinline__ void scan_load(const int32_t *in, int64_t n, int64_t base,
+                                          int32_t t[kScanPer]) {
   static_assert(kScanPer % 4 == 0, "whole 16-byte loads");
-  int32_t a[kScanPer], b[kScanPer];
   if (base + kScanPer <= n) {
 #pragma unroll
     for (int q = 0; q < kScanPer / 4; q++) {
       const int4 u = reinterpret_cast<const int4 *>(in + base)[q];
-      a[4 * q] = u.x;
-      a[4 * q + 1] = u.y;
-      a[4 * q + 2] = u.z;
-      a[4 * q + 3] = u.w;
-      int4 w = make_int4(0, 0, 0, 0);
-      if (in2) w = reinterpret_cast<const int4 *>(in2 + base)[q];
-      b[4 * q] = w.x;
-      b[4 * q + 1] = w.y;
-      b[4 * q + 2] = w.z;
-      b[4 * q + 3] = w.w;
+      t[4 * q] = u.x;
+      t[4 * q + 1] = u.y;
+      t[4 * q + 2] = u.z;
+      t[4 * q + 3] = u.w;
     }
   } else {
 #pragma unroll
-    for (int k = 0; k < kScanPer; k++) {
-      a[k] = base + k < n ? in[base + k] : 0;
-      b[k] = in2 && base + k < n ? in2[base + k] : 0;
-    }
+    for (int k = 0; k < kScanPer; k++) t[k] = base + k < n ? in[base + k] : 0;
   }
-#pragma unroll
-  for (int k = 0; k < kScanPer; k++) t[k] = (int64_t)a[k] + (int64_t)b[k] * 4294967296ll;
 }
 
-__global__ __launch_bounds__(kBlock) void k_scan_sums(const int32_t *in, const int32_t *in2,
-                                                      int64_t n, int64_t *bsum) {
+__global__ __launch_bounds__(kBlock) void k_scan_sums(const int32_t *in, int64_t n,
+                                                      int64_t *bsum) {
   int64_t base = (int64_t)blockIdx.x * kScanChunk + (int64_t)threadIdx.x * kScanPer;
-  int64_t t[kScanPer];
-  scan_load(in, in2, n, base, t);
+  int32_t t[kScanPer];
+  scan_load(in, n, base, t);
   int64_t s = 0;
 #pragma unroll
   for (int k = 0; k < kScanPer; k++) s += t[k];
@@ -103,32 +89,24 @@ __global__ __launch_bounds__(kBlock) void k_scan_top(int64_t *bsum, int64_t nblk
   if (threadIdx.x == 0) bsum[nblk] = carry;
 }
 
-__global__ __launch_bounds__(kBlock) void k_scan_final(const int32_t *in, const int32_t *in2,
-                                                       int64_t n, const int64_t *bsum,
-                                                       int64_t nblk, int64_t *out, int64_t *out2) {
+__global__ __launch_bounds__(kBlock) void k_scan_final(const int32_t *in, int64_t n,
+                                                       const int64_t *bsum, int64_t nblk,
+                                                       int64_t *out) {
   int64_t base = (int64_t)blockIdx.x * kScanChunk + (int64_t)threadIdx.x * kScanPer;
-  int64_t t[kScanPer];
-  scan_load(in, in2, n, base, t);
+  int32_t t[kScanPer];
+  scan_load(in, n, base, t);
   int64_t s = 0;
 #pragma unroll
   for (int k = 0; k < kScanPer; k++) s += t[k];
   int64_t tot;
   int64_t run = block_excl_scan(s, &tot) + bsum[blockIdx.x];
-  auto put = [&](int64_t i, int64_t v) {
-    if (in2) {
-      out[i] = v & 0xffffffffll;
-      out2[i] = v >> 32;
-    } else {
-      out[i] = v;
-    }
-  };
 #pragma unroll
   for (int k = 0; k < kScanPer; k++)
     if (base + k < n) {
-      put(base + k, run);
+      out[base + k] = run;
       run += t[k];
     }
-  if (blockIdx.x == 0 && threadIdx.x == 0) put(n, bsum[nblk]);
+  if (blockIdx.x == 0 && threadIdx.x == 0) out[n] = bsum[nblk];
 }
 
 // ---------------------------------------------------------------- energy
@@ -577,27 +555,15 @@ void launch_zero(void *p, size_t bytes, hipStream_t s) {
 
 int64_t scan_tmp_need(int64_t n) { return (n + kScanChunk - 1) / kScanChunk + 1; }
 
-static void scan_launch(const int32_t *in, const int32_t *in2, int64_t *out, int64_t *out2,
-                        int64_t n, int64_t *tmp, hipStream_t s) {
+void exclusive_scan_i32(const int32_t *in, int64_t *out, int64_t n, int64_t *tmp, hipStream_t s) {
   int64_t nblk = (n + kScanChunk - 1) / kScanChunk;
   if (nblk == 0) {
     launch_zero(out, sizeof(int64_t), s);
-    if (out2) launch_zero(out2, sizeof(int64_t), s);
     return;
   }
-  hipLaunchKernelGGL(k_scan_sums, dim3((unsigned)nblk), dim3(kBlock), 0, s, in, in2, n, tmp);
+  hipLaunchKernelGGL(k_scan_sums, dim3((unsigned)nblk), dim3(kBlock), 0, s, in, n, tmp);
   hipLaunchKernelGGL(k_scan_top, dim3(1), dim3(kBlock), 0, s, tmp, nblk);
-  hipLaunchKernelGGL(k_scan_final, dim3((unsigned)nblk), dim3(kBlock), 0, s, in, in2, n, tmp, nblk,
-                     out, out2);
-}
-
-void exclusive_scan_i32(const int32_t *in, int64_t *out, int64_t n, int64_t *tmp, hipStream_t s) {
-  scan_launch(in, nullptr, out, nullptr, n, tmp, s);
-}
-
-void exclusive_scan2_i32(const int32_t *in, int64_t *out, const int32_t *in2, int64_t *out2,
-                         int64_t n, int64_t *tmp, hipStream_t s) {
-  scan_launch(in, in2, out, out2, n, tmp, s);
+  hipLaunchKernelGGL(k_scan_final, dim3((unsigned)nblk), dim3(kBlock), 0, s, in, n, tmp, nblk, out);
 }
 
 void launch_energy64(emg_ctx *c) {

@@ -67,7 +67,8 @@ typedef struct {
   int32_t tile;        /* FP32_FIXED: tile edge in cells, 4 or 8 (0 = 8 when
                           every axis is a multiple of 8, 4 when a multiple
                           of 4, else 8 if every axis has 8 cells or more,
-                          else 4).  Any grid with at least `tile` cells per
+                          else 4; and 4 where 8 would make fewer than 256
+                          tiles times species).  Any grid with at least `tile` cells per
                           axis and ceil(log2 nx) + ceil(log2 ny) +
                           ceil(log2 nz) <= 32 (the packed cell index) is
                           taken: tiles at the upper faces may be partial.
