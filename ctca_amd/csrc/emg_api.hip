@@ -391,6 +391,7 @@ int emg_destroy(emg_ctx *c) {
   dfree(B.spre);
   dfree(B.spl);
   dfree(c->eb_dev);
+  dfree(c->eb_stage);
   dfree(c->fe_buf);
   dfree(c->sort_rec);
   es_solver_free(c);
@@ -611,25 +612,31 @@ int emg_set_fields(emg_ctx *c, const double *eb, const int32_t lo[3], const int3
     elo[d] = lo[d];
     ext[d] = hi[d] - lo[d] + 1;
   }
-  size_t bytes = sizeof(double) * 6 * (size_t)ext[0] * ext[1] * ext[2];
+  const size_t bytes = sizeof(double) * 6 * (size_t)ext[0] * ext[1] * ext[2];
+  int rc = hip_check(hipStreamSynchronize(c->stream), "stream synchronize");
+  if (rc) return rc;
+  if (bytes > c->eb_stage_bytes) {
+    dfree(c->eb_stage);
+    c->eb_stage = nullptr;
+    c->eb_stage_bytes = 0;
+    if ((rc = dalloc(&c->eb_stage, bytes / sizeof(double), "eb staging"))) return rc;
+    c->eb_stage_bytes = bytes;
+  }
   if (bytes > c->eb_dev_bytes) {
-    int rc = hip_check(hipStreamSynchronize(c->stream), "stream synchronize");
-    if (rc) return rc;
     dfree(c->eb_dev);
     c->eb_dev = nullptr;
     c->eb_dev_bytes = 0;
-    if ((rc = dalloc(&c->eb_dev, bytes / sizeof(double), "eb staging"))) return rc;
+    if ((rc = dalloc(&c->eb_dev, bytes / sizeof(double), "eb"))) return rc;
     c->eb_dev_bytes = bytes;
   }
-  int rc = hip_check(hipStreamSynchronize(c->stream), "stream synchronize");
-  if (rc) return rc;
-  rc = hip_check(hipMemcpy(c->eb_dev, eb, bytes, hipMemcpyHostToDevice), "eb upload");
+  rc = hip_check(hipMemcpy(c->eb_stage, eb, bytes, hipMemcpyHostToDevice), "eb upload");
   if (rc) return rc;
   for (int d = 0; d < 3; d++) {
     c->eb_lo[d] = elo[d];
     c->eb_ext[d] = ext[d];
   }
-  launch_relocate64(c, elo, ext);
+  launch_eb_split(c);
+  launch_relocate64(c);
   c->fields_set = true;
   c->nodes_stale = false;
   return hip_check(hipGetLastError(), "relocate launch");
@@ -646,6 +653,7 @@ int emg_bfield(emg_ctx *c) {
   int rc = need_eb(c);
   if (rc) return rc;
   launch_bfield(c);
+  c->nodes_b_valid = false;
   c->nodes_stale = true;
   return hip_check(hipGetLastError(), "bfield launch");
 }
@@ -664,7 +672,7 @@ int emg_grdcrt(emg_ctx *c) {
   CTX_CHECK(c);
   int rc = need_eb(c);
   if (rc) return rc;
-  launch_relocate64(c, c->eb_lo, c->eb_ext);
+  launch_relocate64(c);
   c->nodes_stale = false;
   return hip_check(hipGetLastError(), "relocate launch");
 }
@@ -704,6 +712,7 @@ int emg_solve_es(emg_ctx *c, double rhobk) {
     if (rc) return rc;
     c->eb_dev_bytes = count * sizeof(double);
     launch_zero(c->eb_dev, c->eb_dev_bytes, c->stream);
+    c->nodes_b_valid = false;
   }
   int rc = solve_es(c, rhobk);
   if (rc) return rc;

@@ -164,6 +164,44 @@ constexpr int kRunSpan = 96;   // cells a block may span and stay whole
 constexpr int kRunCells = 64;  // cells per run of a cut block
 static_assert(kRunSpan >= kRunCells, "a cut block's runs span over kRunCells / 2 cells");
 
+// (i, j, k) of point o of an ex x ey x ... box, x fastest; 32-bit divisions
+// where they do (a 64-bit one takes about four times the instructions)
+__device__ __forceinline__ void point_of(int64_t o, int ex, int ey, int &i, int &j, int &k) {
+  if ((o >> 32) == 0) {
+    const uint32_t u = (uint32_t)o, q = u / (uint32_t)ex, r = q / (uint32_t)ey;
+    i = (int)(u - q * (uint32_t)ex);
+    j = (int)(q - r * (uint32_t)ey);
+    k = (int)r;
+  } else {
+    i = (int)(o % ex);
+    j = (int)((o / ex) % ey);
+    k = (int)(o / ((int64_t)ex * ey));
+  }
+}
+
+// index modulo n for the indices the grid kernels form (a few cells around
+// [0, n)): one compare and add each way, the division only if that misses
+__device__ __forceinline__ int periodic_index(int i, int n) {
+  int r = i < 0 ? i + n : (i >= n ? i - n : i);
+  if ((unsigned)r >= (unsigned)n) r = ((i % n) + n) % n;
+  return r;
+}
+
+// The device copy of eb: component c of point (i, j, k) at c * np + at(i, j, k).
+struct EbView {
+  double *eb;
+  int lo[3], ext[3];
+  int64_t np;
+  Grid g;
+  __device__ __forceinline__ int64_t at(int i, int j, int k) const {
+    return ((int64_t)(k - lo[2]) * ext[1] + (j - lo[1])) * ext[0] + (i - lo[0]);
+  }
+  // periodic image of cell (i, j, k) inside the stored box
+  __device__ __forceinline__ int64_t img(int i, int j, int k) const {
+    return at(periodic_index(i, g.nx), periodic_index(j, g.ny), periodic_index(k, g.nz));
+  }
+};
+
 // Workspace of the adjoint's transposed gather (k_adj.hip): counters and
 // cursors per tile, each tile's first record, the records of one pass.
 struct AdjBins {
@@ -219,15 +257,21 @@ struct emg_ctx {
   emg::FxBuckets fx;
 
   // fields
-  double *eb_dev;   // eb(6, eb_lo : eb_lo + eb_ext - 1), Fortran layout
+  // eb(6, eb_lo : eb_lo + eb_ext - 1) as six component arrays of eb_points
+  // values: an E or a B update writes whole lines, which the six-component
+  // records of the boundary's layout would half fill (EbView)
+  double *eb_dev;
   size_t eb_dev_bytes;
+  double *eb_stage;  // an uploaded eb in the boundary's layout (lazy)
+  size_t eb_stage_bytes;
+  bool nodes_b_valid;  // the nodes' B is the relocation of eb_dev's B
   int eb_lo[3], eb_ext[3];
   bool nodes_stale;  // eb changed on the device since the last relocation
   double *fe_buf;    // field-energy partials and result (lazy)
   emg::EsSolver *es; // FFT plans and arrays of the device Poisson solve (lazy)
   double *bk_dev;    // background charge per periodic node (emg_set_background), or null
   double *node64;  // (nx+1)(ny+1)(nz+1) x 8 doubles, nodes 0..n
-  float *node32;   // nx ny nz x 8 floats, periodic nodes
+  float *node32;   // periodic nodes: nx ny nz x (Ex, Ey, Ez, 0), then as many (Bx, By, Bz, 0)
   bool fields_set;
 
   // deposits
@@ -293,7 +337,7 @@ int64_t scan_tmp_need(int64_t n);
 void exclusive_scan_i32(const int32_t *in, int64_t *out, int64_t n, int64_t *tmp, hipStream_t s);
 
 // kernels: FP64 mirror (k_fp64.hip)
-void launch_relocate64(emg_ctx *c, int elo[3], int eext[3]);
+void launch_relocate64(emg_ctx *c);  // eb_dev -> the form's nodes
 void launch_positn64(emg_ctx *c, int ustep);
 // with resort, the push also moves the particles into the order sort64_rank
 // has counted (into t64; sort64_commit then makes it the live state)
@@ -301,7 +345,9 @@ void launch_push_es64(emg_ctx *c, int ustep, bool resort);
 void launch_deposit64(emg_ctx *c);
 void launch_push_em64(emg_ctx *c, int ustep, bool resort);
 void launch_faces64(emg_ctx *c);  // c->face (zeroed) += upper-face charge
+EbView eb_view(const emg_ctx *c);
 // device Yee update and field energy on eb_dev (k_yee.hip)
+void launch_eb_split(emg_ctx *c);  // eb_stage -> eb_dev
 void launch_bfield(emg_ctx *c);
 void launch_efield(emg_ctx *c, double tcs, double dlt);
 void launch_eb_box(emg_ctx *c, const int lo[3], const int ext[3], double *out_dev);
@@ -314,7 +360,6 @@ int read_potential(emg_ctx *c, double *phi);
 void es_solver_free(emg_ctx *c);
 
 // common kernels (k_common.hip)
-void launch_relocate32(emg_ctx *c);  // node64-independent: from eb_dev
 void launch_energy64(emg_ctx *c);
 void launch_read_rho(emg_ctx *c, int species, double *dst_dev, const int lo[3], const int hi[3]);
 void launch_read_current(emg_ctx *c, int species, double *dst_dev, const int lo[3], const int hi[3]);

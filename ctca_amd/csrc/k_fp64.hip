@@ -120,41 +120,42 @@ __device__ __forceinline__ void wrap_periodic(double &x, double &y, double &z, c
 }
 
 // ---------------------------------------------------------------- grdcrt
-// grdcrt.F90:158-169 (E) and 216-230 (B); writes nodes 0..n (FP64) and, when
-// node32 != nullptr, the periodic FP32 copy (nodes 0..n-1) of the same values.
-__global__ __launch_bounds__(kBlock) void k_relocate(const double *__restrict__ eb, int elx,
-                                                     int ely, int elz, int exx, int exy,
-                                                     double *__restrict__ node64,
-                                                     float *__restrict__ node32, Grid g,
+// grdcrt.F90:158-169 (E) and 216-230 (B); writes nodes 0..n in FP64 (node64) or
+// the periodic nodes 0..n-1 in FP32 (node32) of the same values.
+__global__ __launch_bounds__(kBlock) void k_relocate(EbView v, double *__restrict__ node64,
+                                                     float *__restrict__ node32, int64_t ncell,
                                                      double e0x, double e0y, double e0z,
                                                      double b0x, double b0y, double b0z) {
+  const Grid &g = v.g;
   int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   int64_t nn = (int64_t)(g.nx + 1) * (g.ny + 1) * (g.nz + 1);
   if (idx >= nn) return;
-  int i = (int)(idx % (g.nx + 1));
-  int j = (int)((idx / (g.nx + 1)) % (g.ny + 1));
-  int k = (int)(idx / ((int64_t)(g.nx + 1) * (g.ny + 1)));
-  auto E = [&](int c, int ii, int jj, int kk) -> double {
-    return eb[(((int64_t)(kk - elz) * exy + (jj - ely)) * exx + (ii - elx)) * 6 + c];
-  };
+  int i, j, k;
+  point_of(idx, g.nx + 1, g.ny + 1, i, j, k);
+  if (node32 && (i == g.nx || j == g.ny || k == g.nz)) return;
+  const double *p = v.eb + v.at(i, j, k);
+  const int64_t np = v.np, sy = v.ext[0], sz = (int64_t)v.ext[0] * v.ext[1];
+  const double *ex = p, *ey = p + np, *ez = p + 2 * np, *bx = p + 3 * np, *by = p + 4 * np,
+               *bz = p + 5 * np;
   double o[6];
-  o[0] = 0.5 * (E(0, i, j, k) + E(0, i - 1, j, k)) + e0x;
-  o[1] = 0.5 * (E(1, i, j, k) + E(1, i, j - 1, k)) + e0y;
-  o[2] = 0.5 * (E(2, i, j, k) + E(2, i, j, k - 1)) + e0z;
-  o[3] = 0.25 * (E(3, i, j, k) + E(3, i, j - 1, k) + E(3, i, j, k - 1) + E(3, i, j - 1, k - 1)) + b0x;
-  o[4] = 0.25 * (E(4, i, j, k) + E(4, i - 1, j, k) + E(4, i, j, k - 1) + E(4, i - 1, j, k - 1)) + b0y;
-  o[5] = 0.25 * (E(5, i, j, k) + E(5, i - 1, j, k) + E(5, i, j - 1, k) + E(5, i - 1, j - 1, k)) + b0z;
+  o[0] = 0.5 * (ex[0] + ex[-1]) + e0x;
+  o[1] = 0.5 * (ey[0] + ey[-sy]) + e0y;
+  o[2] = 0.5 * (ez[0] + ez[-sz]) + e0z;
+  o[3] = 0.25 * (bx[0] + bx[-sy] + bx[-sz] + bx[-sy - sz]) + b0x;
+  o[4] = 0.25 * (by[0] + by[-1] + by[-sz] + by[-1 - sz]) + b0y;
+  o[5] = 0.25 * (bz[0] + bz[-1] + bz[-sy] + bz[-1 - sy]) + b0z;
   if (node64) {
-    double *d = node64 + 8 * idx;
-#pragma unroll
-    for (int c = 0; c < 6; c++) d[c] = o[c];
-    d[6] = 0.0;
-    d[7] = 0.0;
+    double2 *d = reinterpret_cast<double2 *>(node64 + 8 * idx);
+    d[0] = make_double2(o[0], o[1]);
+    d[1] = make_double2(o[2], o[3]);
+    d[2] = make_double2(o[4], o[5]);
+    d[3] = make_double2(0.0, 0.0);
   }
-  if (node32 && i < g.nx && j < g.ny && k < g.nz) {
-    float4 *d = reinterpret_cast<float4 *>(node32 + 8 * (((int64_t)k * g.ny + j) * g.nx + i));
-    d[0] = make_float4((float)o[0], (float)o[1], (float)o[2], (float)o[3]);
-    d[1] = make_float4((float)o[4], (float)o[5], 0.f, 0.f);
+  if (node32) {
+    const int64_t c = ((int64_t)k * g.ny + j) * g.nx + i;
+    float4 *d = reinterpret_cast<float4 *>(node32);
+    d[c] = make_float4((float)o[0], (float)o[1], (float)o[2], 0.f);
+    d[ncell + c] = make_float4((float)o[3], (float)o[4], (float)o[5], 0.f);
   }
 }
 
@@ -695,16 +696,17 @@ __global__ __launch_bounds__(kBlock) void k_faces64(State64 s, SpeciesTab sp, Gr
 
 }  // namespace
 
-void launch_relocate64(emg_ctx *c, int elo[3], int eext[3]) {
+void launch_relocate64(emg_ctx *c) {
   int64_t nn = (int64_t)(c->g.nx + 1) * (c->g.ny + 1) * (c->g.nz + 1);
   const emg_config &f = c->cfg;
   timer_begin(c, kTRelocate);
   hipLaunchKernelGGL(k_relocate, dim3((unsigned)((nn + kBlock - 1) / kBlock)), dim3(kBlock), 0,
-                     c->stream, c->eb_dev, elo[0], elo[1], elo[2], eext[0], eext[1],
+                     c->stream, eb_view(c),
                      c->cfg.precision == EMG_PLAIN_FP64 ? c->node64 : nullptr,
-                     c->cfg.precision == EMG_FP32_FIXED ? c->node32 : nullptr, c->g, f.e0[0],
+                     c->cfg.precision == EMG_FP32_FIXED ? c->node32 : nullptr, c->ncell, f.e0[0],
                      f.e0[1], f.e0[2], f.b0[0], f.b0[1], f.b0[2]);
   timer_end(c, kTRelocate);
+  c->nodes_b_valid = true;
 }
 
 void launch_positn64(emg_ctx *c, int ustep) {

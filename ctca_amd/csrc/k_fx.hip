@@ -212,7 +212,8 @@ __device__ __forceinline__ void store_pcl(const StateFx &out, int64_t dst, int c
 }
 
 // rare path (a particle outside its staged tile): one corner at a time
-__device__ __forceinline__ void gather_global(const float *__restrict__ node32, const Grid &g,
+__device__ __forceinline__ void gather_global(const float *__restrict__ node32, int64_t ncell,
+                                              const Grid &g,
                                               int ix, int iy, int iz, float fx, float fy,
                                               float fz, float f[6]) {
   int ix1 = ix + 1 == g.nx ? 0 : ix + 1;
@@ -223,15 +224,15 @@ __device__ __forceinline__ void gather_global(const float *__restrict__ node32, 
   for (int q = 0; q < 8; q++) {
     int a2 = q & 1, b2 = (q >> 1) & 1, c2 = q >> 2;
     float w = (a2 ? fx : 1.f - fx) * (b2 ? fy : 1.f - fy) * (c2 ? fz : 1.f - fz);
-    const float4 *p = reinterpret_cast<const float4 *>(
-        node32 + 8 * (((int64_t)(c2 ? iz1 : iz) * g.ny + (b2 ? iy1 : iy)) * g.nx + (a2 ? ix1 : ix)));
-    float4 A = p[0], B = p[1];
+    const float4 *p = reinterpret_cast<const float4 *>(node32) +
+                      (((int64_t)(c2 ? iz1 : iz) * g.ny + (b2 ? iy1 : iy)) * g.nx + (a2 ? ix1 : ix));
+    float4 A = p[0], B = p[ncell];
     f[0] += w * A.x;
     f[1] += w * A.y;
     f[2] += w * A.z;
-    f[3] += w * A.w;
-    f[4] += w * B.x;
-    f[5] += w * B.y;
+    f[3] += w * B.x;
+    f[4] += w * B.y;
+    f[5] += w * B.z;
   }
 }
 
@@ -537,7 +538,7 @@ __device__ __forceinline__ void fx_one(const FxArgs &a, int s, bool act, const P
         iy = min(iy, g.ny - 1);
         iz = min(iz, g.nz - 1);
       }
-      if (PUSH) gather_global(a.node32, g, ix, iy, iz, fx, fy, fz, f);
+      if (PUSH) gather_global(a.node32, a.ncell, g, ix, iy, iz, fx, fy, fz, f);
     }
   }
   if (PUSH) {
@@ -872,9 +873,11 @@ __global__ __launch_bounds__(T == 8 ? 512 : 256) void k_fx_step(FxArgs a) {
             const int lx = nq % N1, ly = (nq / N1) % N1, lz = nq / (N1 * N1);
             const int gx = wrapc(ox + lx, a.g.nx), gy = wrapc(oy + ly, a.g.ny),
                       gz = wrapc(oz + lz, a.g.nz);
-            const float *pn = a.node32 + 8 * (((int64_t)gz * a.g.ny + gy) * a.g.nx + gx);
-            va[r] = *reinterpret_cast<const float4 *>(pn);
-            vb[r] = *reinterpret_cast<const float2 *>(pn + 4);
+            const float4 *pn = reinterpret_cast<const float4 *>(a.node32) +
+                               (((int64_t)gz * a.g.ny + gy) * a.g.nx + gx);
+            const float4 e = pn[0], m = pn[a.ncell];
+            va[r] = make_float4(e.x, e.y, e.z, m.x);
+            vb[r] = make_float2(m.y, m.z);
           }
         }
 #pragma unroll
