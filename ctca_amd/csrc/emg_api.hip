@@ -774,8 +774,8 @@ static int need_fields(emg_ctx *c) {
 // With `carry` (a push that can move the particles into the new order
 // itself) a re-sort close to the last sort only counts the cells here and
 // *carry is set: the caller launches its push with the re-sort and then
-// calls sort64_commit.
-static int sort_if_due(emg_ctx *c, bool *carry = nullptr) {
+// calls sort64_commit.  which: the run table of the launch that follows.
+static int sort_if_due(emg_ctx *c, int which, bool *carry = nullptr) {
   if (carry) *carry = false;
   if (c->cfg.precision != EMG_PLAIN_FP64 || c->cfg.sort_every <= 0) return EMG_OK;
   if (c->pushes_since_sort < c->cfg.sort_every) {
@@ -784,7 +784,7 @@ static int sort_if_due(emg_ctx *c, bool *carry = nullptr) {
   }
   int rc;
   if (carry && emg::sort64_fusable(c)) {
-    rc = emg::sort64_rank(c);
+    rc = emg::sort64_rank(c, which);
     if (!rc) *carry = true;
   } else {
     rc = sort64(c);
@@ -798,7 +798,7 @@ int emg_positn(emg_ctx *c, int32_t ustep) {
   int rc = need_particles(c);
   if (rc) return rc;
   if (ustep < 0) return set_error(EMG_ERR_ARG, "ustep must be >= 0");
-  if ((rc = sort_if_due(c))) return rc;
+  if ((rc = sort_if_due(c, 0))) return rc;
   if (c->cfg.precision == EMG_PLAIN_FP64) {
     launch_positn64(c, ustep);
     if (c->moves_after_sort < emg::kUnsorted) c->moves_after_sort++;
@@ -818,10 +818,10 @@ int emg_push_es(emg_ctx *c, int32_t ustep) {
   if (rc) return rc;
   if (ustep < 0) return set_error(EMG_ERR_ARG, "ustep must be >= 0");
   bool carry;
-  if ((rc = sort_if_due(c, &carry))) return rc;
+  if ((rc = sort_if_due(c, 0, &carry))) return rc;
   if (c->cfg.precision == EMG_PLAIN_FP64) {
+    if (!carry && (rc = sort64_runs(c, 0))) return rc;
     launch_push_es64(c, ustep, carry);  // push + charge at the new positions
-    // the carried re-sort's buffers are swapped even if its run tables fail
     if (carry) rc = emg::sort64_commit(c);
     if (c->moves_after_sort < emg::kUnsorted) c->moves_after_sort++;
     c->rho_valid = true;
@@ -844,10 +844,12 @@ int emg_deposit_rho(emg_ctx *c, int32_t func) {
   if (rc) return rc;
   if (func < 0 || func > 2) return set_error(EMG_ERR_ARG, "func must be 0, 1 or 2");
   if (!c->rho_valid) {  // a push deposits at its new positions itself
-    if (c->cfg.precision == EMG_PLAIN_FP64)
+    if (c->cfg.precision == EMG_PLAIN_FP64) {
+      if ((rc = sort64_runs(c, 0))) return rc;
       launch_deposit64(c);
-    else
+    } else {
       launch_fx_deposit(c);
+    }
     c->rho_valid = true;
     c->faces_valid = false;
   }
@@ -940,10 +942,10 @@ int emg_push_em(emg_ctx *c, int32_t ustep) {
   if (rc) return rc;
   if (ustep < 1) return set_error(EMG_ERR_ARG, "ustep must be >= 1");
   bool carry;
-  if ((rc = sort_if_due(c, &carry))) return rc;
+  if ((rc = sort_if_due(c, 1, &carry))) return rc;
   if (c->cfg.precision == EMG_PLAIN_FP64) {
+    if (!carry && (rc = sort64_runs(c, 1))) return rc;
     launch_push_em64(c, ustep, carry);
-    // the carried re-sort's buffers are swapped even if its run tables fail
     if (carry) rc = emg::sort64_commit(c);
     if (c->moves_after_sort < emg::kUnsorted) c->moves_after_sort++;
     c->ke_valid = false;
@@ -1096,6 +1098,7 @@ int emg_sort(emg_ctx *c) {
   if (rc) return rc;
   if (c->cfg.precision == EMG_PLAIN_FP64) {
     rc = sort64(c);
+    for (int k = 0; k < 2 && !rc; k++) rc = sort64_runs(c, k);
     if (!rc) c->pushes_since_sort = 0;
   } else {
     rc = fx_rebucket(c);

@@ -101,16 +101,117 @@ struct Timer {
 
 struct EsSolver;  // device field solve (k_poisson.hip)
 
+// An LDS window of the FP64 deposits: nodes o .. o + w - 1 per axis (periodic),
+// w <= n, so no node appears twice.
+struct Win {
+  int32_t wx, wy, wz, ox, oy, oz;
+};
+
+struct Cell3 {
+  int i, j, k;
+};
+
+// most nodes of a window, and the fixed box of a run that no box fits
+struct WinShape {
+  int cap, fx, fy, fz;
+};
+constexpr WinShape kWinEs{3840, 80, 8, 6};  // the charge: 30 KB of int64
+constexpr WinShape kWinEm{1600, 40, 8, 5};  // per component of the current: 3 x 12.8 KB
+static_assert(kWinEs.cap % 2 == 0 && kWinEm.cap % 2 == 0, "cleared two entries at a time");
+
+// widen one axis of a window by a node on each side (or to the whole axis) if
+// its nodes, times `across` of the other axes, stay within cap
+__host__ __device__ inline bool win_grow(int32_t &o, int32_t &w, int n, int across, int cap) {
+  if (w >= n || (w + 2 < n ? w + 2 : n) * across > cap) return false;
+  if (w + 2 >= n) {
+    o = 0;
+    w = n;
+  } else {
+    o = o == 0 ? n - 1 : o - 1;
+    w += 2;
+  }
+  return true;
+}
+
+// The window of a run from cell a to cell b (in the sort order; mid: its middle
+// particle's cell).  The cells of a sorted run go from a to b in z-major order
+// (rows of the y-z plane one after another), so its nodes fit a box of its rows
+// plus one, its layers plus one, and in x the row segment it covers (or, for a
+// run that passes into the next row, the periodic range from its first cell to
+// its last) or whole rows; the rest of the capacity becomes margins in z, y and
+// x for the particles that drift.  A run of more rows than a layer holds, or a
+// box over the capacity, gets the fixed box around its middle.
+__host__ __device__ inline Win run_window(const Cell3 &a, const Cell3 &b, const Cell3 &mid,
+                                          const Grid &g, const WinShape &ws) {
+  Win w;
+  // the run's rows, as consecutive rows of the periodic y-z plane
+  const int64_t plane = (int64_t)g.ny * g.nz;
+  int64_t nrow = ((int64_t)b.k * g.ny + b.j) - ((int64_t)a.k * g.ny + a.j) + 1;
+  if (nrow <= 0) nrow += plane;
+  bool boxed = nrow <= g.ny;
+  if (boxed) {
+    // x: the row segment a..b, or (a run into the next row) a..nx-1 and 0..b
+    // taken as one periodic range; whole rows for longer runs
+    w.ox = a.i;
+    if (nrow == 1 && b.i >= a.i) w.wx = b.i - a.i + 2;
+    else if (nrow == 2 && b.i < a.i) w.wx = b.i + g.nx - a.i + 2;
+    else w.wx = g.nx;
+    // y: rows a .. b (periodic); z: layers a .. b
+    w.oy = a.j;
+    w.wy = (int32_t)nrow + 1;
+    w.oz = a.k;
+    w.wz = (b.k < a.k ? b.k - a.k + g.nz : b.k - a.k) + 2;
+    if (w.wx >= g.nx) {
+      w.ox = 0;
+      w.wx = g.nx;
+    }
+    if (w.wy >= g.ny) {
+      w.oy = 0;
+      w.wy = g.ny;
+    }
+    if (w.wz >= g.nz) {
+      w.oz = 0;
+      w.wz = g.nz;
+    }
+    boxed = (int64_t)w.wx * w.wy * w.wz <= ws.cap;
+  }
+  if (boxed) {  // margins while they fit: z, y, x in turn
+    bool grown = true;
+    while (grown) {
+      grown = win_grow(w.oz, w.wz, g.nz, w.wx * w.wy, ws.cap);
+      grown = win_grow(w.oy, w.wy, g.ny, w.wx * w.wz, ws.cap) || grown;
+      grown = win_grow(w.ox, w.wx, g.nx, w.wy * w.wz, ws.cap) || grown;
+    }
+  } else {
+    w.wx = ws.fx < g.nx ? ws.fx : g.nx;
+    w.wy = ws.fy < g.ny ? ws.fy : g.ny;
+    w.wz = ws.fz < g.nz ? ws.fz : g.nz;
+    auto around = [](int c, int ext, int n) {
+      const int v = c - ext / 2;
+      return v < 0 ? v + n : v;
+    };
+    w.ox = around(mid.i, w.wx, g.nx);
+    w.oy = around(mid.j, w.wy, g.ny);
+    w.oz = around(mid.k, w.wz, g.nz);
+  }
+  return w;
+}
+
 // A block's run of the FP64 kernels after a sort: len consecutive particles
 // of species s from its segment's index beg.  Each species is cut into
 // blocks of `run` particles in the sort order (cells in z-major order); a
 // block whose particles span fewer than kRunSpan cells is one run, a longer
 // one (a sparse region) is cut into np = ceil(span / kRunCells) runs of
-// equal cell ranges, so that every run's LDS window covers its cells.
+// equal cell ranges, so that every run's LDS window covers its cells.  The
+// window is shaped here, from the run's cells, once per sort (shaped by every
+// block from its particles at every push, its loop was 70% of the scalar
+// instructions of the zigzag push and 2-4 us of each block).
 struct Run {
   int64_t beg;
   int32_t len, s;
+  Win w;
 };
+
 // The FP64 sort key of a position: its cell in z-major order, each index the
 // int() of the coordinate clamped into the grid.
 __host__ __device__ inline int64_t slab_key_xyz(double x, double y, double z, const Grid &g) {
@@ -160,6 +261,7 @@ struct SortDest {
 
 constexpr int kRunEs = 4096;   // particles per block of the charge / ES push kernels
 constexpr int kRunEm = 1024;   // of the zigzag push
+constexpr int64_t kRunsUnbuilt = -1;
 constexpr int kRunSpan = 96;   // cells a block may span and stay whole
 constexpr int kRunCells = 64;  // cells per run of a cut block
 static_assert(kRunSpan >= kRunCells, "a cut block's runs span over kRunCells / 2 cells");
@@ -297,7 +399,7 @@ struct emg_ctx {
   int64_t sort_len;
   void *sort_rec;        // cap_total x 64-byte records + cap_total int32 ranks (FP64 sort, lazy)
   emg::Run *runs[2];     // block runs of the last sort: [0] kRunEs, [1] kRunEm particles
-  int64_t nruns[2], runs_cap[2];
+  int64_t nruns[2], runs_cap[2];  // (kRunsUnbuilt: not asked for since the last sort)
   int64_t *run_base;     // scan scratch of the run counts (nspec x chunks + 1)
   int64_t run_base_len;
   bool runs_valid;       // the particles are in the order of the sort the runs describe
@@ -370,8 +472,9 @@ void launch_zero(void *p, size_t bytes, hipStream_t s);
 // push writes every particle to its sorted slot (SortDest), and sort64_commit
 // makes that the live state and builds the blocks' run tables of it.
 int sort64(emg_ctx *c);
+int sort64_runs(emg_ctx *c, int which);  // the run table of kRunEs (0) or kRunEm (1)
 bool sort64_fusable(const emg_ctx *c);
-int sort64_rank(emg_ctx *c);
+int sort64_rank(emg_ctx *c, int which);  // which: the run table of the push that follows
 SortDest sort64_dest(const emg_ctx *c);
 int sort64_commit(emg_ctx *c);
 int init_device(emg_ctx *c, const emg_device_species *spec, int nspec, uint64_t seed);

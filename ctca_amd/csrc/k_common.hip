@@ -480,24 +480,27 @@ struct RunCut {
 // with cf, cl the cells of its first and last particle, it is one run if
 // cl - cf < kRunSpan, else np = ceil((cl - cf + 1) / kRunCells) pieces of
 // equal cell ranges (the first from a, the last to e; empty ones dropped).
-// visit(beg, end) is called for each run in order; returns the count.
+// visit(beg, end, c0, c1) is called for each run in order, its particles in
+// cells c0..c1; returns the count.
 template <typename F>
 __device__ int64_t block_runs(const RunCut &rc, int64_t a, int64_t e, F visit) {
   const int64_t cf = rc.cell_of(a), cl = rc.cell_of(e - 1);
   const int64_t span = cl - cf + 1;
   if (span <= kRunSpan) {
-    visit(a, e);
+    visit(a, e, cf, cl);
     return 1;
   }
   const int64_t np = (span + kRunCells - 1) / kRunCells;
-  int64_t k = 0, pa = a;
+  int64_t k = 0, pa = a, ca = cf;
   for (int64_t q = 1; q <= np; q++) {
-    const int64_t pe = q == np ? e : rc.at(cf + q * span / np);
+    const int64_t ce = cf + q * span / np;  // past the piece's last cell
+    const int64_t pe = q == np ? e : rc.at(ce);
     if (pe > pa) {
-      visit(pa, pe);
+      visit(pa, pe, ca, ce - 1);
       k++;
       pa = pe;
     }
+    ca = ce;
   }
   return k;
 }
@@ -512,7 +515,7 @@ __global__ void k_run_count(const int64_t *start, int64_t nkey, SpeciesTab sp, i
   int32_t n = 0;
   if (a < cnt) {
     const RunCut rc{start + (int64_t)s * nkey, start[(int64_t)s * nkey], nkey};
-    n = (int32_t)block_runs(rc, a, min(a + run, cnt), [](int64_t, int64_t) {});
+    n = (int32_t)block_runs(rc, a, min(a + run, cnt), [](int64_t, int64_t, int64_t, int64_t) {});
   }
   nrun[(int64_t)s * nbmax + b] = n;
 }
@@ -520,7 +523,8 @@ __global__ void k_run_count(const int64_t *start, int64_t nkey, SpeciesTab sp, i
 // ... then, at each block's exclusive prefix, its runs (none written at or
 // past cap, which the count bounds; the host checks the total against it)
 __global__ void k_run_fill(const int64_t *start, int64_t nkey, SpeciesTab sp, int64_t nbmax,
-                           int run, const int64_t *base, Run *runs, int64_t cap) {
+                           int run, const int64_t *base, Run *runs, int64_t cap, Grid g,
+                           WinShape ws) {
   const int s = blockIdx.y;
   const int64_t b = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (b >= nbmax) return;
@@ -528,11 +532,17 @@ __global__ void k_run_fill(const int64_t *start, int64_t nkey, SpeciesTab sp, in
   if (a >= cnt) return;
   const RunCut rc{start + (int64_t)s * nkey, start[(int64_t)s * nkey], nkey};
   int64_t at = base[(int64_t)s * nbmax + b];
-  block_runs(rc, a, min(a + run, cnt), [&](int64_t p0, int64_t p1) {
+  block_runs(rc, a, min(a + run, cnt), [&](int64_t p0, int64_t p1, int64_t c0, int64_t c1) {
     Run r;
     r.beg = p0;
     r.len = (int32_t)(p1 - p0);
     r.s = s;
+    auto cell = [&](int64_t k) {
+      Cell3 c;
+      point_of(k, g.nx, g.ny, c.i, c.j, c.k);
+      return c;
+    };
+    r.w = run_window(cell(c0), cell(c1), cell((c0 + c1) / 2), g, ws);
     if (at < cap) runs[at] = r;
     at++;
   });
@@ -693,71 +703,70 @@ int sort64_count(emg_ctx *c) {
   return hip_check(hipGetLastError(), "sort");
 }
 
-// the sorted order (in t64) becomes the live state, and the blocks' runs of
-// it are built, for both block lengths, from the key starts.  The tables only
-// speed the kernels up: one that cannot be allocated is left unbuilt (its
-// kernels keep their plain slices) and the sort still succeeds.
-int sort64_swap_runs(emg_ctx *c) {
-  const int64_t nkey = c->ncell;
-  const int64_t len = nkey * c->sp.nspec;
+// the sorted order (in t64) becomes the live state; its run tables are built
+// when a kernel first asks for one (sort64_runs)
+int sort64_swap(emg_ctx *c) {
   c->moves_after_sort = 0;
   State64 tmp = c->s64;
   c->s64 = c->t64;
   c->t64 = tmp;
-  c->runs_valid = false;
-  c->nruns[0] = c->nruns[1] = 0;
-  int rc = EMG_OK;
+  c->runs_valid = true;
+  c->nruns[0] = c->nruns[1] = kRunsUnbuilt;
+  return hip_check(hipGetLastError(), "sort");
+}
+
+// Run table `which` from the key starts of the order the state is in; leaves
+// nruns at 0 where the table cannot be had (the kernels keep plain slices).
+int build_runs(emg_ctx *c, int which) {
+  const int64_t nkey = c->ncell;
+  const int64_t len = nkey * c->sp.nspec;
+  c->nruns[which] = 0;
   int64_t mx = 1;
   for (int q = 0; q < c->sp.nspec; q++) mx = c->sp.cnt[q] > mx ? c->sp.cnt[q] : mx;
-  for (int k = 0; k < 2 && !rc; k++) {
-    const int run = k == 0 ? kRunEs : kRunEm;
-    const int64_t nbmax = (mx + run - 1) / run;
-    const int64_t nb = nbmax * c->sp.nspec;
-    // the counts reuse the sort's histogram (nkey nspec entries), which no
-    // later pass reads; with more blocks than cells (over `run` particles
-    // per cell) the kernels keep their plain slices
-    if (nb > len) break;
-    if (c->run_base_len < nb + 1) {
-      if (c->run_base) (void)hipFree(c->run_base);
-      c->run_base_len = 0;
-      if (hipMalloc(&c->run_base, sizeof(int64_t) * (nb + 1)) != hipSuccess) {
-        (void)hipGetLastError();
-        c->run_base = nullptr;
-        break;
-      }
-      c->run_base_len = nb + 1;
+  const int run = which == 0 ? kRunEs : kRunEm;
+  const int64_t nbmax = (mx + run - 1) / run;
+  const int64_t nb = nbmax * c->sp.nspec;
+  // the counts reuse the sort's histogram (nkey nspec entries), which no
+  // later pass reads; with more blocks than cells (over `run` particles
+  // per cell) the kernels keep their plain slices
+  if (nb > len) return EMG_OK;
+  if (c->run_base_len < nb + 1) {
+    if (c->run_base) (void)hipFree(c->run_base);
+    c->run_base_len = 0;
+    if (hipMalloc(&c->run_base, sizeof(int64_t) * (nb + 1)) != hipSuccess) {
+      (void)hipGetLastError();
+      c->run_base = nullptr;
+      return EMG_OK;
     }
-    // a cut block's pieces other than its last end at cell starts more than
-    // kRunCells / 2 cells apart (equal ranges of span / np cells, and
-    // span / np > span kRunCells / (span + kRunCells) >= kRunCells / 2 for
-    // span > kRunSpan >= kRunCells)
-    const int64_t cap = nb + (int64_t)c->sp.nspec * (nkey / (kRunCells / 2) + 2) + 1;
-    if (c->runs_cap[k] < cap) {
-      if (c->runs[k]) (void)hipFree(c->runs[k]);
-      c->runs_cap[k] = 0;
-      if (hipMalloc(&c->runs[k], sizeof(Run) * cap) != hipSuccess) {
-        (void)hipGetLastError();
-        c->runs[k] = nullptr;
-        break;
-      }
-      c->runs_cap[k] = cap;
-    }
-    const dim3 gr((unsigned)((nbmax + kBlock - 1) / kBlock), (unsigned)c->sp.nspec);
-    hipLaunchKernelGGL(k_run_count, gr, dim3(kBlock), 0, c->stream, c->sort_start, nkey, c->sp,
-                       nbmax, run, c->sort_count);
-    exclusive_scan_i32(c->sort_count, c->run_base, nb, c->scan_tmp, c->stream);
-    hipLaunchKernelGGL(k_run_fill, gr, dim3(kBlock), 0, c->stream, c->sort_start, nkey, c->sp,
-                       nbmax, run, c->run_base, c->runs[k], cap);
-    int64_t total = 0;
-    rc = hip_check(hipMemcpyAsync(&total, c->run_base + nb, sizeof(int64_t),
-                                  hipMemcpyDeviceToHost, c->stream), "sort runs");
-    if (!rc) rc = hip_check(hipStreamSynchronize(c->stream), "sort runs");
-    c->nruns[k] = total <= cap ? total : 0;
+    c->run_base_len = nb + 1;
   }
-  // a table left unbuilt has no runs: its kernels keep their plain slices
-  c->runs_valid = rc == EMG_OK;
-  if (rc) return rc;
-  return hip_check(hipGetLastError(), "sort");
+  // a cut block's pieces other than its last end at cell starts more than
+  // kRunCells / 2 cells apart (equal ranges of span / np cells, and
+  // span / np > span kRunCells / (span + kRunCells) >= kRunCells / 2 for
+  // span > kRunSpan >= kRunCells)
+  const int64_t cap = nb + (int64_t)c->sp.nspec * (nkey / (kRunCells / 2) + 2) + 1;
+  if (c->runs_cap[which] < cap) {
+    if (c->runs[which]) (void)hipFree(c->runs[which]);
+    c->runs_cap[which] = 0;
+    if (hipMalloc(&c->runs[which], sizeof(Run) * cap) != hipSuccess) {
+      (void)hipGetLastError();
+      c->runs[which] = nullptr;
+      return EMG_OK;
+    }
+    c->runs_cap[which] = cap;
+  }
+  const dim3 gr((unsigned)((nbmax + kBlock - 1) / kBlock), (unsigned)c->sp.nspec);
+  hipLaunchKernelGGL(k_run_count, gr, dim3(kBlock), 0, c->stream, c->sort_start, nkey, c->sp,
+                     nbmax, run, c->sort_count);
+  exclusive_scan_i32(c->sort_count, c->run_base, nb, c->scan_tmp, c->stream);
+  hipLaunchKernelGGL(k_run_fill, gr, dim3(kBlock), 0, c->stream, c->sort_start, nkey, c->sp, nbmax,
+                     run, c->run_base, c->runs[which], cap, c->g, which == 0 ? kWinEs : kWinEm);
+  int64_t total = 0;
+  int rc = hip_check(hipMemcpyAsync(&total, c->run_base + nb, sizeof(int64_t),
+                                    hipMemcpyDeviceToHost, c->stream), "sort runs");
+  if (!rc) rc = hip_check(hipStreamSynchronize(c->stream), "sort runs");
+  if (!rc && total <= cap) c->nruns[which] = total;
+  return rc;
 }
 
 }  // namespace
@@ -779,8 +788,23 @@ int sort64(emg_ctx *c) {
       hipLaunchKernelGGL(k_sort_split, grid, dim3(kBlock), 0, c->stream,
                          (const uint4 *)c->sort_rec, c->t64, c->sp);
     }
-    rc = sort64_swap_runs(c);
+    rc = sort64_swap(c);
   }
+  timer_end(c, kTSort);
+  return rc;
+}
+
+int sort64_runs(emg_ctx *c, int which) {
+  if (!c->runs_valid || c->nruns[which] != kRunsUnbuilt) return EMG_OK;
+  // building reads a count back, which a captured stream cannot: the launches
+  // recorded now keep plain slices
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(c->stream, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone) {
+    (void)hipGetLastError();
+    return EMG_OK;
+  }
+  timer_begin(c, kTSort);
+  const int rc = build_runs(c, which);
   timer_end(c, kTSort);
   return rc;
 }
@@ -791,12 +815,15 @@ bool sort64_fusable(const emg_ctx *c) {
   return c->moves_after_sort <= kResortDirect && c->t64.x && c->sort_rec && c->runs_valid;
 }
 
-int sort64_rank(emg_ctx *c) {
-  int rc = sort64_alloc(c);
+int sort64_rank(emg_ctx *c, int which) {
+  int rc = sort64_runs(c, which);  // the push's own blocks, before the starts are recounted
+  if (!rc) rc = sort64_alloc(c);
   if (rc) return rc;
   timer_begin(c, kTSort);
   rc = sort64_count(c);
   timer_end(c, kTSort);
+  for (int k = 0; k < 2; k++)
+    if (c->nruns[k] == kRunsUnbuilt) c->nruns[k] = 0;
   return rc;
 }
 
@@ -804,12 +831,7 @@ SortDest sort64_dest(const emg_ctx *c) {
   return SortDest{c->t64, c->sort_start, rank_buf(c), c->ncell};
 }
 
-int sort64_commit(emg_ctx *c) {
-  timer_begin(c, kTSort);
-  const int rc = sort64_swap_runs(c);
-  timer_end(c, kTSort);
-  return rc;
-}
+int sort64_commit(emg_ctx *c) { return sort64_swap(c); }
 
 int init_device_into(emg_ctx *c, State64 &st, const emg_device_species *spec, int nspec,
                      uint64_t seed) {

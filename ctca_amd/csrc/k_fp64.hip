@@ -65,23 +65,65 @@ __device__ __forceinline__ Cic cic(double xl, double yl, double zl, int i, int j
   return w;
 }
 
+// the two nodes of a row (x edge), six components each
+struct Row {
+  double a[6], b[6];
+};
+__device__ __forceinline__ Row load_row(const double *p, int dx) {
+  const double2 *q = reinterpret_cast<const double2 *>(p);
+  const double2 *r = reinterpret_cast<const double2 *>(p + dx);
+  const double2 a = q[0], b = q[1], c = q[2], d = r[0], e = r[1], f = r[2];
+  return {{a.x, a.y, b.x, b.y, c.x, c.y}, {d.x, d.y, e.x, e.y, f.x, f.y}};
+}
+
 // psolve2.F90:195-218: eight-node gather of the six nodal components in the
-// reference's node order v1..v8 and summation order.
+// reference's node order v1..v8 and summation order, a row at a time: left to
+// itself the compiler has all eight nodes (96 registers) in flight.  DEEP
+// keeps two rows in flight, the charge push's 124 VGPRs holding four waves per
+// SIMD; else one row, with which the zigzag push fits 128 and holds four waves
+// instead of three (128^3 charge push 8.41 -> 8.33 ms with DEEP; zigzag push
+// of 18.5M particles 1.42 -> 1.33 ms without).
+template <bool DEEP>
 __device__ __forceinline__ void gather6(const double *__restrict__ node, const Grid &g,
                                         const Cic &w, double f[6]) {
-  int i1 = min(w.i + 1, g.nx), j1 = min(w.j + 1, g.ny), k1 = min(w.k + 1, g.nz);
-  const double *p1 = node + 8 * nidx64(g, w.i, w.j, k1);
-  const double *p2 = node + 8 * nidx64(g, i1, w.j, k1);
-  const double *p3 = node + 8 * nidx64(g, i1, j1, k1);
-  const double *p4 = node + 8 * nidx64(g, w.i, j1, k1);
-  const double *p5 = node + 8 * nidx64(g, w.i, w.j, w.k);
-  const double *p6 = node + 8 * nidx64(g, i1, w.j, w.k);
-  const double *p7 = node + 8 * nidx64(g, i1, j1, w.k);
-  const double *p8 = node + 8 * nidx64(g, w.i, j1, w.k);
+  const double *p = node + 8 * nidx64(g, w.i, w.j, w.k);
+  const int dx = w.i < g.nx ? 8 : 0;
+  const int64_t dj = w.j < g.ny ? 8 * (int64_t)(g.nx + 1) : 0;
+  const int64_t dk = w.k < g.nz ? 8 * (int64_t)(g.nx + 1) * (g.ny + 1) : 0;
+if (DEEP) {
+    const Row r1 = load_row(p + dk, dx);
+    const Row r2 = load_row(p + dk + dj, dx);
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-  for (int c = 0; c < 6; c++)
-    f[c] = p1[c] * w.v1 + p2[c] * w.v2 + p3[c] * w.v3 + p4[c] * w.v4 + p5[c] * w.v5 +
-           p6[c] * w.v6 + p7[c] * w.v7 + p8[c] * w.v8;
+    for (int c = 0; c < 6; c++) f[c] = r1.a[c] * w.v1 + r1.b[c] * w.v2;
+    const Row r3 = load_row(p + 0, dx);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int c = 0; c < 6; c++) f[c] = f[c] + r2.b[c] * w.v3 + r2.a[c] * w.v4;
+    const Row r4 = load_row(p + dj, dx);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int c = 0; c < 6; c++) f[c] = f[c] + r3.a[c] * w.v5 + r3.b[c] * w.v6;
+#pragma unroll
+    for (int c = 0; c < 6; c++) f[c] = f[c] + r4.b[c] * w.v7 + r4.a[c] * w.v8;
+  } else {
+    const Row r1 = load_row(p + dk, dx);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int c = 0; c < 6; c++) f[c] = r1.a[c] * w.v1 + r1.b[c] * w.v2;
+    const Row r2 = load_row(p + dk + dj, dx);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int c = 0; c < 6; c++) f[c] = f[c] + r2.b[c] * w.v3 + r2.a[c] * w.v4;
+    const Row r3 = load_row(p + 0, dx);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int c = 0; c < 6; c++) f[c] = f[c] + r3.a[c] * w.v5 + r3.b[c] * w.v6;
+    const Row r4 = load_row(p + dj, dx);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int c = 0; c < 6; c++) f[c] = f[c] + r4.b[c] * w.v7 + r4.a[c] * w.v8;
+  }
 }
 
 // Buneman-Boris, psolve2.F90:233-257 (ewmodel = 0: the wave field is +0.0).
@@ -192,8 +234,6 @@ __global__ __launch_bounds__(kBlock) void k_positn64(State64 s, SpeciesTab sp, G
 // sum, which the reference's order would give.  The window's shape:
 // run_window; the block's particles: block_run.
 constexpr int kDepPer = 16;
-constexpr int kWinCap = 3840;                    // 30 KB of int64
-constexpr int kWinX = 80, kWinY = 8, kWinZ = 6;  // the fixed box
 constexpr double kRhoFix = 281474976710656.0;   // 2^48 per unit weight
 
 // window index of node l + 1 on an axis of window extent w (full axis: w = n,
@@ -205,113 +245,31 @@ __device__ __forceinline__ bool win_next(int l, int w, int n, int &l1) {
   return w == n && l + 1 == n;
 }
 
-// widen one axis of the window by a node on each side (or to the whole axis)
-__device__ __forceinline__ void win_grow(int &o, int &w, int n) {
-  if (w + 2 >= n) {
-    o = 0;
-    w = n;
-  } else {
-    o = o == 0 ? n - 1 : o - 1;
-    w += 2;
-  }
+// The window of particles a .. b of no run table: from the cells of the first,
+// the last and the middle one.
+__device__ __forceinline__ Win slice_window(const State64 &s, int64_t a, int64_t b, const Grid &g,
+                                            const WinShape &ws) {
+  auto cell = [&](int64_t m) {
+    const double x = s.x[m], y = s.y[m], z = s.z[m];
+    return Cell3{min(max((int)x, 0), g.nx - 1), min(max((int)y, 0), g.ny - 1),
+                 min(max((int)z, 0), g.nz - 1)};
+  };
+  return run_window(cell(a), cell(b), cell(a + (b - a) / 2), g, ws);
 }
 
-// The LDS window of a block's run of particles a .. b (sorted by cell): nodes
-// o .. o + w - 1 per axis (periodic), w <= n, at most cap nodes.  The cells of
-// a sorted run go from its first to its last particle's cell in z-major order
-// (rows of the y-z plane one after another), so its nodes fit a box of its
-// rows plus one, its layers plus one, and in x the row segment it covers (or,
-// for a run that passes into the next row, the periodic range from its first
-// cell to its last) or whole rows; the rest of the capacity becomes margins
-// in z, y and x for the particles that have drifted since the sort.  A run of
-// more rows than a layer holds, or a box over the capacity, gets the fixed
-// box fx x fy x fz around its middle particle.
-__device__ __forceinline__ void run_window(const State64 &s, int64_t a, int64_t b, const Grid &g,
-                                           int cap, int fx, int fy, int fz, int &wx, int &wy,
-                                           int &wz, int &ox, int &oy, int &oz) {
-  auto cell = [&](double v, int n) { return min(max((int)v, 0), n - 1); };
-  const int ia = cell(s.x[a], g.nx), ja = cell(s.y[a], g.ny), ka = cell(s.z[a], g.nz);
-  const int ib = cell(s.x[b], g.nx), jb = cell(s.y[b], g.ny), kb = cell(s.z[b], g.nz);
-  // the run's rows, as consecutive rows of the periodic y-z plane
-  const int64_t ra = (int64_t)ka * g.ny + ja, rb = (int64_t)kb * g.ny + jb;
-  const int64_t nrow = (rb - ra + (int64_t)g.ny * g.nz) % ((int64_t)g.ny * g.nz) + 1;
-  bool boxed = nrow <= g.ny;
-  if (boxed) {
-    // x: the row segment ia..ib, or (a run into the next row) ia..nx-1 and
-    // 0..ib taken as one periodic range; whole rows for longer runs
-    if (nrow == 1 && ib >= ia) {
-      ox = ia;
-      wx = ib - ia + 2;
-    } else if (nrow == 2 && ib < ia) {
-      ox = ia;
-      wx = ib + g.nx - ia + 2;
-    } else {
-      ox = 0;
-      wx = g.nx;
-    }
-    // y: rows ja .. jb (periodic); z: layers ka .. kb
-    oy = ja;
-    wy = (int)min<int64_t>(nrow + 1, g.ny);
-    oz = ka;
-    wz = (kb - ka + g.nz) % g.nz + 2;
-    if (wx >= g.nx) {
-      ox = 0;
-      wx = g.nx;
-    }
-    if (wy >= g.ny) {
-      oy = 0;
-      wy = g.ny;
-    }
-    if (wz >= g.nz) {
-      oz = 0;
-      wz = g.nz;
-    }
-    boxed = (int64_t)wx * wy * wz <= cap;
-  }
-  if (boxed) {  // margins while they fit: z, y, x in turn
-    int o[3] = {ox, oy, oz}, w[3] = {wx, wy, wz};
-    const int n[3] = {g.nx, g.ny, g.nz};
-    for (int d = 2, stuck = 0; stuck < 3; d = d == 0 ? 2 : d - 1) {
-      int o2 = o[d], w2 = w[d];
-      bool grew = false;
-      if (w2 < n[d]) {
-        win_grow(o2, w2, n[d]);
-        if ((int64_t)w2 * w[(d + 1) % 3] * w[(d + 2) % 3] <= cap) {
-          o[d] = o2;
-          w[d] = w2;
-          grew = true;
-        }
-      }
-      stuck = grew ? 0 : stuck + 1;
-    }
-    ox = o[0];
-    oy = o[1];
-    oz = o[2];
-    wx = w[0];
-    wy = w[1];
-    wz = w[2];
-  } else {  // the fixed box around the middle particle
-    wx = min(fx, g.nx);
-    wy = min(fy, g.ny);
-    wz = min(fz, g.nz);
-    const int64_t mid = a + (b - a) / 2;
-    ox = wrapn(cell(s.x[mid], g.nx) - wx / 2 + g.nx, g.nx);
-    oy = wrapn(cell(s.y[mid], g.ny) - wy / 2 + g.ny, g.ny);
-    oz = wrapn(cell(s.z[mid], g.nz) - wz / 2 + g.nz, g.nz);
-  }
-}
-
-// The block's run of particles (indices in the species' segment): after a
-// sort the run table's entry (at most `per` particles over a bounded range
-// of cells), else the per-th slice of species blockIdx.y.  False for a block
-// past the end.
-__device__ __forceinline__ bool block_run(const SpeciesTab &sp, const Run *runs, int per, int &is,
-                                          int64_t &beg, int64_t &end) {
+// The block's run of particles (indices in the species' segment) and its
+// window: after a sort the run table's entry (at most `per` particles over a
+// bounded range of cells), else the per-th slice of species blockIdx.y.  False
+// for a block past the end.
+__device__ __forceinline__ bool block_run(const State64 &s, const SpeciesTab &sp, const Run *runs,
+                                          int per, const Grid &g, const WinShape &ws, int &is,
+                                          int64_t &beg, int64_t &end, Win &W) {
   if (runs) {
     const Run r = runs[blockIdx.x];
     is = r.s;
     beg = r.beg;
     end = r.beg + r.len;
+    W = r.w;
     return true;
   }
   is = blockIdx.y;
@@ -319,16 +277,23 @@ __device__ __forceinline__ bool block_run(const SpeciesTab &sp, const Run *runs,
   const int64_t cnt = sp.cnt[is];
   if (beg >= cnt) return false;
   end = min(beg + (int64_t)per, cnt);
+  W = slice_window(s, sp.off[is] + beg, sp.off[is] + end - 1, g, ws);
   return true;
+}
+
+// v times 2^48 rounded to the nearest integer, |v| < 8: the sum with 1.5 2^52
+// has an ulp of 1, so its mantissa holds the integer; 1.5 2^52 has a zero low
+// word, so taking it off is one 32-bit subtraction (a conversion to int64 is
+// about seven instructions)
+__device__ __forceinline__ unsigned long long win_fix(double v) {
+  const unsigned long long b = (unsigned long long)__double_as_longlong(
+      __builtin_fma(v, 281474976710656.0, 6755399441055744.0));
+  return ((unsigned long long)((uint32_t)(b >> 32) - 0x43380000u) << 32) | (uint32_t)b;
 }
 
 // One particle's CIC weights (charge.F90:152-210) at (x, y, z): into the
 // block's LDS window when its eight nodes lie in it, else into the species'
 // rho r directly.
-struct Win {
-  int wx, wy, wz, ox, oy, oz;
-};
-
 __device__ __forceinline__ void deposit_win(unsigned long long *win, const Win &W, double *r,
                                             const Grid &g, double x, double y, double z,
                                             double qc) {
@@ -341,15 +306,14 @@ __device__ __forceinline__ void deposit_win(unsigned long long *win, const Win &
   if (li < W.wx && lj < W.wy && lk < W.wz && win_next(li, W.wx, g.nx, li1) &&
       win_next(lj, W.wy, g.ny, lj1) && win_next(lk, W.wz, g.nz, lk1)) {
     auto at = [&](int a, int b, int c) { return win + (c * W.wy + b) * W.wx + a; };
-    auto fx = [](double v) { return (unsigned long long)__double2ll_rn(v * kRhoFix); };
-    atomicAdd(at(li, lj, lk1), fx(w.v1));
-    atomicAdd(at(li1, lj, lk1), fx(w.v2));
-    atomicAdd(at(li1, lj1, lk1), fx(w.v3));
-    atomicAdd(at(li, lj1, lk1), fx(w.v4));
-    atomicAdd(at(li, lj, lk), fx(w.v5));
-    atomicAdd(at(li1, lj, lk), fx(w.v6));
-    atomicAdd(at(li1, lj1, lk), fx(w.v7));
-    atomicAdd(at(li, lj1, lk), fx(w.v8));
+    atomicAdd(at(li, lj, lk1), win_fix(w.v1));
+    atomicAdd(at(li1, lj, lk1), win_fix(w.v2));
+    atomicAdd(at(li1, lj1, lk1), win_fix(w.v3));
+    atomicAdd(at(li, lj1, lk1), win_fix(w.v4));
+    atomicAdd(at(li, lj, lk), win_fix(w.v5));
+    atomicAdd(at(li1, lj, lk), win_fix(w.v6));
+    atomicAdd(at(li1, lj1, lk), win_fix(w.v7));
+    atomicAdd(at(li, lj1, lk), win_fix(w.v8));
   } else {
     int i1 = i + 1, j1 = j + 1, k1 = k + 1;
     atomicAdd(r + cidx(g, i, j, k1), w.v1 * qc);
@@ -363,31 +327,64 @@ __device__ __forceinline__ void deposit_win(unsigned long long *win, const Win &
   }
 }
 
-// the window's non-zero nodes into rho, one FP64 atomic each (after a barrier)
-__device__ __forceinline__ void flush_win(const unsigned long long *win, const Win &W, double *r,
-                                          const Grid &g, double qc) {
-  for (int q = threadIdx.x; q < W.wx * W.wy * W.wz; q += kBlock) {
-    const long long v = (long long)win[q];
-    if (v != 0) {
-      int li = q % W.wx, lj = (q / W.wx) % W.wy, lk = q / (W.wx * W.wy);
-      atomicAdd(r + cidx(g, W.ox + li, W.oy + lj, W.oz + lk), (double)v * (qc / kRhoFix));
+// The window's non-zero nodes into the C accumulators r[0..C-1] (sums times
+// scale), one FP64 atomic each, after a barrier; component c of the window
+// starts at c * nodes.  The thread's node moves on by kBlock per pass: its
+// three indices are carried along (four integer divisions per node and
+// component, as many VALU instructions as half of the zigzag push's particle
+// work, were 20% of that kernel's time).
+template <int C>
+__device__ __forceinline__ void flush_win(const unsigned long long *win, const Win &W,
+                                          double *const r[C], const Grid &g, double scale) {
+  const int nodes = W.wx * W.wy * W.wz;
+  int q = threadIdx.x;
+  const int t = q / W.wx, st = kBlock / W.wx;
+  int li = q - t * W.wx, lk = t / W.wy, lj = t - lk * W.wy;
+  const int sx = kBlock - st * W.wx, sz = st / W.wy, sy = st - sz * W.wy;
+  for (; q < nodes; q += kBlock) {
+    long long v[C];
+    bool any = false;
+#pragma unroll
+    for (int c = 0; c < C; c++) {
+      v[c] = (long long)win[c * nodes + q];
+      any = any || v[c] != 0;
+    }
+    if (any) {
+      const int64_t n = cidx(g, W.ox + li, W.oy + lj, W.oz + lk);
+#pragma unroll
+      for (int c = 0; c < C; c++)
+        if (v[c] != 0) atomicAdd(r[c] + n, (double)v[c] * scale);
+    }
+    li += sx;
+    lj += sy;
+    lk += sz;
+    if (li >= W.wx) {
+      li -= W.wx;
+      lj++;
+    }
+    if (lj >= W.wy) {
+      lj -= W.wy;
+      lk++;
     }
   }
+}
+
+// clear the first n of an even number of window entries
+__device__ __forceinline__ void zero_win(unsigned long long *win, int n) {
+  for (int q = threadIdx.x; 2 * q < n; q += kBlock)
+    reinterpret_cast<ulonglong2 *>(win)[q] = make_ulonglong2(0ull, 0ull);
 }
 
 __global__ __launch_bounds__(kBlock) void k_deposit64(State64 s, SpeciesTab sp, Grid g,
                                                       double *__restrict__ rho, int64_t ncell,
                                                       const Run *__restrict__ runs, int *flag) {
-  __shared__ unsigned long long win[kWinCap];
+  __shared__ __align__(16) unsigned long long win[kWinEs.cap];
   int is;
   int64_t beg, end;
-  if (!block_run(sp, runs, kBlock * kDepPer, is, beg, end)) return;  // uniform over the block
-  const int64_t off = sp.off[is];
-  // window: nodes o .. o + w - 1 per axis (w <= n, so no node appears twice)
   Win W;
-  run_window(s, off + beg, off + end - 1, g, kWinCap, kWinX, kWinY, kWinZ, W.wx, W.wy, W.wz, W.ox,
-             W.oy, W.oz);
-  for (int q = threadIdx.x; q < W.wx * W.wy * W.wz; q += kBlock) win[q] = 0ull;
+  if (!block_run(s, sp, runs, kBlock * kDepPer, g, kWinEs, is, beg, end, W)) return;  // uniform
+  const int64_t off = sp.off[is];
+  zero_win(win, W.wx * W.wy * W.wz);
   __syncthreads();
   const double qc = sp.q[is];
   double *r = rho + (int64_t)is * ncell;
@@ -397,7 +394,8 @@ __global__ __launch_bounds__(kBlock) void k_deposit64(State64 s, SpeciesTab sp, 
     deposit_win(win, W, r, g, x, y, z, qc);
   }
   __syncthreads();
-  flush_win(win, W, r, g, qc);
+  double *const acc[1] = {r};
+  flush_win<1>(win, W, acc, g, qc / kRhoFix);
 }
 
 // psolve2 and charge in one pass (psolve2.F90:137-433, then charge.F90:
@@ -417,17 +415,15 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4)))
 void k_push_dep64(State64 s, SpeciesTab sp, const double *__restrict__ node, Grid g, int ustep,
                   double *__restrict__ rho, int64_t ncell, const Run *__restrict__ runs, int *flag,
                   SortDest dst) {
-  __shared__ unsigned long long win[kWinCap];
+  __shared__ __align__(16) unsigned long long win[kWinEs.cap];
   int is;
   int64_t beg, end;
-  if (!block_run(sp, runs, kBlock * kDepPer, is, beg, end)) return;  // uniform over the block
+  Win W;
+  if (!block_run(s, sp, runs, kBlock * kDepPer, g, kWinEs, is, beg, end, W)) return;  // uniform
   const int64_t off = sp.off[is];
   const int64_t key0 = (int64_t)is * dst.nkey;
   const int64_t base = RESORT ? off - dst.start[key0] : 0;
-  Win W;
-  run_window(s, off + beg, off + end - 1, g, kWinCap, kWinX, kWinY, kWinZ, W.wx, W.wy, W.wz, W.ox,
-             W.oy, W.oz);
-  for (int q = threadIdx.x; q < W.wx * W.wy * W.wz; q += kBlock) win[q] = 0ull;
+  zero_win(win, W.wx * W.wy * W.wz);
   __syncthreads();
   const double gustep = (double)ustep;
   const double qmp = sp.qm[is] * gustep * 0.5;
@@ -447,7 +443,7 @@ void k_push_dep64(State64 s, SpeciesTab sp, const double *__restrict__ node, Gri
     int i = (int)x, j = (int)y, k = (int)z;  // int(), psolve2.F90:158-160
     Cic w = cic(x, y, z, i, j, k);
     double f[6];
-    gather6(node, g, w, f);
+    gather6<true>(node, g, w, f);
     boris64(vx, vy, vz, f, qmp);
     double xmove = vx * gustep, ymove = vy * gustep, zmove = vz * gustep;
     x = x + xmove;
@@ -466,7 +462,8 @@ void k_push_dep64(State64 s, SpeciesTab sp, const double *__restrict__ node, Gri
     deposit_win(win, W, r, g, x, y, z, qc);
   }
   __syncthreads();
-  flush_win(win, W, r, g, qc);
+  double *const acc[1] = {r};
+  flush_win<1>(win, W, acc, g, qc / kRhoFix);
 }
 
 // ---------------------------------------------------------------- psolve1
@@ -504,7 +501,7 @@ __device__ __forceinline__ Relay relay_axis(double xnew, double lb, double cb, i
 }
 
 // The zigzag sums of a block's particles go to an LDS window (three
-// components of kEmCap nodes each, shaped from the block's sorted run like the
+// components of kWinEm.cap nodes each, shaped from the block's sorted run like the
 // charge window, or a fixed box around its middle particle) as int64 fixed
 // point at 2^48 per unit, and reach the global FP64 sums once per window
 // node.  A contribution is |vv w| <= 4 in the window (larger fluxes go
@@ -512,33 +509,33 @@ __device__ __forceinline__ Relay relay_axis(double xnew, double lb, double cb, i
 // 2 kBlock kEmPer terms stays below 2^61; the rounding of each term
 // (2^-49) is far below the FP64 summation round-off of the reference's order.
 constexpr int kEmPer = 4;
-constexpr int kEmCap = 1600;                           // 3 x 12.8 KB of int64
-constexpr int kEmWinX = 40, kEmWinY = 8, kEmWinZ = 5;  // the fixed box
 constexpr double kEmFix = 281474976710656.0;          // 2^48
 
-__device__ __forceinline__ long long em_fix(double v) { return __double2ll_rn(v * kEmFix); }
 
-// RESORT as in k_push_dep64.
+// RESORT as in k_push_dep64.  Bound by latency and instruction issue (VALU about
+// 40%, LDS conflicts 30%, HBM 3 TB/s); four waves per SIMD (128 VGPRs).  On the
+// 18.5M-particle two-stream (128 x 64 x 64), 1.42 ms before: one sum per node
+// for a particle that stays in its cell, the flush without divisions and the
+// short fixed-point conversion 1.12; four waves instead of three 1.02; the
+// windows from the run table instead of a scalar loop per block 0.80.  Runs of
+// 2,048 or 4,096 particles, whose windows have no margin left: 1.6 and 1.2 ms.
 template <bool RESORT>
-__global__ __launch_bounds__(kBlock) void k_push_em64(State64 s, SpeciesTab sp,
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4)))
+void k_push_em64(State64 s, SpeciesTab sp,
                                                       const double *__restrict__ node, Grid g,
                                                       int ustep, double *__restrict__ jacc,
                                                       int64_t ncell, const Run *__restrict__ runs,
                                                       int *flag, SortDest dst) {
-  constexpr int WN = kEmCap;
-  __shared__ unsigned long long win[3 * WN];
+  __shared__ __align__(16) unsigned long long win[3 * kWinEm.cap];
   int is;
   int64_t beg, end;
-  if (!block_run(sp, runs, kBlock * kEmPer, is, beg, end)) return;  // uniform over the block
+  Win W;
+  if (!block_run(s, sp, runs, kBlock * kEmPer, g, kWinEm, is, beg, end, W)) return;  // uniform
   const int64_t off = sp.off[is];
   const int64_t key0 = (int64_t)is * dst.nkey;
   const int64_t base = RESORT ? off - dst.start[key0] : 0;
-  // window: nodes o .. o + w - 1 per axis (w <= n, so no node appears twice)
-  int wx, wy, wz, ox, oy, oz;
-  run_window(s, off + beg, off + end - 1, g, WN, kEmWinX, kEmWinY, kEmWinZ, wx, wy, wz, ox, oy,
-             oz);
-  const int wn = wx * wy * wz;  // nodes per component
-  for (int q = threadIdx.x; q < 3 * wn; q += kBlock) win[q] = 0ull;
+  const int wn = W.wx * W.wy * W.wz;  // nodes per component
+  zero_win(win, 3 * wn);
   __syncthreads();
   double gustep = (double)ustep;
   double rustep = 1.0 / gustep;
@@ -562,7 +559,7 @@ __global__ __launch_bounds__(kBlock) void k_push_em64(State64 s, SpeciesTab sp,
     double xb = ib, yb = jb, zb = kb;
     Cic w = cic(xlb, ylb, zlb, ib, jb, kb);
     double f[6];
-    gather6(node, g, w, f);
+    gather6<false>(node, g, w, f);
     boris64(vx, vy, vz, f, qmp);
     double xmove = vx * gustep, ymove = vy * gustep, zmove = vz * gustep;
     x = x + xmove;
@@ -596,62 +593,70 @@ __global__ __launch_bounds__(kBlock) void k_push_em64(State64 s, SpeciesTab sp,
     double vx2w4 = yd2 * zd2, vx2w2 = yd2 - vx2w4, vx2w3 = zd2 - vx2w4, vx2w1 = 1.0 - yd2 - vx2w3;
     double vy2w4 = xd2 * zd2, vy2w2 = xd2 - vy2w4, vy2w3 = zd2 - vy2w4, vy2w1 = 1.0 - xd2 - vy2w3;
     double vz2w4 = xd2 * yd2, vz2w2 = xd2 - vz2w4, vz2w3 = yd2 - vz2w4, vz2w1 = 1.0 - xd2 - vz2w3;
-    // the 12 contributions of each segment (:759-789), in the window when its
-    // cell and the next node along every axis are inside
-    auto seg = [&](int i, int j, int k, double vvx, double vvy, double vvz, const double wx4[4],
-                   const double wy4[4], const double wz4[4]) {
-      const int li = wrapn(i - ox, g.nx), lj = wrapn(j - oy, g.ny), lk = wrapn(k - oz, g.nz);
-      int li1, lj1, lk1;
-      const bool in_win = li < wx && lj < wy && lk < wz && win_next(li, wx, g.nx, li1) &&
-                          win_next(lj, wy, g.ny, lj1) && win_next(lk, wz, g.nz, lk1) &&
-                          fabs(vvx) <= 4.0 && fabs(vvy) <= 4.0 && fabs(vvz) <= 4.0;
-      if (in_win) {
-        auto at = [&](int c, int a, int b, int d) { return win + c * wn + (d * wy + b) * wx + a; };
-        atomicAdd(at(0, li, lj, lk), (unsigned long long)em_fix(vvx * wx4[0]));
-        atomicAdd(at(0, li, lj1, lk), (unsigned long long)em_fix(vvx * wx4[1]));
-        atomicAdd(at(0, li, lj, lk1), (unsigned long long)em_fix(vvx * wx4[2]));
-        atomicAdd(at(0, li, lj1, lk1), (unsigned long long)em_fix(vvx * wx4[3]));
-        atomicAdd(at(1, li, lj, lk), (unsigned long long)em_fix(vvy * wy4[0]));
-        atomicAdd(at(1, li1, lj, lk), (unsigned long long)em_fix(vvy * wy4[1]));
-        atomicAdd(at(1, li, lj, lk1), (unsigned long long)em_fix(vvy * wy4[2]));
-        atomicAdd(at(1, li1, lj, lk1), (unsigned long long)em_fix(vvy * wy4[3]));
-        atomicAdd(at(2, li, lj, lk), (unsigned long long)em_fix(vvz * wz4[0]));
-        atomicAdd(at(2, li1, lj, lk), (unsigned long long)em_fix(vvz * wz4[1]));
-        atomicAdd(at(2, li, lj1, lk), (unsigned long long)em_fix(vvz * wz4[2]));
-        atomicAdd(at(2, li1, lj1, lk), (unsigned long long)em_fix(vvz * wz4[3]));
-      } else {
-        const int i1 = i + 1, j1 = j + 1, k1 = k + 1;
-        atomicAdd(jx + cidx(g, i, j, k), vvx * wx4[0]);
-        atomicAdd(jx + cidx(g, i, j1, k), vvx * wx4[1]);
-        atomicAdd(jx + cidx(g, i, j, k1), vvx * wx4[2]);
-        atomicAdd(jx + cidx(g, i, j1, k1), vvx * wx4[3]);
-        atomicAdd(jy + cidx(g, i, j, k), vvy * wy4[0]);
-        atomicAdd(jy + cidx(g, i1, j, k), vvy * wy4[1]);
-        atomicAdd(jy + cidx(g, i, j, k1), vvy * wy4[2]);
-        atomicAdd(jy + cidx(g, i1, j, k1), vvy * wy4[3]);
-        atomicAdd(jz + cidx(g, i, j, k), vvz * wz4[0]);
-        atomicAdd(jz + cidx(g, i1, j, k), vvz * wz4[1]);
-        atomicAdd(jz + cidx(g, i, j1, k), vvz * wz4[2]);
-        atomicAdd(jz + cidx(g, i1, j1, k), vvz * wz4[3]);
-      }
-    };
     const double ax1[4] = {vx1w1, vx1w2, vx1w3, vx1w4}, ay1[4] = {vy1w1, vy1w2, vy1w3, vy1w4},
                  az1[4] = {vz1w1, vz1w2, vz1w3, vz1w4};
     const double ax2[4] = {vx2w1, vx2w2, vx2w3, vx2w4}, ay2[4] = {vy2w1, vy2w2, vy2w3, vy2w4},
                  az2[4] = {vz2w1, vz2w2, vz2w3, vz2w4};
-    seg(ib, jb, kb, vvx1, vvy1, vvz1, ax1, ay1, az1);
-    seg(rx.ia, ry.ia, rz.ia, vvx2, vvy2, vvz2, ax2, ay2, az2);
+    // the 12 contributions of a segment (:759-789), in the window when its cell
+    // and the next node along every axis are inside; value(c, k) is component
+    // c's contribution with its weight k
+    auto seg = [&](int i, int j, int k, bool fits, auto value) {
+      const int li = wrapn(i - W.ox, g.nx), lj = wrapn(j - W.oy, g.ny), lk = wrapn(k - W.oz, g.nz);
+      int li1, lj1, lk1;
+      if (fits && li < W.wx && lj < W.wy && lk < W.wz && win_next(li, W.wx, g.nx, li1) &&
+          win_next(lj, W.wy, g.ny, lj1) && win_next(lk, W.wz, g.nz, lk1)) {
+        const int dx = li1 - li, dy = (lj1 - lj) * W.wx, dz = (lk1 - lk) * (W.wx * W.wy);
+        unsigned long long *p = win + (lk * W.wy + lj) * W.wx + li;
+        atomicAdd(p, win_fix(value(0, 0)));
+        atomicAdd(p + dy, win_fix(value(0, 1)));
+        atomicAdd(p + dz, win_fix(value(0, 2)));
+        atomicAdd(p + dy + dz, win_fix(value(0, 3)));
+        p += wn;
+        atomicAdd(p, win_fix(value(1, 0)));
+        atomicAdd(p + dx, win_fix(value(1, 1)));
+        atomicAdd(p + dz, win_fix(value(1, 2)));
+        atomicAdd(p + dx + dz, win_fix(value(1, 3)));
+        p += wn;
+        atomicAdd(p, win_fix(value(2, 0)));
+        atomicAdd(p + dx, win_fix(value(2, 1)));
+        atomicAdd(p + dy, win_fix(value(2, 2)));
+        atomicAdd(p + dx + dy, win_fix(value(2, 3)));
+      } else {
+        const int i1 = i + 1, j1 = j + 1, k1 = k + 1;
+        atomicAdd(jx + cidx(g, i, j, k), value(0, 0));
+        atomicAdd(jx + cidx(g, i, j1, k), value(0, 1));
+        atomicAdd(jx + cidx(g, i, j, k1), value(0, 2));
+        atomicAdd(jx + cidx(g, i, j1, k1), value(0, 3));
+        atomicAdd(jy + cidx(g, i, j, k), value(1, 0));
+        atomicAdd(jy + cidx(g, i1, j, k), value(1, 1));
+        atomicAdd(jy + cidx(g, i, j, k1), value(1, 2));
+        atomicAdd(jy + cidx(g, i1, j, k1), value(1, 3));
+        atomicAdd(jz + cidx(g, i, j, k), value(2, 0));
+        atomicAdd(jz + cidx(g, i1, j, k), value(2, 1));
+        atomicAdd(jz + cidx(g, i, j1, k), value(2, 2));
+        atomicAdd(jz + cidx(g, i1, j1, k), value(2, 3));
+      }
+    };
+    auto small = [](double a, double b, double c) {
+      return fabs(a) <= 4.0 && fabs(b) <= 4.0 && fabs(c) <= 4.0;
+    };
+    // a particle that stays in its cell has both segments there: one sum (of
+    // at most 2 cells per step) per node, the second segment's own sums only
+    // for the particles that changed cell
+    const bool same = rx.ia == ib && ry.ia == jb && rz.ia == kb;
+    const double sx2 = same ? vvx2 : 0.0, sy2 = same ? vvy2 : 0.0, sz2 = same ? vvz2 : 0.0;
+    seg(ib, jb, kb, small(vvx1, vvy1, vvz1) && small(sx2, sy2, sz2) , [&](int c, int k) {
+      return c == 0 ? vvx1 * ax1[k] + sx2 * ax2[k]
+                    : (c == 1 ? vvy1 * ay1[k] + sy2 * ay2[k] : vvz1 * az1[k] + sz2 * az2[k]);
+    });
+    if (!same)
+      seg(rx.ia, ry.ia, rz.ia, small(vvx2, vvy2, vvz2), [&](int c, int k) {
+        return c == 0 ? vvx2 * ax2[k] : (c == 1 ? vvy2 * ay2[k] : vvz2 * az2[k]);
+      });
   }
   __syncthreads();
-  for (int q = threadIdx.x; q < 3 * wn; q += kBlock) {
-    const long long v = (long long)win[q];
-    if (v != 0) {
-      const int d = q / wn, r = q - d * wn;
-      const int li = r % wx, lj = (r / wx) % wy, lk = r / (wx * wy);
-      double *jd = d == 0 ? jx : (d == 1 ? jy : jz);
-      atomicAdd(jd + cidx(g, ox + li, oy + lj, oz + lk), (double)v * (1.0 / kEmFix));
-    }
-  }
+  double *const acc[3] = {jx, jy, jz};
+  flush_win<3>(win, W, acc, g, 1.0 / kEmFix);
 }
 
 dim3 species_grid(const SpeciesTab &sp) {
