@@ -31,6 +31,7 @@ SOURCES = [
     ("k_yee.hip", ["-ffp-contract=off"]),
     ("k_poisson.hip", []),
     ("emg_api.hip", []),
+    ("emg_io.hip", []),
 ]
 HOST_SOURCES = [("host_init.cpp", ["-O2", "-fPIC", "-std=c++17", "-ffp-contract=off", "-I", INC])]
 

@@ -95,6 +95,7 @@ namespace {
 
 constexpr int kFlagPreside = 8;
 constexpr int kFlagPid = 16;
+constexpr int kFlagDead = 32;  // a record with nid < 0 in an upload that expected none
 
 // AoS pbuf records -> SoA FP64 state, validating each record
 __global__ __launch_bounds__(kBlock) void k_split(const emg_particle *rec, int64_t n, State64 st,
@@ -102,6 +103,10 @@ __global__ __launch_bounds__(kBlock) void k_split(const emg_particle *rec, int64
   int64_t m = (int64_t)blockIdx.x * kBlock + threadIdx.x;
   if (m >= n) return;
   emg_particle r = rec[m];
+  if (r.nid < 0) {  // the host drops the dead records and uploads again
+    atomicOr(flag, kFlagDead);
+    return;
+  }
   bool ok = (r.x >= 0.0) && (r.x <= g.slx) && (r.y >= 0.0) && (r.y <= g.sly) && (r.z >= 0.0) &&
             (r.z <= g.slz) && (r.vx == r.vx) && (r.vy == r.vy) && (r.vz == r.vz) &&
             (fabs(r.vx) < 1e300) && (fabs(r.vy) < 1e300) && (fabs(r.vz) < 1e300);
@@ -174,14 +179,10 @@ void free_state64(State64 &st) {
   st = State64{};
 }
 
-// synchronise and translate device flags into an error code
-int check_flags(emg_ctx *c) {
-  int rc = hip_check(hipMemcpyAsync(c->hflag, c->dflag, sizeof(int), hipMemcpyDeviceToHost, c->stream),
-                     "flag read");
-  if (rc) return rc;
-  rc = hip_check(hipStreamSynchronize(c->stream), "stream synchronize");
-  if (rc) return rc;
-  int f = *c->hflag;
+}  // namespace
+
+int flags_error(emg_ctx *c) {
+  const int f = *c->hflag;
   if (f == 0) return EMG_OK;
   launch_zero(c->dflag, sizeof(int), c->stream);
   (void)hipStreamSynchronize(c->stream);
@@ -198,7 +199,6 @@ int check_flags(emg_ctx *c) {
   return set_error(EMG_ERR_HIP, "unknown device flag");
 }
 
-}  // namespace
 }  // namespace emg
 
 using namespace emg;
@@ -289,6 +289,7 @@ int emg_create(const emg_config *cfg, emg_ctx **out) {
     return rc;
   }
   c->own_stream = true;
+  io_open(c);
   c->g.nx = cfg->n[0];
   c->g.ny = cfg->n[1];
   c->g.nz = cfg->n[2];
@@ -310,15 +311,19 @@ int emg_create(const emg_config *cfg, emg_ctx **out) {
   c->sp.off[cfg->nspec] = off;
   c->cap_total = off;
   int nsp = cfg->nspec;
-  if ((rc = dalloc(&c->dflag, 1, "flag")) || (rc = dalloc(&c->ke_out, 3 * nsp, "energy")) ||
+  if ((rc = dalloc(&c->dflag, 1, "flag")) ||
       (rc = dalloc((double **)&c->face, (size_t)(face_len(c->g) * nsp), "upper-face charge"))) {
     emg_destroy(c);
     return rc;
   }
-  if (hipHostMalloc((void **)&c->hflag, sizeof(int), hipHostMallocDefault) != hipSuccess) {
+  // the flag, and after it the sums that reduction kernels hand to the host
+  if (hipHostMalloc((void **)&c->hflag, sizeof(double) * (1 + 3 * EMG_MAX_SPECIES),
+                    hipHostMallocDefault) != hipSuccess) {
+    c->hflag = nullptr;
     emg_destroy(c);
     return set_error(EMG_ERR_NOMEM, "pinned flag");
   }
+  c->hsum = reinterpret_cast<double *>(c->hflag) + 1;
   launch_zero(c->dflag, sizeof(int), c->stream);
   if (cfg->precision == EMG_PLAIN_FP64) {
     int64_t nn = (int64_t)(cfg->n[0] + 1) * (cfg->n[1] + 1) * (cfg->n[2] + 1);
@@ -356,7 +361,6 @@ int emg_destroy(emg_ctx *c) {
   for (int k = 0; k < kStateSlots; k++) free_state64(c->slot[k]);
   dfree(c->adj_e);
   dfree(c->adj_g);
-  dfree(c->adj_q);
   dfree(c->adj_sum);
   dfree(c->adj_bins.count);
   dfree(c->adj_bins.start);
@@ -403,7 +407,6 @@ int emg_destroy(emg_ctx *c) {
   dfree(c->j64);
   dfree(c->jfx);
   dfree(c->ke_part);
-  dfree(c->ke_out);
   dfree(c->face);
   dfree(c->runs[0]);
   dfree(c->runs[1]);
@@ -414,6 +417,7 @@ int emg_destroy(emg_ctx *c) {
   dfree(c->scan_tmp);
   dfree(c->dflag);
   if (c->hflag) (void)hipHostFree(c->hflag);
+  io_close(c);
   TimerState *t = tstate(c);
   for (EvPair &p : t->pending) t->free_pairs.push_back(p);
   for (EvPair &p : t->free_pairs) {
@@ -453,7 +457,7 @@ int emg_synchronize(emg_ctx *c) {
   CTX_CHECK(c);
   int rc = hip_check(hipGetLastError(), "kernel launch");
   if (rc) return rc;
-  return check_flags(c);
+  return read_flags(c);
 }
 
 int emg_upload_particles(emg_ctx *c, const emg_particle *pbuf, const int64_t *counts, int32_t nspec) {
@@ -466,18 +470,58 @@ int emg_upload_particles(emg_ctx *c, const emg_particle *pbuf, const int64_t *co
     total += counts[s];
   }
   if (total > 0 && !pbuf) return set_error(EMG_ERR_ARG, "null pbuf");
-  // transbound: keep nid >= 0 in order (host pass; one copy only when needed)
-  std::vector<int64_t> kept(nspec, 0);
-  std::vector<emg_particle> compact;
-  bool need_compact = false;
-  for (int64_t m = 0; m < total; m++)
-    if (pbuf[m].nid < 0) {
-      need_compact = true;
-      break;
+  State64 tgt = c->s64;
+  State64 tmp{};
+  // particles of counts cnt, species-contiguous at src, into tgt
+  auto send = [&](const emg_particle *src, const int64_t *cnt) {
+    int64_t first[EMG_MAX_SPECIES + 1] = {0};
+    for (int s = 0; s < nspec; s++) first[s + 1] = first[s] + cnt[s];
+    const int need_pid0 = c->cfg.precision == EMG_FP32_FIXED && !c->cfg.track_pid ? 1 : 0;
+    for (int s = 0; s < nspec; s++) c->sp.cnt[s] = cnt[s];
+    return io_write(c, src, sizeof(emg_particle) * first[nspec], sizeof(emg_particle),
+                    [&, need_pid0](size_t off, size_t len, void *slot) {
+                      const int64_t m0 = off / sizeof(emg_particle),
+                                    m1 = m0 + len / sizeof(emg_particle);
+                      for (int s = 0; s < nspec; s++) {
+                        const int64_t a = std::max(m0, first[s]), b = std::min(m1, first[s + 1]);
+                        if (a < b)
+                          hipLaunchKernelGGL(k_split, dim3((unsigned)((b - a + kBlock - 1) / kBlock)),
+                                             dim3(kBlock), 0, c->stream,
+                                             static_cast<emg_particle *>(slot) + (a - m0), b - a, tgt,
+                                             c->sp.off[s] + (a - first[s]), c->g, c->dflag,
+                                             need_pid0);
+                      }
+                      return hip_check(hipGetLastError(), "upload split");
+                    });
+  };
+  bool fits = true;
+  for (int s = 0; s < nspec; s++) fits = fits && counts[s] <= c->cfg.capacity[s];
+  int rc = EMG_OK;
+  bool dead = !fits;  // more records than room: only the living have to fit
+  if (fits) {
+    if (c->cfg.precision == EMG_FP32_FIXED) {
+      if ((rc = alloc_state64(tmp, std::max<int64_t>(c->cap_total, 1)))) {
+        free_state64(tmp);
+        return rc;
+      }
+      tgt = tmp;
     }
-  const emg_particle *src = pbuf;
-  if (need_compact) {
-    compact.reserve((size_t)total);
+    rc = send(pbuf, counts);
+    if (!rc) {
+      rc = read_flags(c);
+      dead = rc != EMG_OK && (*c->hflag & kFlagDead) != 0;
+    }
+  }
+  if (dead) {
+    // transbound: keep nid >= 0 in order (flags of the first try are cleared)
+    std::vector<int64_t> kept(nspec, 0);
+    std::vector<emg_particle> compact;
+    try {
+      compact.reserve((size_t)total);
+    } catch (const std::bad_alloc &) {
+      free_state64(tmp);
+      return set_error(EMG_ERR_NOMEM, "host allocation failed");
+    }
     int64_t m = 0;
     for (int s = 0; s < nspec; s++) {
       for (int64_t k = 0; k < counts[s]; k++, m++)
@@ -486,49 +530,23 @@ int emg_upload_particles(emg_ctx *c, const emg_particle *pbuf, const int64_t *co
           kept[s]++;
         }
     }
-    src = compact.data();
-  } else {
-    for (int s = 0; s < nspec; s++) kept[s] = counts[s];
-  }
-  for (int s = 0; s < nspec; s++)
-    if (kept[s] > c->cfg.capacity[s])
-      return set_error(EMG_ERR_CAPACITY, "species count exceeds the context capacity");
-
-  State64 tgt = c->s64;
-  State64 tmp{};
-  int rc;
-  if (c->cfg.precision == EMG_FP32_FIXED) {
-    if ((rc = alloc_state64(tmp, std::max<int64_t>(c->cap_total, 1)))) return rc;
-    tgt = tmp;
-  }
-  const int64_t chunk = 1 << 22;
-  emg_particle *d_rec = nullptr;
-  if ((rc = dalloc(&d_rec, (size_t)std::min<int64_t>(chunk, std::max<int64_t>(total, 1)), "staging"))) {
-    free_state64(tmp);
-    return rc;
-  }
-  int64_t m = 0;
-  for (int s = 0; s < nspec; s++) {
-    for (int64_t k = 0; k < kept[s]; k += chunk) {
-      int64_t n = std::min(chunk, kept[s] - k);
-      rc = hip_check(hipMemcpy(d_rec, src + m + k, sizeof(emg_particle) * n, hipMemcpyHostToDevice),
-                     "upload copy");
-      if (rc) break;
-      hipLaunchKernelGGL(k_split, dim3((unsigned)((n + kBlock - 1) / kBlock)), dim3(kBlock), 0,
-                         c->stream, d_rec, n, tgt, c->sp.off[s] + k, c->g, c->dflag,
-                         (c->cfg.precision == EMG_FP32_FIXED && !c->cfg.track_pid) ? 1 : 0);
-      rc = hip_check(hipStreamSynchronize(c->stream), "upload split");
-      if (rc) break;
+    for (int s = 0; s < nspec; s++)
+      if (kept[s] > c->cfg.capacity[s])
+        return set_error(EMG_ERR_CAPACITY, "species count exceeds the context capacity");
+    rc = EMG_OK;
+    if (c->cfg.precision == EMG_FP32_FIXED && !tmp.x) {
+      if ((rc = alloc_state64(tmp, std::max<int64_t>(c->cap_total, 1)))) {
+        free_state64(tmp);
+        return rc;
+      }
+      tgt = tmp;
     }
-    if (rc) break;
-    m += kept[s];
-    c->sp.cnt[s] = kept[s];
+    rc = send(compact.data(), kept.data());
+    if (!rc) rc = read_flags(c);
   }
-  dfree(d_rec);
-  if (!rc) rc = check_flags(c);
   if (!rc && c->cfg.precision == EMG_FP32_FIXED) {
     rc = fx_from64(c, tmp);
-    if (!rc) rc = check_flags(c);
+    if (!rc) rc = read_flags(c);
   }
   free_state64(tmp);
   if (rc) {
@@ -556,7 +574,7 @@ int emg_particle_counts(emg_ctx *c, int64_t *counts) {
 
 int emg_download_particles(emg_ctx *c, emg_particle *pbuf, int64_t *counts) {
   CTX_CHECK(c);
-  int rc = check_flags(c);
+  int rc = read_flags(c);
   if (rc) return rc;
   int64_t total = 0;
   for (int s = 0; s < c->sp.nspec; s++) total += c->sp.cnt[s];
@@ -567,7 +585,10 @@ int emg_download_particles(emg_ctx *c, emg_particle *pbuf, int64_t *counts) {
   State64 src = c->s64;
   State64 tmp{};
   if (c->cfg.precision == EMG_FP32_FIXED) {
-    if ((rc = alloc_state64(tmp, c->cap_total))) return rc;
+    if ((rc = alloc_state64(tmp, c->cap_total))) {
+      free_state64(tmp);
+      return rc;
+    }
     rc = fx_to64(c, tmp);
     if (rc) {
       free_state64(tmp);
@@ -575,29 +596,22 @@ int emg_download_particles(emg_ctx *c, emg_particle *pbuf, int64_t *counts) {
     }
     src = tmp;
   }
-  const int64_t chunk = 1 << 22;
-  emg_particle *d_rec = nullptr;
-  if ((rc = dalloc(&d_rec, (size_t)std::min<int64_t>(chunk, total), "staging"))) {
-    free_state64(tmp);
-    return rc;
-  }
-  int64_t m = 0;
-  for (int s = 0; s < c->sp.nspec && !rc; s++) {
-    for (int64_t k = 0; k < c->sp.cnt[s]; k += chunk) {
-      int64_t n = std::min(chunk, c->sp.cnt[s] - k);
-      hipLaunchKernelGGL(k_join, dim3((unsigned)((n + kBlock - 1) / kBlock)), dim3(kBlock), 0,
-                         c->stream, src, c->sp.off[s] + k, n, s + 1, d_rec);
-      rc = hip_check(hipStreamSynchronize(c->stream), "download join");
-      if (rc) break;
-      rc = hip_check(hipMemcpy(pbuf + m + k, d_rec, sizeof(emg_particle) * n, hipMemcpyDeviceToHost),
-                     "download copy");
-      if (rc) break;
-    }
-    m += c->sp.cnt[s];
-  }
-  dfree(d_rec);
+  int64_t first[EMG_MAX_SPECIES + 1] = {0};
+  for (int s = 0; s < c->sp.nspec; s++) first[s + 1] = first[s] + c->sp.cnt[s];
+  rc = io_read(c, pbuf, sizeof(emg_particle) * total, sizeof(emg_particle),
+               [&](size_t off, size_t len, void *slot) {
+                 const int64_t m0 = off / sizeof(emg_particle), m1 = m0 + len / sizeof(emg_particle);
+                 for (int s = 0; s < c->sp.nspec; s++) {
+                   const int64_t a = std::max(m0, first[s]), b = std::min(m1, first[s + 1]);
+                   if (a < b)
+                     hipLaunchKernelGGL(k_join, dim3((unsigned)((b - a + kBlock - 1) / kBlock)),
+                                        dim3(kBlock), 0, c->stream, src,
+                                        c->sp.off[s] + (a - first[s]), b - a, s + 1,
+                                        static_cast<emg_particle *>(slot) + (a - m0));
+                 }
+                 return hip_check(hipGetLastError(), "download join");
+               });
   free_state64(tmp);
-  if (!rc) rc = check_flags(c);
   return rc;
 }
 
@@ -687,14 +701,11 @@ int emg_get_fields(emg_ctx *c, double *eb, const int32_t lo[3], const int32_t hi
       return set_error(EMG_ERR_ARG, "eb bounds outside the uploaded array");
   const int l[3] = {lo[0], lo[1], lo[2]};
   const int ext[3] = {hi[0] - lo[0] + 1, hi[1] - lo[1] + 1, hi[2] - lo[2] + 1};
-  const size_t count = (size_t)6 * ext[0] * ext[1] * ext[2];
-  double *d_out = nullptr;
-  if ((rc = dalloc(&d_out, count, "eb read-out"))) return rc;
-  launch_eb_box(c, l, ext, d_out);
-  rc = check_flags(c);
-  if (!rc) rc = hip_check(hipMemcpy(eb, d_out, sizeof(double) * count, hipMemcpyDeviceToHost), "eb download");
-  dfree(d_out);
-  return rc;
+  const size_t count = (size_t)6 * ext[0] * ext[1] * ext[2], unit = 6 * sizeof(double);
+  return io_read(c, eb, sizeof(double) * count, unit, [&](size_t off, size_t len, void *slot) {
+    launch_eb_box(c, l, ext, (int64_t)(off / unit), (int64_t)(len / unit), (double *)slot);
+    return hip_check(hipGetLastError(), "eb read-out");
+  });
 }
 
 int emg_solve_es(emg_ctx *c, double rhobk) {
@@ -743,19 +754,25 @@ int emg_get_potential(emg_ctx *c, double *phi) {
   return read_potential(c, phi);
 }
 
+// wait for a reduction that left its sums in hsum and the flags in hflag
+static int read_sums(emg_ctx *c) {
+  int rc = hip_check(hipGetLastError(), "reduction launch");
+  if (!rc) rc = hip_check(hipStreamSynchronize(c->stream), "stream synchronize");
+  return rc ? rc : flags_error(c);
+}
+
 int emg_field_energy(emg_ctx *c, double cs, double *engeb) {
   CTX_CHECK(c);
   int rc = need_eb(c);
   if (rc) return rc;
   if (!engeb) return set_error(EMG_ERR_ARG, "null argument");
-  if (!c->fe_buf && (rc = dalloc(&c->fe_buf, (size_t)field_energy_part_need() + 2, "field energy")))
+  if (!c->fe_buf && (rc = dalloc(&c->fe_buf, (size_t)field_energy_part_need(), "field energy")))
     return rc;
-  launch_field_energy(c, cs, c->fe_buf, c->fe_buf + field_energy_part_need());
-  rc = check_flags(c);
-  if (!rc)
-    rc = hip_check(hipMemcpy(engeb, c->fe_buf + field_energy_part_need(), 2 * sizeof(double),
-                             hipMemcpyDeviceToHost), "field energy copy");
-  return rc;
+  launch_field_energy(c, cs, c->fe_buf, c->hsum);
+  if ((rc = read_sums(c))) return rc;
+  engeb[0] = c->hsum[0];
+  engeb[1] = c->hsum[1];
+  return EMG_OK;
 }
 
 static int need_particles(emg_ctx *c) {
@@ -856,39 +873,41 @@ int emg_deposit_rho(emg_ctx *c, int32_t func) {
   return hip_check(hipGetLastError(), "deposit launch");
 }
 
-// Read a grid array back: the read-out kernel writes it into a device staging
-// buffer (allocated for the call, or `stage` of `stage_cap` doubles), which
-// is copied to the host.
+// Read a grid array back: in chunks through the pinned slots, or (stage, of
+// stage_cap doubles) whole through a device array with one copy.
 static int read_grid(emg_ctx *c, double *host, const int32_t lo[3], const int32_t hi[3], int comps,
                      int species, bool current, double *stage = nullptr, int64_t stage_cap = 0) {
   if (!host || !lo || !hi) return set_error(EMG_ERR_ARG, "null argument");
   int l[3], h[3];
-  int64_t n = comps;
+  int64_t points = 1;
   for (int d = 0; d < 3; d++) {
     if (hi[d] < lo[d]) return set_error(EMG_ERR_ARG, "hi < lo");
     l[d] = lo[d];
     h[d] = hi[d];
-    n *= (int64_t)(hi[d] - lo[d] + 1);
+    points *= (int64_t)(hi[d] - lo[d] + 1);
   }
-  double *d_out = stage;
-  int rc;
-  if (stage) {
-    if (n > stage_cap)
-      return set_error(EMG_ERR_CAPACITY, "the read-out exceeds the library's static staging "
-                                         "array (2^24 values, 128 MiB): read it with emg_get_rho");
-  } else if ((rc = dalloc(&d_out, (size_t)n, "read-out"))) {
-    return rc;
-  }
-  if (current)
-    launch_read_current(c, species, d_out, l, h);
-  else
-    launch_read_rho(c, species, d_out, l, h);
-  rc = check_flags(c);
+  if (stage && points * comps > stage_cap)
+    return set_error(EMG_ERR_CAPACITY, "the read-out exceeds the library's static staging "
+                                       "array (2^24 values, 128 MiB): read it with emg_get_rho");
+  const bool ghosts = !current && prepare_read_rho(c, l, h);
+  auto launch = [&](int64_t o0, int64_t n, double *dst) {
+    if (current)
+      launch_read_current(c, species, dst, l, h, o0, n);
+    else
+      launch_read_rho(c, species, ghosts, dst, l, h, o0, n);
+    return hip_check(hipGetLastError(), "read-out");
+  };
+  const size_t unit = sizeof(double) * comps;
+  if (!stage)
+    return io_read(c, host, unit * points, unit, [&](size_t off, size_t len, void *slot) {
+      return launch((int64_t)(off / unit), (int64_t)(len / unit), static_cast<double *>(slot));
+    });
+  int rc = launch(0, points, stage);
+  if (!rc) rc = read_flags(c);
   if (!rc)
-    rc = hip_check(hipMemcpyAsync(host, d_out, sizeof(double) * n, hipMemcpyDeviceToHost, c->stream),
+    rc = hip_check(hipMemcpyAsync(host, stage, unit * points, hipMemcpyDeviceToHost, c->stream),
                    "read-out copy");
   if (!rc) rc = hip_check(hipStreamSynchronize(c->stream), "read-out copy");
-  if (!stage) dfree(d_out);
   return rc;
 }
 
@@ -923,12 +942,8 @@ int emg_energy(emg_ctx *c, double *engk) {
     fx_energy_from_push(c);
   else
     launch_fx_energy(c);
-  rc = check_flags(c);
-  if (rc) return rc;
-  double sums[3 * EMG_MAX_SPECIES];
-  rc = hip_check(hipMemcpy(sums, c->ke_out, sizeof(double) * 3 * c->sp.nspec, hipMemcpyDeviceToHost),
-                 "energy copy");
-  if (rc) return rc;
+  if ((rc = read_sums(c))) return rc;
+  const double *sums = c->hsum;
   double vol = c->g.slx * c->g.sly * c->g.slz;
   for (int s = 0; s < c->sp.nspec; s++)
     for (int d = 0; d < 3; d++) engk[3 * s + d] = 0.0 + 0.5 * c->cfg.rm[s] * sums[3 * s + d] / vol;
@@ -999,7 +1014,6 @@ static int need_adjoint(emg_ctx *c) {
   if ((rc = dalloc(&c->lam, 8 * (size_t)c->cap_total, "particle adjoints")) ||
       (rc = dalloc(&c->adj_e, 3 * c->ncell, "adjoint field")) ||
       (rc = dalloc(&c->adj_g, c->ncell, "adjoint density")) ||
-      (rc = dalloc(&c->adj_q, EMG_MAX_SPECIES, "adjoint factors")) ||
       (rc = dalloc(&c->adj_sum, (size_t)adj_vsum_need(), "adjoint sums")))
     return rc;
   launch_zero(c->lam, 8 * sizeof(double) * c->cap_total, c->stream);
@@ -1057,10 +1071,8 @@ int emg_adj_get_field(emg_ctx *c, double *lam_e) {
   CTX_CHECK(c);
   if (!lam_e) return set_error(EMG_ERR_ARG, "null argument");
   int rc = need_adjoint(c);
-  if (!rc) rc = check_flags(c);
   if (rc) return rc;
-  return hip_check(hipMemcpy(lam_e, c->adj_e, sizeof(double) * 3 * c->ncell, hipMemcpyDeviceToHost),
-                   "adjoint field copy");
+  return io_read_array(c, lam_e, c->adj_e, sizeof(double) * 3 * c->ncell);
 }
 
 int emg_adj_add_density(emg_ctx *c, const double *g, const double *qfac) {
@@ -1070,11 +1082,9 @@ int emg_adj_add_density(emg_ctx *c, const double *g, const double *qfac) {
   if (!rc) rc = need_particles(c);
   if (rc) return rc;
   if ((rc = hip_check(hipMemcpyAsync(c->adj_g, g, sizeof(double) * c->ncell, hipMemcpyHostToDevice,
-                                     c->stream), "adjoint density upload")) ||
-      (rc = hip_check(hipMemcpyAsync(c->adj_q, qfac, sizeof(double) * c->sp.nspec,
-                                     hipMemcpyHostToDevice, c->stream), "adjoint factor upload")))
+                                     c->stream), "adjoint density upload")))
     return rc;
-  launch_adj_density64(c, c->adj_q);
+  launch_adj_density64(c, qfac);
   // the host buffers may be reused once this returns
   return hip_check(hipStreamSynchronize(c->stream), "adjoint density");
 }
@@ -1085,11 +1095,10 @@ int emg_adj_velocity_sums(emg_ctx *c, double *out) {
   int rc = need_adjoint(c);
   if (!rc) rc = need_particles(c);
   if (rc) return rc;
-  launch_adj_vsum(c, c->adj_sum);
-  rc = check_flags(c);
-  if (rc) return rc;
-  return hip_check(hipMemcpy(out, c->adj_sum, sizeof(double) * 3 * c->sp.nspec,
-                             hipMemcpyDeviceToHost), "adjoint sums copy");
+  launch_adj_vsum(c, c->adj_sum, c->hsum);
+  if ((rc = read_sums(c))) return rc;
+  for (int k = 0; k < 3 * c->sp.nspec; k++) out[k] = c->hsum[k];
+  return EMG_OK;
 }
 
 int emg_sort(emg_ctx *c) {
@@ -1125,7 +1134,7 @@ int emg_init_device(emg_ctx *c, const emg_device_species *spec, int32_t nspec, u
     if (!rc) rc = hip_check(hipStreamSynchronize(c->stream), "init");
     free_state64(tmp);
   }
-  if (!rc) rc = check_flags(c);
+  if (!rc) rc = read_flags(c);
   if (rc) {
     for (int s = 0; s < nspec; s++) c->sp.cnt[s] = 0;
     return rc;

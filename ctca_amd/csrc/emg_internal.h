@@ -5,6 +5,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
+#include <functional>
 #include <string>
 
 #include "emgpu.h"
@@ -100,6 +101,16 @@ struct Timer {
 };
 
 struct EsSolver;  // device field solve (k_poisson.hip)
+
+// Pinned transfer slots of the host read-outs and uploads (emg_io.hip).
+constexpr int kIoSlots = 8;
+struct HostIo {
+  char *pin;
+  size_t bytes, stride;
+  hipEvent_t ev[kIoSlots];
+  bool pending;  // enqueued work still uses the slots
+  bool open;     // counted among the process's contexts
+};
 
 // An LDS window of the FP64 deposits: nodes o .. o + w - 1 per axis (periodic),
 // w <= n, so no node appears twice.
@@ -389,7 +400,6 @@ struct emg_ctx {
   // energy
   double *ke_part;  // partial sums
   int64_t ke_part_n;
-  double *ke_out;   // [nspec * 3]
   bool ke_valid;
 
   // sort scratch
@@ -408,14 +418,15 @@ struct emg_ctx {
 
   int *dflag;       // device error flags
   int *hflag;       // pinned host mirror
+  double *hsum;     // pinned: energies and adjoint sums, written by their kernels
+  emg::HostIo io;
   double *scratch;  // this device's static staging array (emg_get_rho_noalloc)
 
   // adjoint window (FP64 form)
   double *lam;       // 8 per particle slot: lambda_x, lambda_v, 2 unused (one 64-byte line)
   double *adj_e;     // 3 x ncell: transposed gather of qmp * lambda_a
   double *adj_g;     // ncell: uploaded density adjoint
-  double *adj_q;     // nspec: its factor per species
-  double *adj_sum;   // velocity adjoint sums, then their block partials
+  double *adj_sum;   // block partials of the velocity adjoint sums
   emg::AdjBins adj_bins;
   emg::State64 slot[emg::kStateSlots];  // saved particle states
   int64_t slot_cnt[emg::kStateSlots][EMG_MAX_SPECIES];
@@ -429,6 +440,23 @@ namespace emg {
 // error plumbing (emg_api.hip)
 int set_error(int code, const std::string &msg);
 int hip_check(hipError_t e, const char *what);
+
+int flags_error(emg_ctx *c);  // *hflag as an error code (and dflag cleared)
+
+// Host transfers (emg_io.hip) in chunks of whole units.  fill enqueues on the
+// context's stream what writes bytes [off, off + len) of the result to the
+// pinned slot; io_read copies them to the caller's array and reports the
+// device-side errors first.  use enqueues what reads the slot; the caller's
+// array is free when io_write returns.  Both may call them from several
+// threads at once.
+using IoFn = std::function<int(size_t off, size_t len, void *slot)>;
+int io_read(emg_ctx *c, void *user, size_t bytes, size_t unit, const IoFn &fill);
+int io_write(emg_ctx *c, const void *user, size_t bytes, size_t unit, const IoFn &use);
+int read_flags(emg_ctx *c);  // synchronise and report device-side errors
+// a device array of 8-byte values
+int io_read_array(emg_ctx *c, void *user, const void *dev, size_t bytes);
+void io_open(emg_ctx *c);
+void io_close(emg_ctx *c);
 
 // timers
 void timer_begin(emg_ctx *c, int kind);
@@ -452,9 +480,10 @@ EbView eb_view(const emg_ctx *c);
 void launch_eb_split(emg_ctx *c);  // eb_stage -> eb_dev
 void launch_bfield(emg_ctx *c);
 void launch_efield(emg_ctx *c, double tcs, double dlt);
-void launch_eb_box(emg_ctx *c, const int lo[3], const int ext[3], double *out_dev);
+// points [o0, o0 + n) of the box lo .. lo + ext - 1 (x fastest), 6 values each
+void launch_eb_box(emg_ctx *c, const int lo[3], const int ext[3], int64_t o0, int64_t n, double *out);
 int64_t field_energy_part_need();
-void launch_field_energy(emg_ctx *c, double cs, double *part_dev, double *out_dev);
+void launch_field_energy(emg_ctx *c, double cs, double *part_dev, double *out);
 // device ES field solve (k_poisson.hip): rho of the last deposit + rhobk ->
 // phi -> E into eb_dev -> nodes
 int solve_es(emg_ctx *c, double rhobk);
@@ -462,9 +491,15 @@ int read_potential(emg_ctx *c, double *phi);
 void es_solver_free(emg_ctx *c);
 
 // common kernels (k_common.hip)
+// energy sums (3 per species) into hsum, and the device flags into hflag
 void launch_energy64(emg_ctx *c);
-void launch_read_rho(emg_ctx *c, int species, double *dst_dev, const int lo[3], const int hi[3]);
-void launch_read_current(emg_ctx *c, int species, double *dst_dev, const int lo[3], const int hi[3]);
+// points [o0, o0 + n) of a read-out of lo..hi into dst; prepare_read_rho first:
+// true if the box holds ghost planes, whose charge it then deposits
+bool prepare_read_rho(emg_ctx *c, const int lo[3], const int hi[3]);
+void launch_read_rho(emg_ctx *c, int species, bool ghosts, double *dst, const int lo[3],
+                     const int hi[3], int64_t o0, int64_t n);
+void launch_read_current(emg_ctx *c, int species, double *dst, const int lo[3], const int hi[3],
+                         int64_t o0, int64_t n);
 void launch_zero(void *p, size_t bytes, hipStream_t s);
 // The FP64 cell sort.  sort64 sorts the live state.  A re-sort close to the
 // last sort can ride on the next push instead: sort64_rank counts the
@@ -482,8 +517,8 @@ int init_device(emg_ctx *c, const emg_device_species *spec, int nspec, uint64_t 
 // adjoint of the FP64 ES push (k_adj.hip)
 int adj_bins_alloc(emg_ctx *c);
 void launch_adj_step64(emg_ctx *c, int ustep);  // after adj_bins_alloc
-void launch_adj_density64(emg_ctx *c, const double *qfac_dev);
-void launch_adj_vsum(emg_ctx *c, double *out_dev);  // out_dev: adj_vsum_need() doubles
+void launch_adj_density64(emg_ctx *c, const double *qfac);  // one factor per species
+void launch_adj_vsum(emg_ctx *c, double *part, double *out);  // part: adj_vsum_need() doubles
 int64_t adj_vsum_need();
 
 // FP32 + fixed point (k_fx.hip)

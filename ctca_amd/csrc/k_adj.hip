@@ -304,13 +304,16 @@ __global__ __launch_bounds__(kAdjBlock) void k_adj_step64(double *__restrict__ l
   }
 }
 
+struct SpeciesFactors {
+  double v[EMG_MAX_SPECIES];
+};
+
 // lambda_x += qfac[is] * grad g(x) for the trilinear interpolant of the
 // periodic nodal scalar g (the adjoint of the particle's CIC charge)
 __global__ __launch_bounds__(kBlock) void k_adj_density64(State64 s, double *__restrict__ lam, SpeciesTab sp,
-                                                         Grid g, const double *__restrict__ gn,
-                                                         const double *__restrict__ qfac) {
+                                                         Grid g, const double *__restrict__ gn, SpeciesFactors qfac) {
   int is = blockIdx.y;
-  double f = qfac[is];
+  double f = qfac.v[is];
   if (f == 0.0) return;
   int64_t m = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (m >= sp.cnt[is]) return;
@@ -371,8 +374,10 @@ __global__ __launch_bounds__(kBlock) void k_adj_vsum(const double *__restrict__ 
   vsum_block(v, part + 3 * ((int64_t)is * kVsumBlocks + blockIdx.x));
 }
 
-__global__ __launch_bounds__(kBlock) void k_adj_vsum_final(const double *part, double *out) {
+__global__ __launch_bounds__(kBlock) void k_adj_vsum_final(const double *part, double *out,
+                                                          const int *dflag, int *hflag) {
   const int is = blockIdx.x;
+  if (is == 0 && threadIdx.x == 0) *hflag = *dflag;
   double v[3] = {0.0, 0.0, 0.0};
   for (int k = threadIdx.x; k < kVsumBlocks; k += kBlock)
     for (int d = 0; d < 3; d++) v[d] += part[3 * ((int64_t)is * kVsumBlocks + k) + d];
@@ -479,18 +484,20 @@ void launch_adj_step64(emg_ctx *c, int ustep) {
   }
 }
 
-void launch_adj_density64(emg_ctx *c, const double *qfac_dev) {
+void launch_adj_density64(emg_ctx *c, const double *qfac) {
+  SpeciesFactors f{};
+  for (int s = 0; s < c->sp.nspec; s++) f.v[s] = qfac[s];
   hipLaunchKernelGGL(k_adj_density64, species_blocks(c->sp), dim3(kBlock), 0, c->stream, c->s64,
-                     c->lam, c->sp, c->g, c->adj_g, qfac_dev);
+                     c->lam, c->sp, c->g, c->adj_g, f);
 }
 
-void launch_adj_vsum(emg_ctx *c, double *out_dev) {
+void launch_adj_vsum(emg_ctx *c, double *part, double *out) {
   hipLaunchKernelGGL(k_adj_vsum, dim3(kVsumBlocks, c->sp.nspec), dim3(kBlock), 0, c->stream, c->lam,
-                     c->sp, out_dev + 3 * EMG_MAX_SPECIES);
-  hipLaunchKernelGGL(k_adj_vsum_final, dim3(c->sp.nspec), dim3(kBlock), 0, c->stream,
-                     out_dev + 3 * EMG_MAX_SPECIES, out_dev);
+                     c->sp, part);
+  hipLaunchKernelGGL(k_adj_vsum_final, dim3(c->sp.nspec), dim3(kBlock), 0, c->stream, part, out,
+                     c->dflag, c->hflag);
 }
 
-int64_t adj_vsum_need() { return 3 * EMG_MAX_SPECIES * (1 + kVsumBlocks); }
+int64_t adj_vsum_need() { return (int64_t)3 * EMG_MAX_SPECIES * kVsumBlocks; }
 
 }  // namespace emg

@@ -135,8 +135,10 @@ __global__ __launch_bounds__(kBlock) void k_energy64_part(State64 s, SpeciesTab 
     part[3 * ((int64_t)is * gridDim.x + blockIdx.x) + threadIdx.x] = red[threadIdx.x][0];
 }
 
-__global__ __launch_bounds__(kBlock) void k_energy64_final(const double *part, int nblk, double *out) {
+__global__ __launch_bounds__(kBlock) void k_energy64_final(const double *part, int nblk, double *out,
+                                                          const int *dflag, int *hflag) {
   int is = blockIdx.x;
+  if (is == 0 && threadIdx.x == 0) *hflag = *dflag;
   __shared__ double red[3][kBlock];
   double a[3] = {0.0, 0.0, 0.0};
   for (int k = threadIdx.x; k < nblk; k += kBlock)
@@ -152,11 +154,6 @@ __global__ __launch_bounds__(kBlock) void k_energy64_final(const double *part, i
 }
 
 // ---------------------------------------------------------------- read-out
-__device__ __forceinline__ int pmod(int i, int n) {
-  int r = i % n;
-  return r < 0 ? r + n : r;
-}
-
 struct ReadArgs {
   Grid g;
   int nspec;
@@ -164,6 +161,18 @@ struct ReadArgs {
   double q[EMG_MAX_SPECIES];
   int lo[3], ext[3];
   int64_t ncell;
+  int64_t o0, n;  // the points written: [o0, o0 + n) of the box, x fastest
+  __device__ __forceinline__ bool point(int64_t &o, int &i, int &j, int &k, int64_t &c) const {
+    o = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+    if (o >= n) return false;
+    point_of(o0 + o, ext[0], ext[1], i, j, k);
+    i += lo[0];
+    j += lo[1];
+    k += lo[2];
+    c = ((int64_t)periodic_index(k, g.nz) * g.ny + periodic_index(j, g.ny)) * g.nx +
+        periodic_index(i, g.nx);
+    return true;
+  }
 };
 
 // The raw (unfolded) deposit of species accumulator P at node (a, b, c), a in
@@ -229,12 +238,9 @@ __device__ __forceinline__ bool ghost_node(const ReadArgs &r, int i, int j, int 
 __global__ __launch_bounds__(kBlock) void k_read_rho64(ReadArgs r, const double *rho,
                                                       const double *face, int64_t nf,
                                                       double *out) {
-  int64_t n = (int64_t)r.ext[0] * r.ext[1] * r.ext[2];
-  int64_t o = (int64_t)blockIdx.x * kBlock + threadIdx.x;
-  if (o >= n) return;
-  int i = (int)(o % r.ext[0]) + r.lo[0];
-  int j = (int)((o / r.ext[0]) % r.ext[1]) + r.lo[1];
-  int k = (int)(o / ((int64_t)r.ext[0] * r.ext[1])) + r.lo[2];
+  int64_t o, c;
+  int i, j, k;
+  if (!r.point(o, i, j, k, c)) return;
   double v = 0.0;
   if (face && ghost_node(r, i, j, k)) {
     for (int s = 0; s < r.nspec; s++) {
@@ -244,7 +250,6 @@ __global__ __launch_bounds__(kBlock) void k_read_rho64(ReadArgs r, const double 
     out[o] = v;
     return;
   }
-  int64_t c = ((int64_t)pmod(k, r.g.nz) * r.g.ny + pmod(j, r.g.ny)) * r.g.nx + pmod(i, r.g.nx);
   if (r.species >= 0) {
     v = rho[(int64_t)r.species * r.ncell + c];
   } else {
@@ -256,14 +261,10 @@ __global__ __launch_bounds__(kBlock) void k_read_rho64(ReadArgs r, const double 
 __global__ __launch_bounds__(kBlock) void k_read_rhofx(ReadArgs r, const unsigned long long *rho,
                                                       const unsigned long long *face, int64_t nf,
                                                       double *out) {
-  int64_t n = (int64_t)r.ext[0] * r.ext[1] * r.ext[2];
-  int64_t o = (int64_t)blockIdx.x * kBlock + threadIdx.x;
-  if (o >= n) return;
-  int i = (int)(o % r.ext[0]) + r.lo[0];
-  int j = (int)((o / r.ext[0]) % r.ext[1]) + r.lo[1];
-  int k = (int)(o / ((int64_t)r.ext[0] * r.ext[1])) + r.lo[2];
+  int64_t o, c;
+  int i, j, k;
+  if (!r.point(o, i, j, k, c)) return;
   const bool ghost = face && ghost_node(r, i, j, k);
-  int64_t c = ((int64_t)pmod(k, r.g.nz) * r.g.ny + pmod(j, r.g.ny)) * r.g.nx + pmod(i, r.g.nx);
   double v = 0.0;
   for (int s = 0; s < r.nspec; s++) {
     if (r.species >= 0 && s != r.species) continue;
@@ -280,13 +281,9 @@ __global__ __launch_bounds__(kBlock) void k_read_rhofx(ReadArgs r, const unsigne
 // update that consumes the current)
 template <bool FIX>
 __global__ __launch_bounds__(kBlock) void k_read_current(ReadArgs r, const void *jacc, double *out) {
-  int64_t n = (int64_t)r.ext[0] * r.ext[1] * r.ext[2];
-  int64_t o = (int64_t)blockIdx.x * kBlock + threadIdx.x;
-  if (o >= n) return;
-  int i = (int)(o % r.ext[0]) + r.lo[0];
-  int j = (int)((o / r.ext[0]) % r.ext[1]) + r.lo[1];
-  int k = (int)(o / ((int64_t)r.ext[0] * r.ext[1])) + r.lo[2];
-  int64_t c = ((int64_t)pmod(k, r.g.nz) * r.g.ny + pmod(j, r.g.ny)) * r.g.nx + pmod(i, r.g.nx);
+  int64_t o, c;
+  int i, j, k;
+  if (!r.point(o, i, j, k, c)) return;
   for (int d = 0; d < 3; d++) {
     double v = 0.0;
     for (int s = 0; s < r.nspec; s++) {
@@ -581,13 +578,14 @@ void launch_energy64(emg_ctx *c) {
   hipLaunchKernelGGL(k_energy64_part, dim3(kEnergyBlocks, c->sp.nspec), dim3(kBlock), 0, c->stream,
                      c->s64, c->sp, c->ke_part);
   hipLaunchKernelGGL(k_energy64_final, dim3(c->sp.nspec), dim3(kBlock), 0, c->stream, c->ke_part,
-                     kEnergyBlocks, c->ke_out);
+                     kEnergyBlocks, c->hsum, c->dflag, c->hflag);
   timer_end(c, kTEnergy);
 }
 
 int64_t energy64_part_need(int nspec) { return (int64_t)kEnergyBlocks * nspec * 3; }
 
-static ReadArgs read_args(emg_ctx *c, int species, const int lo[3], const int hi[3]) {
+static ReadArgs read_args(emg_ctx *c, int species, const int lo[3], const int hi[3], int64_t o0,
+                          int64_t n) {
   ReadArgs r;
   r.g = c->g;
   r.nspec = c->sp.nspec;
@@ -598,15 +596,14 @@ static ReadArgs read_args(emg_ctx *c, int species, const int lo[3], const int hi
     r.ext[d] = hi[d] - lo[d] + 1;
   }
   r.ncell = c->ncell;
+  r.o0 = o0;
+  r.n = n;
   return r;
 }
 
-void launch_read_rho(emg_ctx *c, int species, double *dst, const int lo[3], const int hi[3]) {
-  ReadArgs r = read_args(c, species, lo, hi);
-  int64_t n = (int64_t)r.ext[0] * r.ext[1] * r.ext[2];
-  unsigned grid = (unsigned)((n + kBlock - 1) / kBlock);
-  // the reference's ghost planes need the upper-face deposit of the current
-  // positions: computed once per deposit, when a read-out first asks for them
+// the reference's ghost planes need the upper-face deposit of the current
+// positions: computed once per deposit, when a read-out first asks for them
+bool prepare_read_rho(emg_ctx *c, const int lo[3], const int hi[3]) {
   bool ghosts = false;
   for (int d = 0; d < 3; d++) {
     const int nd = d == 0 ? c->g.nx : (d == 1 ? c->g.ny : c->g.nz);
@@ -619,6 +616,13 @@ void launch_read_rho(emg_ctx *c, int species, double *dst, const int lo[3], cons
       launch_fx_faces(c);
     c->faces_valid = true;
   }
+  return ghosts;
+}
+
+void launch_read_rho(emg_ctx *c, int species, bool ghosts, double *dst, const int lo[3],
+                     const int hi[3], int64_t o0, int64_t n) {
+  const ReadArgs r = read_args(c, species, lo, hi, o0, n);
+  const unsigned grid = (unsigned)((n + kBlock - 1) / kBlock);
   const int64_t nf = face_len(c->g);
   if (c->cfg.precision == EMG_PLAIN_FP64)
     hipLaunchKernelGGL(k_read_rho64, dim3(grid), dim3(kBlock), 0, c->stream, r, c->rho64,
@@ -628,10 +632,10 @@ void launch_read_rho(emg_ctx *c, int species, double *dst, const int lo[3], cons
                        ghosts ? (const unsigned long long *)c->face : nullptr, nf, dst);
 }
 
-void launch_read_current(emg_ctx *c, int species, double *dst, const int lo[3], const int hi[3]) {
-  ReadArgs r = read_args(c, species, lo, hi);
-  int64_t n = (int64_t)r.ext[0] * r.ext[1] * r.ext[2];
-  unsigned grid = (unsigned)((n + kBlock - 1) / kBlock);
+void launch_read_current(emg_ctx *c, int species, double *dst, const int lo[3], const int hi[3],
+                         int64_t o0, int64_t n) {
+  const ReadArgs r = read_args(c, species, lo, hi, o0, n);
+  const unsigned grid = (unsigned)((n + kBlock - 1) / kBlock);
   if (c->cfg.precision == EMG_PLAIN_FP64)
     hipLaunchKernelGGL(k_read_current<false>, dim3(grid), dim3(kBlock), 0, c->stream, r,
                        (const void *)c->j64, dst);

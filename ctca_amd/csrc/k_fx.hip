@@ -1538,9 +1538,10 @@ __global__ __launch_bounds__(kBlock) void k_fx_to64(StateFx in, const int64_t *b
 // per-species sum of block partials in a fixed order; partials are indexed by
 // bucket (s * ntiles + t) followed by spill_blocks_per_s entries per species
 __global__ void k_ke_final(const double *part, int ntiles, int nb, int spill_blocks_per_s,
-                           double *out) {
+                           double *out, const int *dflag, int *hflag) {
   __shared__ double red[3][kBlock];
   int s = blockIdx.x;
+  if (s == 0 && threadIdx.x == 0) *hflag = *dflag;
   double v[3] = {0.0, 0.0, 0.0};
   for (int k = threadIdx.x; k < ntiles; k += kBlock)
     for (int d = 0; d < 3; d++) v[d] += part[3 * ((int64_t)s * ntiles + k) + d];
@@ -1931,7 +1932,7 @@ void launch_fx_energy(emg_ctx *c) {
   timer_begin(c, kTEnergy);
   hipLaunchKernelGGL(k_fx_energy, dim3(B.nb + c->sp.nspec), dim3(kBlock), 0, c->stream, a);
   hipLaunchKernelGGL(k_ke_final, dim3(c->sp.nspec), dim3(kBlock), 0, c->stream, c->ke_part,
-                     B.ntiles, B.nb, 1, c->ke_out);
+                     B.ntiles, B.nb, 1, c->hsum, c->dflag, c->hflag);
   timer_end(c, kTEnergy);
 }
 
@@ -1957,7 +1958,7 @@ void launch_fx_faces(emg_ctx *c) {
 void fx_energy_from_push(emg_ctx *c) {
   FxBuckets &B = c->fx;
   hipLaunchKernelGGL(k_ke_final, dim3(c->sp.nspec), dim3(kBlock), 0, c->stream, c->ke_part,
-                     B.ntiles, B.nb, 0, c->ke_out);
+                     B.ntiles, B.nb, 0, c->hsum, c->dflag, c->hflag);
 }
 
 }  // namespace emg

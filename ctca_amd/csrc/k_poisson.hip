@@ -205,11 +205,7 @@ int solve_es(emg_ctx *c, double rhobk) {
 
 int read_potential(emg_ctx *c, double *phi) {
   if (!c->es) return set_error(EMG_ERR_STATE, "no field solve yet");
-  int rc = hip_check(hipStreamSynchronize(c->stream), "stream synchronize");
-  if (!rc)
-    rc = hip_check(hipMemcpy(phi, c->es->rho, sizeof(double) * c->ncell, hipMemcpyDeviceToHost),
-                   "potential copy");
-  return rc;
+  return io_read_array(c, phi, c->es->rho, sizeof(double) * c->ncell);
 }
 
 }  // namespace emg

@@ -105,7 +105,7 @@ __global__ __launch_bounds__(kBlock) void k_efield(EbView v, CurrentView J, doub
 }
 
 // sum E^2 and B^2 over the cells 0..n-1: per-block partials, then one block
-// adds them in block order (deterministic)
+// adds them in a tree (deterministic)
 constexpr int kFeBlocks = 256;
 
 __global__ __launch_bounds__(kBlock) void k_field_energy_part(EbView v, double *part) {
@@ -139,26 +139,35 @@ __global__ __launch_bounds__(kBlock) void k_field_energy_part(EbView v, double *
   }
 }
 
-__global__ void k_field_energy_final(const double *part, double cs, double vol, double *out) {
-  if (threadIdx.x != 0) return;
-  double te = 0.0, tb = 0.0;
-  for (int b = 0; b < kFeBlocks; b++) {
-    te += part[2 * b];
-    tb += part[2 * b + 1];
+__global__ __launch_bounds__(kFeBlocks) void k_field_energy_final(const double *part, double cs,
+                                                                  double vol, double *out,
+                                                                  const int *dflag, int *hflag) {
+  __shared__ double red[2][kFeBlocks];
+  red[0][threadIdx.x] = part[2 * threadIdx.x];
+  red[1][threadIdx.x] = part[2 * threadIdx.x + 1];
+  __syncthreads();
+  for (int o = kFeBlocks / 2; o > 0; o >>= 1) {
+    if (threadIdx.x < (unsigned)o) {
+      red[0][threadIdx.x] += red[0][threadIdx.x + o];
+      red[1][threadIdx.x] += red[1][threadIdx.x + o];
+    }
+    __syncthreads();
   }
-  out[0] = 0.5 * te / vol;
-  out[1] = 0.5 * cs * tb / vol;
+  if (threadIdx.x == 0) {
+    out[0] = 0.5 * red[0][0] / vol;
+    out[1] = 0.5 * cs * red[1][0] / vol;
+    *hflag = *dflag;
+  }
 }
 
-// copy the box lo .. lo + ext - 1 of eb (inside the stored bounds) into a
-// dense out(6, box)
+// copy the points [o0, o0 + n) of the box lo .. lo + ext - 1 of eb (inside the
+// stored bounds) into records out(6, n)
 __global__ __launch_bounds__(kBlock) void k_eb_box(EbView v, int lx, int ly, int lz, int ex, int ey,
-                                                   int ez, double *out) {
-  const int64_t n = (int64_t)ex * ey * ez;
+                                                   int64_t o0, int64_t n, double *out) {
   const int64_t o = (int64_t)blockIdx.x * kBlock + threadIdx.x;
   if (o >= n) return;
   int i, j, k;
-  point_of(o, ex, ey, i, j, k);
+  point_of(o0 + o, ex, ey, i, j, k);
   const double *p = v.eb + v.at(i + lx, j + ly, k + lz);
   double2 *d = reinterpret_cast<double2 *>(out + o * 6);
 #pragma unroll
@@ -210,21 +219,20 @@ void launch_efield(emg_ctx *c, double tcs, double dlt) {
                        dlt);
 }
 
-void launch_eb_box(emg_ctx *c, const int lo[3], const int ext[3], double *out_dev) {
-  const EbView v = eb_view(c);
-  const int64_t n = (int64_t)ext[0] * ext[1] * ext[2];
+void launch_eb_box(emg_ctx *c, const int lo[3], const int ext[3], int64_t o0, int64_t n,
+                   double *out) {
   hipLaunchKernelGGL(k_eb_box, dim3((unsigned)((n + kBlock - 1) / kBlock)), dim3(kBlock), 0,
-                     c->stream, v, lo[0], lo[1], lo[2], ext[0], ext[1], ext[2], out_dev);
+                     c->stream, eb_view(c), lo[0], lo[1], lo[2], ext[0], ext[1], o0, n, out);
 }
 
 int64_t field_energy_part_need() { return 2 * kFeBlocks; }
 
-void launch_field_energy(emg_ctx *c, double cs, double *part_dev, double *out_dev) {
+void launch_field_energy(emg_ctx *c, double cs, double *part_dev, double *out) {
   const EbView v = eb_view(c);
   hipLaunchKernelGGL(k_field_energy_part, dim3(kFeBlocks), dim3(kBlock), 0, c->stream, v, part_dev);
   const double vol = (double)c->g.slx * c->g.sly * c->g.slz;
-  hipLaunchKernelGGL(k_field_energy_final, dim3(1), dim3(64), 0, c->stream, part_dev, cs, vol,
-                     out_dev);
+  hipLaunchKernelGGL(k_field_energy_final, dim3(1), dim3(kFeBlocks), 0, c->stream, part_dev, cs,
+                     vol, out, c->dflag, c->hflag);
 }
 
 }  // namespace emg

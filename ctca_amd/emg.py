@@ -227,7 +227,7 @@ class Context:
 
     def download(self):
         cnt = self.counts()
-        out = np.zeros(int(cnt.sum()), dtype=PARTICLE)
+        out = np.empty(int(cnt.sum()), dtype=PARTICLE)
         cnt2 = np.zeros(self.nspec, dtype=np.int64)
         _chk(lib().emg_download_particles(self.h, _ptr(out), _ptr(cnt2)))
         return out, cnt2
@@ -286,11 +286,11 @@ class Context:
         self.deposit_rho(func)
         lo, hi = (-1, -1, -1), tuple(v + 1 for v in self.n)
         if func in (0, 2):
-            rho[...] = self.rho(lo, hi)
+            self._rho_into(rho, lo, hi, None)
         if func in (1, 2):
-            rhodg[...] = 0.0
+            rhodg[self.nspec:] = 0.0
             for k in range(self.nspec):
-                rhodg[k] = self.rho(lo, hi, species=k)
+                self._rho_into(rhodg[k], lo, hi, k)
 
     def push_em(self, ustep):
         _chk(lib().emg_push_em(self.h, int(ustep)))
@@ -310,7 +310,7 @@ class Context:
         for an eb of the usual extent -1..n+1."""
         if hi is None:
             hi = tuple(v + 1 for v in self.n)
-        out = np.zeros((hi[2] - lo[2] + 1, hi[1] - lo[1] + 1, hi[0] - lo[0] + 1, 6))
+        out = np.empty((hi[2] - lo[2] + 1, hi[1] - lo[1] + 1, hi[0] - lo[0] + 1, 6))
         _chk(lib().emg_get_fields(self.h, _ptr(out), _i3(lo), _i3(hi)))
         return out
 
@@ -331,12 +331,12 @@ class Context:
 
     def potential(self):
         """phi of the last device field solve, numpy [k, j, i]."""
-        out = np.zeros((self.n[2], self.n[1], self.n[0]))
+        out = np.empty((self.n[2], self.n[1], self.n[0]))
         _chk(lib().emg_get_potential(self.h, _ptr(out)))
         return out
 
     def field_energy(self, cs):
-        out = np.zeros(2)
+        out = np.empty(2)
         _chk(lib().emg_field_energy(self.h, float(cs), _ptr(out)))
         return out
 
@@ -356,18 +356,29 @@ class Context:
     def rho(self, lo=None, hi=None, species=None):
         """rho(1, lo:hi)^3 as numpy [k, j, i]; default: the periodic nodes 0..n-1."""
         lo, hi = self._bounds(lo, hi)
-        out = np.zeros((hi[2] - lo[2] + 1, hi[1] - lo[1] + 1, hi[0] - lo[0] + 1))
+        out = np.empty((hi[2] - lo[2] + 1, hi[1] - lo[1] + 1, hi[0] - lo[0] + 1))
         if species is None:
             _chk(lib().emg_get_rho(self.h, _ptr(out), _i3(lo), _i3(hi)))
         else:
             _chk(lib().emg_get_rhodg(self.h, int(species), _ptr(out), _i3(lo), _i3(hi)))
         return out
 
+    def _rho_into(self, dst, lo, hi, species):
+        """rho(lo, hi, species) written into dst, directly where dst's memory
+        is what the library writes."""
+        if dst.dtype == np.float64 and dst.flags.c_contiguous and dst.flags.writeable:
+            if species is None:
+                _chk(lib().emg_get_rho(self.h, _ptr(dst), _i3(lo), _i3(hi)))
+            else:
+                _chk(lib().emg_get_rhodg(self.h, int(species), _ptr(dst), _i3(lo), _i3(hi)))
+        else:
+            dst[...] = self.rho(lo, hi, species)
+
     def rho_noalloc(self, lo=None, hi=None):
         """rho(1, lo:hi)^3 like rho(), read through emg_get_rho_noalloc (no
         device allocation: the library's static staging array)."""
         lo, hi = self._bounds(lo, hi)
-        out = np.zeros((hi[2] - lo[2] + 1, hi[1] - lo[1] + 1, hi[0] - lo[0] + 1))
+        out = np.empty((hi[2] - lo[2] + 1, hi[1] - lo[1] + 1, hi[0] - lo[0] + 1))
         _chk(lib().emg_get_rho_noalloc(self.h, _ptr(out), _i3(lo), _i3(hi)))
         return out
 
@@ -375,7 +386,7 @@ class Context:
         """aj(3, lo:hi)^3 as numpy [k, j, i, 3]; with species, that species'
         ajdg alone."""
         lo, hi = self._bounds(lo, hi)
-        out = np.zeros((hi[2] - lo[2] + 1, hi[1] - lo[1] + 1, hi[0] - lo[0] + 1, 3))
+        out = np.empty((hi[2] - lo[2] + 1, hi[1] - lo[1] + 1, hi[0] - lo[0] + 1, 3))
         if species is None:
             _chk(lib().emg_get_current(self.h, _ptr(out), _i3(lo), _i3(hi)))
         else:
@@ -383,7 +394,7 @@ class Context:
         return out
 
     def energy(self):
-        out = np.zeros(3 * self.nspec)
+        out = np.empty(3 * self.nspec)
         _chk(lib().emg_energy(self.h, _ptr(out)))
         return out.reshape(self.nspec, 3)
 
@@ -402,7 +413,7 @@ class Context:
 
     def adj_field(self):
         """Adjoint of the nodal E: numpy [k, j, i, 3], periodic nodes 0..n-1."""
-        out = np.zeros((self.n[2], self.n[1], self.n[0], 3))
+        out = np.empty((self.n[2], self.n[1], self.n[0], 3))
         _chk(lib().emg_adj_get_field(self.h, _ptr(out)))
         return out
 
@@ -414,7 +425,7 @@ class Context:
         _chk(lib().emg_adj_add_density(self.h, _ptr(g), _ptr(q)))
 
     def adj_velocity_sums(self):
-        out = np.zeros(3 * self.nspec)
+        out = np.empty(3 * self.nspec)
         _chk(lib().emg_adj_velocity_sums(self.h, _ptr(out)))
         return out.reshape(self.nspec, 3)
 
