@@ -804,7 +804,7 @@ static int sort_if_due(emg_ctx *c, int which, bool *carry = nullptr) {
     rc = emg::sort64_rank(c, which);
     if (!rc) *carry = true;
   } else {
-    rc = sort64(c);
+    rc = sort64(c, true);
   }
   if (!rc) c->pushes_since_sort = 1;
   return rc;
@@ -1106,7 +1106,7 @@ int emg_sort(emg_ctx *c) {
   int rc = need_particles(c);
   if (rc) return rc;
   if (c->cfg.precision == EMG_PLAIN_FP64) {
-    rc = sort64(c);
+    rc = sort64(c, false);
     for (int k = 0; k < 2 && !rc; k++) rc = sort64_runs(c, k);
     if (!rc) c->pushes_since_sort = 0;
   } else {

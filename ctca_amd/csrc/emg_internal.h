@@ -126,9 +126,14 @@ struct Cell3 {
 struct WinShape {
   int cap, fx, fy, fz;
 };
-constexpr WinShape kWinEs{3840, 80, 8, 6};  // the charge: 30 KB of int64
-constexpr WinShape kWinEm{1600, 40, 8, 5};  // per component of the current: 3 x 12.8 KB
-static_assert(kWinEs.cap % 2 == 0 && kWinEm.cap % 2 == 0, "cleared two entries at a time");
+// of table 0 (the charge) and 1 (each component of the current), for runs of
+// rows or of particles in no order (30 and 3 x 12.8 KB of int64), and for
+// patches (12 and 3 x 8 KB: the same margins, two or three nodes)
+constexpr WinShape kWinRow[2] = {{3840, 80, 8, 6}, {1600, 40, 8, 5}};
+constexpr int kWinPatch[2] = {1536, 1024};
+constexpr int kFieldCap = 484;  // field nodes staged by a patch's block: 11 x 11 x 4, 23 KB
+static_assert(kWinRow[0].cap % 2 == 0 && kWinRow[1].cap % 2 == 0 && kWinPatch[0] % 2 == 0 &&
+                  kWinPatch[1] % 2 == 0, "cleared two entries at a time");
 
 // widen one axis of a window by a node on each side (or to the whole axis) if
 // its nodes, times `across` of the other axes, stay within cap
@@ -144,7 +149,48 @@ __host__ __device__ inline bool win_grow(int32_t &o, int32_t &w, int n, int acro
   return true;
 }
 
-// The window of a run from cell a to cell b (in the sort order; mid: its middle
+// margins while they fit: z, y, x in turn
+__host__ __device__ inline void win_margins(Win &w, const Grid &g, int cap) {
+  bool grown = true;
+  while (grown) {
+    grown = win_grow(w.oz, w.wz, g.nz, w.wx * w.wy, cap);
+    grown = win_grow(w.oy, w.wy, g.ny, w.wx * w.wz, cap) || grown;
+    grown = win_grow(w.ox, w.wx, g.nx, w.wy * w.wz, cap) || grown;
+  }
+}
+
+// The window of the cells i .. i + ci - 1, j .. j + cj - 1 of layer k.
+__host__ __device__ inline Win patch_window(int i, int j, int k, int ci, int cj, const Grid &g,
+                                            int cap) {
+  Win w{ci + 1, cj + 1, 2, i, j, k};
+  if (w.wx >= g.nx) w.ox = 0, w.wx = g.nx;
+  if (w.wy >= g.ny) w.oy = 0, w.wy = g.ny;
+  if (w.wz >= g.nz) w.oz = 0, w.wz = g.nz;
+  win_margins(w, g, cap);
+  return w;
+}
+
+// The field nodes staged for the same cells: their own, and one more on each side
+// (in z only where that fits) within the nodes 0..n; one node, which serves no
+// cell, if even those of the cells are more than cap.
+__host__ __device__ inline Win patch_fields(int i, int j, int k, int ci, int cj, const Grid &g,
+                                            int cap) {
+  Win w{};
+  for (int m = 2; m >= 0; m--) {  // margins: x, y, z; x, y; none
+    const int mxy = m > 0 ? 1 : 0, mz = m > 1 ? 1 : 0;
+    w.ox = i - mxy < 0 ? 0 : i - mxy;
+    w.oy = j - mxy < 0 ? 0 : j - mxy;
+    w.oz = k - mz < 0 ? 0 : k - mz;
+    w.wx = (i + ci + mxy > g.nx ? g.nx : i + ci + mxy) - w.ox + 1;
+    w.wy = (j + cj + mxy > g.ny ? g.ny : j + cj + mxy) - w.oy + 1;
+    w.wz = (k + 1 + mz > g.nz ? g.nz : k + 1 + mz) - w.oz + 1;
+    if (w.wx * w.wy * w.wz <= cap) return w;
+  }
+  w.wx = w.wy = w.wz = 1;  // a single node: no cell has all its eight
+  return w;
+}
+
+// The window of a run of rows from cell a to cell b (in the sort order; mid: its middle
 // particle's cell).  The cells of a sorted run go from a to b in z-major order
 // (rows of the y-z plane one after another), so its nodes fit a box of its rows
 // plus one, its layers plus one, and in x the row segment it covers (or, for a
@@ -186,13 +232,8 @@ __host__ __device__ inline Win run_window(const Cell3 &a, const Cell3 &b, const 
     }
     boxed = (int64_t)w.wx * w.wy * w.wz <= ws.cap;
   }
-  if (boxed) {  // margins while they fit: z, y, x in turn
-    bool grown = true;
-    while (grown) {
-      grown = win_grow(w.oz, w.wz, g.nz, w.wx * w.wy, ws.cap);
-      grown = win_grow(w.oy, w.wy, g.ny, w.wx * w.wz, ws.cap) || grown;
-      grown = win_grow(w.ox, w.wx, g.nx, w.wy * w.wz, ws.cap) || grown;
-    }
+  if (boxed) {
+    win_margins(w, g, ws.cap);
   } else {
     w.wx = ws.fx < g.nx ? ws.fx : g.nx;
     w.wy = ws.fy < g.ny ? ws.fy : g.ny;
@@ -209,28 +250,46 @@ __host__ __device__ inline Win run_window(const Cell3 &a, const Cell3 &b, const 
 }
 
 // A block's run of the FP64 kernels after a sort: len consecutive particles
-// of species s from its segment's index beg.  Each species is cut into
-// blocks of `run` particles in the sort order (cells in z-major order); a
-// block whose particles span fewer than kRunSpan cells is one run, a longer
-// one (a sparse region) is cut into np = ceil(span / kRunCells) runs of
-// equal cell ranges, so that every run's LDS window covers its cells.  The
-// window is shaped here, from the run's cells, once per sort (shaped by every
-// block from its particles at every push, its loop was 70% of the scalar
+// of species s from its segment's index beg, and their LDS window.
+// After a re-sort in patches a run is a patch's particles, cut evenly where
+// they are more than kRunMax, or up to kPatchMerge patches of a sparse species.
+// After emg_sort each species is cut into blocks of kRunRow particles; a block
+// whose particles span fewer than kRunSpan cells is one run, a longer one (a
+// sparse region) is cut into np = ceil(span / kRunCells) runs of equal cell
+// ranges.  The windows are shaped with the table, once per sort (shaped by
+// every block from its particles at every push, the loop was 70% of the scalar
 // instructions of the zigzag push and 2-4 us of each block).
 struct Run {
   int64_t beg;
   int32_t len, s;
   Win w;
+  Win f;  // patches: the field nodes 0..n staged in LDS (not periodic)
 };
 
-// The FP64 sort key of a position: its cell in z-major order, each index the
-// int() of the coordinate clamped into the grid.
-__host__ __device__ inline int64_t slab_key_xyz(double x, double y, double z, const Grid &g) {
+// The FP64 sort orders, both by z layer first (what the reference's comparator
+// asks of spsort): emg_sort's, cells row by row; and that of the library's own
+// re-sorts (sort_every), whose layers are cut into patches of kPatch x kPatch
+// cells (less at the upper faces), row of patches by row of patches, and each
+// patch's cells row by row.  The particles of 64 consecutive cells then reach
+// 9 x 9 x 2 nodes instead of 65 x 2 x 2, and drift by less of their window.
+constexpr int kPatch = 8;
+
+__host__ __device__ inline int64_t sort_key(int i, int j, int k, const Grid &g, bool patched) {
+  if (!patched) return ((int64_t)k * g.ny + j) * g.nx + i;
+  const int pj = j / kPatch * kPatch, pi = i / kPatch * kPatch;
+  const int h = pj + kPatch <= g.ny ? kPatch : g.ny - pj, w = pi + kPatch <= g.nx ? kPatch : g.nx - pi;
+  return ((int64_t)k * g.ny + pj) * g.nx + (int64_t)pi * h + (j - pj) * w + (i - pi);
+}
+
+// The sort key of a position: of its cell, each index the int() of the
+// coordinate clamped into the grid.
+__host__ __device__ inline int64_t sort_key_xyz(double x, double y, double z, const Grid &g,
+                                                bool patched) {
   int k = (int)z, j = (int)y, i = (int)x;
   k = k < 0 ? 0 : (k >= g.nz ? g.nz - 1 : k);
   j = j < 0 ? 0 : (j >= g.ny ? g.ny - 1 : j);
   i = i < 0 ? 0 : (i >= g.nx ? g.nx - 1 : i);
-  return ((int64_t)k * g.ny + j) * g.nx + i;
+  return sort_key(i, j, k, g, patched);
 }
 
 // The active lanes of a wave grouped by equal key, one ballot per distinct
@@ -270,8 +329,12 @@ struct SortDest {
   int64_t nkey;
 };
 
-constexpr int kRunEs = 4096;   // particles per block of the charge / ES push kernels
-constexpr int kRunEm = 1024;   // of the zigzag push
+// particles per block of table 0 (charge, ES push) and 1 (zigzag push): of a run
+// of rows, or of a slice in no order; and at most of a patch, where a sum of
+// kRunMax fixed-point terms of a node still fits (2^48 each; 8 2^48 twice)
+constexpr int kRunRow[2] = {4096, 1024};
+constexpr int kRunMax[2] = {6144, 2304};
+constexpr int kPatchMerge = 4;
 constexpr int64_t kRunsUnbuilt = -1;
 constexpr int kRunSpan = 96;   // cells a block may span and stay whole
 constexpr int kRunCells = 64;  // cells per run of a cut block
@@ -408,11 +471,12 @@ struct emg_ctx {
   int64_t *sort_start;
   int64_t sort_len;
   void *sort_rec;        // cap_total x 64-byte records + cap_total int32 ranks (FP64 sort, lazy)
-  emg::Run *runs[2];     // block runs of the last sort: [0] kRunEs, [1] kRunEm particles
+  emg::Run *runs[2];     // block runs of the last sort: [0] charge, [1] zigzag
   int64_t nruns[2], runs_cap[2];  // (kRunsUnbuilt: not asked for since the last sort)
   int64_t *run_base;     // scan scratch of the run counts (nspec x chunks + 1)
   int64_t run_base_len;
   bool runs_valid;       // the particles are in the order of the sort the runs describe
+  bool sort_patched;     // the last sort's order: patches, or emg_sort's rows
   int64_t *scan_tmp;
   int64_t scan_tmp_len;
 
@@ -506,8 +570,8 @@ void launch_zero(void *p, size_t bytes, hipStream_t s);
 // current cells (each key's start, each particle's rank in its key), the
 // push writes every particle to its sorted slot (SortDest), and sort64_commit
 // makes that the live state and builds the blocks' run tables of it.
-int sort64(emg_ctx *c);
-int sort64_runs(emg_ctx *c, int which);  // the run table of kRunEs (0) or kRunEm (1)
+int sort64(emg_ctx *c, bool patched);
+int sort64_runs(emg_ctx *c, int which);  // the run table of the charge (0) or the zigzag (1)
 bool sort64_fusable(const emg_ctx *c);
 int sort64_rank(emg_ctx *c, int which);  // which: the run table of the push that follows
 SortDest sort64_dest(const emg_ctx *c);

@@ -304,8 +304,9 @@ __global__ __launch_bounds__(kBlock) void k_read_current(ReadArgs r, const void 
 // inside a slab the cells in order, so that the particles of a workgroup
 // gather from and deposit to a small box of nodes (the order inside a cell is
 // whatever the atomic cursors give).
-__device__ __forceinline__ int64_t slab_key(const State64 &s, int64_t m, const Grid &g) {
-  return slab_key_xyz(s.x[m], s.y[m], s.z[m], g);
+__device__ __forceinline__ int64_t slab_key(const State64 &s, int64_t m, const Grid &g,
+                                            bool patched) {
+  return sort_key_xyz(s.x[m], s.y[m], s.z[m], g, patched);
 }
 
 // count the particles of each key; the count a particle finds is its rank
@@ -318,12 +319,13 @@ __device__ __forceinline__ int64_t slab_key(const State64 &s, int64_t m, const G
 // themselves inside their group from the count it returns.  An input in no
 // known order (up to 64 keys per wave) takes one atomic per lane.
 __global__ __launch_bounds__(kBlock) void k_sort_hist(State64 s, SpeciesTab sp, Grid g, int64_t nkey,
-                                                      int32_t *count, int32_t *rank, bool grouped) {
+                                                      int32_t *count, int32_t *rank, bool grouped,
+                                                      bool patched) {
   const int is = blockIdx.y;
   const int64_t m = (int64_t)blockIdx.x * kBlock + threadIdx.x;
   const bool act = m < sp.cnt[is];  // the whole wave takes part in the ballots
   const int lane = __lane_id();
-  const int64_t key = act ? (int64_t)is * nkey + slab_key(s, m + sp.off[is], g) : -1;
+  const int64_t key = act ? (int64_t)is * nkey + slab_key(s, m + sp.off[is], g, patched) : -1;
   int lead = lane, inner = 0, size = 1;
   if (grouped) wave_groups(key, act, lead, inner, size);  // uniform over the grid
   int base = 0;
@@ -338,12 +340,13 @@ __global__ __launch_bounds__(kBlock) void k_sort_hist(State64 s, SpeciesTab sp, 
 // and a second, coalesced pass splits the records into the arrays.
 __global__ __launch_bounds__(kBlock) void k_sort_scatter(State64 s, uint4 *rec, SpeciesTab sp,
                                                          Grid g, int64_t nkey,
-                                                         const int64_t *start, const int32_t *rank) {
+                                                         const int64_t *start, const int32_t *rank,
+                                                         bool patched) {
   int is = blockIdx.y;
   int64_t m = (int64_t)blockIdx.x * kBlock + threadIdx.x;
   if (m >= sp.cnt[is]) return;
   m += sp.off[is];
-  int64_t key = (int64_t)is * nkey + slab_key(s, m, g);
+  int64_t key = (int64_t)is * nkey + slab_key(s, m, g, patched);
   int64_t d = sp.off[is] + (start[key] - start[(int64_t)is * nkey]) + rank[m];
   auto u2 = [](double a, double b) {
     const unsigned long long ia = (unsigned long long)__double_as_longlong(a),
@@ -363,7 +366,7 @@ __global__ __launch_bounds__(kBlock) void k_sort_scatter(State64 s, uint4 *rec, 
 __global__ __launch_bounds__(kBlock) void k_sort_scatter_direct(State64 s, State64 t, SpeciesTab sp,
                                                                 Grid g, int64_t nkey,
                                                                 const int64_t *start,
-                                                                const int32_t *rank) {
+                                                                const int32_t *rank, bool patched) {
   int is = blockIdx.y;
   int64_t m = (int64_t)blockIdx.x * kBlock + threadIdx.x;
   if (m >= sp.cnt[is]) return;
@@ -372,7 +375,7 @@ __global__ __launch_bounds__(kBlock) void k_sort_scatter_direct(State64 s, State
   // far as the compiler knows, so a load after a store would wait for it
   const double x = s.x[m], y = s.y[m], z = s.z[m], vx = s.vx[m], vy = s.vy[m], vz = s.vz[m];
   const int32_t pid = s.pid[m], rk = rank[m];
-  int64_t key = (int64_t)is * nkey + slab_key(s, m, g);
+  int64_t key = (int64_t)is * nkey + slab_key(s, m, g, patched);
   int64_t d = sp.off[is] + (start[key] - start[(int64_t)is * nkey]) + rk;
   t.x[d] = x;
   t.y[d] = y;
@@ -455,7 +458,64 @@ dim3 species_grid(const SpeciesTab &sp) {
 }
 
 
-// Block runs after a sort.  st(c) = start[s nkey + c] - start[s nkey] is
+// The runs of a species sorted in patches (see Run): group q of `merge` patches
+// of one row of patches holds the cells [key, key + cells) of the order.
+struct PatchGroups {
+  int merge[EMG_MAX_SPECIES];
+  int64_t n[EMG_MAX_SPECIES];  // groups per species
+};
+
+__device__ __forceinline__ int64_t patch_group(const Grid &g, int merge, int64_t q, int &i, int &j,
+                                               int &k, int &ci, int &cj) {
+  const int npx = (g.nx + kPatch - 1) / kPatch, npy = (g.ny + kPatch - 1) / kPatch;
+  const int ngx = (npx + merge - 1) / merge;
+  int gi, pj;
+  point_of(q, ngx, npy, gi, pj, k);
+  i = gi * merge * kPatch;
+  j = pj * kPatch;
+  ci = min(merge * kPatch, g.nx - i);
+  cj = min(kPatch, g.ny - j);
+  return ((int64_t)k * g.ny + j) * g.nx + (int64_t)i * cj;
+}
+
+__global__ void k_patch_count(const int64_t *start, int64_t nkey, Grid g, PatchGroups pg,
+                              int64_t most, int run, int32_t *nrun) {
+  const int s = blockIdx.y;
+  const int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (q >= most) return;
+  int32_t n = 0;
+  if (q < pg.n[s]) {
+    int i, j, k, ci, cj;
+    const int64_t key = s * nkey + patch_group(g, pg.merge[s], q, i, j, k, ci, cj);
+    n = (int32_t)((start[key + (int64_t)ci * cj] - start[key] + run - 1) / run);
+  }
+  nrun[s * most + q] = n;
+}
+
+__global__ void k_patch_fill(const int64_t *start, int64_t nkey, Grid g, PatchGroups pg,
+                             int64_t most, int run, const int64_t *base, Run *runs, int64_t cap,
+                             int wincap) {
+  const int s = blockIdx.y;
+  const int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (q >= pg.n[s]) return;
+  int i, j, k, ci, cj;
+  const int64_t key = s * nkey + patch_group(g, pg.merge[s], q, i, j, k, ci, cj);
+  const int64_t p0 = start[key] - start[s * nkey],
+                cnt = start[key + (int64_t)ci * cj] - start[key], np = (cnt + run - 1) / run;
+  if (np == 0) return;
+  Run r;
+  r.s = s;
+  r.w = patch_window(i, j, k, ci, cj, g, wincap);
+  r.f = patch_fields(i, j, k, ci, cj, g, kFieldCap);
+  const int64_t at = base[s * most + q];
+  for (int64_t t = 0; t < np; t++) {
+    r.beg = p0 + cnt * t / np;
+    r.len = (int32_t)(p0 + cnt * (t + 1) / np - r.beg);
+    if (at + t < cap) runs[at + t] = r;
+  }
+}
+
+// Block runs after a sort by rows.  st(c) = start[s nkey + c] - start[s nkey] is
 // the index (in the species' segment) of the first particle of cell c.
 struct RunCut {
   const int64_t *st;  // start + s nkey
@@ -539,6 +599,7 @@ __global__ void k_run_fill(const int64_t *start, int64_t nkey, SpeciesTab sp, in
       point_of(k, g.nx, g.ny, c.i, c.j, c.k);
       return c;
     };
+    r.f = Win{};
     r.w = run_window(cell(c0), cell(c1), cell((c0 + c1) / 2), g, ws);
     if (at < cap) runs[at] = r;
     at++;
@@ -697,19 +758,21 @@ int sort64_alloc(emg_ctx *c) {
 
 // the sort's keys and ranks: count each key's particles (a particle's rank
 // is the count it finds) and scan the counts into each key's start
-int sort64_count(emg_ctx *c) {
+int sort64_count(emg_ctx *c, bool patched) {
   const int64_t nkey = c->ncell;
   const int64_t len = nkey * c->sp.nspec;
   launch_zero(c->sort_count, sizeof(int32_t) * len, c->stream);
   hipLaunchKernelGGL(k_sort_hist, species_grid(c->sp), dim3(kBlock), 0, c->stream, c->s64, c->sp,
-                     c->g, nkey, c->sort_count, rank_buf(c), c->moves_after_sort <= kResortDirect);
+                     c->g, nkey, c->sort_count, rank_buf(c), c->moves_after_sort <= kResortDirect,
+                     patched);
   exclusive_scan_i32(c->sort_count, c->sort_start, len, c->scan_tmp, c->stream);
   return hip_check(hipGetLastError(), "sort");
 }
 
 // the sorted order (in t64) becomes the live state; its run tables are built
 // when a kernel first asks for one (sort64_runs)
-int sort64_swap(emg_ctx *c) {
+int sort64_swap(emg_ctx *c, bool patched) {
+  c->sort_patched = patched;
   c->moves_after_sort = 0;
   State64 tmp = c->s64;
   c->s64 = c->t64;
@@ -725,14 +788,39 @@ int build_runs(emg_ctx *c, int which) {
   const int64_t nkey = c->ncell;
   const int64_t len = nkey * c->sp.nspec;
   c->nruns[which] = 0;
-  int64_t mx = 1;
-  for (int q = 0; q < c->sp.nspec; q++) mx = c->sp.cnt[q] > mx ? c->sp.cnt[q] : mx;
-  const int run = which == 0 ? kRunEs : kRunEm;
-  const int64_t nbmax = (mx + run - 1) / run;
+  const bool patched = c->sort_patched;
+  const int run = patched ? kRunMax[which] : kRunRow[which];
+  // table entries per species before cutting (nbmax), and the runs they can
+  // become (cap)
+  int64_t nbmax, cap;
+  PatchGroups pg{};
+  if (patched) {
+    // sparse patches are merged, to 256 particles on average if kPatchMerge do
+    nbmax = 1;
+    cap = 1;
+    for (int s = 0; s < c->sp.nspec; s++) {
+      int m = 1;
+      while (m < kPatchMerge && c->sp.cnt[s] * (kPatch * kPatch) * m < 256 * nkey) m *= 2;
+      pg.merge[s] = m;
+      pg.n[s] = (int64_t)(((c->g.nx + kPatch - 1) / kPatch + m - 1) / m) *
+                ((c->g.ny + kPatch - 1) / kPatch) * c->g.nz;
+      nbmax = std::max(nbmax, pg.n[s]);
+      cap += pg.n[s] + c->sp.cnt[s] / run;
+    }
+  } else {
+    int64_t mx = 1;
+    for (int q = 0; q < c->sp.nspec; q++) mx = c->sp.cnt[q] > mx ? c->sp.cnt[q] : mx;
+    nbmax = (mx + run - 1) / run;
+    // a cut block's pieces other than its last end at cell starts more than
+    // kRunCells / 2 cells apart (equal ranges of span / np cells, and
+    // span / np > span kRunCells / (span + kRunCells) >= kRunCells / 2 for
+    // span > kRunSpan >= kRunCells)
+    cap = nbmax * c->sp.nspec + (int64_t)c->sp.nspec * (nkey / (kRunCells / 2) + 2) + 1;
+  }
   const int64_t nb = nbmax * c->sp.nspec;
-  // the counts reuse the sort's histogram (nkey nspec entries), which no
-  // later pass reads; with more blocks than cells (over `run` particles
-  // per cell) the kernels keep their plain slices
+  // the counts reuse the sort's histogram (nkey nspec entries), which no later
+  // pass reads; with more blocks than cells (over `run` particles per cell)
+  // the kernels keep their plain slices
   if (nb > len) return EMG_OK;
   if (c->run_base_len < nb + 1) {
     if (c->run_base) (void)hipFree(c->run_base);
@@ -744,11 +832,6 @@ int build_runs(emg_ctx *c, int which) {
     }
     c->run_base_len = nb + 1;
   }
-  // a cut block's pieces other than its last end at cell starts more than
-  // kRunCells / 2 cells apart (equal ranges of span / np cells, and
-  // span / np > span kRunCells / (span + kRunCells) >= kRunCells / 2 for
-  // span > kRunSpan >= kRunCells)
-  const int64_t cap = nb + (int64_t)c->sp.nspec * (nkey / (kRunCells / 2) + 2) + 1;
   if (c->runs_cap[which] < cap) {
     if (c->runs[which]) (void)hipFree(c->runs[which]);
     c->runs_cap[which] = 0;
@@ -760,11 +843,19 @@ int build_runs(emg_ctx *c, int which) {
     c->runs_cap[which] = cap;
   }
   const dim3 gr((unsigned)((nbmax + kBlock - 1) / kBlock), (unsigned)c->sp.nspec);
-  hipLaunchKernelGGL(k_run_count, gr, dim3(kBlock), 0, c->stream, c->sort_start, nkey, c->sp,
-                     nbmax, run, c->sort_count);
+  if (patched)
+    hipLaunchKernelGGL(k_patch_count, gr, dim3(kBlock), 0, c->stream, c->sort_start, nkey, c->g, pg,
+                       nbmax, run, c->sort_count);
+  else
+    hipLaunchKernelGGL(k_run_count, gr, dim3(kBlock), 0, c->stream, c->sort_start, nkey, c->sp,
+                       nbmax, run, c->sort_count);
   exclusive_scan_i32(c->sort_count, c->run_base, nb, c->scan_tmp, c->stream);
-  hipLaunchKernelGGL(k_run_fill, gr, dim3(kBlock), 0, c->stream, c->sort_start, nkey, c->sp, nbmax,
-                     run, c->run_base, c->runs[which], cap, c->g, which == 0 ? kWinEs : kWinEm);
+  if (patched)
+    hipLaunchKernelGGL(k_patch_fill, gr, dim3(kBlock), 0, c->stream, c->sort_start, nkey, c->g, pg,
+                       nbmax, run, c->run_base, c->runs[which], cap, kWinPatch[which]);
+  else
+    hipLaunchKernelGGL(k_run_fill, gr, dim3(kBlock), 0, c->stream, c->sort_start, nkey, c->sp,
+                       nbmax, run, c->run_base, c->runs[which], cap, c->g, kWinRow[which]);
   int64_t total = 0;
   int rc = hip_check(hipMemcpyAsync(&total, c->run_base + nb, sizeof(int64_t),
                                     hipMemcpyDeviceToHost, c->stream), "sort runs");
@@ -775,24 +866,24 @@ int build_runs(emg_ctx *c, int which) {
 
 }  // namespace
 
-int sort64(emg_ctx *c) {
+int sort64(emg_ctx *c, bool patched) {
   int rc = sort64_alloc(c);
   if (rc) return rc;
   timer_begin(c, kTSort);
-  rc = sort64_count(c);
+  rc = sort64_count(c, patched);
   if (!rc) {
     const int64_t nkey = c->ncell;
     const dim3 grid = species_grid(c->sp);
     if (c->moves_after_sort <= kResortDirect) {
       hipLaunchKernelGGL(k_sort_scatter_direct, grid, dim3(kBlock), 0, c->stream, c->s64, c->t64,
-                         c->sp, c->g, nkey, c->sort_start, rank_buf(c));
+                         c->sp, c->g, nkey, c->sort_start, rank_buf(c), patched);
     } else {
       hipLaunchKernelGGL(k_sort_scatter, grid, dim3(kBlock), 0, c->stream, c->s64,
-                         (uint4 *)c->sort_rec, c->sp, c->g, nkey, c->sort_start, rank_buf(c));
+                         (uint4 *)c->sort_rec, c->sp, c->g, nkey, c->sort_start, rank_buf(c), patched);
       hipLaunchKernelGGL(k_sort_split, grid, dim3(kBlock), 0, c->stream,
                          (const uint4 *)c->sort_rec, c->t64, c->sp);
     }
-    rc = sort64_swap(c);
+    rc = sort64_swap(c, patched);
   }
   timer_end(c, kTSort);
   return rc;
@@ -824,7 +915,7 @@ int sort64_rank(emg_ctx *c, int which) {
   if (!rc) rc = sort64_alloc(c);
   if (rc) return rc;
   timer_begin(c, kTSort);
-  rc = sort64_count(c);
+  rc = sort64_count(c, true);
   timer_end(c, kTSort);
   for (int k = 0; k < 2; k++)
     if (c->nruns[k] == kRunsUnbuilt) c->nruns[k] = 0;
@@ -835,7 +926,7 @@ SortDest sort64_dest(const emg_ctx *c) {
   return SortDest{c->t64, c->sort_start, rank_buf(c), c->ncell};
 }
 
-int sort64_commit(emg_ctx *c) { return sort64_swap(c); }
+int sort64_commit(emg_ctx *c) { return sort64_swap(c, true); }
 
 int init_device_into(emg_ctx *c, State64 &st, const emg_device_species *spec, int nspec,
                      uint64_t seed) {

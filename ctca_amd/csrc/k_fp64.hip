@@ -126,6 +126,49 @@ if (DEEP) {
   }
 }
 
+// The same from the block's staged nodes fs (three double2 per node, box F),
+// for a cell whose eight nodes are among them.
+__device__ __forceinline__ bool staged(const Win &F, const Cic &w) {
+  return (unsigned)(w.i - F.ox) < (unsigned)(F.wx - 1) &&
+         (unsigned)(w.j - F.oy) < (unsigned)(F.wy - 1) &&
+         (unsigned)(w.k - F.oz) < (unsigned)(F.wz - 1);
+}
+
+__device__ __forceinline__ void gather6_lds(const double2 *fs, const Win &F, const Cic &w,
+                                            double f[6]) {
+  const double2 *p = fs + 3 * (((w.k - F.oz) * F.wy + (w.j - F.oy)) * F.wx + (w.i - F.ox));
+  const int dj = 3 * F.wx, dk = dj * F.wy;
+  auto row = [](const double2 *q) {
+    const double2 a = q[0], b = q[1], c = q[2], d = q[3], e = q[4], g = q[5];
+    return Row{{a.x, a.y, b.x, b.y, c.x, c.y}, {d.x, d.y, e.x, e.y, g.x, g.y}};
+  };
+  const Row r1 = row(p + dk), r2 = row(p + dk + dj);
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int c = 0; c < 6; c++) f[c] = r1.a[c] * w.v1 + r1.b[c] * w.v2;
+  const Row r3 = row(p);
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int c = 0; c < 6; c++) f[c] = f[c] + r2.b[c] * w.v3 + r2.a[c] * w.v4;
+  const Row r4 = row(p + dj);
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int c = 0; c < 6; c++) f[c] = f[c] + r3.a[c] * w.v5 + r3.b[c] * w.v6;
+#pragma unroll
+  for (int c = 0; c < 6; c++) f[c] = f[c] + r4.b[c] * w.v7 + r4.a[c] * w.v8;
+}
+
+__device__ __forceinline__ void stage_fields(double2 *fs, const Win &F,
+                                             const double *__restrict__ node, const Grid &g) {
+  const int n = 3 * F.wx * F.wy * F.wz;
+  for (int q = threadIdx.x; q < n; q += blockDim.x) {
+    const int v = q / 3, r = v / F.wx;
+    const int k = r / F.wy;
+    const double *p = node + 8 * nidx64(g, F.ox + v - r * F.wx, F.oy + r - k * F.wy, F.oz + k);
+    fs[q] = reinterpret_cast<const double2 *>(p)[q - 3 * v];
+  }
+}
+
 // Buneman-Boris, psolve2.F90:233-257 (ewmodel = 0: the wave field is +0.0).
 __device__ __forceinline__ void boris64(double &vx, double &vy, double &vz, const double f[6],
                                         double qmp) {
@@ -223,17 +266,16 @@ __global__ __launch_bounds__(kBlock) void k_positn64(State64 s, SpeciesTab sp, G
 // ---------------------------------------------------------------- charge
 // charge.F90:59-83 + distribute_charge 197-210; rho[is][node mod n] += v_k q(is)
 // charge.F90:152-210 per particle; the particles of a block are a contiguous
-// run of a species (kDepPer per thread).  The sort orders particles by cell
-// and they drift slowly, so most of a block's particles lie in a box of
-// nodes: the block sums their weights in an LDS window of that box, as int64
-// fixed point at 2^48 per unit weight (at most kBlock kDepPer terms of at
-// most 2^48 per node, below 2^61), and adds each non-zero window node
+// run of a species.  The sort orders particles by cell and they drift slowly,
+// so most of a block's particles lie in a box of nodes: the block sums their
+// weights in an LDS window of that box, as int64 fixed point at 2^48 per unit
+// weight (at most kRunMax[0] terms of at most 2^48 per node, below 2^61), and
+// adds each non-zero window node
 // times q(is) to rho with one global FP64 atomic; a particle whose eight
 // nodes are not all in the window adds its weights to rho directly.  The
 // rounding of a weight (2^-49) is below the FP64 round-off of the sequential
-// sum, which the reference's order would give.  The window's shape:
-// run_window; the block's particles: block_run.
-constexpr int kDepPer = 16;
+// sum, which the reference's order would give.  The block's particles and its
+// window: block_run.
 constexpr double kRhoFix = 281474976710656.0;   // 2^48 per unit weight
 
 // window index of node l + 1 on an axis of window extent w (full axis: w = n,
@@ -263,13 +305,14 @@ __device__ __forceinline__ Win slice_window(const State64 &s, int64_t a, int64_t
 // for a block past the end.
 __device__ __forceinline__ bool block_run(const State64 &s, const SpeciesTab &sp, const Run *runs,
                                           int per, const Grid &g, const WinShape &ws, int &is,
-                                          int64_t &beg, int64_t &end, Win &W) {
+                                          int64_t &beg, int64_t &end, Win &W, Win &F) {
   if (runs) {
     const Run r = runs[blockIdx.x];
     is = r.s;
     beg = r.beg;
     end = r.beg + r.len;
     W = r.w;
+    F = r.f;
     return true;
   }
   is = blockIdx.y;
@@ -371,18 +414,18 @@ __device__ __forceinline__ void flush_win(const unsigned long long *win, const W
 
 // clear the first n of an even number of window entries
 __device__ __forceinline__ void zero_win(unsigned long long *win, int n) {
-  for (int q = threadIdx.x; 2 * q < n; q += kBlock)
+  for (int q = threadIdx.x; 2 * q < n; q += blockDim.x)
     reinterpret_cast<ulonglong2 *>(win)[q] = make_ulonglong2(0ull, 0ull);
 }
 
 __global__ __launch_bounds__(kBlock) void k_deposit64(State64 s, SpeciesTab sp, Grid g,
                                                       double *__restrict__ rho, int64_t ncell,
                                                       const Run *__restrict__ runs, int *flag) {
-  __shared__ __align__(16) unsigned long long win[kWinEs.cap];
+  extern __shared__ __align__(16) unsigned long long win[];
   int is;
   int64_t beg, end;
-  Win W;
-  if (!block_run(s, sp, runs, kBlock * kDepPer, g, kWinEs, is, beg, end, W)) return;  // uniform
+  Win W, F;
+  if (!block_run(s, sp, runs, kRunRow[0], g, kWinRow[0], is, beg, end, W, F)) return;  // uniform
   const int64_t off = sp.off[is];
   zero_win(win, W.wx * W.wy * W.wz);
   __syncthreads();
@@ -410,20 +453,28 @@ __global__ __launch_bounds__(kBlock) void k_deposit64(State64 s, SpeciesTab sp, 
 // instead of back to its own slot; the arithmetic is the same.  Four waves
 // per SIMD (at most 128 VGPRs) for both forms: the plain one needs 122, the
 // re-sorting one would take 132 and drop to three.
-template <bool RESORT>
+// STAGED (runs of patches): the patch's field nodes are copied to LDS first and
+// the gather reads them there.  From memory it moves 24 x 16 bytes per particle
+// through the vector cache, 384 of its cycles per wave and round, whatever the
+// lanes share.  On 128^3 cells with 64 particles per cell and species, per step
+// with the re-sorts: rows 8.31 ms, patches 8.73, patches with staged fields
+// 7.49; 64^3 with 16 per cell 426, 408 and 327 us.
+template <bool RESORT, bool STAGED>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4)))
 void k_push_dep64(State64 s, SpeciesTab sp, const double *__restrict__ node, Grid g, int ustep,
                   double *__restrict__ rho, int64_t ncell, const Run *__restrict__ runs, int *flag,
                   SortDest dst) {
-  __shared__ __align__(16) unsigned long long win[kWinEs.cap];
+  extern __shared__ __align__(16) unsigned long long win[];
   int is;
   int64_t beg, end;
-  Win W;
-  if (!block_run(s, sp, runs, kBlock * kDepPer, g, kWinEs, is, beg, end, W)) return;  // uniform
+  Win W, F;
+  if (!block_run(s, sp, runs, kRunRow[0], g, kWinRow[0], is, beg, end, W, F)) return;  // uniform
   const int64_t off = sp.off[is];
   const int64_t key0 = (int64_t)is * dst.nkey;
   const int64_t base = RESORT ? off - dst.start[key0] : 0;
+  double2 *fs = reinterpret_cast<double2 *>(win + kWinPatch[0]);
   zero_win(win, W.wx * W.wy * W.wz);
+  if (STAGED) stage_fields(fs, F, node, g);
   __syncthreads();
   const double gustep = (double)ustep;
   const double qmp = sp.qm[is] * gustep * 0.5;
@@ -437,13 +488,14 @@ void k_push_dep64(State64 s, SpeciesTab sp, const double *__restrict__ node, Gri
     int32_t pid = 0;
     if (RESORT) {
       pid = s.pid[m];
-      d = base + dst.start[key0 + slab_key_xyz(x, y, z, g)] + dst.rank[m];
+      d = base + dst.start[key0 + sort_key_xyz(x, y, z, g, true)] + dst.rank[m];
     }
     domain_guard(x, y, z, g, flag);
     int i = (int)x, j = (int)y, k = (int)z;  // int(), psolve2.F90:158-160
     Cic w = cic(x, y, z, i, j, k);
     double f[6];
-    gather6<true>(node, g, w, f);
+    if (STAGED && staged(F, w)) gather6_lds(fs, F, w, f);
+    else gather6<!STAGED>(node, g, w, f);
     boris64(vx, vy, vz, f, qmp);
     double xmove = vx * gustep, ymove = vy * gustep, zmove = vz * gustep;
     x = x + xmove;
@@ -501,24 +553,22 @@ __device__ __forceinline__ Relay relay_axis(double xnew, double lb, double cb, i
 }
 
 // The zigzag sums of a block's particles go to an LDS window (three
-// components of kWinEm.cap nodes each, shaped from the block's sorted run like the
-// charge window, or a fixed box around its middle particle) as int64 fixed
+// components, shaped like the charge window) as int64 fixed
 // point at 2^48 per unit, and reach the global FP64 sums once per window
 // node.  A contribution is |vv w| <= 4 in the window (larger fluxes go
 // straight to the global sums), so a node's window sum of at most
-// 2 kBlock kEmPer terms stays below 2^61; the rounding of each term
+// kRunMax[1] particles' terms (twice 8 2^48) stays below 2^63; the rounding of each term
 // (2^-49) is far below the FP64 summation round-off of the reference's order.
-constexpr int kEmPer = 4;
 constexpr double kEmFix = 281474976710656.0;          // 2^48
-
 
 // RESORT as in k_push_dep64.  Bound by latency and instruction issue (VALU about
 // 40%, LDS conflicts 30%, HBM 3 TB/s); four waves per SIMD (128 VGPRs).  On the
 // 18.5M-particle two-stream (128 x 64 x 64), 1.42 ms before: one sum per node
 // for a particle that stays in its cell, the flush without divisions and the
 // short fixed-point conversion 1.12; four waves instead of three 1.02; the
-// windows from the run table instead of a scalar loop per block 0.80.  Runs of
-// 2,048 or 4,096 particles, whose windows have no margin left: 1.6 and 1.2 ms.
+// windows from the run table instead of a scalar loop per block 0.83, patches
+// instead of rows 0.78.  With staged fields (as k_push_dep64) 0.91: the LDS is
+// the busier side here.
 template <bool RESORT>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4)))
 void k_push_em64(State64 s, SpeciesTab sp,
@@ -526,11 +576,11 @@ void k_push_em64(State64 s, SpeciesTab sp,
                                                       int ustep, double *__restrict__ jacc,
                                                       int64_t ncell, const Run *__restrict__ runs,
                                                       int *flag, SortDest dst) {
-  __shared__ __align__(16) unsigned long long win[3 * kWinEm.cap];
+  extern __shared__ __align__(16) unsigned long long win[];
   int is;
   int64_t beg, end;
-  Win W;
-  if (!block_run(s, sp, runs, kBlock * kEmPer, g, kWinEm, is, beg, end, W)) return;  // uniform
+  Win W, F;
+  if (!block_run(s, sp, runs, kRunRow[1], g, kWinRow[1], is, beg, end, W, F)) return;  // uniform
   const int64_t off = sp.off[is];
   const int64_t key0 = (int64_t)is * dst.nkey;
   const int64_t base = RESORT ? off - dst.start[key0] : 0;
@@ -551,7 +601,7 @@ void k_push_em64(State64 s, SpeciesTab sp,
     int32_t pid = 0;
     if (RESORT) {
       pid = s.pid[m];
-      d = base + dst.start[key0 + slab_key_xyz(x, y, z, g)] + dst.rank[m];
+      d = base + dst.start[key0 + sort_key_xyz(x, y, z, g, true)] + dst.rank[m];
     }
     domain_guard(x, y, z, g, flag);
     double xlb = x, ylb = y, zlb = z;
@@ -721,34 +771,40 @@ void launch_positn64(emg_ctx *c, int ustep) {
   timer_end(c, kTPush);
 }
 
-// The grid of a kernel whose blocks take `per` particles each: the run table
-// `which` of the last sort when it is valid (one block per run), else
-// (slices of `per` particles, species) with runs = nullptr.
-static dim3 block_grid(const emg_ctx *c, int per, int which, const Run *&runs) {
-  static_assert(kBlock * kDepPer == kRunEs && kBlock * kEmPer == kRunEm,
-                "run lengths are the kernels' particles per block");
-  if (c->runs_valid && c->nruns[which] > 0) {
+// The grid of a kernel of table `which`: the last sort's run table when it is
+// there (one block per run), else (slices, species) with runs = nullptr; and
+// its LDS: `comps` windows of the runs' shape, and (patched, fields) the staged
+// field nodes.
+static dim3 block_grid(const emg_ctx *c, int which, int comps, bool fields, const Run *&runs,
+                       size_t &lds, bool &patched) {
+  const bool table = c->runs_valid && c->nruns[which] > 0;
+  patched = table && c->sort_patched;
+  lds = sizeof(unsigned long long) * comps * (patched ? kWinPatch[which] : kWinRow[which].cap);
+  if (patched && fields) lds += sizeof(double2) * 3 * kFieldCap;
+  if (table) {
     runs = c->runs[which];
     return dim3((unsigned)c->nruns[which]);
   }
   runs = nullptr;
   int64_t mx = 1;
   for (int q = 0; q < c->sp.nspec; q++) mx = c->sp.cnt[q] > mx ? c->sp.cnt[q] : mx;
-  return dim3((unsigned)((mx + per - 1) / per), c->sp.nspec);
+  return dim3((unsigned)((mx + kRunRow[which] - 1) / kRunRow[which]), c->sp.nspec);
 }
 
 void launch_push_es64(emg_ctx *c, int ustep, bool resort) {
   launch_zero(c->rho64, sizeof(double) * c->ncell * c->sp.nspec, c->stream);
   timer_begin(c, kTPush);
   const Run *runs;
-  const dim3 grid = block_grid(c, kBlock * kDepPer, 0, runs);
-  if (resort)
-    hipLaunchKernelGGL(k_push_dep64<true>, grid, dim3(kBlock), 0, c->stream, c->s64, c->sp,
-                       c->node64, c->g, ustep, c->rho64, c->ncell, runs, c->dflag,
-                       sort64_dest(c));
-  else
-    hipLaunchKernelGGL(k_push_dep64<false>, grid, dim3(kBlock), 0, c->stream, c->s64, c->sp,
-                       c->node64, c->g, ustep, c->rho64, c->ncell, runs, c->dflag, SortDest{});
+  size_t lds;
+  bool patched;
+  const dim3 grid = block_grid(c, 0, 1, true, runs, lds, patched);
+  const SortDest dst = resort ? sort64_dest(c) : SortDest{};
+  auto go = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, grid, dim3(kBlock), lds, c->stream, c->s64, c->sp, c->node64, c->g,
+                       ustep, c->rho64, c->ncell, runs, c->dflag, dst);
+  };
+  if (patched) resort ? go(k_push_dep64<true, true>) : go(k_push_dep64<false, true>);
+  else resort ? go(k_push_dep64<true, false>) : go(k_push_dep64<false, false>);
   timer_end(c, kTPush);
 }
 
@@ -756,8 +812,10 @@ void launch_deposit64(emg_ctx *c) {
   launch_zero(c->rho64, sizeof(double) * c->ncell * c->sp.nspec, c->stream);
   timer_begin(c, kTDeposit);
   const Run *runs;
-  const dim3 grid = block_grid(c, kBlock * kDepPer, 0, runs);
-  hipLaunchKernelGGL(k_deposit64, grid, dim3(kBlock), 0, c->stream, c->s64, c->sp, c->g, c->rho64,
+  size_t lds;
+  bool patched;
+  const dim3 grid = block_grid(c, 0, 1, false, runs, lds, patched);
+  hipLaunchKernelGGL(k_deposit64, grid, dim3(kBlock), lds, c->stream, c->s64, c->sp, c->g, c->rho64,
                      c->ncell, runs, c->dflag);
   timer_end(c, kTDeposit);
 }
@@ -766,13 +824,15 @@ void launch_push_em64(emg_ctx *c, int ustep, bool resort) {
   launch_zero(c->j64, sizeof(double) * 3 * c->ncell * c->sp.nspec, c->stream);
   timer_begin(c, kTPush);
   const Run *runs;
-  const dim3 grid = block_grid(c, kBlock * kEmPer, 1, runs);
-  if (resort)
-    hipLaunchKernelGGL(k_push_em64<true>, grid, dim3(kBlock), 0, c->stream, c->s64, c->sp,
-                       c->node64, c->g, ustep, c->j64, c->ncell, runs, c->dflag, sort64_dest(c));
-  else
-    hipLaunchKernelGGL(k_push_em64<false>, grid, dim3(kBlock), 0, c->stream, c->s64, c->sp,
-                       c->node64, c->g, ustep, c->j64, c->ncell, runs, c->dflag, SortDest{});
+  size_t lds;
+  bool patched;
+  const dim3 grid = block_grid(c, 1, 3, false, runs, lds, patched);
+  const SortDest dst = resort ? sort64_dest(c) : SortDest{};
+  auto go = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, grid, dim3(kBlock), lds, c->stream, c->s64, c->sp, c->node64, c->g,
+                       ustep, c->j64, c->ncell, runs, c->dflag, dst);
+  };
+  resort ? go(k_push_em64<true>) : go(k_push_em64<false>);
   timer_end(c, kTPush);
 }
 

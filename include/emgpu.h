@@ -76,9 +76,10 @@ typedef struct {
                           EMG_PLAIN_FP64, which takes any grid)              */
   int32_t track_pid;   /* FP32_FIXED: carry pid through every move (+8 B per
                           particle-step); without it download returns pid 0  */
-  int32_t sort_every;  /* PLAIN_FP64: re-sort by cell (emg_sort) before every
-                          sort_every-th push, and before the first push
-                          after an upload; 0 = only when emg_sort is called
+  int32_t sort_every;  /* PLAIN_FP64: re-sort before every sort_every-th push,
+                          and before the first push after an upload, by z
+                          layer like emg_sort and inside a layer by patches
+                          of 8 x 8 cells; 0 = only when emg_sort is called
                           (the reference's isort cadence).  A sort only
                           permutes the particles.  FP32_FIXED: must be 0
                           (its tile buckets are re-formed every step)       */
