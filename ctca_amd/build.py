@@ -28,6 +28,7 @@ SOURCES = [
     ("k_common.hip", []),
     ("k_fx.hip", []),
     ("k_adj.hip", []),
+    ("k_bin.hip", []),
     ("k_yee.hip", ["-ffp-contract=off"]),
     ("k_poisson.hip", []),
     ("emg_api.hip", []),

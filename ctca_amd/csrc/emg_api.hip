@@ -98,11 +98,23 @@ constexpr int kFlagPid = 16;
 constexpr int kFlagDead = 32;  // a record with nid < 0 in an upload that expected none
 
 // AoS pbuf records -> SoA FP64 state, validating each record
+// (near += the records that lie in the 8^3 tile of the one before them, over
+// every kNearSample-th block)
+constexpr int kNearSample = 8;
 __global__ __launch_bounds__(kBlock) void k_split(const emg_particle *rec, int64_t n, State64 st,
-                                                  int64_t dst0, Grid g, int *flag, int need_pid0) {
+                                                  int64_t dst0, Grid g, int *flag, int need_pid0,
+                                                  int *near) {
   int64_t m = (int64_t)blockIdx.x * kBlock + threadIdx.x;
-  if (m >= n) return;
-  emg_particle r = rec[m];
+  const bool act = m < n;
+  emg_particle r{};
+  if (act) r = rec[m];
+  if (blockIdx.x % kNearSample == 0) {
+    const int tile = ((int)r.z >> 3) * 1048573 + ((int)r.y >> 3) * 1021 + ((int)r.x >> 3);
+    const bool eq = __shfl_up(tile, 1) == tile;
+    const int same = __popcll(__ballot(act && eq && __lane_id() != 0));
+    if (__lane_id() == 0 && same) atomicAdd(near, same);
+  }
+  if (!act) return;
   if (r.nid < 0) {  // the host drops the dead records and uploads again
     atomicOr(flag, kFlagDead);
     return;
@@ -311,7 +323,7 @@ int emg_create(const emg_config *cfg, emg_ctx **out) {
   c->sp.off[cfg->nspec] = off;
   c->cap_total = off;
   int nsp = cfg->nspec;
-  if ((rc = dalloc(&c->dflag, 1, "flag")) ||
+  if ((rc = dalloc(&c->dflag, 2, "flag")) ||
       (rc = dalloc((double **)&c->face, (size_t)(face_len(c->g) * nsp), "upper-face charge"))) {
     emg_destroy(c);
     return rc;
@@ -324,7 +336,7 @@ int emg_create(const emg_config *cfg, emg_ctx **out) {
     return set_error(EMG_ERR_NOMEM, "pinned flag");
   }
   c->hsum = reinterpret_cast<double *>(c->hflag) + 1;
-  launch_zero(c->dflag, sizeof(int), c->stream);
+  launch_zero(c->dflag, 2 * sizeof(int), c->stream);
   if (cfg->precision == EMG_PLAIN_FP64) {
     int64_t nn = (int64_t)(cfg->n[0] + 1) * (cfg->n[1] + 1) * (cfg->n[2] + 1);
     if ((rc = alloc_state64(c->s64, c->cap_total)) || (rc = dalloc(&c->node64, 8 * nn, "nodal E/B")) ||
@@ -362,9 +374,9 @@ int emg_destroy(emg_ctx *c) {
   dfree(c->adj_e);
   dfree(c->adj_g);
   dfree(c->adj_sum);
-  dfree(c->adj_bins.count);
-  dfree(c->adj_bins.start);
-  dfree(c->adj_bins.rec);
+  dfree(c->bins.count);
+  dfree(c->bins.start);
+  dfree(c->bins.rec);
   FxBuckets &B = c->fx;
   for (int k = 0; k < 2; k++) {
     dfree(B.st[k].cell);
@@ -472,6 +484,7 @@ int emg_upload_particles(emg_ctx *c, const emg_particle *pbuf, const int64_t *co
   if (total > 0 && !pbuf) return set_error(EMG_ERR_ARG, "null pbuf");
   State64 tgt = c->s64;
   State64 tmp{};
+  launch_zero(c->dflag + 1, sizeof(int), c->stream);
   // particles of counts cnt, species-contiguous at src, into tgt
   auto send = [&](const emg_particle *src, const int64_t *cnt) {
     int64_t first[EMG_MAX_SPECIES + 1] = {0};
@@ -489,7 +502,7 @@ int emg_upload_particles(emg_ctx *c, const emg_particle *pbuf, const int64_t *co
                                              dim3(kBlock), 0, c->stream,
                                              static_cast<emg_particle *>(slot) + (a - m0), b - a, tgt,
                                              c->sp.off[s] + (a - first[s]), c->g, c->dflag,
-                                             need_pid0);
+                                             need_pid0, c->dflag + 1);
                       }
                       return hip_check(hipGetLastError(), "upload split");
                     });
@@ -555,6 +568,8 @@ int emg_upload_particles(emg_ctx *c, const emg_particle *pbuf, const int64_t *co
     return rc;
   }
   c->have_particles = true;
+  // most neighbours in the order share a tile: the blocks' windows catch them
+  c->ordered = (int64_t)c->hflag[1] * kNearSample * 2 > total;
   c->pushes_since_sort = c->cfg.sort_every;  // unsorted: sort before the first push
   c->moves_after_sort = emg::kUnsorted;
   c->runs_valid = false;
@@ -1062,7 +1077,7 @@ int emg_adj_step(emg_ctx *c, int32_t ustep) {
   if (!rc) rc = need_fields(c);
   if (rc) return rc;
   if (ustep < 0) return set_error(EMG_ERR_ARG, "ustep must be >= 0");
-  if ((rc = adj_bins_alloc(c))) return rc;
+  if ((rc = bins_alloc(c))) return rc;
   launch_adj_step64(c, ustep);
   return hip_check(hipGetLastError(), "adjoint step launch");
 }
@@ -1140,6 +1155,7 @@ int emg_init_device(emg_ctx *c, const emg_device_species *spec, int32_t nspec, u
     return rc;
   }
   c->have_particles = true;
+  c->ordered = false;
   c->pushes_since_sort = c->cfg.sort_every;  // unsorted: sort before the first push
   c->moves_after_sort = emg::kUnsorted;
   c->runs_valid = false;

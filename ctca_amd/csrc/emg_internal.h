@@ -378,13 +378,22 @@ struct EbView {
   }
 };
 
-// Workspace of the adjoint's transposed gather (k_adj.hip): counters and
-// cursors per tile, each tile's first record, the records of one pass.
-struct AdjBins {
+// Particles binned by tiles (k_bin.hip): counters and cursors per tile, each
+// tile's first record, the records of one pass.
+constexpr int kBinTile = 8;
+struct BinRec {
+  double x, y, z;
+  int64_t ms;  // the particle's index | species << 56
+};
+static_assert(sizeof(BinRec) == 32, "two 16-byte accesses");
+struct TileBins {
   int32_t *count;
   int64_t *start;
-  void *rec;
+  BinRec *rec;
   int64_t len;  // records
+};
+struct BinTiles {
+  int ntx, nty, ntz, n;
 };
 
 // Upper-face accumulators of the charge.  The periodic accumulators add the
@@ -428,6 +437,9 @@ struct emg_ctx {
   bool have_particles;
   int pushes_since_sort;  // PLAIN_FP64 pushes since the last cell sort (sort_every)
   int moves_after_sort;   // PLAIN_FP64 pushes since the state was last sorted, or kUnsorted
+
+  bool ordered;           // the uploaded order keeps neighbours together
+  emg::TileBins bins;     // workspace (lazy)
 
   // FP32 state
   emg::FxBuckets fx;
@@ -480,7 +492,7 @@ struct emg_ctx {
   int64_t *scan_tmp;
   int64_t scan_tmp_len;
 
-  int *dflag;       // device error flags
+  int *dflag;       // device error flags, and an upload's count of near neighbours
   int *hflag;       // pinned host mirror
   double *hsum;     // pinned: energies and adjoint sums, written by their kernels
   emg::HostIo io;
@@ -491,7 +503,6 @@ struct emg_ctx {
   double *adj_e;     // 3 x ncell: transposed gather of qmp * lambda_a
   double *adj_g;     // ncell: uploaded density adjoint
   double *adj_sum;   // block partials of the velocity adjoint sums
-  emg::AdjBins adj_bins;
   emg::State64 slot[emg::kStateSlots];  // saved particle states
   int64_t slot_cnt[emg::kStateSlots][EMG_MAX_SPECIES];
 
@@ -578,9 +589,15 @@ SortDest sort64_dest(const emg_ctx *c);
 int sort64_commit(emg_ctx *c);
 int init_device(emg_ctx *c, const emg_device_species *spec, int nspec, uint64_t seed);
 
+// binning by tiles (k_bin.hip): bin_pass bins the next particles of every
+// species, after done[] of it, into bins.rec and bins.start, and returns how
+// many (0: none left)
+BinTiles bin_tiles(const Grid &g);
+int bins_alloc(emg_ctx *c);
+int64_t bin_pass(emg_ctx *c, int64_t done[EMG_MAX_SPECIES]);
+
 // adjoint of the FP64 ES push (k_adj.hip)
-int adj_bins_alloc(emg_ctx *c);
-void launch_adj_step64(emg_ctx *c, int ustep);  // after adj_bins_alloc
+void launch_adj_step64(emg_ctx *c, int ustep);  // after bins_alloc
 void launch_adj_density64(emg_ctx *c, const double *qfac);  // one factor per species
 void launch_adj_vsum(emg_ctx *c, double *part, double *out);  // part: adj_vsum_need() doubles
 int64_t adj_vsum_need();

@@ -32,7 +32,10 @@ __global__ __launch_bounds__(kBlock) void k_copy8(const unsigned long long *src,
   if (o < n) dst[o] = src[o];
 }
 
-__global__ void k_flag(const int *dflag, int *hflag) { *hflag = *dflag; }
+__global__ void k_flag(const int *dflag, int *hflag) {
+  hflag[0] = dflag[0];
+  hflag[1] = dflag[1];
+}
 
 // Pinned memory is slow to get (0.3 ms per MB), so a context that ends leaves
 // its slots to the next one on its device: at most kPoolRings of them, given

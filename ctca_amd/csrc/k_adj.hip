@@ -84,129 +84,15 @@ __device__ __forceinline__ void rotate(double u[3], const double b[3]) {
 // every saved state).  Stepped in that order, the kernel gathered 24 x 16 bytes
 // from random cells and sent one global FP64 atomic per particle, node and
 // component, at 22 G atomics/s: 9.28 ms for 8.8M particles on 64^3 cells, whose
-// state is 0.2 ms of traffic.  So a step bins the particles by tiles of
-// kAdjTile^3 cells first:
-//   k_adj_count   particles per tile (a block's counts in LDS, one atomic per
-//                 block and tile), then a scan;
-//   k_adj_bin     position and index of each particle, 32 bytes, to its tile's
-//                 range, a block's records of one tile in one run;
-//   k_adj_step64  one workgroup per tile: its nodes' E and B staged in LDS, the
-//                 reverse step of its particles (their adjoints are 64-byte
-//                 records, so an access at a random particle is one line), the
-//                 transposed gather summed in an LDS tile of FP64 nodes, each
-//                 of which reaches memory once.
-// At the same size: 0.08 + 0.26 + 0.50 ms, bound by the random 64-byte lines of
-// the adjoints.  (Binning only the scatter, with the gather in slot order, took
-// 0.08 + 2.22 + 0.18 ms.)  With more than kAdjLdsTiles tiles a
-// block's LDS counters would not fit, and each particle takes one global
-// atomic on its tile's counter.
-constexpr int kAdjTile = 8;
-constexpr int kAdjNode = kAdjTile + 1;        // nodes per axis of a tile
-constexpr int kAdjLdsTiles = 4096;            // 16 KB of LDS counters
-constexpr int64_t kAdjRecMax = int64_t(1) << 24;  // records per pass (512 MB)
+// state is 0.2 ms of traffic.  So a step bins the particles by tiles first
+// (k_bin.hip), and k_adj_step64 takes one workgroup per tile: its nodes' E and B
+// staged in LDS, the reverse step of its particles (their adjoints are 64-byte
+// records, so an access at a random particle is one line), the transposed
+// gather summed in an LDS tile of FP64 nodes, each of which reaches memory once.
+// At the same size: 0.08 (count) + 0.26 (bin) + 0.50 ms, bound by the random
+// 64-byte lines of the adjoints.  (Binning only the scatter, with the gather in
+// slot order, took 0.08 + 2.22 + 0.18 ms.)
 constexpr int kAdjBlock = 512;
-
-// position, and the particle's index | species << 56
-struct AdjRec {
-  double x, y, z;
-  int64_t ms;
-};
-static_assert(sizeof(AdjRec) == 32, "two 16-byte accesses");
-
-struct AdjTiles {
-  int ntx, nty, ntz, n;
-};
-
-__device__ __forceinline__ int adj_tile(const AdjTiles &a, int i, int j, int k) {
-  return ((k / kAdjTile) * a.nty + j / kAdjTile) * a.ntx + i / kAdjTile;
-}
-
-// The particles of a pass: [lo, hi) of each species, as indices of the state
-// arrays.  A block takes kBlock P of species blockIdx.y.
-struct AdjPass {
-  int64_t lo[EMG_MAX_SPECIES], hi[EMG_MAX_SPECIES];
-};
-
-template <int P>
-__global__ __launch_bounds__(kBlock) void k_adj_count(State64 s, AdjPass ps, AdjTiles at, Grid g,
-                                                      int32_t *count) {
-  extern __shared__ int32_t hist[];
-  const int is = blockIdx.y;
-  const int64_t beg = ps.lo[is] + (int64_t)blockIdx.x * (kBlock * P);
-  if (beg >= ps.hi[is]) return;  // uniform over the block
-  const bool lds = at.n <= kAdjLdsTiles;
-  if (lds) {
-    for (int t = threadIdx.x; t < at.n; t += kBlock) hist[t] = 0;
-    __syncthreads();
-  }
-#pragma unroll 4
-  for (int q = 0; q < P; q++) {
-    const int64_t m = beg + q * kBlock + threadIdx.x;
-    if (m < ps.hi[is]) {
-      const Tri t = tri(s.x[m], s.y[m], s.z[m], g);
-      const int tl = adj_tile(at, t.i, t.j, t.k);
-      if (lds) atomicAdd(&hist[tl], 1);
-      else atomicAdd(&count[tl], 1);
-    }
-  }
-  if (lds) {
-    __syncthreads();
-    for (int t = threadIdx.x; t < at.n; t += kBlock)
-      if (hist[t]) atomicAdd(&count[t], hist[t]);
-  }
-}
-
-template <int P>
-__global__ __launch_bounds__(kBlock) void k_adj_bin(State64 s, AdjPass ps, AdjTiles at, Grid g,
-                                                    const int64_t *__restrict__ start,
-                                                    int32_t *__restrict__ cursor,
-                                                    AdjRec *__restrict__ rec) {
-  // a tile's count, then its first record of this block; then each particle's
-  // tile and rank
-  extern __shared__ int32_t hist[];
-  static_assert(kAdjLdsTiles <= 1 << 16 && kBlock * P <= 1 << 16, "tile and rank in one word");
-  uint32_t *mine = reinterpret_cast<uint32_t *>(hist + at.n) + threadIdx.x;
-  const int is = blockIdx.y;
-  const int64_t beg = ps.lo[is] + (int64_t)blockIdx.x * (kBlock * P);
-  if (beg >= ps.hi[is]) return;  // uniform over the block
-  const bool lds = at.n <= kAdjLdsTiles;
-  if (lds) {
-    for (int t = threadIdx.x; t < at.n; t += kBlock) hist[t] = 0;
-    __syncthreads();
-#pragma unroll 4
-    for (int q = 0; q < P; q++) {
-      const int64_t m = beg + q * kBlock + threadIdx.x;
-      if (m < ps.hi[is]) {
-        const Tri t = tri(s.x[m], s.y[m], s.z[m], g);
-        const int tl = adj_tile(at, t.i, t.j, t.k);
-        mine[q * kBlock] = ((uint32_t)tl << 16) | (uint32_t)atomicAdd(&hist[tl], 1);
-      }
-    }
-    __syncthreads();
-    for (int t = threadIdx.x; t < at.n; t += kBlock)
-      if (hist[t]) hist[t] = (int32_t)start[t] + atomicAdd(&cursor[t], hist[t]);
-    __syncthreads();
-  }
-#pragma unroll 4
-  for (int q = 0; q < P; q++) {
-    const int64_t m = beg + q * kBlock + threadIdx.x;
-    if (m < ps.hi[is]) {
-      const double x = s.x[m], y = s.y[m], z = s.z[m];
-      int64_t d;
-      if (lds) {
-        const uint32_t tr = mine[q * kBlock];
-        d = hist[tr >> 16] + (int)(tr & 0xffffu);
-      } else {
-        const Tri t = tri(x, y, z, g);
-        const int tl = adj_tile(at, t.i, t.j, t.k);
-        d = start[tl] + atomicAdd(&cursor[tl], 1);
-      }
-      double2 *r = reinterpret_cast<double2 *>(rec + d);
-      r[0] = make_double2(x, y);
-      r[1] = make_double2(z, __longlong_as_double(m | ((int64_t)is << 56)));
-    }
-  }
-}
 
 // The reverse step of tile blockIdx.x's records (slice blockIdx.y of
 // gridDim.y).  A node strictly inside the tile belongs to this tile alone:
@@ -214,21 +100,21 @@ __global__ __launch_bounds__(kBlock) void k_adj_bin(State64 s, AdjPass ps, AdjTi
 __global__ __launch_bounds__(kAdjBlock) void k_adj_step64(double *__restrict__ lam, SpeciesTab sp,
                                                          const double *__restrict__ node, Grid g,
                                                          int ustep,
-                                                         const AdjRec *__restrict__ rec,
+                                                         const BinRec *__restrict__ rec,
                                                          const int64_t *__restrict__ start,
-                                                         AdjTiles at,
+                                                         BinTiles at,
                                                          double *__restrict__ adj_e) {
-  constexpr int N = kAdjNode, NN = N * N * N;
+  constexpr int N = kBinTile + 1, NN = N * N * N;
   __shared__ double2 fs[3 * NN];  // E and B of the tile's nodes
   __shared__ double acc[3 * NN];
   const int tl = blockIdx.x;
   const int64_t beg = start[tl], end = start[tl + 1];
   const int64_t step = (int64_t)gridDim.y * kAdjBlock;
   if (beg + (int64_t)blockIdx.y * kAdjBlock >= end) return;  // uniform over the block
-  const int ox = (tl % at.ntx) * kAdjTile, oy = (tl / at.ntx) % at.nty * kAdjTile,
-            oz = tl / (at.ntx * at.nty) * kAdjTile;
-  const int tx = min(kAdjTile, g.nx - ox), ty = min(kAdjTile, g.ny - oy),
-            tz = min(kAdjTile, g.nz - oz);
+  const int ox = (tl % at.ntx) * kBinTile, oy = (tl / at.ntx) % at.nty * kBinTile,
+            oz = tl / (at.ntx * at.nty) * kBinTile;
+  const int tx = min(kBinTile, g.nx - ox), ty = min(kBinTile, g.ny - oy),
+            tz = min(kBinTile, g.nz - oz);
   for (int q = threadIdx.x; q < 3 * NN; q += kAdjBlock) {
     acc[q] = 0.0;
     const int nq = q / 3, c = q - 3 * nq;
@@ -390,97 +276,19 @@ dim3 species_blocks(const SpeciesTab &sp) {
   return dim3((unsigned)((mx + kBlock - 1) / kBlock), sp.nspec);
 }
 
-AdjTiles adj_tiles(const Grid &g) {
-  AdjTiles a;
-  a.ntx = (g.nx + kAdjTile - 1) / kAdjTile;
-  a.nty = (g.ny + kAdjTile - 1) / kAdjTile;
-  a.ntz = (g.nz + kAdjTile - 1) / kAdjTile;
-  a.n = a.ntx * a.nty * a.ntz;
-  return a;
-}
-
 }  // namespace
-
-// the workspace of the binned transposed gather, kept with the context: the
-// tile counters and starts, and the records of one pass (halved until they
-// can be allocated: a step then takes more passes)
-int adj_bins_alloc(emg_ctx *c) {
-  AdjBins &B = c->adj_bins;
-  if (B.rec) return EMG_OK;
-  const int64_t n = adj_tiles(c->g).n;
-  if (!B.count && hipMalloc(&B.count, sizeof(int32_t) * 2 * n) != hipSuccess) {
-    B.count = nullptr;
-    return set_error(EMG_ERR_NOMEM, "adjoint tile counters");
-  }
-  if (!B.start && hipMalloc(&B.start, sizeof(int64_t) * (n + 1)) != hipSuccess) {
-    B.start = nullptr;
-    return set_error(EMG_ERR_NOMEM, "adjoint tile starts");
-  }
-  const int64_t need = scan_tmp_need(n);
-  if (need > c->scan_tmp_len) {
-    if (c->scan_tmp) (void)hipFree(c->scan_tmp);
-    c->scan_tmp_len = 0;
-    if (hipMalloc(&c->scan_tmp, sizeof(int64_t) * need) != hipSuccess) {
-      c->scan_tmp = nullptr;
-      return set_error(EMG_ERR_NOMEM, "scan scratch");
-    }
-    c->scan_tmp_len = need;
-  }
-  int64_t len = c->cap_total < 1 ? 1 : (c->cap_total < kAdjRecMax ? c->cap_total : kAdjRecMax);
-  while (hipMalloc(&B.rec, sizeof(AdjRec) * len) != hipSuccess) {
-    (void)hipGetLastError();
-    B.rec = nullptr;
-    if (len <= 65536) return set_error(EMG_ERR_NOMEM, "adjoint records");
-    len /= 2;
-  }
-  B.len = len;
-  return EMG_OK;
-}
-
-template <int P>
-static void adj_pass(emg_ctx *c, int ustep, const AdjPass &ps, int64_t most, int64_t total) {
-  const AdjBins &B = c->adj_bins;
-  const AdjTiles at = adj_tiles(c->g);
-  const dim3 grid((unsigned)((most + kBlock * P - 1) / (kBlock * P)), c->sp.nspec);
-  const bool counted = at.n <= kAdjLdsTiles;
-  const size_t lds = counted ? sizeof(int32_t) * at.n : 0;
-  launch_zero(B.count, sizeof(int32_t) * 2 * at.n, c->stream);
-  hipLaunchKernelGGL(k_adj_count<P>, grid, dim3(kBlock), lds, c->stream, c->s64, ps, at, c->g,
-                     B.count);
-  exclusive_scan_i32(B.count, B.start, at.n, c->scan_tmp, c->stream);
-  hipLaunchKernelGGL(k_adj_bin<P>, grid, dim3(kBlock),
-                     counted ? lds + sizeof(int32_t) * kBlock * P : 0, c->stream, c->s64, ps, at,
-                     c->g, B.start, B.count + at.n, static_cast<AdjRec *>(B.rec));
-  // about 512 workgroups or more (two per CU), of 16 rounds of records at least
-  int64_t split = (512 + at.n - 1) / at.n;
-  split = std::min<int64_t>(split, total / ((int64_t)at.n * kAdjBlock * 16) + 1);
-  hipLaunchKernelGGL(k_adj_step64, dim3(at.n, (unsigned)split), dim3(kAdjBlock), 0, c->stream,
-                     c->lam, c->sp, c->node64, c->g, ustep, static_cast<const AdjRec *>(B.rec),
-                     B.start, at, c->adj_e);
-}
 
 void launch_adj_step64(emg_ctx *c, int ustep) {
   launch_zero(c->adj_e, sizeof(double) * 3 * c->ncell, c->stream);
+  const BinTiles at = bin_tiles(c->g);
   int64_t done[EMG_MAX_SPECIES] = {};
-  for (;;) {  // passes of at most adj_bins.len particles
-    AdjPass ps{};
-    int64_t room = c->adj_bins.len, most = 0;
-    for (int s = 0; s < c->sp.nspec; s++) {
-      const int64_t k = std::min(room, c->sp.cnt[s] - done[s]);
-      ps.lo[s] = c->sp.off[s] + done[s];
-      ps.hi[s] = ps.lo[s] + k;
-      done[s] += k;
-      room -= k;
-      most = std::max(most, k);
-    }
-    if (most == 0) break;
-    const int64_t total = c->adj_bins.len - room;
-    // 16 particles per thread make a block's records of a tile a run of
-    // several; small populations need the blocks more
-    if (total >= (int64_t)kBlock * 16 * 512)
-      adj_pass<16>(c, ustep, ps, most, total);
-    else
-      adj_pass<4>(c, ustep, ps, most, total);
+  while (const int64_t total = bin_pass(c, done)) {
+    // about 512 workgroups or more (two per CU), of 16 rounds of records at least
+    int64_t split = (512 + at.n - 1) / at.n;
+    split = std::min<int64_t>(split, total / ((int64_t)at.n * kAdjBlock * 16) + 1);
+    hipLaunchKernelGGL(k_adj_step64, dim3(at.n, (unsigned)split), dim3(kAdjBlock), 0, c->stream,
+                       c->lam, c->sp, c->node64, c->g, ustep, c->bins.rec, c->bins.start, at,
+                       c->adj_e);
   }
 }
 
