@@ -36,10 +36,10 @@ def build_oracle():
 
 
 def build_ref():
-    if not os.path.isdir(REF):
+    srcs = [os.path.join(REF, "lib/mtarm/mt19937arm.c"), os.path.join(REF, "lib/psort/psort-struct.c")]
+    if not all(os.path.isfile(s) for s in srcs):
         return None
     os.makedirs(os.path.dirname(REF_LIB), exist_ok=True)
-    srcs = [os.path.join(REF, "lib/mtarm/mt19937arm.c"), os.path.join(REF, "lib/psort/psort-struct.c")]
     inc = os.path.join(REF, "lib/ohhelp/ohhelp-1.1.1")
     tmp = REF_LIB + ".tmp"
     _run(["gcc", "-O2", "-fPIC", "-shared", "-I", inc] + srcs + ["-o", tmp])
