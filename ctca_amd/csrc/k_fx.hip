@@ -35,6 +35,7 @@
 //     one atomic per non-zero node.  Integer sums are associative, so rho is
 //     bitwise independent of particle order, scheduling and launch shape.
 #include <algorithm>
+#include <type_traits>
 
 #include "emg_internal.h"
 
@@ -43,12 +44,14 @@ namespace {
 
 constexpr int kSpillBlocksPerSpecies = 64;
 // Movers staged per bucket: the global outboxes hold kObStride records per
-// bucket; a step kernel stages up to ob_cap of them in LDS (the current's
-// three LDS tiles leave room for 512 at two blocks per CU; the charge kernel
-// takes 1024, above the ~490 movers per bucket of a 268M-particle step)
+// bucket; a step kernel stages up to OB of them in LDS (the current's three LDS
+// tiles leave room for 512 at two blocks per CU; the charge kernel takes 1024,
+// above the ~490 movers per bucket of a 268M-particle step).  The sparse
+// buckets' kernel stages 320, so that four of its blocks fit a CU, and keeps
+// the rest of the 1024 in the bucket's own global outbox until it groups them.
 constexpr int kObStride = 1024;
-template <int DEP>
-constexpr int ob_cap() { return DEP == 2 ? 512 : 1024; }
+constexpr int kObCharge = kObStride, kObCurrent = 512, kObSparse = 320;
+constexpr int ob_kept(int ob) { return ob == kObSparse ? kObStride : ob; }
 constexpr int kExtra = 16;    // slots per bucket for direct arrivals
 // bucket capacities are multiples of 32 slots, so every bucket starts on a
 // 128-byte line of each state array and every wave's load of a round covers
@@ -513,13 +516,13 @@ __device__ __forceinline__ void zig_seg_global(unsigned long long *j3, int64_t n
 // common path issues the same memory instructions whatever the data.  `act`
 // is false for lanes past the end of a round; full rounds pass a literal true.
 // DEP: 0 no deposit, 1 charge (psolve2 + charge), 2 zigzag current (psolve1).
-template <int T, bool PUSH, int DEP, bool PID>
+template <int T, bool PUSH, int DEP, bool PID, int OB>
 __device__ __forceinline__ void fx_one(const FxArgs &a, int s, bool act, const Pcl &p, int ox,
                                        int oy, int oz, int twx, int twy, int twz, bool lds_ok,
                                        const StateFx &outb,
                                        int32_t nrec,
                                        int *n_stay, int *n_out, FxRec *outbox,
-                                       unsigned char *ocode, const float4 *fA, const float2 *fB,
+                                       FxRec *obover, unsigned char *ocode, const float4 *fA, const float2 *fB,
                                        unsigned long long *rh, double ke[3]) {
   constexpr int N1 = T + 1, N3 = T + 3;
   const Grid &g = a.g;
@@ -650,7 +653,7 @@ __device__ __forceinline__ void fx_one(const FxArgs &a, int s, bool act, const P
     obase = __builtin_amdgcn_readlane(obase, leader);
     int k = obase + __builtin_amdgcn_mbcnt_hi((uint32_t)(mv >> 32),
                                               __builtin_amdgcn_mbcnt_lo((uint32_t)mv, 0));
-    const bool boxed = mover && lds_ok && k < ob_cap<DEP>();
+    const bool boxed = mover && lds_ok && k < ob_kept(OB);
     if (boxed) {
       FxRec r;
       r.cell = cell;
@@ -661,7 +664,10 @@ __device__ __forceinline__ void fx_one(const FxArgs &a, int s, bool act, const P
       r.vy = vy;
       r.vz = vz;
       r.pid = p.pid;
-      outbox[k] = r;
+      if (ob_kept(OB) == OB || k < OB)
+        outbox[k] = r;
+      else
+        obover[k] = r;
       // direction of the new tile: the tile coordinate of each axis is 0, 1
       // or 2 for the tile before, the own tile or the tile after; moves
       // beyond a neighbouring tile are placed directly at the end
@@ -769,19 +775,16 @@ __device__ __forceinline__ int64_t arrival_rec(const int64_t *seg_src, const int
   return seg_src[lo] + (j - seg_pre[lo]);
 }
 
-template <int T, bool PUSH, int DEP, bool PID>
-__global__ __launch_bounds__(T == 8 ? 512 : 256) void k_fx_step(FxArgs a) {
-  constexpr int NT = T == 8 ? 512 : 256;  // threads: T^3 cells x 64 particles per cell
+template <int T, bool PUSH, int DEP, bool PID, int NT, int OB>
+__global__ __launch_bounds__(NT) void k_fx_step(FxArgs a) {
   constexpr int N1 = T + 1, N3 = T + 3;
-  constexpr int kOb = ob_cap<DEP>();
-  constexpr int kPer = kOb / NT;
-  static_assert(kOb % NT == 0, "the outbox is written kPer records per thread");
+  constexpr int kKept = ob_kept(OB);
   __shared__ float4 fA[PUSH ? N1 * N1 * N1 : 1];
   __shared__ float2 fB[PUSH ? N1 * N1 * N1 : 1];
   constexpr int kTileNodes = DEP == 1 ? N3 * N3 * N3 : (DEP == 2 ? 3 * N3 * N3 * N3 : 1);
   __shared__ unsigned long long rh[kTileNodes];  // charge tile, or the three current tiles
-  __shared__ FxRec outbox[kOb];
-  __shared__ unsigned char ocode[kOb];
+  __shared__ FxRec outbox[OB];
+  __shared__ unsigned char ocode[kKept];
   __shared__ int64_t seg_src[kCodes];
   __shared__ int seg_pre[kPre];
   __shared__ int n_stay, n_out;
@@ -809,6 +812,7 @@ __global__ __launch_bounds__(T == 8 ? 512 : 256) void k_fx_step(FxArgs a) {
     const StateFx inb = shifted(a.in, a.start_in[b]);
     const StateFx outb = shifted(a.out, a.start_out[b]);
     const int32_t nrec = a.cap_out[b] * 4;
+    FxRec *obover = a.ob_out + (int64_t)b * kObStride;
     auto off_of = [&](int i) -> uint32_t {
       return ((uint32_t)i + (i >= nst ? gap32 : 0u)) << 2;
     };
@@ -836,9 +840,8 @@ __global__ __launch_bounds__(T == 8 ? 512 : 256) void k_fx_step(FxArgs a) {
       }
     };
     auto one = [&](bool act, const Pcl &p) {
-      fx_one<T, PUSH, DEP, PID>(a, s, act, p, ox, oy, oz, twx, twy, twz, true, outb, nrec,
-                                &n_stay, &n_out,
-                                    outbox, ocode, fA, fB, rh, ke);
+      fx_one<T, PUSH, DEP, PID, OB>(a, s, act, p, ox, oy, oz, twx, twy, twz, true, outb, nrec,
+                                    &n_stay, &n_out, outbox, obover, ocode, fA, fB, rh, ke);
     };
     // Software pipelined three deep: while a lane pushes particle k, the loads
     // of particles k + 1 and k + 2 (the next rounds of the list) are in
@@ -939,50 +942,67 @@ __global__ __launch_bounds__(T == 8 ? 512 : 256) void k_fx_step(FxArgs a) {
   // ---- write the outbox grouped by direction
   __syncthreads();
   if (b >= 0) {
-    const int nout = min(n_out, kOb);
+    const int nout = min(n_out, kKept);
     const int t = b - s * a.ntiles;
-    int cq[kPer], rq[kPer];
+    FxRec *ob = a.ob_out + (int64_t)b * kObStride;
+    // N records, a compile-time constant of which each thread takes its share:
+    // those past the staged ones are read back before any is written
+    auto group = [&](auto n_records) {
+      constexpr int N = decltype(n_records)::value;
+      constexpr int kPer = (N + NT - 1) / NT;  // records per thread
+      int cq[kPer], rq[kPer];
+      FxRec over[N > OB ? kPer : 1];
 #pragma unroll
-    for (int k = 0; k < kPer; k++) {
-      const int q = (int)threadIdx.x + k * NT;
-      cq[k] = kFar;
-      rq[k] = 0;
-      if (q < nout) {
-        cq[k] = ocode[q];
-        if (cq[k] < kFar) rq[k] = atomicAdd(&hist[cq[k]], 1);
-      }
-    }
-    __syncthreads();
-    if (threadIdx.x < 64) {
-      const int c = threadIdx.x;
-      int v = c < kCodes ? hist[c] : 0;
-      int incl = v;
-#pragma unroll
-      for (int o = 1; o < 32; o <<= 1) {
-        int u = __shfl_up(incl, o);
-        if (c >= o) incl += u;
-      }
-      if (c < kPre) {
-        int ex = incl - v;  // c = 27: the total
-        opre[c] = ex;
-        a.pre_out[(int64_t)b * kPre + c] = ex;
-      }
-    }
-    if (threadIdx.x == 0) a.stay_out[b] = n_stay;
-    __syncthreads();
-#pragma unroll
-    for (int k = 0; k < kPer; k++) {
-      const int q = (int)threadIdx.x + k * NT;
-      if (q < nout) {
-        const FxRec r = outbox[q];
-        if (cq[k] < kFar) {
-          a.ob_out[(int64_t)b * kObStride + opre[cq[k]] + rq[k]] = r;
-        } else {
-          place_direct(a, s * a.ntiles + tile_of_cell<T>(r.cell, a.g, a.ntx, a.nty), r.cell, r.pid,
-                       r.fx, r.fy, r.fz, r.vx, r.vy, r.vz);
+      for (int k = 0; k < kPer; k++) {
+        const int q = (int)threadIdx.x + k * NT;
+        cq[k] = kFar;
+        rq[k] = 0;
+        if (q < nout) {
+          cq[k] = ocode[q];
+          if (cq[k] < kFar) rq[k] = atomicAdd(&hist[cq[k]], 1);
+          if constexpr (N > OB) over[k] = q < OB ? outbox[q] : ob[q];
         }
       }
-    }
+      __syncthreads();
+      if (threadIdx.x < 64) {
+        const int c = threadIdx.x;
+        int v = c < kCodes ? hist[c] : 0;
+        int incl = v;
+#pragma unroll
+        for (int o = 1; o < 32; o <<= 1) {
+          int u = __shfl_up(incl, o);
+          if (c >= o) incl += u;
+        }
+        if (c < kPre) {
+          int ex = incl - v;  // c = 27: the total
+          opre[c] = ex;
+          a.pre_out[(int64_t)b * kPre + c] = ex;
+        }
+      }
+      if (threadIdx.x == 0) a.stay_out[b] = n_stay;
+      __syncthreads();
+#pragma unroll
+      for (int k = 0; k < kPer; k++) {
+        const int q = (int)threadIdx.x + k * NT;
+        if (q < nout) {
+          FxRec r;
+          if constexpr (N > OB)
+            r = over[k];
+          else
+            r = outbox[q];
+          if (cq[k] < kFar) {
+            ob[opre[cq[k]] + rq[k]] = r;
+          } else {
+            place_direct(a, s * a.ntiles + tile_of_cell<T>(r.cell, a.g, a.ntx, a.nty), r.cell,
+                         r.pid, r.fx, r.fy, r.fz, r.vx, r.vy, r.vz);
+          }
+        }
+      }
+    };
+    if (kKept == OB || nout <= OB)
+      group(std::integral_constant<int, OB>());
+    else
+      group(std::integral_constant<int, kKept>());
   }
   if (PUSH) {
     block_reduce3<NT>(ke, a.ke_part + 3 * (int64_t)part);
@@ -1646,15 +1666,33 @@ FxArgs make_args(emg_ctx *c) {
 // (psolve1), move only (positn)
 template <int T, bool PID>
 void step_tp(emg_ctx *c, const FxArgs &a, bool push, int dep, unsigned grid) {
-  if (push && dep == 1)
-    hipLaunchKernelGGL((k_fx_step<T, true, 1, PID>), dim3(grid), dim3(T == 8 ? 512 : 256), 0,
-                       c->stream, a);
-  else if (push && dep == 2)
-    hipLaunchKernelGGL((k_fx_step<T, true, 2, PID>), dim3(grid), dim3(T == 8 ? 512 : 256), 0,
-                       c->stream, a);
-  else
-    hipLaunchKernelGGL((k_fx_step<T, false, 0, PID>), dim3(grid), dim3(T == 8 ? 512 : 256), 0,
-                       c->stream, a);
+  constexpr int NT = T == 8 ? 512 : 256;  // threads: about T^3 cells
+  auto go = [&](auto kernel, int nt) {
+    hipLaunchKernelGGL(kernel, dim3(grid), dim3(nt), 0, c->stream, a);
+  };
+  int64_t total = 0;
+  for (int s = 0; s < c->sp.nspec; s++) total += c->sp.cnt[s];
+  if (push && dep == 1) {
+    // Sparse 8^3 tiles: four 256-thread blocks per CU instead of two of 512
+    // (with a smaller staged outbox, so that their LDS fits), so that more of
+    // them hide each other's set-up and flush.  512 against 256 threads at an
+    // average of 2,048 particles per bucket: 338 : 283 us (128^3 cells), at
+    // 4,096 510 : 475, at 6,144 690 : 677, at 8,192 865 : 882; with 432
+    // buckets 38 : 42.  Hot buckets gain as much, though their movers overflow
+    // the staged outbox (2,048 per bucket of which a quarter leave: 287 : 226).
+    if constexpr (T == 8) {
+      if (total <= (int64_t)4608 * a.nb && a.nb >= 1024)
+        go(k_fx_step<T, true, 1, PID, 256, kObSparse>, 256);
+      else
+        go(k_fx_step<T, true, 1, PID, NT, kObCharge>, NT);
+    } else {
+      go(k_fx_step<T, true, 1, PID, NT, kObCharge>, NT);
+    }
+  } else if (push && dep == 2) {
+    go(k_fx_step<T, true, 2, PID, NT, kObCurrent>, NT);
+  } else {
+    go(k_fx_step<T, false, 0, PID, NT, kObCharge>, NT);
+  }
 }
 
 template <int T>

@@ -8,6 +8,13 @@ import pytest
 pytestmark = pytest.mark.gpu
 
 
+@pytest.fixture(scope="module", autouse=True)
+def torch_first():
+    """torch has to see the device before the library initialises it."""
+    import torch
+    torch.cuda.is_available()
+
+
 def _setup(n, ppc, vth, seed=3):
     from ctca_amd import emg
     rng = np.random.default_rng(seed)
@@ -21,13 +28,16 @@ def _setup(n, ppc, vth, seed=3):
     return rec, [cnt, cnt]
 
 
-# 2 species; tiles of 4 or 8 cells: 54, 256, 2 x 129 = 258, 2,880, 16,384 and 1,024 buckets
+# 2 species; tiles of 4 or 8 cells: 54, 256, 2 x 129 = 258, 2,880, 16,384, 1,024 (twice), 1,296 and 1,024 buckets
 @pytest.mark.parametrize("n,tile,ppc,vth", [
     ((12, 12, 12), 4, 6.0, 0.3),
     ((16, 16, 32), 4, 6.0, 0.05),
     ((12, 172, 4), 4, 6.0, 0.3),
     ((40, 96, 24), 4, 4.0, 0.45),      # fast: about 3% of the particles spill
-    ((256, 256, 64), 8, 0.5, 0.3),
+    ((256, 256, 64), 8, 0.5, 0.3),     # sparse 8^3 tiles (256-thread blocks)
+    ((64, 64, 64), 8, 8.9, 0.05),      # just under the sparse rule's 4,608 per bucket
+    ((64, 64, 64), 8, 9.1, 0.05),      # just over it
+    ((66, 65, 57), 8, 4.0, 0.45),      # sparse, partial tiles, staged outboxes overflow
     ((32, 32, 32), 0, 4.0, 0.45),       # the default tile of a small grid
 ])
 def test_steps_keep_every_particle_where_it_should_be(n, tile, ppc, vth):
@@ -70,7 +80,8 @@ def test_plan_replayed_from_a_graph():
     """Eight captured steps (the first after a re-bucketing, so nine plans),
     replayed three times with eager steps between, against eager steps."""
     import torch
-    assert torch.cuda.is_available()
+    if not torch.cuda.is_available():
+        pytest.skip("the library initialised the device before torch")
     from ctca_amd import emg
     n = (40, 48, 48)
     rec, counts = _setup(n, 3.0, 0.5)
