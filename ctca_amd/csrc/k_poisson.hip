@@ -6,7 +6,8 @@
 //   phi    : -lap7 phi = rho, spectrally: the 7-point Laplacian has the
 //            eigenvalues kappa = sum_d (2 sin(pi k_d / n_d))^2
 //            (inifft.F90:390-404), the zero mode is dropped
-//            (poissn.F90:398-410); real-to-complex FFTs from hipFFT;
+//            (poissn.F90:398-410); in three kernels where an x-y plane's lines
+//            fit in LDS, else real-to-complex FFTs from hipFFT;
 //   E      = -grad phi on the staggered points (esfild.F90:351-367):
 //            EX(i) = phi(i) - phi(i+1), etc., written into the device eb
 //            (every point, ghosts as periodic images; B untouched) and, in
@@ -16,13 +17,17 @@
 // is pinned by the spectral closed form and the 7-point residual.
 #include <hipfft/hipfft.h>
 
+#include <algorithm>
 #include <cmath>
 #include <new>
 #include <string>
 
 #include "emg_internal.h"
+#include "fft_lines.h"
 
 namespace emg {
+
+constexpr int kPlaneThreads = 1024, kColumnThreads = 512;  // at most
 
 struct EsSolver {
   hipfftHandle fwd = 0, inv = 0;
@@ -30,36 +35,60 @@ struct EsSolver {
   double *rho = nullptr;    // nz ny nx, then phi in place of it
   double2 *spec = nullptr;  // nz ny (nx/2 + 1)
   double *eig = nullptr;    // (2 sin(pi k / n))^2 of x, y, z: nx + ny + nz values
+  bool planes = false;      // the three kernels below instead of hipFFT
+  int kind = 0;             // of the axes' radices
+  FftAxis *ax = nullptr;    // x, y, z
+  double2 *tw = nullptr;    // e^(-2 pi i k / n) of x, y, z
 };
 
 namespace {
 
-__global__ __launch_bounds__(kBlock) void k_rho_total(const double *rho64,
-                                                      const unsigned long long *rhofx,
-                                                      SpeciesTab sp, int64_t ncell,
-                                                      const double *bkarr, double bk,
-                                                      double *out) {
-  const int64_t c = (int64_t)blockIdx.x * kBlock + threadIdx.x;
-  if (c >= ncell) return;
+// Where the charge comes from: rho64 or rhofx of every species, and the
+// background
+struct RhoSum {
+  const double *rho64;
+  const unsigned long long *rhofx;
+  int64_t ncell;
+  const double *bkarr;
+  double bk;
+  int nspec;
+  double q[EMG_MAX_SPECIES];
+};
+
+__device__ __forceinline__ double rho_total(const RhoSum &a, int64_t c) {
+  auto of = [&](int s) {
+    return a.rho64
+               ? a.rho64[(int64_t)s * a.ncell + c]
+               : a.q[s] *
+                     ((double)(long long)a.rhofx[(int64_t)s * a.ncell + c] * (1.0 / kFixScale));
+  };
+  const double back = a.bkarr ? a.bkarr[c] : 0.0;
   double v = 0.0;
-  for (int s = 0; s < sp.nspec; s++) {
-    if (rho64)
-      v = v + rho64[(int64_t)s * ncell + c];
-    else
-      v = v + sp.q[s] * ((double)(long long)rhofx[(int64_t)s * ncell + c] * (1.0 / kFixScale));
+  int s = 0;
+  for (; s + 1 < a.nspec; s += 2) {  // two loads in flight
+    const double v0 = of(s), v1 = of(s + 1);
+    v = v + v0 + v1;
   }
-  if (bkarr) v = v + bkarr[c];
-  out[c] = v + bk;
+  if (s < a.nspec) v = v + of(s);
+  if (a.bkarr) v = v + back;
+  return v + a.bk;
+}
+
+__global__ __launch_bounds__(kBlock) void k_rho_total(RhoSum a, double *out) {
+  const int64_t c = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+  if (c < a.ncell) out[c] = rho_total(a, c);
 }
 
 // the eigenvalues of every axis, once per context (three sines per mode and solve
-// made the division take 24 us on 256 x 256 x 64 cells, 13 now)
+// made the division take 24 us on 256 x 256 x 64 cells, 13 now).  By the smaller
+// of k and n - k: near half a turn a sine loses its low bits, which the largest
+// modes of phi then lack.
 __global__ __launch_bounds__(kBlock) void k_poisson_eig(double *eig, Grid g) {
   const int o = blockIdx.x * kBlock + threadIdx.x;
   if (o >= g.nx + g.ny + g.nz) return;
   const int k = o < g.nx ? o : (o < g.nx + g.ny ? o - g.nx : o - g.nx - g.ny);
   const int n = o < g.nx ? g.nx : (o < g.nx + g.ny ? g.ny : g.nz);
-  const double s = 2.0 * sin(3.141592653589793 * k / n);
+  const double s = 2.0 * sinpi((double)min(k, n - k) / n);
   eig[o] = s * s;
 }
 
@@ -84,6 +113,207 @@ __global__ __launch_bounds__(kBlock) void k_poisson_divide(double2 *spec,
     v.y *= f;
   }
   spec[o] = v;
+}
+
+// e^(-2 pi i k / n) of every axis, the angle folded to at most an eighth of a
+// turn by whole numbers first, so that only the sine and cosine round
+__global__ __launch_bounds__(kBlock) void k_poisson_twiddle(double2 *tw, Grid g, FftAxis x,
+                                                            FftAxis y, FftAxis z, FftAxis *ax) {
+  const int o = blockIdx.x * kBlock + threadIdx.x;
+  if (o == 0) {
+    ax[0] = x;
+    ax[1] = y;
+    ax[2] = z;
+  }
+  if (o >= g.nx + g.ny + g.nz) return;
+  const int k = o < g.nx ? o : (o < g.nx + g.ny ? o - g.nx : o - g.nx - g.ny);
+  const int n = o < g.nx ? g.nx : (o < g.nx + g.ny ? g.ny : g.nz);
+  const int quarter = (8 * k + n) / (2 * n);  // the nearest quarter turn
+  double s, c;
+  sincospi(0.5 * (4 * k - quarter * n) / n, &s, &c);
+  switch (quarter & 3) {
+    case 0: tw[o] = make_double2(c, -s); break;
+    case 1: tw[o] = make_double2(-s, -c); break;
+    case 2: tw[o] = make_double2(-c, s); break;
+    default: tw[o] = make_double2(s, c);
+  }
+}
+
+// The solve of a small grid in three kernels, the lines of which stay in LDS:
+// the charge of an x-y plane and its transform, every (kx, ky) column's
+// transform, division and inverse, and the planes' inverse.  hipFFT's four
+// kernels, the charge sum and the division moved each value six times through
+// launches of 3 to 6 us that do little work.  A block's time is its chain of
+// latencies (16^3 cells: three kernels of 5 us): its tables and its data are
+// loaded together, it has a thread per element where that is at most 1024, and
+// each kernel holds the code of its radices only.
+struct PlaneArgs {
+  const FftAxis *ax;
+  const double2 *tw;
+  int ny;
+  FastDiv nx, np, hx;  // np: pairs of x lines
+  int stride, buf;     // of the pairs (odd: no bank conflicts); elements per buffer
+};
+constexpr int kAxisWords = sizeof(FftAxis) / 4;
+
+// one axis' passes; the result's buffer comes back in x
+template <bool INV, int KIND>
+__device__ __forceinline__ void fft_axis_lines(const FftAxis &a, double2 *&x, double2 *&y,
+                                               const FastDiv &lines, int stride,
+                                               const double2 *tw) {
+  const int npass = __builtin_amdgcn_readfirstlane(a.npass);
+  for (int p = 0; p < npass; p++) {
+    fft_pass_of<INV, KIND>(a, p, x, y, lines, stride, tw, threadIdx.x, blockDim.x);
+    __syncthreads();
+    double2 *z = x;
+    x = y;
+    y = z;
+  }
+}
+
+extern __shared__ double2 fft_lds[];
+
+// put(t, get(t)) for this thread's t < n, U loads in flight
+template <int U, class Get, class Put>
+__device__ __forceinline__ void stage(int n, Get get, Put put) {
+  const int nt = blockDim.x;
+  for (int t0 = threadIdx.x; t0 < n; t0 += U * nt) {
+    double2 v[U];
+#pragma unroll
+    for (int u = 0; u < U; u++)
+      if (t0 + u * nt < n) v[u] = get(t0 + u * nt);
+#pragma unroll
+    for (int u = 0; u < U; u++)
+      if (t0 + u * nt < n) put(t0 + u * nt, v[u]);
+  }
+}
+
+// The tables of a block, n axes' and m twiddles, on their way to LDS: get()
+// issues the loads, put() (after the loads of the data) stores, so that one
+// memory latency covers all.  Blocks have at least 2 kAxisWords threads.
+struct Tables {
+  int word;
+  double2 w;
+  __device__ __forceinline__ void get(const FftAxis *ax, int n, const double2 *tw, int m) {
+    const int tid = threadIdx.x;
+    if (tid < n * kAxisWords) word = reinterpret_cast<const int *>(ax)[tid];
+    if (tid < m) w = tw[tid];
+  }
+  __device__ __forceinline__ void put(FftAxis *ax, int n, const double2 *tw, double2 *out, int m) {
+    const int tid = threadIdx.x;
+    if (tid < n * kAxisWords) reinterpret_cast<int *>(ax)[tid] = word;
+    if (tid < m) out[tid] = w;
+    for (int q = tid + blockDim.x; q < m; q += blockDim.x) out[q] = tw[q];
+  }
+};
+
+template <int KIND>
+__global__ __launch_bounds__(kPlaneThreads) void k_plane_forward(PlaneArgs a, RhoSum rho, double2 *spec) {
+  __shared__ FftAxis ax[2];
+  double2 *x = fft_lds, *y = x + a.buf, *tw = y + a.buf;
+  const int nx = a.nx.d, ny = a.ny, tid = threadIdx.x, nt = blockDim.x;
+  Tables tab;
+  tab.get(a.ax, 2, a.tw, nx + ny);
+  const int64_t c0 = (int64_t)blockIdx.x * nx * ny;
+  stage<1>(
+      nx * a.np.d,
+      [&](int t) {
+        const int p = div(t, a.nx), i = t - p * nx;
+        const int64_t c = c0 + 2 * p * nx + i;
+        const double v = rho_total(rho, 2 * p + 1 < ny ? c + nx : c);
+        return make_double2(rho_total(rho, c), 2 * p + 1 < ny ? v : 0.0);
+      },
+      [&](int t, double2 v) {
+        const int p = div(t, a.nx), i = t - p * nx;
+        x[i * a.stride + p] = v;
+      });
+  tab.put(ax, 2, a.tw, tw, nx + ny);
+  __syncthreads();
+  fft_axis_lines<false, KIND>(ax[0], x, y, a.np, a.stride, tw);
+  split_pairs(x, a.stride, y, nx, ny, a.np, tid, nt);
+  __syncthreads();
+  fft_axis_lines<false, KIND>(ax[1], y, x, a.hx, a.hx.d, tw + nx);
+  const int n = a.hx.d * ny;
+  for (int t = tid; t < n; t += nt) spec[(int64_t)blockIdx.x * n + t] = y[t];
+}
+
+template <int KIND>
+__global__ __launch_bounds__(kPlaneThreads) void k_plane_inverse(PlaneArgs a, const double2 *spec,
+                                                       double *phi) {
+  __shared__ FftAxis ax[2];
+  double2 *x = fft_lds, *y = x + a.buf, *tw = y + a.buf;
+  const int nx = a.nx.d, ny = a.ny, tid = threadIdx.x, nt = blockDim.x;
+  Tables tab;
+  tab.get(a.ax, 2, a.tw, nx + ny);
+  const int n = a.hx.d * ny;
+  const double2 *in = spec + (int64_t)blockIdx.x * n;
+  stage<4>(n, [&](int t) { return in[t]; }, [&](int t, double2 v) { x[t] = v; });
+  tab.put(ax, 2, a.tw, tw, nx + ny);
+  __syncthreads();
+  fft_axis_lines<true, KIND>(ax[1], x, y, a.hx, a.hx.d, tw + nx);
+  join_pairs(x, y, a.stride, nx, ny, a.np, tid, nt);
+  __syncthreads();
+  fft_axis_lines<true, KIND>(ax[0], y, x, a.np, a.stride, tw);
+  const int64_t c0 = (int64_t)blockIdx.x * nx * ny;
+  for (int t = tid; t < nx * a.np.d; t += nt) {
+    const int p = div(t, a.nx), i = t - p * nx;
+    const double2 v = y[i * a.stride + p];
+    const int64_t c = c0 + 2 * p * nx + i;
+    phi[c] = v.x;
+    if (2 * p + 1 < ny) phi[c + nx] = v.y;
+  }
+}
+
+// kColumns neighbouring (kx, ky) columns per block: 128 bytes of each plane
+constexpr int kColumns = 8;
+struct ColumnArgs {
+  const FftAxis *ax;
+  const double2 *tw;
+  const double *ez, *ey, *ex;  // eigenvalues
+  int nz, ncol;
+  FastDiv hx;
+  double cells;
+};
+template <int KIND>
+__global__ __launch_bounds__(kColumnThreads) void k_column_solve(ColumnArgs a, double2 *spec) {
+  __shared__ FftAxis ax;
+  const int col0 = blockIdx.x * kColumns, nz = a.nz, nt = blockDim.x, tid = threadIdx.x;
+  double2 *x = fft_lds, *y = x + nz * kColumns, *tw = y + nz * kColumns;
+  double *ez = reinterpret_cast<double *>(tw + nz);
+  // a thread's column is the same all through (nt is a multiple of kColumns)
+  const int l = tid % kColumns, col = min(col0 + l, a.ncol - 1);
+  const bool mine = col0 + l < a.ncol;
+  const int ky = div(col, a.hx), kx = col - ky * a.hx.d;
+  Tables tab;
+  tab.get(a.ax, 1, a.tw, nz);
+  const double e0 = tid < nz ? a.ez[tid] : 0.0, ey = a.ey[ky], ex = a.ex[kx];
+  double2 *own = spec + col;
+  stage<4>(
+      nz * kColumns, [&](int t) { return own[(int64_t)(t / kColumns) * a.ncol]; },
+      [&](int t, double2 v) { x[t] = v; });
+  tab.put(&ax, 1, a.tw, tw, nz);
+  if (tid < nz) ez[tid] = e0;
+  for (int q = tid + nt; q < nz; q += nt) ez[q] = a.ez[q];
+  __syncthreads();
+  const FastDiv cols{(uint32_t)((1ull << 32) / kColumns), kColumns};
+  fft_axis_lines<false, KIND>(ax, x, y, cols, kColumns, tw);
+  for (int t = tid; t < nz * kColumns; t += nt) {
+    const double kappa = ez[t / kColumns] + ey + ex;
+    double2 v = x[t];
+    if (col == 0 && t < kColumns) {
+      v.x = 0.0;
+      v.y = 0.0;
+    } else {
+      const double f = 1.0 / (kappa * a.cells);
+      v.x *= f;
+      v.y *= f;
+    }
+    x[t] = v;
+  }
+  __syncthreads();
+  fft_axis_lines<true, KIND>(ax, x, y, cols, kColumns, tw);
+  if (mine)
+    for (int t = tid; t < nz * kColumns; t += nt) own[(int64_t)(t / kColumns) * a.ncol] = x[t];
 }
 
 // E = -grad phi at every point of eb, and at the nodes 0..n its relocation
@@ -128,6 +358,13 @@ __global__ __launch_bounds__(kBlock) void k_es_efield(const double *__restrict__
 
 }  // namespace
 
+constexpr size_t kPlaneLds = 159 * 1024;  // of 160 KB, less the static part
+constexpr int kLargestRadix = 61;         // (a prime r costs r products per element)
+// a thread per element where they fit
+static int threads_for(int elems, int most) {
+  return std::min(most, std::max(128, (elems + 63) / 64 * 64));
+}
+
 static int fft_check(hipfftResult r, const char *what) {
   if (r == HIPFFT_SUCCESS) return EMG_OK;
   return set_error(EMG_ERR_HIP, std::string(what) + ": hipFFT error " + std::to_string((int)r));
@@ -141,8 +378,63 @@ void es_solver_free(emg_ctx *c) {
   if (s->rho) (void)hipFree(s->rho);
   if (s->spec) (void)hipFree(s->spec);
   if (s->eig) (void)hipFree(s->eig);
+  if (s->tw) (void)hipFree(s->tw);
+  if (s->ax) (void)hipFree(s->ax);
   delete s;
   c->es = nullptr;
+}
+
+// elements of a buffer of k_plane_*, and their LDS and k_column_solve's
+static int plane_elems(const Grid &g) {
+  const int np = (g.ny + 1) / 2;
+  return std::max(g.nx * (np | 1), g.ny * (g.nx / 2 + 1));
+}
+static size_t plane_lds(const Grid &g) {
+  return sizeof(double2) * (2 * (size_t)plane_elems(g) + g.nx + g.ny);
+}
+static size_t column_lds(const Grid &g) {
+  return (sizeof(double2) * (2 * kColumns + 1) + sizeof(double)) * (size_t)g.nz;
+}
+
+// Can the three kernels do this grid, and are they faster than hipFFT?  Solve,
+// E included, hipFFT against planes: 16^3 cells 21.4 : 18.5 us, 32^3 24.7 :
+// 20.0, 48^3 32.5 : 27.1, 64^3 37.4 : 31.0, 80^3 52.6 : 47.1, 96^3 78.9 :
+// 56.8, 128x64x64 52.7 : 46.6, 20x20x160 26.8 : 23.0, 77x63x70 72 : 44.
+// From a prime factor of 19 on hipFFT changes to a longer algorithm (31x37x41
+// 121 : 35, 61x59x47 156 : 79).  Large planes with factors of 7 to 17 are the
+// exception (90x70x51 46.9 : 49.7, 98x98x50 52.3 : 59.3, but 85x68x34 72 : 56).
+// The first solve also has no kernels to compile at run time (1.6 s : 0.2 ms).
+static bool plane_solve_fits(const Grid &g, FftAxis ax[3]) {
+  if (g.nx > 1024 || g.ny > 1024 || g.nz > 1024) return false;
+  if (plane_lds(g) > kPlaneLds || column_lds(g) > kPlaneLds) return false;
+  int largest = 0, kind = 0;
+  const int n[3] = {g.nx, g.ny, g.nz};
+  for (int d = 0; d < 3; d++) {
+    if (!fft_axis(n[d], kLargestRadix, &ax[d])) return false;
+    kind = std::max(kind, radix_kind(ax[d]));
+    for (int p = 0; p < ax[d].npass; p++) largest = std::max(largest, ax[d].r[p]);
+  }
+  return kind < 2 || largest >= 19 || plane_elems(g) <= 3000;
+}
+
+template <class F>
+static void with_kind(int kind, F f) {
+  if (kind == 0)
+    f(std::integral_constant<int, 0>());
+  else if (kind == 1)
+    f(std::integral_constant<int, 1>());
+  else
+    f(std::integral_constant<int, 2>());
+}
+
+static int es_fft_plans(emg_ctx *c, EsSolver *s) {
+  int rc = fft_check(hipfftPlan3d(&s->fwd, c->g.nz, c->g.ny, c->g.nx, HIPFFT_D2Z), "plan D2Z");
+  if (!rc) s->have_fwd = true;
+  if (!rc) rc = fft_check(hipfftPlan3d(&s->inv, c->g.nz, c->g.ny, c->g.nx, HIPFFT_Z2D), "plan Z2D");
+  if (!rc) s->have_inv = true;
+  if (!rc) rc = fft_check(hipfftSetStream(s->fwd, c->stream), "set stream");
+  if (!rc) rc = fft_check(hipfftSetStream(s->inv, c->stream), "set stream");
+  return rc;
 }
 
 static int es_solver_get(emg_ctx *c, EsSolver **out) {
@@ -160,38 +452,84 @@ static int es_solver_get(emg_ctx *c, EsSolver **out) {
       hipMalloc(&s->spec, sizeof(double2) * c->g.nz * c->g.ny * hx) != hipSuccess ||
       hipMalloc(&s->eig, sizeof(double) * neig) != hipSuccess)
     rc = set_error(EMG_ERR_NOMEM, "field solver arrays");
-  if (!rc) rc = fft_check(hipfftPlan3d(&s->fwd, c->g.nz, c->g.ny, c->g.nx, HIPFFT_D2Z), "plan D2Z");
-  if (!rc) s->have_fwd = true;
-  if (!rc) rc = fft_check(hipfftPlan3d(&s->inv, c->g.nz, c->g.ny, c->g.nx, HIPFFT_Z2D), "plan Z2D");
-  if (!rc) s->have_inv = true;
-  if (!rc) rc = fft_check(hipfftSetStream(s->fwd, c->stream), "set stream");
-  if (!rc) rc = fft_check(hipfftSetStream(s->inv, c->stream), "set stream");
+  FftAxis ax[3];
+  s->planes = plane_solve_fits(c->g, ax);
+  if (!rc && s->planes) {
+    if (hipMalloc(&s->tw, sizeof(double2) * neig) != hipSuccess ||
+        hipMalloc(&s->ax, sizeof(ax)) != hipSuccess)
+      rc = set_error(EMG_ERR_NOMEM, "field solver arrays");
+    for (int d = 0; d < 3; d++) s->kind = std::max(s->kind, radix_kind(ax[d]));
+    auto allow = [&](auto kernel) {
+      if (!rc)
+        rc = hip_check(hipFuncSetAttribute(reinterpret_cast<const void *>(kernel),
+                                           hipFuncAttributeMaxDynamicSharedMemorySize,
+                                           (int)kPlaneLds),
+                       "field solver LDS");
+    };
+    with_kind(s->kind, [&](auto kind) {
+      constexpr int K = decltype(kind)::value;
+      allow(k_plane_forward<K>);
+      allow(k_column_solve<K>);
+      allow(k_plane_inverse<K>);
+    });
+  }
+  if (!rc && !s->planes) rc = es_fft_plans(c, s);
   if (rc) {
     es_solver_free(c);
     return rc;
   }
-  hipLaunchKernelGGL(k_poisson_eig, dim3((unsigned)((neig + kBlock - 1) / kBlock)), dim3(kBlock), 0,
-                     c->stream, s->eig, c->g);
+  const dim3 ge((unsigned)((neig + kBlock - 1) / kBlock));
+  hipLaunchKernelGGL(k_poisson_eig, ge, dim3(kBlock), 0, c->stream, s->eig, c->g);
+  if (s->planes)
+    hipLaunchKernelGGL(k_poisson_twiddle, ge, dim3(kBlock), 0, c->stream, s->tw, c->g, ax[0], ax[1],
+                       ax[2], s->ax);
   *out = s;
   return EMG_OK;
+}
+static void plane_solve(emg_ctx *c, EsSolver *s, const RhoSum &sum) {
+  const Grid &g = c->g;
+  const int hx = g.nx / 2 + 1, np = (g.ny + 1) / 2;
+  const PlaneArgs a{s->ax, s->tw, g.ny, fast_div(g.nx), fast_div(np), fast_div(hx), np | 1,
+                    plane_elems(g)};
+  const ColumnArgs ca{s->ax + 2,  s->tw + g.nx + g.ny, s->eig + g.nx + g.ny, s->eig + g.nx,
+                      s->eig,     g.nz,                hx * g.ny,            fast_div(hx),
+                      (double)g.nx * g.ny * g.nz};
+  const dim3 planes(g.nz), columns((ca.ncol + kColumns - 1) / kColumns);
+  const dim3 tp(threads_for(g.nx * np, kPlaneThreads)),
+      tc(threads_for(g.nz * kColumns, kColumnThreads));
+  with_kind(s->kind, [&](auto kind) {
+    constexpr int K = decltype(kind)::value;
+    hipLaunchKernelGGL(k_plane_forward<K>, planes, tp, plane_lds(g), c->stream, a, sum, s->spec);
+    hipLaunchKernelGGL(k_column_solve<K>, columns, tc, column_lds(g), c->stream, ca, s->spec);
+    hipLaunchKernelGGL(k_plane_inverse<K>, planes, tp, plane_lds(g), c->stream, a, s->spec, s->rho);
+  });
+}
+
+static int fft_solve(emg_ctx *c, EsSolver *s, const RhoSum &sum) {
+  const unsigned gc = (unsigned)((c->ncell + kBlock - 1) / kBlock);
+  hipLaunchKernelGGL(k_rho_total, dim3(gc), dim3(kBlock), 0, c->stream, sum, s->rho);
+  int rc = fft_check(hipfftExecD2Z(s->fwd, s->rho, reinterpret_cast<hipfftDoubleComplex *>(s->spec)),
+                     "D2Z");
+  if (rc) return rc;
+  const int64_t ns = (int64_t)c->g.nz * c->g.ny * (c->g.nx / 2 + 1);
+  hipLaunchKernelGGL(k_poisson_divide, dim3((unsigned)((ns + kBlock - 1) / kBlock)), dim3(kBlock),
+                     0, c->stream, s->spec, s->eig, c->g);
+  return fft_check(hipfftExecZ2D(s->inv, reinterpret_cast<hipfftDoubleComplex *>(s->spec), s->rho),
+                   "Z2D");
 }
 
 int solve_es(emg_ctx *c, double rhobk) {
   EsSolver *s = nullptr;
   int rc = es_solver_get(c, &s);
   if (rc) return rc;
-  const unsigned gc = (unsigned)((c->ncell + kBlock - 1) / kBlock);
   const bool fix = c->cfg.precision == EMG_FP32_FIXED;
-  hipLaunchKernelGGL(k_rho_total, dim3(gc), dim3(kBlock), 0, c->stream, fix ? nullptr : c->rho64,
-                     fix ? c->rhofx : nullptr, c->sp, c->ncell, c->bk_dev, rhobk, s->rho);
-  rc = fft_check(hipfftExecD2Z(s->fwd, s->rho, reinterpret_cast<hipfftDoubleComplex *>(s->spec)),
-                 "D2Z");
-  if (rc) return rc;
-  const int64_t ns = (int64_t)c->g.nz * c->g.ny * (c->g.nx / 2 + 1);
-  hipLaunchKernelGGL(k_poisson_divide, dim3((unsigned)((ns + kBlock - 1) / kBlock)), dim3(kBlock),
-                     0, c->stream, s->spec, s->eig, c->g);
-  rc = fft_check(hipfftExecZ2D(s->inv, reinterpret_cast<hipfftDoubleComplex *>(s->spec), s->rho),
-                 "Z2D");
+  RhoSum sum{fix ? nullptr : c->rho64, fix ? c->rhofx : nullptr, c->ncell, c->bk_dev, rhobk,
+             c->sp.nspec, {}};
+  for (int k = 0; k < c->sp.nspec; k++) sum.q[k] = c->sp.q[k];
+  if (s->planes)
+    plane_solve(c, s, sum);
+  else
+    rc = fft_solve(c, s, sum);
   if (rc) return rc;
   const EbView v = eb_view(c);
   timer_begin(c, kTRelocate);
