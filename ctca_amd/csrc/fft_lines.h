@@ -10,8 +10,9 @@
 // w^(p k n / (ns r)), w = e^(-2 pi i / n), transforms those r values, and
 // writes result q to (j / ns) ns r + k + q ns.
 //
-// Radices 2, 3, 4, 5, 7, 8, 11 and 13 transform in registers; any other prime sums its r
-// products per output straight from LDS.
+// Radices 2, 3, 4, 5, 7, 8, 11 and 13 transform in registers; any other prime sums
+// its products straight from LDS, and comes first (ns = 1, no twiddles), where
+// results q and r - q share theirs.
 //
 // The functions do the work of thread tid of nt; the caller separates them with
 // barriers.
@@ -38,7 +39,8 @@ __host__ __device__ inline int div(int t, const FastDiv &f) {
   return f.d == 1 ? t : (int)(((uint64_t)(uint32_t)t * f.m) >> 32);
 }
 
-// An axis' length, its radices, before each the product of those done, and 1 / r
+// An axis' length, its radices, before each the product of those done, and the
+// divisions by r (of pass 0, by n / r)
 struct FftAxis {
   int n, npass;
   int r[kMaxPasses];
@@ -53,25 +55,25 @@ inline int radix_kind(const FftAxis &a) {
   return kind;
 }
 
-// Splits n into radices; false if a prime factor is above `largest`
+// Splits n into radices; false if a prime factor is above 13 and `largest`
 inline bool fft_axis(int n, int largest, FftAxis *a) {
   a->n = n;
   a->npass = 0;
   auto take = [&](int r) {
     while (n % r == 0 && a->npass < kMaxPasses) {
       a->ns[a->npass] = fast_div(a->n / n);
-      a->rd[a->npass] = fast_div(r);
+      a->rd[a->npass] = fast_div(a->npass == 0 ? a->n / r : r);
       a->r[a->npass++] = r;
       n /= r;
     }
   };
+  for (int p = 17; p <= largest; p += 2) take(p);
   // 16 = 4 x 4 and not 8 x 2
   if (n % 16 == 0 && n % 32 != 0) take(4);
   take(8);
   take(4);
   take(2);
-  take(3);
-  for (int p = 5; p <= largest; p += 2) take(p);
+  for (int p = 3; p <= 13; p += 2) take(p);
   return n == 1;
 }
 
@@ -258,6 +260,38 @@ __host__ __device__ inline void fft_pass_any(const double2 *x, double2 *y, int n
   }
 }
 
+// the first pass of an odd radix r: results q and r - q of each j, from the sums
+// and differences of inputs p and r - p
+template <bool INV>
+__host__ __device__ inline void fft_pass_first(const double2 *x, double2 *y, int n, int r,
+                                               FastDiv lines, FastDiv nrd, int stride,
+                                               const double2 *tw, int tid, int nt) {
+  const int nr = nrd.d, h = r / 2;
+  for (int t = tid; t < nr * lines.d * (h + 1); t += nt) {
+    const int jq = div(t, lines), l = t - jq * lines.d;
+    const int q = div(jq, nrd), j = jq - q * nr;
+    const double2 *a = x + j * stride + l, *b = a + n * stride;
+    const int step = q * nr, by = nr * stride;
+    double2 m = *a, d = make_double2(0.0, 0.0);
+    int e = 0;
+    for (int p = 1; p <= h; p++) {
+      a += by;
+      b -= by;
+      e += step;
+      if (e >= n) e -= n;
+      const double2 w = tw[e], u = *a, v = *b;  // (cos, -sin)
+      m.x += w.x * (u.x + v.x);
+      m.y += w.x * (u.y + v.y);
+      d.x -= w.y * (u.x - v.x);
+      d.y -= w.y * (u.y - v.y);
+    }
+    d = crot<INV>(d);
+    double2 *o = y + j * r * stride + l;
+    o[q * stride] = cadd(m, d);
+    if (q > 0) o[(r - q) * stride] = csub(m, d);
+  }
+}
+
 // a value that is the same for the whole wave, as a scalar
 __host__ __device__ inline int uniform(int v) {
 #ifdef __HIP_DEVICE_COMPILE__
@@ -293,7 +327,10 @@ __host__ __device__ inline void fft_pass_of(const FftAxis &a, int pass, const do
     if (r == 7) return go(std::integral_constant<int, 7>());
     if (r == 11) return go(std::integral_constant<int, 11>());
     if (r == 13) return go(std::integral_constant<int, 13>());
-    fft_pass_any<INV>(x, y, n, r, ns, uniform(a.rd[pass]), lines, stride, tw, tid, nt);
+    if (pass == 0)
+      fft_pass_first<INV>(x, y, n, r, lines, uniform(a.rd[0]), stride, tw, tid, nt);
+    else
+      fft_pass_any<INV>(x, y, n, r, ns, uniform(a.rd[pass]), lines, stride, tw, tid, nt);
   }
 }
 
@@ -305,7 +342,7 @@ __host__ __device__ inline void split_pairs(const double2 *z, int stride, double
   for (int t = tid; t < hx * np.d; t += nt) {
     const int k = div(t, np), p = t - k * np.d;
     const double2 u = z[k * stride + p], w = z[(k == 0 ? 0 : nx - k) * stride + p];
-    y[2 * p * hx + k] = make_double2(0.5 * (u.x + w.x), 0.5 * (u.y - w.y));
+    if (2 * p < ny) y[2 * p * hx + k] = make_double2(0.5 * (u.x + w.x), 0.5 * (u.y - w.y));
     if (2 * p + 1 < ny)
       y[(2 * p + 1) * hx + k] = make_double2(0.5 * (u.y + w.y), 0.5 * (w.x - u.x));
   }
@@ -318,7 +355,7 @@ __host__ __device__ inline void join_pairs(const double2 *y, double2 *z, int str
   const int hx = nx / 2 + 1;
   for (int t = tid; t < hx * np.d; t += nt) {
     const int k = div(t, np), p = t - k * np.d;
-    double2 a = y[2 * p * hx + k];
+    double2 a = 2 * p < ny ? y[2 * p * hx + k] : make_double2(0.0, 0.0);
     double2 b = 2 * p + 1 < ny ? y[(2 * p + 1) * hx + k] : make_double2(0.0, 0.0);
     const bool real = k == 0 || 2 * k == nx;
     if (real) a.y = b.y = 0.0;

@@ -6,8 +6,8 @@
 //   phi    : -lap7 phi = rho, spectrally: the 7-point Laplacian has the
 //            eigenvalues kappa = sum_d (2 sin(pi k_d / n_d))^2
 //            (inifft.F90:390-404), the zero mode is dropped
-//            (poissn.F90:398-410); in three kernels where an x-y plane's lines
-//            fit in LDS, else real-to-complex FFTs from hipFFT;
+//            (poissn.F90:398-410); in three or five kernels of LDS lines where
+//            they are faster, else real-to-complex FFTs from hipFFT;
 //   E      = -grad phi on the staggered points (esfild.F90:351-367):
 //            EX(i) = phi(i) - phi(i+1), etc., written into the device eb
 //            (every point, ghosts as periodic images; B untouched) and, in
@@ -35,7 +35,7 @@ struct EsSolver {
   double *rho = nullptr;    // nz ny nx, then phi in place of it
   double2 *spec = nullptr;  // nz ny (nx/2 + 1)
   double *eig = nullptr;    // (2 sin(pi k / n))^2 of x, y, z: nx + ny + nz values
-  bool planes = false;      // the three kernels below instead of hipFFT
+  int path = 0;             // SolvePath
   int kind = 0;             // of the axes' radices
   FftAxis *ax = nullptr;    // x, y, z
   double2 *tw = nullptr;    // e^(-2 pi i k / n) of x, y, z
@@ -150,7 +150,7 @@ __global__ __launch_bounds__(kBlock) void k_poisson_twiddle(double2 *tw, Grid g,
 struct PlaneArgs {
   const FftAxis *ax;
   const double2 *tw;
-  int ny;
+  int ny, rows;        // rows per block: a whole plane, or some of its x lines
   FastDiv nx, np, hx;  // np: pairs of x lines
   int stride, buf;     // of the pairs (odd: no bank conflicts); elements per buffer
 };
@@ -207,19 +207,23 @@ struct Tables {
   }
 };
 
-template <int KIND>
-__global__ __launch_bounds__(kPlaneThreads) void k_plane_forward(PlaneArgs a, RhoSum rho, double2 *spec) {
+// YAXIS: the block's rows are a whole plane, which goes through y as well
+template <int KIND, bool YAXIS>
+__global__ __launch_bounds__(kPlaneThreads) void k_plane_forward(PlaneArgs a, RhoSum rho,
+                                                                 double2 *spec) {
   __shared__ FftAxis ax[2];
   double2 *x = fft_lds, *y = x + a.buf, *tw = y + a.buf;
-  const int nx = a.nx.d, ny = a.ny, tid = threadIdx.x, nt = blockDim.x;
+  const int nx = a.nx.d, tid = threadIdx.x, nt = blockDim.x;
+  const int naxes = YAXIS ? 2 : 1, ntw = YAXIS ? nx + a.ny : nx;
+  const int row0 = YAXIS ? 0 : blockIdx.y * a.rows, ny = YAXIS ? a.ny : min(a.rows, a.ny - row0);
+  const int64_t line0 = (int64_t)blockIdx.x * a.ny + row0;
   Tables tab;
-  tab.get(a.ax, 2, a.tw, nx + ny);
-  const int64_t c0 = (int64_t)blockIdx.x * nx * ny;
+  tab.get(a.ax, naxes, a.tw, ntw);
   stage<1>(
       nx * a.np.d,
       [&](int t) {
         const int p = div(t, a.nx), i = t - p * nx;
-        const int64_t c = c0 + 2 * p * nx + i;
+        const int64_t c = (line0 + min(2 * p, ny - 1)) * nx + i;
         const double v = rho_total(rho, 2 * p + 1 < ny ? c + nx : c);
         return make_double2(rho_total(rho, c), 2 * p + 1 < ny ? v : 0.0);
       },
@@ -227,93 +231,108 @@ __global__ __launch_bounds__(kPlaneThreads) void k_plane_forward(PlaneArgs a, Rh
         const int p = div(t, a.nx), i = t - p * nx;
         x[i * a.stride + p] = v;
       });
-  tab.put(ax, 2, a.tw, tw, nx + ny);
+  tab.put(ax, naxes, a.tw, tw, ntw);
   __syncthreads();
   fft_axis_lines<false, KIND>(ax[0], x, y, a.np, a.stride, tw);
   split_pairs(x, a.stride, y, nx, ny, a.np, tid, nt);
   __syncthreads();
-  fft_axis_lines<false, KIND>(ax[1], y, x, a.hx, a.hx.d, tw + nx);
+  if (YAXIS) fft_axis_lines<false, KIND>(ax[1], y, x, a.hx, a.hx.d, tw + nx);
   const int n = a.hx.d * ny;
-  for (int t = tid; t < n; t += nt) spec[(int64_t)blockIdx.x * n + t] = y[t];
+  double2 *out = spec + line0 * a.hx.d;
+  for (int t = tid; t < n; t += nt) out[t] = y[t];
 }
 
-template <int KIND>
+template <int KIND, bool YAXIS>
 __global__ __launch_bounds__(kPlaneThreads) void k_plane_inverse(PlaneArgs a, const double2 *spec,
-                                                       double *phi) {
+                                                                 double *phi) {
   __shared__ FftAxis ax[2];
   double2 *x = fft_lds, *y = x + a.buf, *tw = y + a.buf;
-  const int nx = a.nx.d, ny = a.ny, tid = threadIdx.x, nt = blockDim.x;
+  const int nx = a.nx.d, tid = threadIdx.x, nt = blockDim.x;
+  const int naxes = YAXIS ? 2 : 1, ntw = YAXIS ? nx + a.ny : nx;
+  const int row0 = YAXIS ? 0 : blockIdx.y * a.rows, ny = YAXIS ? a.ny : min(a.rows, a.ny - row0);
+  const int64_t line0 = (int64_t)blockIdx.x * a.ny + row0;
   Tables tab;
-  tab.get(a.ax, 2, a.tw, nx + ny);
-  const int n = a.hx.d * ny;
-  const double2 *in = spec + (int64_t)blockIdx.x * n;
-  stage<4>(n, [&](int t) { return in[t]; }, [&](int t, double2 v) { x[t] = v; });
-  tab.put(ax, 2, a.tw, tw, nx + ny);
+  tab.get(a.ax, naxes, a.tw, ntw);
+  const double2 *in = spec + line0 * a.hx.d;
+  stage<4>(a.hx.d * ny, [&](int t) { return in[t]; }, [&](int t, double2 v) { x[t] = v; });
+  tab.put(ax, naxes, a.tw, tw, ntw);
   __syncthreads();
-  fft_axis_lines<true, KIND>(ax[1], x, y, a.hx, a.hx.d, tw + nx);
+  if (YAXIS) fft_axis_lines<true, KIND>(ax[1], x, y, a.hx, a.hx.d, tw + nx);
   join_pairs(x, y, a.stride, nx, ny, a.np, tid, nt);
   __syncthreads();
   fft_axis_lines<true, KIND>(ax[0], y, x, a.np, a.stride, tw);
-  const int64_t c0 = (int64_t)blockIdx.x * nx * ny;
   for (int t = tid; t < nx * a.np.d; t += nt) {
     const int p = div(t, a.nx), i = t - p * nx;
     const double2 v = y[i * a.stride + p];
-    const int64_t c = c0 + 2 * p * nx + i;
-    phi[c] = v.x;
+    const int64_t c = (line0 + 2 * p) * nx + i;
+    if (2 * p < ny) phi[c] = v.x;
     if (2 * p + 1 < ny) phi[c + nx] = v.y;
   }
 }
 
-// kColumns neighbouring (kx, ky) columns per block: 128 bytes of each plane
+// The transforms of kColumns neighbouring columns per block (128 bytes of each
+// of their elements): of z, with the division and the inverse (SOLVE), or of y
+// one way.  Element k of column c of part blockIdx.y is spec[part y + k ncol + c].
 constexpr int kColumns = 8;
+enum ColumnMode { kForward, kInverse, kSolve };
 struct ColumnArgs {
   const FftAxis *ax;
   const double2 *tw;
-  const double *ez, *ey, *ex;  // eigenvalues
-  int nz, ncol;
-  FastDiv hx;
+  int n, ncol;
+  int64_t part;
+  const double *ez, *ey, *ex;  // kSolve: the eigenvalues
+  int hx;
   double cells;
 };
-template <int KIND>
-__global__ __launch_bounds__(kColumnThreads) void k_column_solve(ColumnArgs a, double2 *spec) {
+template <int KIND, ColumnMode MODE>
+__global__ __launch_bounds__(kColumnThreads) void k_columns(ColumnArgs a, double2 *spec) {
   __shared__ FftAxis ax;
-  const int col0 = blockIdx.x * kColumns, nz = a.nz, nt = blockDim.x, tid = threadIdx.x;
-  double2 *x = fft_lds, *y = x + nz * kColumns, *tw = y + nz * kColumns;
-  double *ez = reinterpret_cast<double *>(tw + nz);
+  const int col0 = blockIdx.x * kColumns, n = a.n, nt = blockDim.x, tid = threadIdx.x;
+  double2 *x = fft_lds, *y = x + n * kColumns, *tw = y + n * kColumns;
+  double *ez = reinterpret_cast<double *>(tw + n);
   // a thread's column is the same all through (nt is a multiple of kColumns)
   const int l = tid % kColumns, col = min(col0 + l, a.ncol - 1);
   const bool mine = col0 + l < a.ncol;
-  const int ky = div(col, a.hx), kx = col - ky * a.hx.d;
   Tables tab;
-  tab.get(a.ax, 1, a.tw, nz);
-  const double e0 = tid < nz ? a.ez[tid] : 0.0, ey = a.ey[ky], ex = a.ex[kx];
-  double2 *own = spec + col;
+  tab.get(a.ax, 1, a.tw, n);
+  double e0 = 0.0, ey = 0.0, ex = 0.0;
+  if (MODE == kSolve) {
+    const int ky = col / a.hx, kx = col - ky * a.hx;
+    if (tid < n) e0 = a.ez[tid];
+    ey = a.ey[ky];
+    ex = a.ex[kx];
+  }
+  double2 *own = spec + blockIdx.y * a.part + col;
   stage<4>(
-      nz * kColumns, [&](int t) { return own[(int64_t)(t / kColumns) * a.ncol]; },
+      n * kColumns, [&](int t) { return own[(int64_t)(t / kColumns) * a.ncol]; },
       [&](int t, double2 v) { x[t] = v; });
-  tab.put(&ax, 1, a.tw, tw, nz);
-  if (tid < nz) ez[tid] = e0;
-  for (int q = tid + nt; q < nz; q += nt) ez[q] = a.ez[q];
-  __syncthreads();
-  const FastDiv cols{(uint32_t)((1ull << 32) / kColumns), kColumns};
-  fft_axis_lines<false, KIND>(ax, x, y, cols, kColumns, tw);
-  for (int t = tid; t < nz * kColumns; t += nt) {
-    const double kappa = ez[t / kColumns] + ey + ex;
-    double2 v = x[t];
-    if (col == 0 && t < kColumns) {
-      v.x = 0.0;
-      v.y = 0.0;
-    } else {
-      const double f = 1.0 / (kappa * a.cells);
-      v.x *= f;
-      v.y *= f;
-    }
-    x[t] = v;
+  tab.put(&ax, 1, a.tw, tw, n);
+  if (MODE == kSolve) {
+    if (tid < n) ez[tid] = e0;
+    for (int q = tid + nt; q < n; q += nt) ez[q] = a.ez[q];
   }
   __syncthreads();
-  fft_axis_lines<true, KIND>(ax, x, y, cols, kColumns, tw);
+  const FastDiv cols{(uint32_t)((1ull << 32) / kColumns), kColumns};
+  fft_axis_lines<MODE == kInverse, KIND>(ax, x, y, cols, kColumns, tw);
+  if (MODE == kSolve) {
+    for (int t = tid; t < n * kColumns; t += nt) {
+      const double kappa = ez[t / kColumns] + ey + ex;
+      double2 v = x[t];
+      if (col == 0 && t < kColumns) {
+        v.x = 0.0;
+        v.y = 0.0;
+      } else {
+        const double f = 1.0 / (kappa * a.cells);
+        v.x *= f;
+        v.y *= f;
+      }
+      x[t] = v;
+    }
+    __syncthreads();
+    fft_axis_lines<true, KIND>(ax, x, y, cols, kColumns, tw);
+  }
   if (mine)
-    for (int t = tid; t < nz * kColumns; t += nt) own[(int64_t)(t / kColumns) * a.ncol] = x[t];
+    for (int t = tid; t < n * kColumns; t += nt) own[(int64_t)(t / kColumns) * a.ncol] = x[t];
 }
 
 // E = -grad phi at every point of eb, and at the nodes 0..n its relocation
@@ -359,7 +378,11 @@ __global__ __launch_bounds__(kBlock) void k_es_efield(const double *__restrict__
 }  // namespace
 
 constexpr size_t kPlaneLds = 159 * 1024;  // of 160 KB, less the static part
-constexpr int kLargestRadix = 61;         // (a prime r costs r products per element)
+constexpr int kLargestRadix = 211;        // (a prime r costs r / 2 products per element)
+constexpr int kLongestLine = 512;         // (two buffers of 8 columns in LDS)
+// kLines: pairs of x lines per block, of about kRowElems elements.  (199x40x40
+// cells 78 us with 256 threads, 61 with 512; 2048 elements 82.)
+constexpr int kRowElems = 1024, kRowThreads = 512;
 // a thread per element where they fit
 static int threads_for(int elems, int most) {
   return std::min(most, std::max(128, (elems + 63) / 64 * 64));
@@ -384,37 +407,48 @@ void es_solver_free(emg_ctx *c) {
   c->es = nullptr;
 }
 
-// elements of a buffer of k_plane_*, and their LDS and k_column_solve's
-static int plane_elems(const Grid &g) {
-  const int np = (g.ny + 1) / 2;
-  return std::max(g.nx * (np | 1), g.ny * (g.nx / 2 + 1));
+// How the field solve runs: kPlanes as above; kLines with x and y in kernels of
+// their own (five kernels, for planes that LDS does not hold); kLibrary
+enum SolvePath { kLibrary, kPlanes, kLines };
+
+// rows per block, elements per buffer, and LDS bytes of k_plane_*
+static int plane_rows(const Grid &g, SolvePath path) {
+  return path == kPlanes ? g.ny : std::min((g.ny + 1) / 2 * 2, 2 * std::max(1, kRowElems / g.nx));
 }
-static size_t plane_lds(const Grid &g) {
-  return sizeof(double2) * (2 * (size_t)plane_elems(g) + g.nx + g.ny);
+static int plane_elems(const Grid &g, SolvePath path) {
+  const int rows = plane_rows(g, path), np = (rows + 1) / 2;
+  return std::max(g.nx * (np | 1), rows * (g.nx / 2 + 1));
 }
-static size_t column_lds(const Grid &g) {
-  return (sizeof(double2) * (2 * kColumns + 1) + sizeof(double)) * (size_t)g.nz;
+static size_t plane_lds(const Grid &g, SolvePath path) {
+  return sizeof(double2) *
+         (2 * (size_t)plane_elems(g, path) + g.nx + (path == kPlanes ? g.ny : 0));
+}
+static size_t column_lds(int n) {
+  return (sizeof(double2) * (2 * kColumns + 1) + sizeof(double)) * (size_t)n;
 }
 
-// Can the three kernels do this grid, and are they faster than hipFFT?  Solve,
-// E included, hipFFT against planes: 16^3 cells 21.4 : 18.5 us, 32^3 24.7 :
-// 20.0, 48^3 32.5 : 27.1, 64^3 37.4 : 31.0, 80^3 52.6 : 47.1, 96^3 78.9 :
-// 56.8, 128x64x64 52.7 : 46.6, 20x20x160 26.8 : 23.0, 77x63x70 72 : 44.
-// From a prime factor of 19 on hipFFT changes to a longer algorithm (31x37x41
-// 121 : 35, 61x59x47 156 : 79).  Large planes with factors of 7 to 17 are the
-// exception (90x70x51 46.9 : 49.7, 98x98x50 52.3 : 59.3, but 85x68x34 72 : 56).
-// The first solve also has no kernels to compile at run time (1.6 s : 0.2 ms).
-static bool plane_solve_fits(const Grid &g, FftAxis ax[3]) {
-  if (g.nx > 1024 || g.ny > 1024 || g.nz > 1024) return false;
-  if (plane_lds(g) > kPlaneLds || column_lds(g) > kPlaneLds) return false;
-  int largest = 0, kind = 0;
+// Which one is the fastest.  Solve, E included, hipFFT against planes: 16^3 cells
+// 21.4 : 18.5 us, 32^3 24.7 : 20.0, 48^3 32.5 : 27.1, 64^3 37.4 : 31.0, 80^3
+// 52.6 : 47.1, 96^3 78.9 : 56.8, 128x64x64 52.7 : 46.6, 77x63x70 72 : 44; larger
+// planes with factors of 7 to 17 are the exception (90x70x51 46.9 : 49.7,
+// 98x98x50 52.3 : 59.3).  From a prime factor of 19 on hipFFT changes to a longer
+// algorithm: 31^3 83 : 24, 53^3 152 : 37; there the lines do the planes' work
+// from 3000 elements of a plane on (hipFFT : planes : lines, 62^3 129 : 40 : 41,
+// 95x66x40 87 : 49 : 41; 114x95x133 252 : - : 111, 191x181x173 1148 : - : 619).
+// Without such a factor the lines gain nothing (256x256x64 206 : 214, 180x150x170
+// 233 : 288).  The first solve also has no kernels to compile at run time (1.6 s :
+// 0.2 ms).
+static SolvePath solve_path(const Grid &g, FftAxis ax[3]) {
   const int n[3] = {g.nx, g.ny, g.nz};
+  int largest = 0, kind = 0;
   for (int d = 0; d < 3; d++) {
-    if (!fft_axis(n[d], kLargestRadix, &ax[d])) return false;
+    if (n[d] > kLongestLine || !fft_axis(n[d], kLargestRadix, &ax[d])) return kLibrary;
     kind = std::max(kind, radix_kind(ax[d]));
     for (int p = 0; p < ax[d].npass; p++) largest = std::max(largest, ax[d].r[p]);
   }
-  return kind < 2 || largest >= 19 || plane_elems(g) <= 3000;
+  if (plane_lds(g, kPlanes) <= kPlaneLds && (kind < 2 || plane_elems(g, kPlanes) <= 3000))
+    return kPlanes;
+  return largest >= 19 ? kLines : kLibrary;
 }
 
 template <class F>
@@ -453,8 +487,8 @@ static int es_solver_get(emg_ctx *c, EsSolver **out) {
       hipMalloc(&s->eig, sizeof(double) * neig) != hipSuccess)
     rc = set_error(EMG_ERR_NOMEM, "field solver arrays");
   FftAxis ax[3];
-  s->planes = plane_solve_fits(c->g, ax);
-  if (!rc && s->planes) {
+  s->path = solve_path(c->g, ax);
+  if (!rc && s->path != kLibrary) {
     if (hipMalloc(&s->tw, sizeof(double2) * neig) != hipSuccess ||
         hipMalloc(&s->ax, sizeof(ax)) != hipSuccess)
       rc = set_error(EMG_ERR_NOMEM, "field solver arrays");
@@ -468,19 +502,26 @@ static int es_solver_get(emg_ctx *c, EsSolver **out) {
     };
     with_kind(s->kind, [&](auto kind) {
       constexpr int K = decltype(kind)::value;
-      allow(k_plane_forward<K>);
-      allow(k_column_solve<K>);
-      allow(k_plane_inverse<K>);
+      if (s->path == kPlanes) {
+        allow(k_plane_forward<K, true>);
+        allow(k_plane_inverse<K, true>);
+      } else {
+        allow(k_plane_forward<K, false>);
+        allow(k_plane_inverse<K, false>);
+        allow(k_columns<K, kForward>);
+        allow(k_columns<K, kInverse>);
+      }
+      allow(k_columns<K, kSolve>);
     });
   }
-  if (!rc && !s->planes) rc = es_fft_plans(c, s);
+  if (!rc && s->path == kLibrary) rc = es_fft_plans(c, s);
   if (rc) {
     es_solver_free(c);
     return rc;
   }
   const dim3 ge((unsigned)((neig + kBlock - 1) / kBlock));
   hipLaunchKernelGGL(k_poisson_eig, ge, dim3(kBlock), 0, c->stream, s->eig, c->g);
-  if (s->planes)
+  if (s->path != kLibrary)
     hipLaunchKernelGGL(k_poisson_twiddle, ge, dim3(kBlock), 0, c->stream, s->tw, c->g, ax[0], ax[1],
                        ax[2], s->ax);
   *out = s;
@@ -488,20 +529,44 @@ static int es_solver_get(emg_ctx *c, EsSolver **out) {
 }
 static void plane_solve(emg_ctx *c, EsSolver *s, const RhoSum &sum) {
   const Grid &g = c->g;
-  const int hx = g.nx / 2 + 1, np = (g.ny + 1) / 2;
-  const PlaneArgs a{s->ax, s->tw, g.ny, fast_div(g.nx), fast_div(np), fast_div(hx), np | 1,
-                    plane_elems(g)};
-  const ColumnArgs ca{s->ax + 2,  s->tw + g.nx + g.ny, s->eig + g.nx + g.ny, s->eig + g.nx,
-                      s->eig,     g.nz,                hx * g.ny,            fast_div(hx),
+  const SolvePath path = (SolvePath)s->path;
+  const int hx = g.nx / 2 + 1, rows = plane_rows(g, path), np = (rows + 1) / 2;
+  const PlaneArgs a{s->ax, s->tw, g.ny, rows, fast_div(g.nx), fast_div(np), fast_div(hx), np | 1,
+                    plane_elems(g, path)};
+  const ColumnArgs az{s->ax + 2,
+                      s->tw + g.nx + g.ny,
+                      g.nz,
+                      hx * g.ny,
+                      0,
+                      s->eig + g.nx + g.ny,
+                      s->eig + g.nx,
+                      s->eig,
+                      hx,
                       (double)g.nx * g.ny * g.nz};
-  const dim3 planes(g.nz), columns((ca.ncol + kColumns - 1) / kColumns);
-  const dim3 tp(threads_for(g.nx * np, kPlaneThreads)),
-      tc(threads_for(g.nz * kColumns, kColumnThreads));
+  const ColumnArgs ay{s->ax + 1, s->tw + g.nx, g.ny,    hx,  (int64_t)hx * g.ny,
+                      nullptr,   nullptr,      nullptr, hx, 0.0};
+  const size_t lp = plane_lds(g, path);
+  const dim3 gp(g.nz, (g.ny + rows - 1) / rows), gz((az.ncol + kColumns - 1) / kColumns),
+      gy((hx + kColumns - 1) / kColumns, g.nz);
+  const dim3 tp(threads_for(g.nx * np, path == kPlanes ? kPlaneThreads : kRowThreads)),
+      ty(threads_for(g.ny * kColumns, kColumnThreads)),
+      tz(threads_for(g.nz * kColumns, kColumnThreads));
   with_kind(s->kind, [&](auto kind) {
     constexpr int K = decltype(kind)::value;
-    hipLaunchKernelGGL(k_plane_forward<K>, planes, tp, plane_lds(g), c->stream, a, sum, s->spec);
-    hipLaunchKernelGGL(k_column_solve<K>, columns, tc, column_lds(g), c->stream, ca, s->spec);
-    hipLaunchKernelGGL(k_plane_inverse<K>, planes, tp, plane_lds(g), c->stream, a, s->spec, s->rho);
+    auto columns = [&](auto kernel, dim3 grid, dim3 threads, const ColumnArgs &ca) {
+      hipLaunchKernelGGL(kernel, grid, threads, column_lds(ca.n), c->stream, ca, s->spec);
+    };
+    if (path == kPlanes) {
+      hipLaunchKernelGGL((k_plane_forward<K, true>), gp, tp, lp, c->stream, a, sum, s->spec);
+      columns(k_columns<K, kSolve>, gz, tz, az);
+      hipLaunchKernelGGL((k_plane_inverse<K, true>), gp, tp, lp, c->stream, a, s->spec, s->rho);
+    } else {
+      hipLaunchKernelGGL((k_plane_forward<K, false>), gp, tp, lp, c->stream, a, sum, s->spec);
+      columns(k_columns<K, kForward>, gy, ty, ay);
+      columns(k_columns<K, kSolve>, gz, tz, az);
+      columns(k_columns<K, kInverse>, gy, ty, ay);
+      hipLaunchKernelGGL((k_plane_inverse<K, false>), gp, tp, lp, c->stream, a, s->spec, s->rho);
+    }
   });
 }
 
@@ -526,7 +591,7 @@ int solve_es(emg_ctx *c, double rhobk) {
   RhoSum sum{fix ? nullptr : c->rho64, fix ? c->rhofx : nullptr, c->ncell, c->bk_dev, rhobk,
              c->sp.nspec, {}};
   for (int k = 0; k < c->sp.nspec; k++) sum.q[k] = c->sp.q[k];
-  if (s->planes)
+  if (s->path != kLibrary)
     plane_solve(c, s, sum);
   else
     rc = fft_solve(c, s, sum);

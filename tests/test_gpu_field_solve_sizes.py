@@ -13,9 +13,10 @@ pytestmark = pytest.mark.gpu
     (2, 2, 2), (3, 2, 5), (2, 3, 64), (4, 16, 8), (16, 4, 9),
     (32, 32, 32), (64, 64, 64), (15, 13, 11), (17, 19, 61), (53, 7, 3), (24, 40, 6),
     (77, 63, 14), (90, 70, 9), (7, 26, 22),
-    (67, 8, 8), (8, 8, 134),   # a prime factor above the largest radix
+    (67, 8, 8), (8, 8, 211), (8, 223, 8),  # the largest radix, and a prime above it
     (100, 97, 8),              # the largest plane that LDS holds, and one above
     (100, 98, 8),
+    (111, 97, 10), (95, 66, 8), (19, 510, 4), (512, 38, 6),   # x lines in ragged groups
     (12, 10, 512), (6, 10, 640),
 ])
 @pytest.mark.parametrize("precision", [emg.PLAIN_FP64, emg.FP32_FIXED])
@@ -40,6 +41,6 @@ def test_solve_matches_numpy(n, precision):
             ctx.solve_es(bk)
             phi = ctx.potential()
             ref = oracle.fields.poisson_periodic(rho)
-            # two transforms of at most 21 additions per output and pass round
-            # to some 1e-15 of the largest value
+            # the transforms' passes, of at most 211 terms, round to some
+            # 1e-15 of the largest value
             assert np.abs(phi - ref).max() <= 1e-12 * np.abs(ref).max()
