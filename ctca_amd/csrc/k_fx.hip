@@ -697,6 +697,19 @@ __device__ __forceinline__ void fx_one(const FxArgs &a, int s, bool act, const P
   store_masked<PID>(outb, nrec, off, cell, p.pid, fx, fy, fz, vx, vy, vz);
 }
 
+// v plus the value that the DPP control brings from another lane (0 where none)
+template <int CTRL, int ROWS>
+__device__ __forceinline__ double dpp_add(double v) {
+  const unsigned long long b = (unsigned long long)__double_as_longlong(v);
+  const int lo = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)b, CTRL, ROWS, 0xf, false);
+  const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), CTRL, ROWS, 0xf, false);
+  return v + __longlong_as_double((long long)(((unsigned long long)(uint32_t)hi << 32) |
+                                              (uint32_t)lo));
+}
+
+// The sums of ke over the block.  In the wave by DPP (row shifts by 1, 2, 4 and 8,
+// then rows 0 and 2 into 1 and 3, and 0-1 into 2-3: lane 63 has the sum): through
+// LDS shuffles it was 0.9 us of a block's 15 to 20.
 template <int NT>
 __device__ __forceinline__ void block_reduce3(double ke[3], double *out) {
   __shared__ double red[3][NT / 64];
@@ -704,9 +717,13 @@ __device__ __forceinline__ void block_reduce3(double ke[3], double *out) {
 #pragma unroll
   for (int d = 0; d < 3; d++) {
     double v = ke[d];
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_down(v, o);
-    if (lane == 0) red[d][w] = v;
+    v = dpp_add<0x111, 0xf>(v);
+    v = dpp_add<0x112, 0xf>(v);
+    v = dpp_add<0x114, 0xf>(v);
+    v = dpp_add<0x118, 0xf>(v);
+    v = dpp_add<0x142, 0xa>(v);
+    v = dpp_add<0x143, 0xc>(v);
+    if (lane == 63) red[d][w] = v;
   }
   __syncthreads();
   if (threadIdx.x < 3) {
@@ -1681,6 +1698,11 @@ void step_tp(emg_ctx *c, const FxArgs &a, bool push, int dep, unsigned grid) {
   };
   int64_t total = 0;
   for (int s = 0; s < c->sp.nspec; s++) total += c->sp.cnt[s];
+  // At most one 4^3 tile per CU: more threads, and so fewer rounds one after
+  // another in a block.  Charge step, 256 : 512 : 1024 threads: 16^3 cells with 16
+  // per cell and species (128 buckets) 18.3 : 15.7 : 14.9 us, with 64 35.6 : 26.8 :
+  // 24.9; 24^3 (432 buckets) 20.9 : 20.9; 32^3 (1024) 28.2 : 35.4.
+  const bool few = T == 4 && a.nb <= 256;
   if (push && dep == 1) {
     // Sparse 8^3 tiles: four 256-thread blocks per CU instead of two of 512
     // (with a smaller staged outbox, so that their LDS fits), so that more of
@@ -1695,9 +1717,15 @@ void step_tp(emg_ctx *c, const FxArgs &a, bool push, int dep, unsigned grid) {
       else
         go(k_fx_step<T, true, 1, PID, NT, kObCharge>, NT);
     } else {
-      go(k_fx_step<T, true, 1, PID, NT, kObCharge>, NT);
+      if (few)
+        go(k_fx_step<T, true, 1, PID, 1024, kObCharge>, 1024);
+      else
+        go(k_fx_step<T, true, 1, PID, NT, kObCharge>, NT);
     }
   } else if (push && dep == 2) {
+    if constexpr (T == 4) {
+      if (few) return go(k_fx_step<T, true, 2, PID, 1024, kObCurrent>, 1024);
+    }
     go(k_fx_step<T, true, 2, PID, NT, kObCurrent>, NT);
   } else {
     go(k_fx_step<T, false, 0, PID, NT, kObCharge>, NT);

@@ -28,10 +28,11 @@ def _setup(n, ppc, vth, seed=3):
     return rec, [cnt, cnt]
 
 
-# 2 species; tiles of 4 or 8 cells: 54, 256, 2 x 129 = 258, 2,880, 16,384, 1,024 (twice), 1,296 and 1,024 buckets
+# 2 species; tiles of 4 or 8 cells: 54, 256, 128, 2 x 129 = 258, 2,880, 16,384, 1,024 (twice), 1,296 and 1,024 buckets
 @pytest.mark.parametrize("n,tile,ppc,vth", [
     ((12, 12, 12), 4, 6.0, 0.3),
     ((16, 16, 32), 4, 6.0, 0.05),
+    ((16, 16, 16), 4, 40.0, 0.1),      # few tiles of several 1024-thread rounds
     ((12, 172, 4), 4, 6.0, 0.3),
     ((40, 96, 24), 4, 4.0, 0.45),      # fast: about 3% of the particles spill
     ((256, 256, 64), 8, 0.5, 0.3),     # sparse 8^3 tiles (256-thread blocks)
