@@ -310,6 +310,7 @@ __device__ __forceinline__ bool block_run(const State64 &s, const SpeciesTab &sp
                                           int64_t &beg, int64_t &end, Win &W, Win &F) {
   if (runs) {
     const Run r = runs[blockIdx.x];
+    if (r.len == 0) return false;
     is = r.s;
     beg = r.beg;
     end = r.beg + r.len;

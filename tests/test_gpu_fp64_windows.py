@@ -14,6 +14,7 @@ pytestmark = pytest.mark.gpu
     ((130, 3, 2), (5000, 40), 0.1),          # rows longer than a wave
     ((17, 13, 11), (60000, 900), 0.4),       # cut runs of a sparse species
     ((33, 31, 8), (1030, 1023), 1.3),        # one particle past a block; fast
+    ((64, 64, 9), (90, 0), 0.3),             # most patches and run entries empty
 ])
 @pytest.mark.parametrize("em", [False, True])
 def test_pushes_after_a_sort_equal_unsorted_ones(n, counts, drift, em):
