@@ -742,7 +742,7 @@ def main():
                    "device_resident_step": {
                        "ms_per_step": el_full / nfull * 1e3, "steps": nfull,
                        "particle_steps_per_s": npart * nfull / el_full,
-                       "what": "emg_solve_es (charge + background -> hipFFT Poisson -> E -> "
+                       "what": "emg_solve_es (charge + background -> spectral Poisson -> E -> "
                                "grdcrt) + emg_push_es (fused push + charge), fields on the "
                                "device"},
                    "fp64": fp64,
