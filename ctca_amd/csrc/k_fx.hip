@@ -1472,8 +1472,8 @@ __device__ __forceinline__ void range_load(const RangeDesc &d, const StateFx &in
 // bucket runs or an outbox puts a wave's lanes in one or a few buckets: each
 // group of equal buckets takes one atomic (one atomic per lane on one
 // counter made a re-bucketing of 268M particles take 145 ms instead of
-// 3.9).  The flat segments (an upload, the spill) are in no tile order, and
-// their lanes keep an atomic each.
+// 3.9).  The spill's lanes, in no tile order, keep an atomic each (a flat
+// upload's too where k_fx_*_flat do not take it).
 template <int T>
 __global__ __launch_bounds__(kBlock) void k_fx_hist(RangeDesc d, StateFx in, Grid g, int ntx,
                                                     int nty, int32_t *hist) {
@@ -1520,6 +1520,65 @@ __global__ __launch_bounds__(kBlock) void k_fx_scatter(RangeDesc d, StateFx in, 
     if (grouped) base = __shfl(base, lead);
     if (act)
       store_pcl(out, start[b] + base + inner, p.cell, p.pid, p.fx, p.fy, p.fz, p.vx, p.vy, p.vz);
+  }
+}
+
+// The same for an upload's flat segments, in no tile order: a block counts its
+// chunk's particles per tile in LDS and adds each tile's count with one atomic;
+// the scatter's atomics reserve the block's slots, which its particles then take
+// in LDS.  With one atomic per particle, many on each counter, the count took 209
+// us for 2 x 0.5M particles in 1,024 buckets and 3.9 ms for 2 x 33.6M in 8,192,
+// now 7 and 95 us.
+constexpr int kFlatPer = 4;
+template <int T>
+__device__ __forceinline__ void flat_count(const RangeDesc &d, const StateFx &in, const Grid &g,
+                                           int ntx, int nty, int s, int64_t beg, int64_t end,
+                                           int32_t *cnt) {
+  for (int t = threadIdx.x; t < d.ntiles; t += kBlock) cnt[t] = 0;
+  __syncthreads();
+  for (int64_t i0 = beg + threadIdx.x; i0 < end; i0 += kFlatPer * kBlock) {
+    int cell[kFlatPer];
+#pragma unroll
+    for (int u = 0; u < kFlatPer; u++)
+      cell[u] = in.cell[d.seg_start[s] + min(i0 + u * kBlock, end - 1)];
+#pragma unroll
+    for (int u = 0; u < kFlatPer; u++)
+      if (i0 + u * kBlock < end) atomicAdd(&cnt[tile_of_cell<T>(cell[u], g, ntx, nty)], 1);
+  }
+  __syncthreads();
+}
+
+template <int T>
+__global__ __launch_bounds__(kBlock) void k_fx_hist_flat(RangeDesc d, StateFx in, Grid g, int ntx,
+                                                         int nty, int64_t chunk, int32_t *hist) {
+  extern __shared__ int32_t cnt[];
+  const int s = blockIdx.y;
+  const int64_t beg = blockIdx.x * chunk, end = min(beg + chunk, d.seg_count[s]);
+  if (beg >= end) return;  // uniform
+  flat_count<T>(d, in, g, ntx, nty, s, beg, end, cnt);
+  for (int t = threadIdx.x; t < d.ntiles; t += kBlock)
+    if (cnt[t] > 0) atomicAdd(&hist[s * d.ntiles + t], cnt[t]);
+}
+
+template <int T>
+__global__ __launch_bounds__(kBlock) void k_fx_scatter_flat(RangeDesc d, StateFx in, StateFx out,
+                                                            Grid g, int ntx, int nty, int64_t chunk,
+                                                            const int64_t *start,
+                                                            int32_t *cursor) {
+  extern __shared__ int32_t cnt[];
+  const int s = blockIdx.y;
+  const int64_t beg = blockIdx.x * chunk, end = min(beg + chunk, d.seg_count[s]);
+  if (beg >= end) return;  // uniform
+  flat_count<T>(d, in, g, ntx, nty, s, beg, end, cnt);
+  for (int t = threadIdx.x; t < d.ntiles; t += kBlock)
+    if (cnt[t] > 0) cnt[t] = atomicAdd(&cursor[s * d.ntiles + t], cnt[t]);
+  __syncthreads();
+  for (int64_t i = beg + threadIdx.x; i < end; i += kBlock) {
+    Pcl p;
+    load_pcl(in, d.seg_start[s] + i, p);
+    const int t = tile_of_cell<T>(p.cell, g, ntx, nty);
+    store_pcl(out, start[s * d.ntiles + t] + atomicAdd(&cnt[t], 1), p.cell, p.pid, p.fx, p.fy, p.fz,
+              p.vx, p.vy, p.vz);
   }
 }
 
@@ -1741,6 +1800,28 @@ void step_t(emg_ctx *c, const FxArgs &a, bool push, int dep, unsigned grid) {
 }
 
 // bucket the particles described by d (reading buffer 'src') into buffer 1 - src
+constexpr int kFlatTiles = 16384;  // 64 KB of LDS counters
+// Particles per species up to which the flat scatter is the better one (an atomic
+// per particle : per block and tile, 2 x 0.9M in 432 buckets 797 : 128 us, 2 x
+// 6.4M in 1,512 2695 : 1791, 2 x 33.6M in 8,192 8340 : 11200): beyond the caches
+// the blocks' slots, reserved ahead, leave more lines written in parts.
+constexpr int64_t kFlatScatter = 1 << 23;
+
+template <int T>
+void launch_hist_flat(emg_ctx *c, const RangeDesc &d, int src, dim3 grid, size_t lds,
+                      int64_t chunk) {
+  FxBuckets &B = c->fx;
+  hipLaunchKernelGGL(k_fx_hist_flat<T>, grid, dim3(kBlock), lds, c->stream, d, B.st[src], c->g,
+                     B.ntx, B.nty, chunk, B.hist);
+}
+template <int T>
+void launch_scatter_flat(emg_ctx *c, const RangeDesc &d, int src, dim3 grid, size_t lds,
+                         int64_t chunk) {
+  FxBuckets &B = c->fx;
+  hipLaunchKernelGGL(k_fx_scatter_flat<T>, grid, dim3(kBlock), lds, c->stream, d, B.st[src],
+                     B.st[1 - src], c->g, B.ntx, B.nty, chunk, B.start[1 - src], B.cursor);
+}
+
 int bucket_ranges(emg_ctx *c, RangeDesc d, int nr, int rb, int src) {
   FxBuckets &B = c->fx;
   int dst = 1 - src;
@@ -1748,7 +1829,19 @@ int bucket_ranges(emg_ctx *c, RangeDesc d, int nr, int rb, int src) {
   unsigned grid = (unsigned)((int64_t)nr * rb);
   unsigned gb = (unsigned)((B.nb + kBlock - 1) / kBlock);
   launch_zero(B.hist, sizeof(int32_t) * B.nb, c->stream);
-  switch (B.tile) {
+  // an upload's chunks: for the count 1,024 per species at most, of 4,096 particles
+  // and four per tile at least
+  int64_t most = 0;
+  for (int s = 0; s < d.nspec; s++) most = std::max(most, d.seg_count[s]);
+  const bool flat = d.nrb == 0 && d.nob == 0 && !d.seg_count_dev && d.ntiles <= kFlatTiles;
+  const int64_t chunk =
+      std::max<int64_t>({4096, (int64_t)4 * d.ntiles, (most + 1023) / 1024});
+  const dim3 fg((unsigned)std::max<int64_t>(1, (most + chunk - 1) / chunk), (unsigned)d.nspec);
+  const size_t flds = sizeof(int32_t) * d.ntiles;
+  if (flat)
+    B.tile == 4 ? launch_hist_flat<4>(c, d, src, fg, flds, chunk)
+                : launch_hist_flat<8>(c, d, src, fg, flds, chunk);
+  else switch (B.tile) {
     case 4:
       hipLaunchKernelGGL(k_fx_hist<4>, dim3(grid), dim3(kBlock), 0, c->stream, d, B.st[src], c->g,
                          B.ntx, B.nty, B.hist);
@@ -1764,7 +1857,12 @@ int bucket_ranges(emg_ctx *c, RangeDesc d, int nr, int rb, int src) {
                      B.spill[dst], B.shist[dst], B.nb, c->sp.nspec);
   hipLaunchKernelGGL(k_fill_i32, dim3(gb), dim3(kBlock), 0, c->stream, B.cursor, (int64_t)B.nb, 0);
   exclusive_scan_i32(B.cap[dst], B.start[dst], B.nb, c->scan_tmp, c->stream);
-  switch (B.tile) {
+  const int64_t schunk = std::max<int64_t>(2048, d.ntiles);
+  const dim3 sg((unsigned)std::max<int64_t>(1, (most + schunk - 1) / schunk), (unsigned)d.nspec);
+  if (flat && most <= kFlatScatter)
+    B.tile == 4 ? launch_scatter_flat<4>(c, d, src, sg, flds, schunk)
+                : launch_scatter_flat<8>(c, d, src, sg, flds, schunk);
+  else switch (B.tile) {
     case 4:
       hipLaunchKernelGGL(k_fx_scatter<4>, dim3(grid), dim3(kBlock), 0, c->stream, d, B.st[src],
                          B.st[dst], c->g, B.ntx, B.nty, B.start[dst], B.cursor);

@@ -129,3 +129,36 @@ def test_plan_replayed_from_a_graph():
     ctx.close()
     for a, b in zip(got, want):
         assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("n,counts,tile", [
+    ((16, 16, 16), (1, 0), 4),
+    ((16, 12, 8), (2049, 2047), 4),          # chunk edges
+    ((40, 40, 40), (30000, 4097), 4),        # many tiles, few particles in each
+    ((128, 128, 64), (5000, 20000), 4),      # as many tiles as LDS counters, and more
+    ((128, 104, 80), (5000, 20000), 4),
+    ((24, 24, 24), (8388609, 10), 8),        # past the flat scatter's particles
+])
+def test_upload_reaches_the_buckets(n, counts, tile):
+    """Every uploaded particle in its bucket: the charge of each species and the
+    records that come back."""
+    from ctca_amd import emg
+    rng = np.random.default_rng(sum(counts))
+    total = sum(counts)
+    rec = np.zeros(total, dtype=emg.PARTICLE)
+    for c, m in zip("xyz", n):
+        rec[c] = rng.integers(0, m * 4096, total) / 4096.0   # exact in FP32
+    rec["vx"] = np.arange(total) % 4093 / 4096.0
+    rec["pid"] = np.arange(total)
+    with emg.Context(n, [1.0, -1.0], [0.0, 0.0], [1.0, 1.0], counts, precision=emg.FP32_FIXED,
+                     tile=tile, track_pid=True) as ctx:
+        ctx.upload(rec, counts)
+        ctx.deposit_rho(0)
+        for s in range(2):
+            assert abs(ctx.rho(species=s)).sum() == pytest.approx(counts[s], rel=1e-12)
+        got, cnt = ctx.download()
+    assert list(cnt) == list(counts)
+    back = np.empty_like(got)
+    back[got["pid"]] = got
+    for f in ("x", "y", "z", "vx", "pid"):
+        assert np.array_equal(back[f], rec[f])
