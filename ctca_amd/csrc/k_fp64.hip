@@ -618,9 +618,13 @@ __device__ __forceinline__ Relay relay_axis(double xnew, double lb, double cb, i
 // The zigzag sums of a block's particles go to an LDS window (three
 // components, shaped like the charge window) as int64 fixed
 // point at 2^48 per unit, and reach the global FP64 sums once per window
-// node.  A contribution is |vv w| <= 4 in the window (larger fluxes go
-// straight to the global sums), so a node's window sum of at most
-// kRunMax[1] particles' terms (twice 8 2^48) stays below 2^63; the rounding of each term
+// node.  A segment is summed in the window if its midpoint's offsets from the
+// cell are in [-1/2, 3/2] on all axes, as they are for moves of up to two cells
+// that stay in the box (a longer one has its relay point at the far cell or face,
+// and weights as large as the move; it goes straight to the global sums).  Its
+// length is then at most 3 per axis and its weights at most (3/2)^2, so |vv w| <=
+// 6.75 < 8 as win_fix needs, and a node's sum of at most kRunMax[1] particles'
+// terms (two of 6.75 2^48 each) stays below 2^63; the rounding of each term
 // (2^-49) is far below the FP64 summation round-off of the reference's order.
 constexpr double kEmFix = 281474976710656.0;          // 2^48
 
@@ -750,20 +754,21 @@ void k_push_em64(State64 s, SpeciesTab sp,
         atomicAdd(jz + cidx(g, i1, j1, k), value(2, 3));
       }
     };
-    auto small = [](double a, double b, double c) {
-      return fabs(a) <= 4.0 && fabs(b) <= 4.0 && fabs(c) <= 4.0;
+    auto near = [](double a, double b, double c) {
+      return fabs(a - 0.5) <= 1.0 && fabs(b - 0.5) <= 1.0 && fabs(c - 0.5) <= 1.0;
     };
-    // a particle that stays in its cell has both segments there: one sum (of
-    // at most 2 cells per step) per node, the second segment's own sums only
-    // for the particles that changed cell
+    const bool near2 = near(xd2, yd2, zd2);
+    // a particle that stays in its cell has both segments there: one sum (of a
+    // move within the cell, or beyond the face from a position of exactly L) per
+    // node, the second segment's own sums only for the particles that changed cell
     const bool same = rx.ia == ib && ry.ia == jb && rz.ia == kb;
     const double sx2 = same ? vvx2 : 0.0, sy2 = same ? vvy2 : 0.0, sz2 = same ? vvz2 : 0.0;
-    seg(ib, jb, kb, small(vvx1, vvy1, vvz1) && small(sx2, sy2, sz2) , [&](int c, int k) {
+    seg(ib, jb, kb, near(xd1, yd1, zd1) && (!same || near2), [&](int c, int k) {
       return c == 0 ? vvx1 * ax1[k] + sx2 * ax2[k]
                     : (c == 1 ? vvy1 * ay1[k] + sy2 * ay2[k] : vvz1 * az1[k] + sz2 * az2[k]);
     });
     if (!same)
-      seg(rx.ia, ry.ia, rz.ia, small(vvx2, vvy2, vvz2), [&](int c, int k) {
+      seg(rx.ia, ry.ia, rz.ia, near2, [&](int c, int k) {
         return c == 0 ? vvx2 * ax2[k] : (c == 1 ? vvy2 * ay2[k] : vvz2 * az2[k]);
       });
   }
