@@ -87,7 +87,6 @@ struct FxBuckets {
   FxRec *spl;          // [nspec * spill_cap] the spill particles sorted by bucket
   StateFx st[2];
   int cur;             // buffer holding the live particles
-  bool planned;        // the other buffer is laid out for the next step
   unsigned long long *plan_word;    // [plan blocks] look-back words
   unsigned long long *plan_ticket;  // blocks of plan launches started so far
 };

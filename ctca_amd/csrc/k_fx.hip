@@ -1670,7 +1670,9 @@ __global__ void k_copy_i32(const int32_t *src, int n, int32_t *dst) {
 int64_t plan_blocks(int nb) { return (nb + kBlock - 1) / kBlock; }
 
 // lay out the buffer that the next step writes (finish: close the step that
-// wrote the live buffer)
+// wrote the live buffer).  Whatever changes the live buffer ends with this, so
+// that a step needs no other launches after an upload or a sort than after a
+// step: a graph recorded at one of these points may be replayed at another.
 void launch_plan(emg_ctx *c, bool finish) {
   FxBuckets &B = c->fx;
   const int L = B.cur, X = 1 - B.cur;
@@ -1699,7 +1701,6 @@ void launch_plan(emg_ctx *c, bool finish) {
   p.word = B.plan_word;
   p.ticket = B.plan_ticket;
   hipLaunchKernelGGL(k_fx_plan, dim3((unsigned)plan_blocks(B.nb)), dim3(kBlock), 0, c->stream, p);
-  B.planned = true;
 }
 
 FxArgs make_args(emg_ctx *c) {
@@ -1879,7 +1880,6 @@ int bucket_ranges(emg_ctx *c, RangeDesc d, int nr, int rb, int src) {
   hipLaunchKernelGGL(k_fill_i32, dim3((unsigned)((npre + kBlock - 1) / kBlock)), dim3(kBlock), 0,
                      c->stream, B.pre[dst], npre, 0);
   B.cur = dst;
-  B.planned = false;
   return hip_check(hipGetLastError(), "bucketing");
 }
 
@@ -2013,7 +2013,6 @@ int fx_alloc(emg_ctx *c, int64_t ntotal) {
     return set_error(EMG_ERR_NOMEM, "energy partials");
   c->ke_part_n = kp;
   B.cur = 0;
-  B.planned = false;
   return EMG_OK;
 }
 
@@ -2034,22 +2033,32 @@ int fx_from64(emg_ctx *c, const State64 &src) {
     d.seg_start[s] = c->sp.off[s];
     d.seg_count[s] = c->sp.cnt[s];
   }
-  return bucket_ranges(c, d, c->sp.nspec, 2048, flat);
+  const int rc = bucket_ranges(c, d, c->sp.nspec, 2048, flat);
+  if (!rc) launch_plan(c, false);
+  return rc;
 }
 
 // bucketed FP32 (runs, outboxes, spill) -> one run per bucket, nothing pending
-int fx_rebucket(emg_ctx *c) {
+static int gather_buckets(emg_ctx *c) {
   return bucket_ranges(c, bucket_desc(c), 2 * c->fx.nb + c->sp.nspec, 1, c->fx.cur);
+}
+
+int fx_rebucket(emg_ctx *c) {
+  const int rc = gather_buckets(c);
+  if (!rc) launch_plan(c, false);
+  return rc;
 }
 
 int fx_to64(emg_ctx *c, State64 &dst) {
   FxBuckets &B = c->fx;
-  int rc = fx_rebucket(c);
+  int rc = gather_buckets(c);
   if (rc) return rc;
+  // (the scan's output is the other buffer's bucket starts: laid out after it)
   exclusive_scan_i32(B.count[B.cur], B.start[1 - B.cur], B.nb, c->scan_tmp, c->stream);
   hipLaunchKernelGGL(k_fx_to64, dim3(B.nb), dim3(kBlock), 0, c->stream, B.st[B.cur],
                      B.start[B.cur], B.count[B.cur], B.start[1 - B.cur], B.ntiles, c->sp, c->g,
                      dst);
+  launch_plan(c, false);
   return hip_check(hipGetLastError(), "fx_to64");
 }
 
@@ -2059,7 +2068,6 @@ void launch_fx_step(emg_ctx *c, int ustep, bool push, bool deposit, bool em) {
   FxBuckets &B = c->fx;
   const int dep = em ? 2 : (deposit ? 1 : 0);
   const int in = B.cur;
-  if (!B.planned) launch_plan(c, false);  // after a bucketing
   const int64_t words = dep == 0 ? 0 : (dep == 1 ? 1 : 3) * c->ncell * c->sp.nspec;
   const int zb = (int)std::min<int64_t>((words / 2 + kBlock - 1) / kBlock + (words & 1), 4096);
   const dim3 pg((unsigned)(zb + kSpillBlocksPerSpecies * c->sp.nspec));

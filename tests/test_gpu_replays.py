@@ -1,0 +1,83 @@
+"""Graphs of steps replayed after the program has changed the particles or the
+fields eagerly: equal to the same calls without a graph."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+class Recorded:
+    """What `calls` launches on a context, recorded once and replayed."""
+
+    def __init__(self, ctx, calls):
+        import torch
+        from ctca_amd import emg
+        self.torch, self.stream = torch, torch.cuda.Stream()
+        emg.lib().emg_set_stream(ctx.h, self.stream.cuda_stream)
+        self.graph = torch.cuda.CUDAGraph()
+        with torch.cuda.stream(self.stream):
+            self.graph.capture_begin()
+            calls()
+            self.graph.capture_end()
+
+    def __call__(self):
+        with self.torch.cuda.stream(self.stream):
+            self.graph.replay()
+
+
+def need_torch():
+    import torch
+    if not torch.cuda.is_available():
+        pytest.skip("the library initialised the device before torch")
+
+
+@pytest.mark.parametrize("em", [False, True])
+def test_fp32_steps_recorded_after_a_step_and_replayed_after_an_upload(em):
+    need_torch()
+    from ctca_amd import emg
+    n, counts = (24, 20, 16), (30000, 9000)
+    rng = np.random.default_rng(31)
+    eb = np.zeros((n[2] + 3, n[1] + 3, n[0] + 3, 6))
+
+    def records(part):
+        """particles in `part` of the box, with moves of up to a cell or two"""
+        r = np.zeros(sum(counts), dtype=emg.PARTICLE)
+        for c, m in zip("xyz", n):
+            r[c] = rng.random(sum(counts)) * m * part
+            r["v" + c] = rng.normal(size=sum(counts)) * 0.15
+        return r
+
+    sets = [records(1.0), records(0.4), records(0.7)]
+
+    def program(ctx, recorded):
+        push = ctx.push_em if em else ctx.push_es
+
+        def steps():
+            for _ in range(4):     # an even number: two state buffers
+                push(2)
+
+        out = []
+        ctx.upload(sets[0], counts)
+        ctx.set_fields(eb)
+        push(2)
+        push(2)
+        four = Recorded(ctx, steps) if recorded else steps
+        for k in range(4):
+            four()
+            push(2)
+            push(2)
+            out.append(ctx.current() if em else ctx.rho())
+            if k < 2:
+                ctx.upload(sets[k + 1], counts)
+            else:
+                ctx.sort()
+                ctx.sort()
+        return out
+
+    got = []
+    for recorded in (False, True):
+        with emg.Context(n, [1.0, -1.0], [0.0, 0.0], [1.0, 1.0], counts,
+                         precision=emg.FP32_FIXED) as ctx:
+            got.append(program(ctx, recorded))
+    for a, b in zip(*got):         # integer sums: in any order
+        assert np.array_equal(a, b)
