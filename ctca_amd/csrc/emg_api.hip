@@ -211,6 +211,14 @@ int flags_error(emg_ctx *c) {
   return set_error(EMG_ERR_HIP, "unknown device flag");
 }
 
+bool capturing(emg_ctx *c) {
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(c->stream, &st) == hipSuccess && st == hipStreamCaptureStatusNone)
+    return false;
+  (void)hipGetLastError();
+  return true;
+}
+
 }  // namespace emg
 
 using namespace emg;
@@ -683,6 +691,7 @@ int emg_bfield(emg_ctx *c) {
   if (rc) return rc;
   launch_bfield(c);
   c->nodes_b_valid = false;
+  c->b_recorded = c->b_recorded || capturing(c);
   c->nodes_stale = true;
   return hip_check(hipGetLastError(), "bfield launch");
 }

@@ -452,6 +452,7 @@ struct emg_ctx {
   double *eb_stage;  // an uploaded eb in the boundary's layout (lazy)
   size_t eb_stage_bytes;
   bool nodes_b_valid;  // the nodes' B is the relocation of eb_dev's B
+  bool b_recorded;     // a graph holds an emg_bfield: its replays change eb_dev's B unseen
   int eb_lo[3], eb_ext[3];
   bool nodes_stale;  // eb changed on the device since the last relocation
   double *fe_buf;    // field-energy partials and result (lazy)
@@ -516,6 +517,7 @@ int set_error(int code, const std::string &msg);
 int hip_check(hipError_t e, const char *what);
 
 int flags_error(emg_ctx *c);  // *hflag as an error code (and dflag cleared)
+bool capturing(emg_ctx *c);   // whether the stream's work is being recorded into a graph
 
 // Host transfers (emg_io.hip) in chunks of whole units.  fill enqueues on the
 // context's stream what writes bytes [off, off + len) of the result to the

@@ -908,11 +908,7 @@ int sort64_runs(emg_ctx *c, int which) {
   if (!c->runs_valid || c->nruns[which] != kRunsUnbuilt) return EMG_OK;
   // building reads a count back, which a captured stream cannot: the launches
   // recorded now keep plain slices
-  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-  if (hipStreamIsCapturing(c->stream, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone) {
-    (void)hipGetLastError();
-    return EMG_OK;
-  }
+  if (capturing(c)) return EMG_OK;
   timer_begin(c, kTSort);
   const int rc = build_runs(c, which);
   timer_end(c, kTSort);

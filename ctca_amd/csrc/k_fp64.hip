@@ -903,7 +903,7 @@ void launch_relocate64(emg_ctx *c) {
                      c->cfg.precision == EMG_FP32_FIXED ? c->node32 : nullptr, c->ncell, f.e0[0],
                      f.e0[1], f.e0[2], f.b0[0], f.b0[1], f.b0[2]);
   timer_end(c, kTRelocate);
-  c->nodes_b_valid = true;
+  if (!capturing(c)) c->nodes_b_valid = true;  // (recorded, not done)
 }
 
 void launch_positn64(emg_ctx *c, int ustep) {
@@ -944,9 +944,8 @@ static bool tiles64(emg_ctx *c) {
   for (int s = 0; s < c->sp.nspec; s++) total += c->sp.cnt[s];
   if (c->runs_valid || c->ordered || total < kTileMin) return false;
   if (!c->bins.rec) {
-    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(c->stream, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone ||
-        bins_alloc(c) != EMG_OK) {
+    if (capturing(c)) return false;
+    if (bins_alloc(c) != EMG_OK) {
       (void)hipGetLastError();
       return false;
     }

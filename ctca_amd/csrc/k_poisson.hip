@@ -602,7 +602,9 @@ int solve_es(emg_ctx *c, double rhobk) {
                      c->stream, s->rho, v, fix ? nullptr : c->node64, fix ? c->node32 : nullptr,
                      c->ncell, c->cfg.e0[0], c->cfg.e0[1], c->cfg.e0[2]);
   timer_end(c, kTRelocate);
-  if (!c->nodes_b_valid) launch_relocate64(c);
+  // the nodes' B as well where it may be another one; always in a recorded solve,
+  // which may be replayed after a B update that this call cannot know of
+  if (!c->nodes_b_valid || c->b_recorded || capturing(c)) launch_relocate64(c);
   return hip_check(hipGetLastError(), "field solve launch");
 }
 

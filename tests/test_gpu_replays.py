@@ -3,6 +3,12 @@ fields eagerly: equal to the same calls without a graph."""
 import numpy as np
 import pytest
 
+try:
+    import torch
+    torch.cuda.is_available()   # before the library initialises the device
+except ImportError:
+    pass
+
 pytestmark = pytest.mark.gpu
 
 
@@ -81,3 +87,52 @@ def test_fp32_steps_recorded_after_a_step_and_replayed_after_an_upload(em):
             got.append(program(ctx, recorded))
     for a, b in zip(*got):         # integer sums: in any order
         assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+def test_recorded_solves_replayed_after_b_updates(precision):
+    need_torch()
+    from ctca_amd import emg
+    n, counts = (16, 20, 12), (9000, 4000)
+    rng = np.random.default_rng(5)
+    core = rng.normal(size=(n[2], n[1], n[0], 6)) * 0.1
+    at = [np.arange(-1, v + 2) % v for v in n]
+    eb = np.ascontiguousarray(core[np.ix_(at[2], at[1], at[0])])
+    rec = np.zeros(sum(counts), dtype=emg.PARTICLE)
+    for c, m in zip("xyz", n):
+        rec[c] = rng.random(sum(counts)) * m
+        rec["v" + c] = rng.normal(size=sum(counts)) * 0.1
+
+    def program(ctx, recorded):
+        def steps():
+            for _ in range(2):
+                ctx.solve_es(0.1)
+                ctx.push_es(2)
+
+        ctx.upload(rec, counts)
+        ctx.set_fields(eb)
+        ctx.deposit_rho(0)
+        ctx.solve_es(0.1)
+        ctx.push_es(2)
+        ctx.push_es(2)
+        two = Recorded(ctx, steps) if recorded else steps
+        two()
+        ctx.set_fields(eb)     # E anew, so that B changes by its curl
+        ctx.bfield()
+        ctx.grdcrt()
+        ctx.push_es(2)
+        ctx.push_es(2)
+        ctx.bfield()
+        two()
+        two()
+        return ctx.energy(), ctx.fields()
+
+    out = []
+    for recorded in (False, True):
+        with emg.Context(n, [0.02, -0.02], [1.0, -1.0], [1.0, 1.0], counts,
+                         precision=emg.PLAIN_FP64 if precision == "fp64" else emg.FP32_FIXED) as c:
+            out.append(program(c, recorded))
+    # the same kernels: sums of atomics in another order at most (FP64), or the
+    # energy's partial sums of particles in another order (FP32)
+    for a, b in zip(*out):
+        assert np.abs(a - b).max() <= 1e-12 * np.abs(a).max()

@@ -21,3 +21,34 @@ def test_fp32_steps_launch_the_same_after_every_change_of_the_particles(tmp_path
                     change()
                     assert launches(push, 2) == first
     """)
+
+
+def test_a_field_solve_relocates_b_where_a_replay_may_meet_another_one(tmp_path):
+    fake_hip.run(tmp_path, """
+        n, counts = (16, 16, 16), (2000, 1000)
+        for precision in (emg.PLAIN_FP64, emg.FP32_FIXED):
+            with emg.Context(n, [1.0, -1.0], [1.0, 1.0], [1.0, 1.0], counts,
+                             precision=precision) as c:
+                def all_nodes(f, *a):
+                    return "k_relocate" in launches(f, *a)
+
+                c.upload(records(3000, n), counts)
+                c.set_fields(np.zeros((19, 19, 19, 6)))
+                c.push_es(2)
+                assert not all_nodes(c.solve_es, 0.0)  # B is that of set_fields
+                fake.fake_capture(1)
+                assert all_nodes(c.solve_es, 0.0)
+                fake.fake_capture(0)
+                assert not all_nodes(c.solve_es, 0.0)
+                c.bfield()
+                fake.fake_capture(1)
+                c.grdcrt()                             # recorded, not done
+                fake.fake_capture(0)
+                assert all_nodes(c.solve_es, 0.0)
+                assert not all_nodes(c.solve_es, 0.0)
+                fake.fake_capture(1)
+                c.bfield()
+                fake.fake_capture(0)
+                c.grdcrt()
+                assert all_nodes(c.solve_es, 0.0)      # a replay may have been here
+    """)
