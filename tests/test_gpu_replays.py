@@ -3,13 +3,14 @@ fields eagerly: equal to the same calls without a graph."""
 import numpy as np
 import pytest
 
-try:
-    import torch
-    torch.cuda.is_available()   # before the library initialises the device
-except ImportError:
-    pass
-
 pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module", autouse=True)
+def torch_first():
+    """torch has to see the device before the library initialises it."""
+    import torch
+    torch.cuda.is_available()
 
 
 class Recorded:
