@@ -286,11 +286,11 @@ class Context:
         self.deposit_rho(func)
         lo, hi = (-1, -1, -1), tuple(v + 1 for v in self.n)
         if func in (0, 2):
-            self._rho_into(rho, lo, hi, None)
+            self._rho_into(rho, ..., lo, hi, None)
         if func in (1, 2):
             rhodg[self.nspec:] = 0.0
             for k in range(self.nspec):
-                self._rho_into(rhodg[k], lo, hi, k)
+                self._rho_into(rhodg, k, lo, hi, k)
 
     def push_em(self, ustep):
         _chk(lib().emg_push_em(self.h, int(ustep)))
@@ -363,16 +363,19 @@ class Context:
             _chk(lib().emg_get_rhodg(self.h, int(species), _ptr(out), _i3(lo), _i3(hi)))
         return out
 
-    def _rho_into(self, dst, lo, hi, species):
-        """rho(lo, hi, species) written into dst, directly where dst's memory
-        is what the library writes."""
-        if dst.dtype == np.float64 and dst.flags.c_contiguous and dst.flags.writeable:
+    def _rho_into(self, arr, at, lo, hi, species):
+        """arr[at] = rho(lo, hi, species), written there directly where that is
+        memory of a plain numpy array as the library fills it (another kind of
+        array may hand out a copy, or keep more than its values)."""
+        dst = arr[at] if type(arr) is np.ndarray else None
+        if dst is not None and dst.dtype == np.float64 and dst.flags.c_contiguous \
+                and dst.flags.writeable:
             if species is None:
                 _chk(lib().emg_get_rho(self.h, _ptr(dst), _i3(lo), _i3(hi)))
             else:
                 _chk(lib().emg_get_rhodg(self.h, int(species), _ptr(dst), _i3(lo), _i3(hi)))
         else:
-            dst[...] = self.rho(lo, hi, species)
+            arr[at] = self.rho(lo, hi, species)
 
     def rho_noalloc(self, lo=None, hi=None):
         """rho(1, lo:hi)^3 like rho(), read through emg_get_rho_noalloc (no
