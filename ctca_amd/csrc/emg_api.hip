@@ -470,7 +470,7 @@ int emg_set_stream(emg_ctx *c, void *stream) {
     if (rc) return rc;
     c->own_stream = true;
   }
-  return EMG_OK;
+  return es_solver_stream(c);
 }
 
 int emg_synchronize(emg_ctx *c) {

@@ -564,6 +564,7 @@ void launch_field_energy(emg_ctx *c, double cs, double *part_dev, double *out);
 // phi -> E into eb_dev -> nodes
 int solve_es(emg_ctx *c, double rhobk);
 int read_potential(emg_ctx *c, double *phi);
+int es_solver_stream(emg_ctx *c);  // after c->stream has changed
 void es_solver_free(emg_ctx *c);
 
 // common kernels (k_common.hip)

@@ -461,14 +461,21 @@ static void with_kind(int kind, F f) {
     f(std::integral_constant<int, 2>());
 }
 
+// the plans keep the stream they are given: again when the context's changes
+int es_solver_stream(emg_ctx *c) {
+  EsSolver *s = c->es;
+  int rc = EMG_OK;
+  if (s && s->have_fwd) rc = fft_check(hipfftSetStream(s->fwd, c->stream), "set stream");
+  if (!rc && s && s->have_inv) rc = fft_check(hipfftSetStream(s->inv, c->stream), "set stream");
+  return rc;
+}
+
 static int es_fft_plans(emg_ctx *c, EsSolver *s) {
   int rc = fft_check(hipfftPlan3d(&s->fwd, c->g.nz, c->g.ny, c->g.nx, HIPFFT_D2Z), "plan D2Z");
   if (!rc) s->have_fwd = true;
   if (!rc) rc = fft_check(hipfftPlan3d(&s->inv, c->g.nz, c->g.ny, c->g.nx, HIPFFT_Z2D), "plan Z2D");
   if (!rc) s->have_inv = true;
-  if (!rc) rc = fft_check(hipfftSetStream(s->fwd, c->stream), "set stream");
-  if (!rc) rc = fft_check(hipfftSetStream(s->inv, c->stream), "set stream");
-  return rc;
+  return rc ? rc : es_solver_stream(c);
 }
 
 static int es_solver_get(emg_ctx *c, EsSolver **out) {
