@@ -67,7 +67,10 @@ inline bool fft_axis(int n, int largest, FftAxis *a) {
       n /= r;
     }
   };
-  for (int p = 17; p <= largest; p += 2) take(p);
+  // the large primes (an odd p without these factors is one, or a product of
+  // primes that have been taken)
+  for (int p = 17; p <= largest; p += 2)
+    if (p % 3 && p % 5 && p % 7 && p % 11 && p % 13) take(p);
   // 16 = 4 x 4 and not 8 x 2
   if (n % 16 == 0 && n % 32 != 0) take(4);
   take(8);

@@ -427,28 +427,33 @@ static size_t column_lds(int n) {
   return (sizeof(double2) * (2 * kColumns + 1) + sizeof(double)) * (size_t)n;
 }
 
-// Which one is the fastest.  Solve, E included, hipFFT against planes: 16^3 cells
-// 21.4 : 18.5 us, 32^3 24.7 : 20.0, 48^3 32.5 : 27.1, 64^3 37.4 : 31.0, 80^3
-// 52.6 : 47.1, 96^3 78.9 : 56.8, 128x64x64 52.7 : 46.6, 77x63x70 72 : 44; larger
-// planes with factors of 7 to 17 are the exception (90x70x51 46.9 : 49.7,
-// 98x98x50 52.3 : 59.3).  From a prime factor of 19 on hipFFT changes to a longer
-// algorithm: 31^3 83 : 24, 53^3 152 : 37; there the lines do the planes' work
-// from 3000 elements of a plane on (hipFFT : planes : lines, 62^3 129 : 40 : 41,
-// 95x66x40 87 : 49 : 41; 114x95x133 252 : - : 111, 191x181x173 1148 : - : 619).
-// Without such a factor the lines gain nothing (256x256x64 206 : 214, 180x150x170
-// 233 : 288).  The first solve also has no kernels to compile at run time (1.6 s :
-// 0.2 ms).
+// Which one is the fastest.  Solve, E included, hipFFT : planes : lines in us.
+// Planes where LDS holds them: 16^3 cells 19.3 : 17.7 : 22.0, 32^3 22.3 : 19.4 :
+// 24.1, 64^3 36.7 : 29.9 : 36.4, 90x70x51 46.8 : 44.9 : 46.5, 77x63x70 72 : 42 :
+// 47, 84^3 57 : 50 : 58, 88^3 69 : 47 : 64, 96^3 73 : 54 : 63 (98x98x50 is the
+// exception, 51 : 57 : 57).
+// From a prime factor of 19 on hipFFT changes to a longer algorithm: 31^3 117 : 23
+// : 28, 53^3 150 : 36 : 43; there the lines do the work of planes of more than
+// 3000 elements (62^3 128 : 38 : 38, 101x40x40 74 : 38 : 40, 95x66x40 87 : 43 : 38,
+// 97x98x50 113 : 78 : 62) and of those that LDS does not hold (114x95x133 252 : -
+// : 112, 191x181x173 1141 : - : 596).
+// An odd nx costs hipFFT's real transforms about twice an even one, and the lines
+// nothing: 105x100x100 131 : - : 88, 125^3 154 : - : 99, 143x119x130 217 : - : 133,
+// 225^3 1204 : - : 503.  Else the two are close (110^3 106 : - : 99, 112^3 94 : - :
+// 102, 126^3 127 : - : 109, 130x143x119 129 : - : 145, 150^3 155 : - : 152,
+// 180x150x170 219 : - : 251, 200^3 323 : - : 326, 256x256x64 194 : - : 200).
+// The first solve of planes and lines also has no kernels to compile at run time
+// (1.6 s : 0.2 ms).
 static SolvePath solve_path(const Grid &g, FftAxis ax[3]) {
   const int n[3] = {g.nx, g.ny, g.nz};
-  int largest = 0, kind = 0;
+  int largest = 0;
   for (int d = 0; d < 3; d++) {
     if (n[d] > kLongestLine || !fft_axis(n[d], kLargestRadix, &ax[d])) return kLibrary;
-    kind = std::max(kind, radix_kind(ax[d]));
     for (int p = 0; p < ax[d].npass; p++) largest = std::max(largest, ax[d].r[p]);
   }
-  if (plane_lds(g, kPlanes) <= kPlaneLds && (kind < 2 || plane_elems(g, kPlanes) <= 3000))
+  if (plane_lds(g, kPlanes) <= kPlaneLds && (largest < 19 || plane_elems(g, kPlanes) <= 3000))
     return kPlanes;
-  return largest >= 19 ? kLines : kLibrary;
+  return largest >= 19 || g.nx % 2 ? kLines : kLibrary;
 }
 
 template <class F>
