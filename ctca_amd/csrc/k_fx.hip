@@ -1907,6 +1907,8 @@ int fx_alloc(emg_ctx *c, int64_t ntotal) {
   FxBuckets &B = c->fx;
   const Grid &g = c->g;
   int T = c->cfg.tile;
+  int64_t nt8 = 0;
+  bool few = false;
   if (T <= 0) {  // default
     const bool m8 = g.nx % 8 == 0 && g.ny % 8 == 0 && g.nz % 8 == 0;
     const bool m4 = g.nx % 4 == 0 && g.ny % 4 == 0 && g.nz % 4 == 0;
@@ -1916,9 +1918,9 @@ int fx_alloc(emg_ctx *c, int64_t ntotal) {
     // (the results do not depend on the tile).  Step kernel, 8^3 against 4^3
     // tiles: 16^3 cells 39 : 19 us, 24^3 42 : 21, 32^3 48 : 28 (16 blocks, 54,
     // 128); 48^3 67 : 70, 64^3 138 : 163 (432, 1024).
-    const int64_t nb8 = (int64_t)((g.nx + 7) / 8) * ((g.ny + 7) / 8) * ((g.nz + 7) / 8) *
-                        c->sp.nspec;
-    if (T == 8 && nb8 < 256) T = 4;
+    nt8 = (int64_t)((g.nx + 7) / 8) * ((g.ny + 7) / 8) * ((g.nz + 7) / 8);
+    few = T == 8 && nt8 * c->sp.nspec < 256;
+    if (few) T = 4;
   }
   if (T != 4 && T != 8) return set_error(EMG_ERR_ARG, "tile must be 4 or 8");
   // a grid that is not a multiple of T ends in partial tiles; the tile and
@@ -1944,7 +1946,12 @@ int fx_alloc(emg_ctx *c, int64_t ntotal) {
   B.area = align_up(ntotal + (int64_t)(kExtra + kAlign - 1) * B.nb);
   int64_t maxs = 0;
   for (int s = 0; s < c->sp.nspec; s++) maxs = c->cfg.capacity[s] > maxs ? c->cfg.capacity[s] : maxs;
-  B.spill_cap = align_up(maxs / 16 + 4096);
+  B.spill_cap = maxs / 16 + 4096;
+  // 4^3 tiles in place of 8^3 ones keep what those would: evenly spread particles
+  // leave a tile of 4, or pass the cell beyond it, at most twice as often as one
+  // of 8, which has kObStride + kExtra places and its share of the spill for them
+  if (few) B.spill_cap = std::min(maxs, 2 * (B.spill_cap + (kObStride + kExtra) * nt8));
+  B.spill_cap = align_up(B.spill_cap);
   if (B.spill_cap > (1 << 28)) B.spill_cap = 1 << 28;
   B.cap_total = B.area + B.spill_cap * c->sp.nspec;
   // the step's capacity scan packs two sums into one 64-bit term (the first
