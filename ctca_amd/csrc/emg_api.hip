@@ -156,28 +156,13 @@ __global__ __launch_bounds__(kBlock) void k_join(State64 st, int64_t src0, int64
 
 template <typename T>
 int dalloc(T **p, size_t count, const char *what) {
-  *p = nullptr;
   if (count == 0) count = 1;
-  hipError_t e = hipMalloc((void **)p, sizeof(T) * count);
-  if (e != hipSuccess) {
-    *p = nullptr;
-    return set_error(EMG_ERR_NOMEM, std::string("device allocation failed: ") + what);
-  }
-  return EMG_OK;
+  if (dev_malloc(p, sizeof(T) * count)) return EMG_OK;
+  return set_error(EMG_ERR_NOMEM, std::string("device allocation failed: ") + what);
 }
 
 void dfree(void *p) {
   if (p) (void)hipFree(p);
-}
-
-int alloc_state64(State64 &st, int64_t cap) {
-  int rc;
-  if ((rc = dalloc(&st.x, cap, "x")) || (rc = dalloc(&st.y, cap, "y")) ||
-      (rc = dalloc(&st.z, cap, "z")) || (rc = dalloc(&st.vx, cap, "vx")) ||
-      (rc = dalloc(&st.vy, cap, "vy")) || (rc = dalloc(&st.vz, cap, "vz")) ||
-      (rc = dalloc(&st.pid, cap, "pid")))
-    return rc;
-  return EMG_OK;
 }
 
 void free_state64(State64 &st) {
@@ -189,6 +174,17 @@ void free_state64(State64 &st) {
   dfree(st.vz);
   dfree(st.pid);
   st = State64{};
+}
+
+// all of a state's arrays or none
+int alloc_state64(State64 &st, int64_t cap) {
+  int rc;
+  if ((rc = dalloc(&st.x, cap, "x")) || (rc = dalloc(&st.y, cap, "y")) ||
+      (rc = dalloc(&st.z, cap, "z")) || (rc = dalloc(&st.vx, cap, "vx")) ||
+      (rc = dalloc(&st.vy, cap, "vy")) || (rc = dalloc(&st.vz, cap, "vz")) ||
+      (rc = dalloc(&st.pid, cap, "pid")))
+    free_state64(st);
+  return rc;
 }
 
 }  // namespace
@@ -521,10 +517,7 @@ int emg_upload_particles(emg_ctx *c, const emg_particle *pbuf, const int64_t *co
   bool dead = !fits;  // more records than room: only the living have to fit
   if (fits) {
     if (c->cfg.precision == EMG_FP32_FIXED) {
-      if ((rc = alloc_state64(tmp, std::max<int64_t>(c->cap_total, 1)))) {
-        free_state64(tmp);
-        return rc;
-      }
+      if ((rc = alloc_state64(tmp, std::max<int64_t>(c->cap_total, 1)))) return rc;
       tgt = tmp;
     }
     rc = send(pbuf, counts);
@@ -556,10 +549,7 @@ int emg_upload_particles(emg_ctx *c, const emg_particle *pbuf, const int64_t *co
         return set_error(EMG_ERR_CAPACITY, "species count exceeds the context capacity");
     rc = EMG_OK;
     if (c->cfg.precision == EMG_FP32_FIXED && !tmp.x) {
-      if ((rc = alloc_state64(tmp, std::max<int64_t>(c->cap_total, 1)))) {
-        free_state64(tmp);
-        return rc;
-      }
+      if ((rc = alloc_state64(tmp, std::max<int64_t>(c->cap_total, 1)))) return rc;
       tgt = tmp;
     }
     rc = send(compact.data(), kept.data());
@@ -608,10 +598,7 @@ int emg_download_particles(emg_ctx *c, emg_particle *pbuf, int64_t *counts) {
   State64 src = c->s64;
   State64 tmp{};
   if (c->cfg.precision == EMG_FP32_FIXED) {
-    if ((rc = alloc_state64(tmp, c->cap_total))) {
-      free_state64(tmp);
-      return rc;
-    }
+    if ((rc = alloc_state64(tmp, c->cap_total))) return rc;
     rc = fx_to64(c, tmp);
     if (rc) {
       free_state64(tmp);
@@ -1034,10 +1021,10 @@ static int copy_state(const State64 &src, const State64 &dst, int64_t n, hipStre
 static int need_adjoint(emg_ctx *c) {
   int rc = need_fp64(c);
   if (rc) return rc;
-  if (c->lam) return EMG_OK;
-  if ((rc = dalloc(&c->lam, 8 * (size_t)c->cap_total, "particle adjoints")) ||
-      (rc = dalloc(&c->adj_e, 3 * c->ncell, "adjoint field")) ||
-      (rc = dalloc(&c->adj_g, c->ncell, "adjoint density")) ||
+  if (c->adj_sum) return EMG_OK;  // the last one: then all are there
+  if ((!c->lam && (rc = dalloc(&c->lam, 8 * (size_t)c->cap_total, "particle adjoints"))) ||
+      (!c->adj_e && (rc = dalloc(&c->adj_e, 3 * c->ncell, "adjoint field"))) ||
+      (!c->adj_g && (rc = dalloc(&c->adj_g, c->ncell, "adjoint density"))) ||
       (rc = dalloc(&c->adj_sum, (size_t)adj_vsum_need(), "adjoint sums")))
     return rc;
   launch_zero(c->lam, 8 * sizeof(double) * c->cap_total, c->stream);
@@ -1146,13 +1133,13 @@ int emg_init_device(emg_ctx *c, const emg_device_species *spec, int32_t nspec, u
     if (spec[s].count < 0 || spec[s].count > c->cfg.capacity[s])
       return set_error(EMG_ERR_CAPACITY, "species count exceeds the context capacity");
   }
-  for (int s = 0; s < nspec; s++) c->sp.cnt[s] = spec[s].count;
   int rc;
+  State64 tmp{};
+  if (c->cfg.precision != EMG_PLAIN_FP64 && (rc = alloc_state64(tmp, c->cap_total))) return rc;
+  for (int s = 0; s < nspec; s++) c->sp.cnt[s] = spec[s].count;
   if (c->cfg.precision == EMG_PLAIN_FP64) {
     rc = init_device_into(c, c->s64, spec, nspec, seed);
   } else {
-    State64 tmp{};
-    if ((rc = alloc_state64(tmp, c->cap_total))) return rc;
     rc = init_device_into(c, tmp, spec, nspec, seed);
     if (!rc) rc = fx_from64(c, tmp);
     if (!rc) rc = hip_check(hipStreamSynchronize(c->stream), "init");

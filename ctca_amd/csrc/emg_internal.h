@@ -516,6 +516,16 @@ namespace emg {
 int set_error(int code, const std::string &msg);
 int hip_check(hipError_t e, const char *what);
 
+// device memory; where there is none a null pointer, and no error left for the
+// next launch's check to find
+template <typename T>
+bool dev_malloc(T **p, size_t bytes) {
+  if (hipMalloc((void **)p, bytes) == hipSuccess) return true;
+  (void)hipGetLastError();
+  *p = nullptr;
+  return false;
+}
+
 int flags_error(emg_ctx *c);  // *hflag as an error code (and dflag cleared)
 bool capturing(emg_ctx *c);   // whether the stream's work is being recorded into a graph
 
@@ -538,9 +548,9 @@ void io_close(emg_ctx *c);
 void timer_begin(emg_ctx *c, int kind);
 void timer_end(emg_ctx *c, int kind);
 
-// scan: exclusive prefix sum of n int32 values into int64 out[0..n]; tmp >= scan_tmp_need(n)
-int64_t scan_tmp_need(int64_t n);
+// scan: exclusive prefix sum of n int32 values into int64 out[0..n]; tmp: scan_tmp_alloc
 void exclusive_scan_i32(const int32_t *in, int64_t *out, int64_t n, int64_t *tmp, hipStream_t s);
+int scan_tmp_alloc(emg_ctx *c, int64_t n);  // c->scan_tmp for scans of n values
 
 // kernels: FP64 mirror (k_fp64.hip)
 void launch_relocate64(emg_ctx *c);  // eb_dev -> the form's nodes

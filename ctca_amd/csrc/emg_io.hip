@@ -64,7 +64,10 @@ char *ring_get(int device, size_t need, size_t &bytes) {
       }
   }
   char *p = nullptr;
-  if (hipHostMalloc((void **)&p, need, hipHostMallocDefault) != hipSuccess) return nullptr;
+  if (hipHostMalloc((void **)&p, need, hipHostMallocDefault) != hipSuccess) {
+    (void)hipGetLastError();
+    return nullptr;
+  }
   bytes = need;
   return p;
 }

@@ -140,28 +140,14 @@ int bins_alloc(emg_ctx *c) {
   TileBins &B = c->bins;
   if (B.rec) return EMG_OK;
   const int64_t n = bin_tiles(c->g).n;
-  if (!B.count && hipMalloc(&B.count, sizeof(int32_t) * 2 * n) != hipSuccess) {
-    B.count = nullptr;
+  if (!B.count && !dev_malloc(&B.count, sizeof(int32_t) * 2 * n))
     return set_error(EMG_ERR_NOMEM, "tile counters");
-  }
-  if (!B.start && hipMalloc(&B.start, sizeof(int64_t) * (n + 1)) != hipSuccess) {
-    B.start = nullptr;
+  if (!B.start && !dev_malloc(&B.start, sizeof(int64_t) * (n + 1)))
     return set_error(EMG_ERR_NOMEM, "tile starts");
-  }
-  const int64_t need = scan_tmp_need(n);
-  if (need > c->scan_tmp_len) {
-    if (c->scan_tmp) (void)hipFree(c->scan_tmp);
-    c->scan_tmp_len = 0;
-    if (hipMalloc(&c->scan_tmp, sizeof(int64_t) * need) != hipSuccess) {
-      c->scan_tmp = nullptr;
-      return set_error(EMG_ERR_NOMEM, "scan scratch");
-    }
-    c->scan_tmp_len = need;
-  }
+  const int rc = scan_tmp_alloc(c, n);
+  if (rc) return rc;
   int64_t len = std::min(std::max<int64_t>(c->cap_total, 1), kBinMax);
-  while (hipMalloc(&B.rec, sizeof(BinRec) * len) != hipSuccess) {
-    (void)hipGetLastError();
-    B.rec = nullptr;
+  while (!dev_malloc(&B.rec, sizeof(BinRec) * len)) {
     if (len <= 65536) return set_error(EMG_ERR_NOMEM, "tile records");
     len /= 2;
   }

@@ -943,14 +943,7 @@ static bool tiles64(emg_ctx *c) {
   int64_t total = 0;
   for (int s = 0; s < c->sp.nspec; s++) total += c->sp.cnt[s];
   if (c->runs_valid || c->ordered || total < kTileMin) return false;
-  if (!c->bins.rec) {
-    if (capturing(c)) return false;
-    if (bins_alloc(c) != EMG_OK) {
-      (void)hipGetLastError();
-      return false;
-    }
-  }
-  return true;
+  return c->bins.rec || (!capturing(c) && bins_alloc(c) == EMG_OK);
 }
 
 static void launch_tiles64(emg_ctx *c) {

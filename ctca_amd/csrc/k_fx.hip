@@ -1960,29 +1960,22 @@ int fx_alloc(emg_ctx *c, int64_t ntotal) {
     return set_error(EMG_ERR_ARG, "FP32_FIXED holds at most 2^32 particle slots per context");
   for (int k = 0; k < 2; k++) {
     StateFx &S = B.st[k];
-    void *p[7];
-    for (int q = 0; q < 7; q++) {
-      if (hipMalloc(&p[q], sizeof(float) * B.cap_total) != hipSuccess)
-        return set_error(EMG_ERR_NOMEM, "FP32 particle buffers");
-    }
-    S.cell = (int32_t *)p[0];
-    S.fx = (float *)p[1];
-    S.fy = (float *)p[2];
-    S.fz = (float *)p[3];
-    S.vx = (float *)p[4];
-    S.vy = (float *)p[5];
-    S.vz = (float *)p[6];
+    const size_t bytes = sizeof(float) * B.cap_total;
+    if (!dev_malloc(&S.cell, bytes) || !dev_malloc(&S.fx, bytes) || !dev_malloc(&S.fy, bytes) ||
+        !dev_malloc(&S.fz, bytes) || !dev_malloc(&S.vx, bytes) || !dev_malloc(&S.vy, bytes) ||
+        !dev_malloc(&S.vz, bytes))
+      return set_error(EMG_ERR_NOMEM, "FP32 particle buffers");
     S.pid = nullptr;
-    if (c->cfg.track_pid && hipMalloc(&S.pid, sizeof(int32_t) * B.cap_total) != hipSuccess)
+    if (c->cfg.track_pid && !dev_malloc(&S.pid, sizeof(int32_t) * B.cap_total))
       return set_error(EMG_ERR_NOMEM, "FP32 pid buffers");
-    if (hipMalloc(&B.start[k], sizeof(int64_t) * (B.nb + 1)) != hipSuccess ||
-        hipMalloc(&B.count[k], sizeof(int32_t) * B.nb) != hipSuccess ||
-        hipMalloc(&B.nst[k], sizeof(int32_t) * B.nb) != hipSuccess ||
-        hipMalloc(&B.cap[k], sizeof(int32_t) * B.nb) != hipSuccess ||
-        hipMalloc(&B.spill[k], sizeof(int32_t) * EMG_MAX_SPECIES) != hipSuccess ||
-        hipMalloc(&B.pre[k], sizeof(int32_t) * B.nb * kPre) != hipSuccess)
+    if (!dev_malloc(&B.start[k], sizeof(int64_t) * (B.nb + 1)) ||
+        !dev_malloc(&B.count[k], sizeof(int32_t) * B.nb) ||
+        !dev_malloc(&B.nst[k], sizeof(int32_t) * B.nb) ||
+        !dev_malloc(&B.cap[k], sizeof(int32_t) * B.nb) ||
+        !dev_malloc(&B.spill[k], sizeof(int32_t) * EMG_MAX_SPECIES) ||
+        !dev_malloc(&B.pre[k], sizeof(int32_t) * B.nb * kPre))
       return set_error(EMG_ERR_NOMEM, "bucket tables");
-    if (hipMalloc(&B.ob[k], sizeof(FxRec) * B.nb * kObStride) != hipSuccess)
+    if (!dev_malloc(&B.ob[k], sizeof(FxRec) * B.nb * kObStride))
       return set_error(EMG_ERR_NOMEM, "bucket outboxes");
     launch_zero(B.count[k], sizeof(int32_t) * B.nb, c->stream);
     launch_zero(B.nst[k], sizeof(int32_t) * B.nb, c->stream);
@@ -1991,32 +1984,27 @@ int fx_alloc(emg_ctx *c, int64_t ntotal) {
     launch_zero(B.start[k], sizeof(int64_t) * (B.nb + 1), c->stream);
     launch_zero(B.pre[k], sizeof(int32_t) * B.nb * kPre, c->stream);
   }
-  if (hipMalloc(&B.stay, sizeof(int32_t) * B.nb) != hipSuccess ||
-      hipMalloc(&B.extra, sizeof(int32_t) * B.nb) != hipSuccess ||
-      hipMalloc(&B.hist, sizeof(int32_t) * B.nb) != hipSuccess ||
-      hipMalloc(&B.cursor, sizeof(int32_t) * B.nb) != hipSuccess ||
-      hipMalloc(&B.shist[0], sizeof(int32_t) * B.nb) != hipSuccess ||
-      hipMalloc(&B.shist[1], sizeof(int32_t) * B.nb) != hipSuccess ||
-      hipMalloc(&B.plan_word, sizeof(unsigned long long) * plan_blocks(B.nb)) != hipSuccess ||
-      hipMalloc(&B.plan_ticket, sizeof(unsigned long long)) != hipSuccess ||
-      hipMalloc(&B.scur, sizeof(int32_t) * B.nb) != hipSuccess ||
-      hipMalloc(&B.spre, sizeof(int64_t) * (B.nb + 1)) != hipSuccess)
+  if (!dev_malloc(&B.stay, sizeof(int32_t) * B.nb) ||
+      !dev_malloc(&B.extra, sizeof(int32_t) * B.nb) ||
+      !dev_malloc(&B.hist, sizeof(int32_t) * B.nb) ||
+      !dev_malloc(&B.cursor, sizeof(int32_t) * B.nb) ||
+      !dev_malloc(&B.shist[0], sizeof(int32_t) * B.nb) ||
+      !dev_malloc(&B.shist[1], sizeof(int32_t) * B.nb) ||
+      !dev_malloc(&B.plan_word, sizeof(unsigned long long) * plan_blocks(B.nb)) ||
+      !dev_malloc(&B.plan_ticket, sizeof(unsigned long long)) ||
+      !dev_malloc(&B.scur, sizeof(int32_t) * B.nb) ||
+      !dev_malloc(&B.spre, sizeof(int64_t) * (B.nb + 1)))
     return set_error(EMG_ERR_NOMEM, "bucket tables");
-  if (hipMalloc(&B.spl, sizeof(FxRec) * B.spill_cap * c->sp.nspec) != hipSuccess)
+  if (!dev_malloc(&B.spl, sizeof(FxRec) * B.spill_cap * c->sp.nspec))
     return set_error(EMG_ERR_NOMEM, "sorted spill buffer");
   for (int k = 0; k < 2; k++) launch_zero(B.shist[k], sizeof(int32_t) * B.nb, c->stream);
   launch_zero(B.plan_word, sizeof(unsigned long long) * plan_blocks(B.nb), c->stream);
   launch_zero(B.plan_ticket, sizeof(unsigned long long), c->stream);
   launch_zero(B.scur, sizeof(int32_t) * B.nb, c->stream);
-  int64_t need = scan_tmp_need(B.nb);
-  if (need > c->scan_tmp_len) {
-    if (c->scan_tmp) (void)hipFree(c->scan_tmp);
-    if (hipMalloc(&c->scan_tmp, sizeof(int64_t) * need) != hipSuccess)
-      return set_error(EMG_ERR_NOMEM, "scan scratch");
-    c->scan_tmp_len = need;
-  }
+  const int rc = scan_tmp_alloc(c, B.nb);
+  if (rc) return rc;
   int64_t kp = (int64_t)(B.nb + c->sp.nspec * kSpillBlocksPerSpecies) * 3;
-  if (hipMalloc(&c->ke_part, sizeof(double) * kp) != hipSuccess)
+  if (!dev_malloc(&c->ke_part, sizeof(double) * kp))
     return set_error(EMG_ERR_NOMEM, "energy partials");
   c->ke_part_n = kp;
   B.cur = 0;

@@ -13,15 +13,20 @@
 #include <map>
 #include <mutex>
 #include <string>
+#include <vector>
 
 namespace {
 std::mutex mu;
-std::map<char *, size_t> live;            // device allocations
-std::map<const void *, std::string> name; // host stub -> kernel
+std::map<char *, size_t> live, dead;      // device allocations; freed ones (kept)
+struct Kernel {
+  std::string name;
+  std::vector<bool> pointer;              // its parameters
+};
+std::map<const void *, Kernel> kernels;   // by host stub
 std::string launches;
 size_t used = 0, peak = 0, limit = SIZE_MAX;
 long fail_in = -1;                        // this allocation from now fails
-int bad_frees = 0, bad_copies = 0, mallocs = 0, capturing = 0, last_error = 0;
+int bad_frees = 0, bad_copies = 0, bad_args = 0, mallocs = 0, capturing = 0, last_error = 0;
 int flags[2] = {0, 0};                    // what the next k_flag reports
 struct Dim3 {
   uint32_t x, y, z;
@@ -32,13 +37,18 @@ thread_local struct {
   void *stream;
 } config;
 int fail(int e) { return last_error = e; }
-// [p, p + n) within one allocation, or in none (host memory)
-bool within(const void *v, size_t n) {
-  char *p = (char *)v;
-  auto it = live.upper_bound(p);
-  if (it == live.begin()) return true;
+bool inside(const std::map<char *, size_t> &m, char *p, size_t &left) {
+  auto it = m.upper_bound(p);
+  if (it == m.begin()) return false;
   --it;
-  return p >= it->first + it->second || p + n <= it->first + it->second;
+  left = p < it->first + it->second ? it->first + it->second - p : 0;
+  return left > 0;
+}
+// [p, p + n) within one allocation, or in none, freed ones included (host memory)
+bool within(const void *v, size_t n) {
+  size_t left;
+  if (inside(dead, (char *)v, left)) return false;
+  return !inside(live, (char *)v, left) || n <= left;
 }
 void note(const std::string &what) { launches += what + "\n"; }
 }  // namespace
@@ -55,6 +65,7 @@ API size_t fake_peak(int reset) { const size_t p = peak; if (reset) peak = used;
 API int fake_mallocs() { return mallocs; }
 API int fake_bad_frees() { return bad_frees; }
 API int fake_bad_copies() { return bad_copies; }
+API int fake_bad_args() { return bad_args; }  // kernels given freed memory
 API void fake_capture(int on) { capturing = on; }
 API void fake_flags(int a, int b) { flags[0] = a; flags[1] = b; }
 
@@ -81,8 +92,8 @@ API int hipFree(void *p) {
     return fail(1);
   }
   used -= it->second;
+  dead[it->first] = it->second;
   live.erase(it);
-  std::free(p);
   return 0;
 }
 API int hipHostMalloc(void **p, size_t n, unsigned) { *p = std::calloc(n, 1); return *p ? 0 : 2; }
@@ -114,14 +125,16 @@ API int __hipPopCallConfiguration(Dim3 *g, Dim3 *b, size_t *shm, void **stream) 
 }
 API int hipLaunchKernel(const void *f, Dim3, Dim3, void **args, size_t, void *) {
   std::lock_guard<std::mutex> l(mu);
-  const std::string &k = name[f];
-  if (k == "k_flag") {
+  const Kernel &k = kernels[f];
+  for (size_t i = 0; i < k.pointer.size(); i++)
+    if (k.pointer[i] && !within(*(void **)args[i], 1)) bad_args++;
+  if (k.name == "k_flag") {
     int *h = *(int **)args[1];
     h[0] = flags[0];
     h[1] = flags[1];
     flags[0] = flags[1] = 0;
   }
-  note(k);
+  note(k.name);
   return 0;
 }
 API void **__hipRegisterFatBinary(const void *) { static void *h; return &h; }
@@ -136,10 +149,18 @@ API void __hipRegisterFunction(void **, const void *host, char *, const char *de
   // "void emg::(anonymous namespace)::k_x<8, true>(args)" -> "k_x<8, true>"
   const size_t at = s.find("k_");
   s = at == std::string::npos ? s : s.substr(at);
-  size_t end = 0;
-  for (int depth = 0; end < s.size() && (depth > 0 || s[end] != '('); end++)
-    depth += s[end] == '<' ? 1 : (s[end] == '>' ? -1 : 0);
-  name[host] = s.substr(0, end);
+  Kernel k;
+  int depth = 0;
+  for (size_t i = 0; i < s.size(); i++) {
+    const bool top = depth == (k.name.empty() ? 0 : 1);
+    if (k.name.empty() && top && s[i] == '(') {
+      k.name = s.substr(0, i);
+    } else if (!k.name.empty() && top && (s[i] == ',' || s[i] == ')')) {
+      k.pointer.push_back(s[i - 1] == '*');
+    }
+    depth += s[i] == '<' || s[i] == '(' ? 1 : (s[i] == '>' || s[i] == ')' ? -1 : 0);
+  }
+  kernels[host] = k;
 }
 
 // ---- the rest
