@@ -1018,10 +1018,12 @@ static int copy_state(const State64 &src, const State64 &dst, int64_t n, hipStre
   return EMG_OK;
 }
 
+// the adjoint arrays and the step's bins, so that only the window's first call
+// allocates and a step can be recorded after any other call of it
 static int need_adjoint(emg_ctx *c) {
   int rc = need_fp64(c);
   if (rc) return rc;
-  if (c->adj_sum) return EMG_OK;  // the last one: then all are there
+  if (c->adj_sum) return bins_alloc(c);  // the last one: then all are there
   if ((!c->lam && (rc = dalloc(&c->lam, 8 * (size_t)c->cap_total, "particle adjoints"))) ||
       (!c->adj_e && (rc = dalloc(&c->adj_e, 3 * c->ncell, "adjoint field"))) ||
       (!c->adj_g && (rc = dalloc(&c->adj_g, c->ncell, "adjoint density"))) ||
@@ -1029,7 +1031,8 @@ static int need_adjoint(emg_ctx *c) {
     return rc;
   launch_zero(c->lam, 8 * sizeof(double) * c->cap_total, c->stream);
   launch_zero(c->adj_e, sizeof(double) * 3 * c->ncell, c->stream);
-  return hip_check(hipGetLastError(), "adjoint allocation");
+  if ((rc = hip_check(hipGetLastError(), "adjoint allocation"))) return rc;
+  return bins_alloc(c);
 }
 
 int emg_state_save(emg_ctx *c, int32_t slot) {
@@ -1073,7 +1076,6 @@ int emg_adj_step(emg_ctx *c, int32_t ustep) {
   if (!rc) rc = need_fields(c);
   if (rc) return rc;
   if (ustep < 0) return set_error(EMG_ERR_ARG, "ustep must be >= 0");
-  if ((rc = bins_alloc(c))) return rc;
   launch_adj_step64(c, ustep);
   return hip_check(hipGetLastError(), "adjoint step launch");
 }

@@ -137,3 +137,39 @@ def test_recorded_solves_replayed_after_b_updates(precision):
     # energy's partial sums of particles in another order (FP32)
     for a, b in zip(*out):
         assert np.abs(a - b).max() <= 1e-12 * np.abs(a).max()
+
+
+def test_adjoint_steps_recorded_after_a_reset():
+    need_torch()
+    from ctca_amd import emg
+    n, counts = (16, 20, 12), (9000, 4000)
+    rng = np.random.default_rng(8)
+    rec = np.zeros(sum(counts), dtype=emg.PARTICLE)
+    for c, m in zip("xyz", n):
+        rec[c] = rng.random(sum(counts)) * m
+    core = rng.normal(size=(n[2], n[1], n[0], 6)) * 0.1
+    at = [np.arange(-1, v + 2) % v for v in n]
+    eb = np.ascontiguousarray(core[np.ix_(at[2], at[1], at[0])])
+    g = rng.normal(size=n[::-1])
+
+    def program(ctx, recorded):
+        ctx.upload(rec, counts)
+        ctx.set_fields(eb)
+        ctx.adj_reset()
+        step = (lambda: ctx.adj_step(2))
+        if recorded:
+            step = Recorded(ctx, step)
+        out = []
+        for _ in range(3):
+            ctx.adj_add_density(g, (0.5, -0.25))
+            step()
+            out.append(ctx.adj_velocity_sums())
+            out.append(ctx.adj_field())
+        return out
+
+    got = []
+    for recorded in (False, True):
+        with emg.Context(n, [0.02, -0.02], [1.0, -1.0], [1.0, 1.0], counts) as ctx:
+            got.append(program(ctx, recorded))
+    for a, b in zip(*got):         # FP64 sums of some thousand terms in another order
+        assert np.abs(a - b).max() <= 1e-11 * np.abs(a).max()

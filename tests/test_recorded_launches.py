@@ -52,3 +52,19 @@ def test_a_field_solve_relocates_b_where_a_replay_may_meet_another_one(tmp_path)
                 c.grdcrt()
                 assert all_nodes(c.solve_es, 0.0)      # a replay may have been here
     """)
+
+
+def test_an_adjoint_step_allocates_nothing_after_the_window_has_begun(tmp_path):
+    fake_hip.run(tmp_path, """
+        n, counts = (16, 16, 16), (200000, 1000)
+        for begin in (lambda c: c.adj_reset(), lambda c: c.adj_field()):
+            with emg.Context(n, [1.0, -1.0], [1.0, 1.0], [1.0, 1.0], counts) as c:
+                c.upload(records(201000, n), counts)
+                c.set_fields(np.zeros((19, 19, 19, 6)))
+                begin(c)
+                before = fake.fake_mallocs()
+                fake.fake_capture(1)
+                c.adj_step(2)
+                fake.fake_capture(0)
+                assert fake.fake_mallocs() == before
+    """)
