@@ -1,5 +1,6 @@
 // emg_api.hip -- the extern "C" entry points of libemgpu (include/emgpu.h).
 #include <algorithm>
+#include <atomic>
 #include <cmath>
 #include <cstdio>
 #include <cstring>
@@ -188,6 +189,41 @@ int alloc_state64(State64 &st, int64_t cap) {
 }
 
 }  // namespace
+
+// The records of an upload with nid >= 0: how many come before a record, and a
+// range of them without the others.
+struct LivingRecords {
+  static constexpr int64_t kStep = 1024;
+  const emg_particle *rec = nullptr;
+  std::vector<int64_t> at;  // living records before every kStep-th one
+  int count(emg_ctx *c, const emg_particle *r, int64_t n) {
+    rec = r;
+    const int64_t steps = (n + kStep - 1) / kStep;
+    try {
+      at.assign((size_t)steps + 1, 0);
+    } catch (const std::bad_alloc &) {
+      return set_error(EMG_ERR_NOMEM, "host allocation failed");
+    }
+    const int rc = io_ranges(c, steps, sizeof(emg_particle) * kStep, [&](int64_t a, int64_t b) {
+      for (int64_t k = a; k < b; k++) at[k + 1] = alive(k * kStep, std::min(n, (k + 1) * kStep));
+    });
+    for (int64_t k = 0; k < steps; k++) at[k + 1] += at[k];
+    return rc;
+  }
+  int64_t alive(int64_t a, int64_t b) const {
+    int64_t k = 0;
+    for (; a < b; a++) k += rec[a].nid >= 0;
+    return k;
+  }
+  int64_t before(int64_t m) const { return at[m / kStep] + alive(m / kStep * kStep, m); }
+  // the living ones of n records from m on, to out; their bytes
+  size_t copy(int64_t m, int64_t n, emg_particle *out) const {
+    int64_t k = 0;
+    for (int64_t a = m; a < m + n; a++)
+      if (rec[a].nid >= 0) out[k++] = rec[a];
+    return sizeof(emg_particle) * (size_t)k;
+  }
+};
 
 int flags_error(emg_ctx *c) {
   const int f = *c->hflag;
@@ -488,72 +524,73 @@ int emg_upload_particles(emg_ctx *c, const emg_particle *pbuf, const int64_t *co
   if (total > 0 && !pbuf) return set_error(EMG_ERR_ARG, "null pbuf");
   State64 tgt = c->s64;
   State64 tmp{};
-  launch_zero(c->dflag + 1, sizeof(int), c->stream);
-  // particles of counts cnt, species-contiguous at src, into tgt
-  auto send = [&](const emg_particle *src, const int64_t *cnt) {
+  const SpeciesTab before = c->sp;
+  std::atomic<bool> touched{false};  // records of the new state have been sent
+  *c->hflag = 0;
+  // the records (with `living`, those of them), cnt[s] of species s, into tgt
+  auto send = [&](const int64_t *cnt, const LivingRecords *living) {
     int64_t first[EMG_MAX_SPECIES + 1] = {0};
     for (int s = 0; s < nspec; s++) first[s + 1] = first[s] + cnt[s];
     const int need_pid0 = c->cfg.precision == EMG_FP32_FIXED && !c->cfg.track_pid ? 1 : 0;
     for (int s = 0; s < nspec; s++) c->sp.cnt[s] = cnt[s];
-    return io_write(c, src, sizeof(emg_particle) * first[nspec], sizeof(emg_particle),
-                    [&, need_pid0](size_t off, size_t len, void *slot) {
-                      const int64_t m0 = off / sizeof(emg_particle),
-                                    m1 = m0 + len / sizeof(emg_particle);
-                      for (int s = 0; s < nspec; s++) {
-                        const int64_t a = std::max(m0, first[s]), b = std::min(m1, first[s + 1]);
-                        if (a < b)
-                          hipLaunchKernelGGL(k_split, dim3((unsigned)((b - a + kBlock - 1) / kBlock)),
-                                             dim3(kBlock), 0, c->stream,
-                                             static_cast<emg_particle *>(slot) + (a - m0), b - a, tgt,
-                                             c->sp.off[s] + (a - first[s]), c->g, c->dflag,
-                                             need_pid0, c->dflag + 1);
-                      }
-                      return hip_check(hipGetLastError(), "upload split");
-                    });
+    launch_zero(c->dflag + 1, sizeof(int), c->stream);
+    const IoFn use = [&](size_t off, size_t len, void *slot) {
+      const int64_t at = off / sizeof(emg_particle), m0 = living ? living->before(at) : at,
+                    m1 = m0 + len / sizeof(emg_particle);
+      touched = true;
+      for (int s = 0; s < nspec; s++) {
+        const int64_t a = std::max(m0, first[s]), b = std::min(m1, first[s + 1]);
+        if (a < b)
+          hipLaunchKernelGGL(k_split, dim3((unsigned)((b - a + kBlock - 1) / kBlock)), dim3(kBlock),
+                             0, c->stream, static_cast<emg_particle *>(slot) + (a - m0), b - a, tgt,
+                             c->sp.off[s] + (a - first[s]), c->g, c->dflag, need_pid0,
+                             c->dflag + 1);
+      }
+      return hip_check(hipGetLastError(), "upload split");
+    };
+    IoCopy copy;
+    if (living)
+      copy = [&](size_t off, size_t len, void *slot) {
+        return living->copy(off / sizeof(emg_particle), len / sizeof(emg_particle),
+                            static_cast<emg_particle *>(slot));
+      };
+    return io_write(c, pbuf, sizeof(emg_particle) * total, sizeof(emg_particle), use, copy);
   };
   bool fits = true;
   for (int s = 0; s < nspec; s++) fits = fits && counts[s] <= c->cfg.capacity[s];
   int rc = EMG_OK;
   bool dead = !fits;  // more records than room: only the living have to fit
+  int64_t sent = total;
+  if (c->cfg.precision == EMG_FP32_FIXED) {
+    if ((rc = alloc_state64(tmp, std::max<int64_t>(c->cap_total, 1)))) return rc;
+    tgt = tmp;
+  }
   if (fits) {
-    if (c->cfg.precision == EMG_FP32_FIXED) {
-      if ((rc = alloc_state64(tmp, std::max<int64_t>(c->cap_total, 1)))) return rc;
-      tgt = tmp;
-    }
-    rc = send(pbuf, counts);
+    rc = send(counts, nullptr);
     if (!rc) {
       rc = read_flags(c);
-      dead = rc != EMG_OK && (*c->hflag & kFlagDead) != 0;
+      dead = rc != EMG_OK && *c->hflag == kFlagDead;  // (and no other error)
     }
   }
   if (dead) {
-    // transbound: keep nid >= 0 in order (flags of the first try are cleared)
-    std::vector<int64_t> kept(nspec, 0);
-    std::vector<emg_particle> compact;
-    try {
-      compact.reserve((size_t)total);
-    } catch (const std::bad_alloc &) {
-      free_state64(tmp);
-      return set_error(EMG_ERR_NOMEM, "host allocation failed");
-    }
-    int64_t m = 0;
-    for (int s = 0; s < nspec; s++) {
-      for (int64_t k = 0; k < counts[s]; k++, m++)
-        if (pbuf[m].nid >= 0) {
-          compact.push_back(pbuf[m]);
-          kept[s]++;
-        }
-    }
-    for (int s = 0; s < nspec; s++)
+    // transbound: keep nid >= 0 in order
+    LivingRecords living;
+    int64_t kept[EMG_MAX_SPECIES] = {0};
+    rc = living.count(c, pbuf, total);
+    sent = 0;
+    for (int64_t s = 0, m = 0; s < nspec && !rc; m += counts[s], s++) {
+      kept[s] = living.before(m + counts[s]) - living.before(m);
+      sent += kept[s];
       if (kept[s] > c->cfg.capacity[s])
-        return set_error(EMG_ERR_CAPACITY, "species count exceeds the context capacity");
-    rc = EMG_OK;
-    if (c->cfg.precision == EMG_FP32_FIXED && !tmp.x) {
-      if ((rc = alloc_state64(tmp, std::max<int64_t>(c->cap_total, 1)))) return rc;
-      tgt = tmp;
+        rc = set_error(EMG_ERR_CAPACITY, "species count exceeds the context capacity");
     }
-    rc = send(compact.data(), kept.data());
+    if (!rc) rc = send(kept, &living);
     if (!rc) rc = read_flags(c);
+  }
+  if (rc && !touched && *c->hflag == 0) {  // nothing has been sent: the old state stands
+    free_state64(tmp);
+    c->sp = before;
+    return rc;
   }
   if (!rc && c->cfg.precision == EMG_FP32_FIXED) {
     rc = fx_from64(c, tmp);
@@ -567,7 +604,7 @@ int emg_upload_particles(emg_ctx *c, const emg_particle *pbuf, const int64_t *co
   }
   c->have_particles = true;
   // most neighbours in the order share a tile: the blocks' windows catch them
-  c->ordered = (int64_t)c->hflag[1] * kNearSample * 2 > total;
+  c->ordered = (int64_t)c->hflag[1] * kNearSample * 2 > sent;
   c->pushes_since_sort = c->cfg.sort_every;  // unsorted: sort before the first push
   c->moves_after_sort = emg::kUnsorted;
   c->runs_valid = false;

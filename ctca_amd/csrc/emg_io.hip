@@ -88,6 +88,11 @@ struct Plan {
   int n, threads;
 };
 
+int threads_for(size_t bytes) {
+  const unsigned hc = std::thread::hardware_concurrency();
+  return bytes >= kIoMany && (hc == 0 || hc >= (unsigned)kIoThreads) ? kIoThreads : 1;
+}
+
 Plan plan_of(size_t bytes, size_t unit) {
   Plan p;
   p.bytes = bytes;
@@ -100,8 +105,7 @@ Plan plan_of(size_t bytes, size_t unit) {
   }
   p.chunk = chunk;
   p.n = (int)((bytes + chunk - 1) / chunk);
-  const unsigned hc = std::thread::hardware_concurrency();
-  p.threads = bytes >= kIoMany && (hc == 0 || hc >= (unsigned)kIoThreads) ? kIoThreads : 1;
+  p.threads = threads_for(bytes);
   return p;
 }
 
@@ -247,7 +251,17 @@ int io_read_array(emg_ctx *c, void *user, const void *dev, size_t bytes) {
   });
 }
 
-int io_write(emg_ctx *c, const void *user, size_t bytes, size_t unit, const IoFn &use) {
+int io_ranges(emg_ctx *c, int64_t n, size_t bytes,
+              const std::function<void(int64_t, int64_t)> &f) {
+  const int threads = threads_for(bytes * (size_t)n);
+  return on_threads(c, threads, [&](int t) {
+    f(n * t / threads, n * (t + 1) / threads);
+    return EMG_OK;
+  });
+}
+
+int io_write(emg_ctx *c, const void *user, size_t bytes, size_t unit, const IoFn &use,
+             const IoCopy &copy) {
   if (bytes == 0) return EMG_OK;
   const Plan p = plan_of(bytes, unit);
   int rc = ring(c, p, true);
@@ -261,8 +275,13 @@ int io_write(emg_ctx *c, const void *user, size_t bytes, size_t unit, const IoFn
       const int s = i % slots;
       if (i >= slots) r = hip_check(hipEventSynchronize(io.ev[s]), "transfer");
       if (r) break;
-      std::memcpy(io.pin + s * io.stride, static_cast<const char *>(user) + off, len);
-      r = use(off, len, io.pin + s * io.stride);
+      char *slot = io.pin + s * io.stride;
+      size_t got = len;
+      if (copy)
+        got = copy(off, len, slot);
+      else
+        std::memcpy(slot, static_cast<const char *>(user) + off, len);
+      if (got > 0) r = use(off, got, slot);
       if (!r && i + slots < p.n)
         r = hip_check(hipEventRecord(io.ev[s], c->stream), "transfer event");
     }

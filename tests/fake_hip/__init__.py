@@ -1,6 +1,7 @@
 """libemgpu.so's host logic without a GPU: a child process loads a stand-in for
 the HIP runtime (fake_hip.cpp) before the library and runs a test's code there,
 with `fake` (the stand-in's own entry points) and `emg` at hand."""
+import functools
 import os
 import shutil
 import subprocess
@@ -40,14 +41,20 @@ def records(total, n, pid=False):
 """
 
 
+@functools.lru_cache(None)
+def library(folder):
+    so = os.path.join(folder, "libfakehip.so")
+    subprocess.run(["g++", "-std=c++17", "-O1", "-shared", "-fPIC",
+                    os.path.join(HERE, "fake_hip.cpp"), "-o", so],
+                   check=True, capture_output=True, text=True)
+    return so
+
+
 def run(tmp_path, code):
     """Run `code` in a child process; the test fails where it does."""
     if shutil.which("g++") is None:
         pytest.skip("g++ not found")
-    so = str(tmp_path / "libfakehip.so")
-    subprocess.run(["g++", "-std=c++17", "-O1", "-shared", "-fPIC",
-                    os.path.join(HERE, "fake_hip.cpp"), "-o", so],
-                   check=True, capture_output=True, text=True)
+    so = library(str(tmp_path.parent))      # one for the session
     r = subprocess.run([sys.executable, "-c", PRELUDE + textwrap.dedent(code), so], cwd=ROOT,
                        capture_output=True, text=True, timeout=120)
     assert r.returncode == 0, (r.stdout + r.stderr)[-4000:]

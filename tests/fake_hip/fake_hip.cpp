@@ -28,6 +28,7 @@ size_t used = 0, peak = 0, limit = SIZE_MAX;
 long fail_in = -1;                        // this allocation from now fails
 int bad_frees = 0, bad_copies = 0, bad_args = 0, mallocs = 0, capturing = 0, last_error = 0;
 int flags[2] = {0, 0};                    // what the next k_flag reports
+std::map<int64_t, int> split;             // pid of the record that k_split puts where
 struct Dim3 {
   uint32_t x, y, z;
 };
@@ -68,6 +69,19 @@ API int fake_bad_copies() { return bad_copies; }
 API int fake_bad_args() { return bad_args; }  // kernels given freed memory
 API void fake_capture(int on) { capturing = on; }
 API void fake_flags(int a, int b) { flags[0] = a; flags[1] = b; }
+
+API int64_t fake_split(int64_t *slot, int *pid, int64_t n) {  // and start anew
+  std::lock_guard<std::mutex> l(mu);
+  int64_t k = 0;
+  for (auto &e : split)
+    if (k < n) {
+      slot[k] = e.first;
+      pid[k++] = e.second;
+    }
+  k = (int64_t)split.size();
+  split.clear();
+  return k;
+}
 
 // ---- memory
 API int hipMalloc(void **p, size_t n) {
@@ -133,6 +147,11 @@ API int hipLaunchKernel(const void *f, Dim3, Dim3, void **args, size_t, void *) 
     h[0] = flags[0];
     h[1] = flags[1];
     flags[0] = flags[1] = 0;
+  }
+  if (k.name == "k_split") {
+    const char *rec = *(char **)args[0];
+    for (int64_t i = 0; i < *(int64_t *)args[1]; i++)
+      std::memcpy(&split[*(int64_t *)args[3] + i], rec + 64 * i + 48, 4);
   }
   note(k.name);
   return 0;
