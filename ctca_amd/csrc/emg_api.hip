@@ -447,7 +447,6 @@ int emg_destroy(emg_ctx *c) {
   dfree(B.spre);
   dfree(B.spl);
   dfree(c->eb_dev);
-  dfree(c->eb_stage);
   dfree(c->fe_buf);
   dfree(c->sort_rec);
   es_solver_free(c);
@@ -676,13 +675,6 @@ int emg_set_fields(emg_ctx *c, const double *eb, const int32_t lo[3], const int3
   const size_t bytes = sizeof(double) * 6 * (size_t)ext[0] * ext[1] * ext[2];
   int rc = hip_check(hipStreamSynchronize(c->stream), "stream synchronize");
   if (rc) return rc;
-  if (bytes > c->eb_stage_bytes) {
-    dfree(c->eb_stage);
-    c->eb_stage = nullptr;
-    c->eb_stage_bytes = 0;
-    if ((rc = dalloc(&c->eb_stage, bytes / sizeof(double), "eb staging"))) return rc;
-    c->eb_stage_bytes = bytes;
-  }
   if (bytes > c->eb_dev_bytes) {
     dfree(c->eb_dev);
     c->eb_dev = nullptr;
@@ -690,13 +682,16 @@ int emg_set_fields(emg_ctx *c, const double *eb, const int32_t lo[3], const int3
     if ((rc = dalloc(&c->eb_dev, bytes / sizeof(double), "eb"))) return rc;
     c->eb_dev_bytes = bytes;
   }
-  rc = hip_check(hipMemcpy(c->eb_stage, eb, bytes, hipMemcpyHostToDevice), "eb upload");
-  if (rc) return rc;
   for (int d = 0; d < 3; d++) {
     c->eb_lo[d] = elo[d];
     c->eb_ext[d] = ext[d];
   }
-  launch_eb_split(c);
+  const size_t unit = 6 * sizeof(double);
+  rc = io_write(c, eb, bytes, unit, [&](size_t off, size_t len, void *slot) {
+    launch_eb_split(c, (const double *)slot, (int64_t)(off / unit), (int64_t)(len / unit));
+    return hip_check(hipGetLastError(), "eb upload");
+  });
+  if (rc) return rc;
   launch_relocate64(c);
   c->fields_set = true;
   c->nodes_stale = false;

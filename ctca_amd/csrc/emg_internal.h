@@ -449,8 +449,6 @@ struct emg_ctx {
   // records of the boundary's layout would half fill (EbView)
   double *eb_dev;
   size_t eb_dev_bytes;
-  double *eb_stage;  // an uploaded eb in the boundary's layout (lazy)
-  size_t eb_stage_bytes;
   bool nodes_b_valid;  // the nodes' B is the relocation of eb_dev's B
   bool b_recorded;     // a graph holds an emg_bfield: its replays change eb_dev's B unseen
   int eb_lo[3], eb_ext[3];
@@ -571,7 +569,8 @@ void launch_push_em64(emg_ctx *c, int ustep, bool resort);
 void launch_faces64(emg_ctx *c);  // c->face (zeroed) += upper-face charge
 EbView eb_view(const emg_ctx *c);
 // device Yee update and field energy on eb_dev (k_yee.hip)
-void launch_eb_split(emg_ctx *c);  // eb_stage -> eb_dev
+// n points from point o0 on, in the boundary's layout at rec, into eb_dev
+void launch_eb_split(emg_ctx *c, const double *rec, int64_t o0, int64_t n);
 void launch_bfield(emg_ctx *c);
 void launch_efield(emg_ctx *c, double tcs, double dlt);
 // points [o0, o0 + n) of the box lo .. lo + ext - 1 (x fastest), 6 values each

@@ -30,16 +30,20 @@ __device__ __forceinline__ bool my_point(const EbView &v, int64_t &o, int &i, in
   return true;
 }
 
-// the uploaded records (six components per point) into the component arrays
-__global__ __launch_bounds__(kBlock) void k_eb_split(const double *__restrict__ rec, EbView v) {
+// n uploaded records (six components per point) into the component arrays from
+// point o0 on
+__global__ __launch_bounds__(kBlock) void k_eb_split(const double *__restrict__ rec, EbView v,
+                                                     int64_t o0, int64_t n) {
   const int64_t o = (int64_t)blockIdx.x * kBlock + threadIdx.x;
-  if (o >= v.np) return;
+  if (o >= n) return;
   const double2 *r = reinterpret_cast<const double2 *>(rec + 6 * o);
+  double2 a[3];
+#pragma unroll
+  for (int q = 0; q < 3; q++) a[q] = r[q];
 #pragma unroll
   for (int q = 0; q < 3; q++) {
-    const double2 a = r[q];
-    v.eb[(2 * q) * v.np + o] = a.x;
-    v.eb[(2 * q + 1) * v.np + o] = a.y;
+    v.eb[(2 * q) * v.np + o0 + o] = a[q].x;
+    v.eb[(2 * q + 1) * v.np + o0 + o] = a[q].y;
   }
 }
 
@@ -193,9 +197,9 @@ EbView eb_view(const emg_ctx *c) {
   return v;
 }
 
-void launch_eb_split(emg_ctx *c) {
-  const EbView v = eb_view(c);
-  hipLaunchKernelGGL(k_eb_split, dim3(blocks_of(v)), dim3(kBlock), 0, c->stream, c->eb_stage, v);
+void launch_eb_split(emg_ctx *c, const double *rec, int64_t o0, int64_t n) {
+  hipLaunchKernelGGL(k_eb_split, dim3((unsigned)((n + kBlock - 1) / kBlock)), dim3(kBlock), 0,
+                     c->stream, rec, eb_view(c), o0, n);
 }
 
 void launch_bfield(emg_ctx *c) {
