@@ -156,9 +156,9 @@ __global__ __launch_bounds__(kBlock) void k_join(State64 st, int64_t src0, int64
 }
 
 template <typename T>
-int dalloc(T **p, size_t count, const char *what) {
+int dalloc(emg_ctx *c, T **p, size_t count, const char *what) {
   if (count == 0) count = 1;
-  if (dev_malloc(p, sizeof(T) * count)) return EMG_OK;
+  if (dev_malloc(c, p, sizeof(T) * count)) return EMG_OK;
   return set_error(EMG_ERR_NOMEM, std::string("device allocation failed: ") + what);
 }
 
@@ -178,12 +178,12 @@ void free_state64(State64 &st) {
 }
 
 // all of a state's arrays or none
-int alloc_state64(State64 &st, int64_t cap) {
+int alloc_state64(emg_ctx *c, State64 &st, int64_t cap) {
   int rc;
-  if ((rc = dalloc(&st.x, cap, "x")) || (rc = dalloc(&st.y, cap, "y")) ||
-      (rc = dalloc(&st.z, cap, "z")) || (rc = dalloc(&st.vx, cap, "vx")) ||
-      (rc = dalloc(&st.vy, cap, "vy")) || (rc = dalloc(&st.vz, cap, "vz")) ||
-      (rc = dalloc(&st.pid, cap, "pid")))
+  if ((rc = dalloc(c, &st.x, cap, "x")) || (rc = dalloc(c, &st.y, cap, "y")) ||
+      (rc = dalloc(c, &st.z, cap, "z")) || (rc = dalloc(c, &st.vx, cap, "vx")) ||
+      (rc = dalloc(c, &st.vy, cap, "vy")) || (rc = dalloc(c, &st.vz, cap, "vz")) ||
+      (rc = dalloc(c, &st.pid, cap, "pid")))
     free_state64(st);
   return rc;
 }
@@ -363,8 +363,8 @@ int emg_create(const emg_config *cfg, emg_ctx **out) {
   c->sp.off[cfg->nspec] = off;
   c->cap_total = off;
   int nsp = cfg->nspec;
-  if ((rc = dalloc(&c->dflag, 2, "flag")) ||
-      (rc = dalloc((double **)&c->face, (size_t)(face_len(c->g) * nsp), "upper-face charge"))) {
+  if ((rc = dalloc(c, &c->dflag, 2, "flag")) ||
+      (rc = dalloc(c, (double **)&c->face, (size_t)(face_len(c->g) * nsp), "upper-face charge"))) {
     emg_destroy(c);
     return rc;
   }
@@ -379,17 +379,17 @@ int emg_create(const emg_config *cfg, emg_ctx **out) {
   launch_zero(c->dflag, 2 * sizeof(int), c->stream);
   if (cfg->precision == EMG_PLAIN_FP64) {
     int64_t nn = (int64_t)(cfg->n[0] + 1) * (cfg->n[1] + 1) * (cfg->n[2] + 1);
-    if ((rc = alloc_state64(c->s64, c->cap_total)) || (rc = dalloc(&c->node64, 8 * nn, "nodal E/B")) ||
-        (rc = dalloc(&c->rho64, c->ncell * nsp, "rho")) ||
-        (rc = dalloc(&c->j64, 3 * c->ncell * nsp, "current")) ||
-        (rc = dalloc(&c->ke_part, energy64_part_need(nsp), "energy partials"))) {
+    if ((rc = alloc_state64(c, c->s64, c->cap_total)) || (rc = dalloc(c, &c->node64, 8 * nn, "nodal E/B")) ||
+        (rc = dalloc(c, &c->rho64, c->ncell * nsp, "rho")) ||
+        (rc = dalloc(c, &c->j64, 3 * c->ncell * nsp, "current")) ||
+        (rc = dalloc(c, &c->ke_part, energy64_part_need(nsp), "energy partials"))) {
       emg_destroy(c);
       return rc;
     }
   } else {
-    if ((rc = fx_alloc(c, c->cap_total)) || (rc = dalloc(&c->node32, 8 * c->ncell, "nodal E/B")) ||
-        (rc = dalloc(&c->rhofx, c->ncell * nsp, "rho")) ||
-        (rc = dalloc(&c->jfx, 3 * c->ncell * nsp, "current"))) {
+    if ((rc = fx_alloc(c, c->cap_total)) || (rc = dalloc(c, &c->node32, 8 * c->ncell, "nodal E/B")) ||
+        (rc = dalloc(c, &c->rhofx, c->ncell * nsp, "rho")) ||
+        (rc = dalloc(c, &c->jfx, 3 * c->ncell * nsp, "current"))) {
       emg_destroy(c);
       return rc;
     }
@@ -561,7 +561,7 @@ int emg_upload_particles(emg_ctx *c, const emg_particle *pbuf, const int64_t *co
   bool dead = !fits;  // more records than room: only the living have to fit
   int64_t sent = total;
   if (c->cfg.precision == EMG_FP32_FIXED) {
-    if ((rc = alloc_state64(tmp, std::max<int64_t>(c->cap_total, 1)))) return rc;
+    if ((rc = alloc_state64(c, tmp, std::max<int64_t>(c->cap_total, 1)))) return rc;
     tgt = tmp;
   }
   if (fits) {
@@ -634,7 +634,7 @@ int emg_download_particles(emg_ctx *c, emg_particle *pbuf, int64_t *counts) {
   State64 src = c->s64;
   State64 tmp{};
   if (c->cfg.precision == EMG_FP32_FIXED) {
-    if ((rc = alloc_state64(tmp, c->cap_total))) return rc;
+    if ((rc = alloc_state64(c, tmp, c->cap_total))) return rc;
     rc = fx_to64(c, tmp);
     if (rc) {
       free_state64(tmp);
@@ -679,7 +679,7 @@ int emg_set_fields(emg_ctx *c, const double *eb, const int32_t lo[3], const int3
     dfree(c->eb_dev);
     c->eb_dev = nullptr;
     c->eb_dev_bytes = 0;
-    if ((rc = dalloc(&c->eb_dev, bytes / sizeof(double), "eb"))) return rc;
+    if ((rc = dalloc(c, &c->eb_dev, bytes / sizeof(double), "eb"))) return rc;
     c->eb_dev_bytes = bytes;
   }
   for (int d = 0; d < 3; d++) {
@@ -762,7 +762,7 @@ int emg_solve_es(emg_ctx *c, double rhobk) {
       c->eb_ext[d] = n[d] + 3;
       count *= (size_t)c->eb_ext[d];
     }
-    int rc = dalloc(&c->eb_dev, count, "eb");
+    int rc = dalloc(c, &c->eb_dev, count, "eb");
     if (rc) return rc;
     c->eb_dev_bytes = count * sizeof(double);
     launch_zero(c->eb_dev, c->eb_dev_bytes, c->stream);
@@ -783,7 +783,7 @@ int emg_set_background(emg_ctx *c, const double *rhobk) {
     return EMG_OK;
   }
   int rc;
-  if (!c->bk_dev && (rc = dalloc(&c->bk_dev, (size_t)c->ncell, "background charge"))) return rc;
+  if (!c->bk_dev && (rc = dalloc(c, &c->bk_dev, (size_t)c->ncell, "background charge"))) return rc;
   rc = hip_check(hipMemcpyAsync(c->bk_dev, rhobk, sizeof(double) * c->ncell,
                                 hipMemcpyHostToDevice, c->stream),
                  "background copy");
@@ -809,7 +809,7 @@ int emg_field_energy(emg_ctx *c, double cs, double *engeb) {
   int rc = need_eb(c);
   if (rc) return rc;
   if (!engeb) return set_error(EMG_ERR_ARG, "null argument");
-  if (!c->fe_buf && (rc = dalloc(&c->fe_buf, (size_t)field_energy_part_need(), "field energy")))
+  if (!c->fe_buf && (rc = dalloc(c, &c->fe_buf, (size_t)field_energy_part_need(), "field energy")))
     return rc;
   launch_field_energy(c, cs, c->fe_buf, c->hsum);
   if ((rc = read_sums(c))) return rc;
@@ -1056,10 +1056,10 @@ static int need_adjoint(emg_ctx *c) {
   int rc = need_fp64(c);
   if (rc) return rc;
   if (c->adj_sum) return bins_alloc(c);  // the last one: then all are there
-  if ((!c->lam && (rc = dalloc(&c->lam, 8 * (size_t)c->cap_total, "particle adjoints"))) ||
-      (!c->adj_e && (rc = dalloc(&c->adj_e, 3 * c->ncell, "adjoint field"))) ||
-      (!c->adj_g && (rc = dalloc(&c->adj_g, c->ncell, "adjoint density"))) ||
-      (rc = dalloc(&c->adj_sum, (size_t)adj_vsum_need(), "adjoint sums")))
+  if ((!c->lam && (rc = dalloc(c, &c->lam, 8 * (size_t)c->cap_total, "particle adjoints"))) ||
+      (!c->adj_e && (rc = dalloc(c, &c->adj_e, 3 * c->ncell, "adjoint field"))) ||
+      (!c->adj_g && (rc = dalloc(c, &c->adj_g, c->ncell, "adjoint density"))) ||
+      (rc = dalloc(c, &c->adj_sum, (size_t)adj_vsum_need(), "adjoint sums")))
     return rc;
   launch_zero(c->lam, 8 * sizeof(double) * c->cap_total, c->stream);
   launch_zero(c->adj_e, sizeof(double) * 3 * c->ncell, c->stream);
@@ -1073,7 +1073,7 @@ int emg_state_save(emg_ctx *c, int32_t slot) {
   if (!rc) rc = need_particles(c);
   if (rc) return rc;
   if (slot < 0 || slot >= kStateSlots) return set_error(EMG_ERR_ARG, "slot must be 0..63");
-  if (!c->slot[slot].x && (rc = alloc_state64(c->slot[slot], c->cap_total))) return rc;
+  if (!c->slot[slot].x && (rc = alloc_state64(c, c->slot[slot], c->cap_total))) return rc;
   for (int s = 0; s < c->sp.nspec; s++) c->slot_cnt[slot][s] = c->sp.cnt[s];
   return copy_state(c->s64, c->slot[slot], c->cap_total, c->stream);
 }
@@ -1169,7 +1169,7 @@ int emg_init_device(emg_ctx *c, const emg_device_species *spec, int32_t nspec, u
   }
   int rc;
   State64 tmp{};
-  if (c->cfg.precision != EMG_PLAIN_FP64 && (rc = alloc_state64(tmp, c->cap_total))) return rc;
+  if (c->cfg.precision != EMG_PLAIN_FP64 && (rc = alloc_state64(c, tmp, c->cap_total))) return rc;
   for (int s = 0; s < nspec; s++) c->sp.cnt[s] = spec[s].count;
   if (c->cfg.precision == EMG_PLAIN_FP64) {
     rc = init_device_into(c, c->s64, spec, nspec, seed);

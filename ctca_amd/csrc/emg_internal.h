@@ -390,6 +390,7 @@ struct TileBins {
   int64_t *start;
   BinRec *rec;
   int64_t len;  // records
+  bool recorded;  // a graph uses them
 };
 struct BinTiles {
   int ntx, nty, ntz, n;
@@ -513,13 +514,16 @@ namespace emg {
 // error plumbing (emg_api.hip)
 int set_error(int code, const std::string &msg);
 int hip_check(hipError_t e, const char *what);
+bool bins_give_back(emg_ctx *c);  // frees bins.rec; false if there is nothing to free
 
-// device memory; where there is none a null pointer, and no error left for the
-// next launch's check to find
+// device memory, the tile records' if there is no other; where there is none a
+// null pointer, and no error left for the next launch's check to find
 template <typename T>
-bool dev_malloc(T **p, size_t bytes) {
-  if (hipMalloc((void **)p, bytes) == hipSuccess) return true;
-  (void)hipGetLastError();
+bool dev_malloc(emg_ctx *c, T **p, size_t bytes) {
+  do {
+    if (hipMalloc((void **)p, bytes) == hipSuccess) return true;
+    (void)hipGetLastError();
+  } while (bins_give_back(c));
   *p = nullptr;
   return false;
 }

@@ -140,19 +140,32 @@ int bins_alloc(emg_ctx *c) {
   TileBins &B = c->bins;
   if (B.rec) return EMG_OK;
   const int64_t n = bin_tiles(c->g).n;
-  if (!B.count && !dev_malloc(&B.count, sizeof(int32_t) * 2 * n))
+  if (!B.count && !dev_malloc(c, &B.count, sizeof(int32_t) * 2 * n))
     return set_error(EMG_ERR_NOMEM, "tile counters");
-  if (!B.start && !dev_malloc(&B.start, sizeof(int64_t) * (n + 1)))
+  if (!B.start && !dev_malloc(c, &B.start, sizeof(int64_t) * (n + 1)))
     return set_error(EMG_ERR_NOMEM, "tile starts");
   const int rc = scan_tmp_alloc(c, n);
   if (rc) return rc;
   int64_t len = std::min(std::max<int64_t>(c->cap_total, 1), kBinMax);
-  while (!dev_malloc(&B.rec, sizeof(BinRec) * len)) {
+  while (!dev_malloc(c, &B.rec, sizeof(BinRec) * len)) {
     if (len <= 65536) return set_error(EMG_ERR_NOMEM, "tile records");
     len /= 2;
   }
   B.len = len;
   return EMG_OK;
+}
+
+// The records, up to 512 MB, are a workspace that is had again when it is next
+// needed: what else the context allocates comes first (unless a graph holds their
+// address).
+bool bins_give_back(emg_ctx *c) {
+  TileBins &B = c->bins;
+  if (!B.rec || B.recorded || capturing(c)) return false;
+  (void)hipStreamSynchronize(c->stream);
+  (void)hipFree(B.rec);
+  B.rec = nullptr;
+  B.len = 0;
+  return true;
 }
 
 int64_t bin_pass(emg_ctx *c, int64_t done[EMG_MAX_SPECIES]) {
@@ -167,6 +180,7 @@ int64_t bin_pass(emg_ctx *c, int64_t done[EMG_MAX_SPECIES]) {
     most = std::max(most, k);
   }
   if (most == 0) return 0;
+  c->bins.recorded = c->bins.recorded || capturing(c);
   const int64_t total = c->bins.len - room;
   // 16 particles per thread make a block's records of a tile a run of several;
   // small populations need the blocks more

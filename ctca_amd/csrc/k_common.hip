@@ -634,7 +634,7 @@ int scan_tmp_alloc(emg_ctx *c, int64_t n) {
   if (need <= c->scan_tmp_len) return EMG_OK;
   if (c->scan_tmp) (void)hipFree(c->scan_tmp);
   c->scan_tmp_len = 0;
-  if (!dev_malloc(&c->scan_tmp, sizeof(int64_t) * need))
+  if (!dev_malloc(c, &c->scan_tmp, sizeof(int64_t) * need))
     return set_error(EMG_ERR_NOMEM, "scan scratch");
   c->scan_tmp_len = need;
   return EMG_OK;
@@ -743,9 +743,9 @@ int sort64_alloc(emg_ctx *c) {
     c->sort_cursor = nullptr;
     c->sort_start = nullptr;
     c->sort_len = 0;
-    if (!dev_malloc(&c->sort_count, sizeof(int32_t) * len) ||
-        !dev_malloc(&c->sort_cursor, sizeof(int32_t) * len) ||
-        !dev_malloc(&c->sort_start, sizeof(int64_t) * (len + 1)))
+    if (!dev_malloc(c, &c->sort_count, sizeof(int32_t) * len) ||
+        !dev_malloc(c, &c->sort_cursor, sizeof(int32_t) * len) ||
+        !dev_malloc(c, &c->sort_start, sizeof(int64_t) * (len + 1)))
       return set_error(EMG_ERR_NOMEM, "sort scratch");
     c->sort_len = len;
   }
@@ -754,14 +754,14 @@ int sort64_alloc(emg_ctx *c) {
   if (!c->t64.x) {
     void *p[7];
     for (int q = 0; q < 7; q++)
-      if (!dev_malloc(&p[q], (q < 6 ? sizeof(double) : sizeof(int32_t)) * c->cap_total)) {
+      if (!dev_malloc(c, &p[q], (q < 6 ? sizeof(double) : sizeof(int32_t)) * c->cap_total)) {
         for (int r = 0; r < q; r++) (void)hipFree(p[r]);
         return set_error(EMG_ERR_NOMEM, "sort buffers");
       }
     c->t64 = State64{(double *)p[0], (double *)p[1], (double *)p[2], (double *)p[3],
                      (double *)p[4], (double *)p[5], (int32_t *)p[6]};
   }
-  if (!c->sort_rec && !dev_malloc(&c->sort_rec, 68 * (size_t)c->cap_total))
+  if (!c->sort_rec && !dev_malloc(c, &c->sort_rec, 68 * (size_t)c->cap_total))
     return set_error(EMG_ERR_NOMEM, "sort records");
   return EMG_OK;
 }
@@ -835,13 +835,13 @@ int build_runs(emg_ctx *c, int which) {
   if (c->run_base_len < nb + 1) {
     if (c->run_base) (void)hipFree(c->run_base);
     c->run_base_len = 0;
-    if (!dev_malloc(&c->run_base, sizeof(int64_t) * (nb + 1))) return EMG_OK;
+    if (!dev_malloc(c, &c->run_base, sizeof(int64_t) * (nb + 1))) return EMG_OK;
     c->run_base_len = nb + 1;
   }
   if (c->runs_cap[which] < cap) {
     if (c->runs[which]) (void)hipFree(c->runs[which]);
     c->runs_cap[which] = 0;
-    if (!dev_malloc(&c->runs[which], sizeof(Run) * cap)) return EMG_OK;
+    if (!dev_malloc(c, &c->runs[which], sizeof(Run) * cap)) return EMG_OK;
     c->runs_cap[which] = cap;
   }
   const dim3 gr((unsigned)((nbmax + kBlock - 1) / kBlock), (unsigned)c->sp.nspec);

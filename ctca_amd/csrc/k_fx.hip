@@ -1961,21 +1961,21 @@ int fx_alloc(emg_ctx *c, int64_t ntotal) {
   for (int k = 0; k < 2; k++) {
     StateFx &S = B.st[k];
     const size_t bytes = sizeof(float) * B.cap_total;
-    if (!dev_malloc(&S.cell, bytes) || !dev_malloc(&S.fx, bytes) || !dev_malloc(&S.fy, bytes) ||
-        !dev_malloc(&S.fz, bytes) || !dev_malloc(&S.vx, bytes) || !dev_malloc(&S.vy, bytes) ||
-        !dev_malloc(&S.vz, bytes))
+    if (!dev_malloc(c, &S.cell, bytes) || !dev_malloc(c, &S.fx, bytes) || !dev_malloc(c, &S.fy, bytes) ||
+        !dev_malloc(c, &S.fz, bytes) || !dev_malloc(c, &S.vx, bytes) || !dev_malloc(c, &S.vy, bytes) ||
+        !dev_malloc(c, &S.vz, bytes))
       return set_error(EMG_ERR_NOMEM, "FP32 particle buffers");
     S.pid = nullptr;
-    if (c->cfg.track_pid && !dev_malloc(&S.pid, sizeof(int32_t) * B.cap_total))
+    if (c->cfg.track_pid && !dev_malloc(c, &S.pid, sizeof(int32_t) * B.cap_total))
       return set_error(EMG_ERR_NOMEM, "FP32 pid buffers");
-    if (!dev_malloc(&B.start[k], sizeof(int64_t) * (B.nb + 1)) ||
-        !dev_malloc(&B.count[k], sizeof(int32_t) * B.nb) ||
-        !dev_malloc(&B.nst[k], sizeof(int32_t) * B.nb) ||
-        !dev_malloc(&B.cap[k], sizeof(int32_t) * B.nb) ||
-        !dev_malloc(&B.spill[k], sizeof(int32_t) * EMG_MAX_SPECIES) ||
-        !dev_malloc(&B.pre[k], sizeof(int32_t) * B.nb * kPre))
+    if (!dev_malloc(c, &B.start[k], sizeof(int64_t) * (B.nb + 1)) ||
+        !dev_malloc(c, &B.count[k], sizeof(int32_t) * B.nb) ||
+        !dev_malloc(c, &B.nst[k], sizeof(int32_t) * B.nb) ||
+        !dev_malloc(c, &B.cap[k], sizeof(int32_t) * B.nb) ||
+        !dev_malloc(c, &B.spill[k], sizeof(int32_t) * EMG_MAX_SPECIES) ||
+        !dev_malloc(c, &B.pre[k], sizeof(int32_t) * B.nb * kPre))
       return set_error(EMG_ERR_NOMEM, "bucket tables");
-    if (!dev_malloc(&B.ob[k], sizeof(FxRec) * B.nb * kObStride))
+    if (!dev_malloc(c, &B.ob[k], sizeof(FxRec) * B.nb * kObStride))
       return set_error(EMG_ERR_NOMEM, "bucket outboxes");
     launch_zero(B.count[k], sizeof(int32_t) * B.nb, c->stream);
     launch_zero(B.nst[k], sizeof(int32_t) * B.nb, c->stream);
@@ -1984,18 +1984,18 @@ int fx_alloc(emg_ctx *c, int64_t ntotal) {
     launch_zero(B.start[k], sizeof(int64_t) * (B.nb + 1), c->stream);
     launch_zero(B.pre[k], sizeof(int32_t) * B.nb * kPre, c->stream);
   }
-  if (!dev_malloc(&B.stay, sizeof(int32_t) * B.nb) ||
-      !dev_malloc(&B.extra, sizeof(int32_t) * B.nb) ||
-      !dev_malloc(&B.hist, sizeof(int32_t) * B.nb) ||
-      !dev_malloc(&B.cursor, sizeof(int32_t) * B.nb) ||
-      !dev_malloc(&B.shist[0], sizeof(int32_t) * B.nb) ||
-      !dev_malloc(&B.shist[1], sizeof(int32_t) * B.nb) ||
-      !dev_malloc(&B.plan_word, sizeof(unsigned long long) * plan_blocks(B.nb)) ||
-      !dev_malloc(&B.plan_ticket, sizeof(unsigned long long)) ||
-      !dev_malloc(&B.scur, sizeof(int32_t) * B.nb) ||
-      !dev_malloc(&B.spre, sizeof(int64_t) * (B.nb + 1)))
+  if (!dev_malloc(c, &B.stay, sizeof(int32_t) * B.nb) ||
+      !dev_malloc(c, &B.extra, sizeof(int32_t) * B.nb) ||
+      !dev_malloc(c, &B.hist, sizeof(int32_t) * B.nb) ||
+      !dev_malloc(c, &B.cursor, sizeof(int32_t) * B.nb) ||
+      !dev_malloc(c, &B.shist[0], sizeof(int32_t) * B.nb) ||
+      !dev_malloc(c, &B.shist[1], sizeof(int32_t) * B.nb) ||
+      !dev_malloc(c, &B.plan_word, sizeof(unsigned long long) * plan_blocks(B.nb)) ||
+      !dev_malloc(c, &B.plan_ticket, sizeof(unsigned long long)) ||
+      !dev_malloc(c, &B.scur, sizeof(int32_t) * B.nb) ||
+      !dev_malloc(c, &B.spre, sizeof(int64_t) * (B.nb + 1)))
     return set_error(EMG_ERR_NOMEM, "bucket tables");
-  if (!dev_malloc(&B.spl, sizeof(FxRec) * B.spill_cap * c->sp.nspec))
+  if (!dev_malloc(c, &B.spl, sizeof(FxRec) * B.spill_cap * c->sp.nspec))
     return set_error(EMG_ERR_NOMEM, "sorted spill buffer");
   for (int k = 0; k < 2; k++) launch_zero(B.shist[k], sizeof(int32_t) * B.nb, c->stream);
   launch_zero(B.plan_word, sizeof(unsigned long long) * plan_blocks(B.nb), c->stream);
@@ -2004,7 +2004,7 @@ int fx_alloc(emg_ctx *c, int64_t ntotal) {
   const int rc = scan_tmp_alloc(c, B.nb);
   if (rc) return rc;
   int64_t kp = (int64_t)(B.nb + c->sp.nspec * kSpillBlocksPerSpecies) * 3;
-  if (!dev_malloc(&c->ke_part, sizeof(double) * kp))
+  if (!dev_malloc(c, &c->ke_part, sizeof(double) * kp))
     return set_error(EMG_ERR_NOMEM, "energy partials");
   c->ke_part_n = kp;
   B.cur = 0;

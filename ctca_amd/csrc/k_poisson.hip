@@ -494,15 +494,15 @@ static int es_solver_get(emg_ctx *c, EsSolver **out) {
   const int64_t hx = c->g.nx / 2 + 1;
   const int neig = c->g.nx + c->g.ny + c->g.nz;
   int rc = EMG_OK;
-  if (!dev_malloc(&s->rho, sizeof(double) * c->ncell) ||
-      !dev_malloc(&s->spec, sizeof(double2) * c->g.nz * c->g.ny * hx) ||
-      !dev_malloc(&s->eig, sizeof(double) * neig))
+  if (!dev_malloc(c, &s->rho, sizeof(double) * c->ncell) ||
+      !dev_malloc(c, &s->spec, sizeof(double2) * c->g.nz * c->g.ny * hx) ||
+      !dev_malloc(c, &s->eig, sizeof(double) * neig))
     rc = set_error(EMG_ERR_NOMEM, "field solver arrays");
   FftAxis ax[3];
   s->path = solve_path(c->g, ax);
   if (!rc && s->path != kLibrary) {
-    if (!dev_malloc(&s->tw, sizeof(double2) * neig) ||
-        !dev_malloc(&s->ax, sizeof(ax)))
+    if (!dev_malloc(c, &s->tw, sizeof(double2) * neig) ||
+        !dev_malloc(c, &s->ax, sizeof(ax)))
       rc = set_error(EMG_ERR_NOMEM, "field solver arrays");
     for (int d = 0; d < 3; d++) s->kind = std::max(s->kind, radix_kind(ax[d]));
     auto allow = [&](auto kernel) {
