@@ -20,7 +20,7 @@ fake.fake_log.restype = ctypes.c_char_p
 for f in (fake.fake_used, fake.fake_peak):
     f.restype = ctypes.c_size_t
 fake.fake_limit.argtypes = [ctypes.c_size_t]
-fake.fake_fail_in.argtypes = [ctypes.c_long]
+fake.fake_fail_in.argtypes = [ctypes.c_long] * 2
 import numpy as np
 import pytest
 from ctca_amd import emg

@@ -25,7 +25,7 @@ struct Kernel {
 std::map<const void *, Kernel> kernels;   // by host stub
 std::string launches;
 size_t used = 0, peak = 0, limit = SIZE_MAX;
-long fail_in = -1;                        // this allocation from now fails
+long fail_in = -1, fail_times = 0;        // this allocation from now fails, and so many in all
 int bad_frees = 0, bad_copies = 0, bad_args = 0, mallocs = 0, capturing = 0, last_error = 0;
 int flags[2] = {0, 0};                    // what the next k_flag reports
 std::map<int64_t, int> split;             // pid of the record that k_split puts where
@@ -60,7 +60,7 @@ void note(const std::string &what) { launches += what + "\n"; }
 API void fake_log_clear() { std::lock_guard<std::mutex> l(mu); launches.clear(); }
 API const char *fake_log() { return launches.c_str(); }
 API void fake_limit(size_t bytes) { limit = bytes; }
-API void fake_fail_in(long n) { fail_in = n; }
+API void fake_fail_in(long n, long times) { fail_in = n; fail_times = times; }
 API size_t fake_used() { return used; }
 API size_t fake_peak(int reset) { const size_t p = peak; if (reset) peak = used; return p; }
 API int fake_mallocs() { return mallocs; }
@@ -88,7 +88,12 @@ API int hipMalloc(void **p, size_t n) {
   std::lock_guard<std::mutex> l(mu);
   mallocs++;
   if (capturing) return fail(900);  // not while a stream is captured
-  if ((fail_in > 0 && --fail_in == 0) || n > limit || used > limit - n) return fail(2);
+  if (fail_in > 0 && fail_times > 0 && --fail_in == 0) {
+    fail_in = 1;
+    fail_times--;
+    return fail(2);
+  }
+  if (n > limit || used > limit - n) return fail(2);
   char *q = (char *)std::malloc(n ? n : 1);
   if (!q) return fail(2);
   live[q] = n;
