@@ -1075,6 +1075,7 @@ int emg_state_save(emg_ctx *c, int32_t slot) {
   if (slot < 0 || slot >= kStateSlots) return set_error(EMG_ERR_ARG, "slot must be 0..63");
   if (!c->slot[slot].x && (rc = alloc_state64(c, c->slot[slot], c->cap_total))) return rc;
   for (int s = 0; s < c->sp.nspec; s++) c->slot_cnt[slot][s] = c->sp.cnt[s];
+  c->slot_ordered[slot] = c->ordered || c->runs_valid;
   return copy_state(c->s64, c->slot[slot], c->cap_total, c->stream);
 }
 
@@ -1086,6 +1087,7 @@ int emg_state_load(emg_ctx *c, int32_t slot) {
     return set_error(EMG_ERR_ARG, "slot holds no saved state");
   for (int s = 0; s < c->sp.nspec; s++) c->sp.cnt[s] = c->slot_cnt[slot][s];
   c->have_particles = true;
+  c->ordered = c->slot_ordered[slot];
   c->moves_after_sort = emg::kUnsorted;
   c->runs_valid = false;
   c->rho_valid = c->j_valid = c->ke_valid = false;

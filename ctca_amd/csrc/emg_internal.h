@@ -438,7 +438,7 @@ struct emg_ctx {
   int pushes_since_sort;  // PLAIN_FP64 pushes since the last cell sort (sort_every)
   int moves_after_sort;   // PLAIN_FP64 pushes since the state was last sorted, or kUnsorted
 
-  bool ordered;           // the uploaded order keeps neighbours together
+  bool ordered;           // the order that was uploaded or loaded keeps neighbours together
   emg::TileBins bins;     // workspace (lazy)
 
   // FP32 state
@@ -504,6 +504,7 @@ struct emg_ctx {
   double *adj_sum;   // block partials of the velocity adjoint sums
   emg::State64 slot[emg::kStateSlots];  // saved particle states
   int64_t slot_cnt[emg::kStateSlots][EMG_MAX_SPECIES];
+  bool slot_ordered[emg::kStateSlots];
 
   bool timing;
   emg::Timer timers[emg::kTNum];
