@@ -428,32 +428,39 @@ static size_t column_lds(int n) {
 }
 
 // Which one is the fastest.  Solve, E included, hipFFT : planes : lines in us.
-// Planes where LDS holds them: 16^3 cells 19.3 : 17.7 : 22.0, 32^3 22.3 : 19.4 :
-// 24.1, 64^3 36.7 : 29.9 : 36.4, 90x70x51 46.8 : 44.9 : 46.5, 77x63x70 72 : 42 :
-// 47, 84^3 57 : 50 : 58, 88^3 69 : 47 : 64, 96^3 73 : 54 : 63 (98x98x50 is the
-// exception, 51 : 57 : 57).
-// From a prime factor of 19 on hipFFT changes to a longer algorithm: 31^3 117 : 23
-// : 28, 53^3 150 : 36 : 43; there the lines do the work of planes of more than
-// 3000 elements (62^3 128 : 38 : 38, 101x40x40 74 : 38 : 40, 95x66x40 87 : 43 : 38,
-// 97x98x50 113 : 78 : 62) and of those that LDS does not hold (114x95x133 252 : -
-// : 112, 191x181x173 1141 : - : 596).
+// Small planes: 16^3 cells 19.3 : 17.7 : 22.0, 32^3 22.3 : 19.4 : 24.1, 64^3 36.7 :
+// 29.9 : 36.4, 64x64x4 26.7 : 22.2 : 24.8.  Above 3000 elements a plane is a long
+// chain for its one block, which pays where there are many: 90x100 cells by 4 27.6
+// : 36.4 : 28.5, by 32 41.7 : 44.8 : 39.6, by 48 52.5 : 48.9 : 46.7, by 96 75.5 :
+// 56.9 : 63.9; 84x84 by 4 34 : 32 : 29, by 48 48 : 44 : 46; 60x140 by 4 52 : 35 : 30,
+// by 48 65 : 51 : 52; 90x70x51 46.8 : 44.9 : 46.5; 96^3 73 : 54 : 63.
+// From a prime factor of 19 on hipFFT changes to a longer algorithm, and the lines
+// do the work of the larger planes: 31^3 117 : 23 : 28, 53^3 150 : 36 : 43, 62^3
+// 128 : 38 : 38, 101x40x40 74 : 38 : 40, 95x66x40 87 : 43 : 38, 97x98x50 113 : 78 : 62,
+// 114x95x133 252 : - : 112, 191x181x173 1141 : - : 596.
 // An odd nx costs hipFFT's real transforms about twice an even one, and the lines
-// nothing: 105x100x100 131 : - : 88, 125^3 154 : - : 99, 143x119x130 217 : - : 133,
-// 225^3 1204 : - : 503.  Else the two are close (110^3 106 : - : 99, 112^3 94 : - :
-// 102, 126^3 127 : - : 109, 130x143x119 129 : - : 145, 150^3 155 : - : 152,
-// 180x150x170 219 : - : 251, 200^3 323 : - : 326, 256x256x64 194 : - : 200).
+// nothing: 105x100x100 131 : - : 88, 125^3 154 : - : 99, 225^3 1204 : - : 503.
+// Else, with factors 2, 3 and 5, the lines up to some 2 million cells (100x100x16
+// 49 : - : 33, 100^3 83 : - : 69, 48x200x96 80 : - : 63, 128^3 117 : - : 106, 256x64x96
+// 110 : - : 90, but 512x64x64 111 : - : 118), beyond that about equal (150^3 155 : - :
+// 152, 160^3 169 : - : 170, 256x256x64 194 : - : 200); with 7, 11 or 13 now this, now
+// that (110^3 106 : - : 99, 126^3 127 : - : 109, 112^3 94 : - : 102, 98x112x112 84 : -
+// : 94, 154x143x91 124 : - : 135, 180x150x170 219 : - : 251).
 // The first solve of planes and lines also has no kernels to compile at run time
 // (1.6 s : 0.2 ms).
 static SolvePath solve_path(const Grid &g, FftAxis ax[3]) {
   const int n[3] = {g.nx, g.ny, g.nz};
-  int largest = 0;
+  int largest = 0, kind = 0;
   for (int d = 0; d < 3; d++) {
     if (n[d] > kLongestLine || !fft_axis(n[d], kLargestRadix, &ax[d])) return kLibrary;
+    kind = std::max(kind, radix_kind(ax[d]));
     for (int p = 0; p < ax[d].npass; p++) largest = std::max(largest, ax[d].r[p]);
   }
-  if (plane_lds(g, kPlanes) <= kPlaneLds && (largest < 19 || plane_elems(g, kPlanes) <= 3000))
-    return kPlanes;
-  return largest >= 19 || g.nx % 2 ? kLines : kLibrary;
+  if (plane_lds(g, kPlanes) <= kPlaneLds)
+    return plane_elems(g, kPlanes) <= 3000 || (largest < 19 && g.nz >= 48) ? kPlanes : kLines;
+  if (largest >= 19 || g.nx % 2) return kLines;
+  const bool small = (int64_t)g.nx * g.ny * g.nz <= 1 << 21 && std::max({n[0], n[1], n[2]}) < 512;
+  return kind < 2 && small ? kLines : kLibrary;
 }
 
 template <class F>

@@ -53,12 +53,14 @@ def test_axes_split_into_small_radices_and_large_primes(tmp_path):
 
 
 @pytest.mark.parametrize("path,sizes", [
-    ("planes", [(16, 16, 16), (45, 45, 45), (49, 50, 63), (90, 70, 51), (77, 77, 10), (98, 98, 50),
-                (96, 96, 96), (31, 31, 31), (62, 62, 62), (100, 91, 14), (9, 9, 211)]),
+    ("planes", [(16, 16, 16), (45, 45, 45), (49, 50, 63), (90, 70, 51), (77, 77, 60), (98, 98, 48),
+                (96, 96, 96), (31, 31, 31), (62, 62, 62), (72, 72, 4), (9, 9, 211), (512, 9, 2)]),
     ("lines", [(95, 66, 40), (114, 95, 133), (199, 40, 40), (62, 127, 9), (105, 100, 100),
-               (125, 125, 125), (225, 64, 64), (99, 121, 98)]),
-    ("library", [(100, 100, 100), (150, 150, 150), (200, 200, 40), (180, 150, 170),
-                 (128, 125, 135), (256, 256, 64), (110, 121, 100), (8, 223, 8), (6, 10, 640)]),
+               (125, 125, 125), (225, 64, 64), (99, 121, 98), (90, 100, 47), (60, 140, 4),
+               (100, 100, 16), (100, 100, 100), (128, 128, 128), (400, 40, 40)]),
+    ("library", [(150, 150, 150), (200, 200, 60), (180, 150, 170), (128, 126, 135),
+                 (256, 256, 64), (110, 121, 100), (112, 112, 112), (512, 64, 64), (8, 223, 8),
+                 (6, 10, 640)]),
 ])
 def test_grids_take_the_path_that_was_measured_for_them(tmp_path, path, sizes):
     fake_hip.run(tmp_path, f"""

@@ -7,7 +7,7 @@ import pytest
 
 def test_fft_plans_follow_the_context_stream(tmp_path):
     fake_hip.run(tmp_path, """
-        n = (128, 128, 8)
+        n = (112, 112, 8)
         with emg.Context(n, [1.0], [1.0], [1.0], (10,)) as c:
             c.upload(records(10, n), (10,))
             c.deposit_rho(0)
@@ -30,7 +30,7 @@ def test_library_solve_after_the_stream_has_changed():
         pytest.skip("the library initialised the device before torch")
     import oracle
     from ctca_amd import emg
-    n, count = (128, 128, 8), 50000
+    n, count = (112, 112, 8), 50000
     rng = np.random.default_rng(17)
     rec = np.zeros(count, dtype=emg.PARTICLE)
     for c, m in zip("xyz", n):
