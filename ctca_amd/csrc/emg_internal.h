@@ -534,7 +534,7 @@ bool capturing(emg_ctx *c);   // whether the stream's work is being recorded int
 
 // Host transfers (emg_io.hip) in chunks of whole units.  fill enqueues on the
 // context's stream what writes bytes [off, off + len) of the result to the
-// pinned slot; io_read copies them to the caller's array and reports the
+// pinned slot; io_read copies them to the caller's array and (flags) reports the
 // device-side errors first.  use enqueues what reads the slot; the caller's
 // array is free when io_write returns.  copy, if given, fills the slot with what
 // takes the place of those bytes, at most as many, and returns their number, which
@@ -542,7 +542,7 @@ bool capturing(emg_ctx *c);   // whether the stream's work is being recorded int
 // threads at once.
 using IoFn = std::function<int(size_t off, size_t len, void *slot)>;
 using IoCopy = std::function<size_t(size_t off, size_t len, void *slot)>;
-int io_read(emg_ctx *c, void *user, size_t bytes, size_t unit, const IoFn &fill);
+int io_read(emg_ctx *c, void *user, size_t bytes, size_t unit, const IoFn &fill, bool flags = true);
 int io_write(emg_ctx *c, const void *user, size_t bytes, size_t unit, const IoFn &use,
              const IoCopy &copy = nullptr);
 // f(a, b) over ranges that make up [0, n), each entry standing for `bytes` of host
@@ -551,7 +551,7 @@ int io_ranges(emg_ctx *c, int64_t n, size_t bytes,
               const std::function<void(int64_t, int64_t)> &f);
 int read_flags(emg_ctx *c);  // synchronise and report device-side errors
 // a device array of 8-byte values
-int io_read_array(emg_ctx *c, void *user, const void *dev, size_t bytes);
+int io_read_array(emg_ctx *c, void *user, const void *dev, size_t bytes, bool flags = true);
 void io_open(emg_ctx *c);
 void io_close(emg_ctx *c);
 

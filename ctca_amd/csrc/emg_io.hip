@@ -198,8 +198,8 @@ int read_flags(emg_ctx *c) {
   return rc ? rc : flags_error(c);
 }
 
-int io_read(emg_ctx *c, void *user, size_t bytes, size_t unit, const IoFn &fill) {
-  if (bytes == 0) return read_flags(c);
+int io_read(emg_ctx *c, void *user, size_t bytes, size_t unit, const IoFn &fill, bool flags) {
+  if (bytes == 0) return flags ? read_flags(c) : EMG_OK;
   const Plan p = plan_of(bytes, unit);
   int rc = ring(c, p, false);
   if (rc) return rc;
@@ -212,13 +212,13 @@ int io_read(emg_ctx *c, void *user, size_t bytes, size_t unit, const IoFn &fill)
     if (!r && p.n > 1) r = hip_check(hipEventRecord(io.ev[s], c->stream), "transfer event");
     return r;
   };
-  hipLaunchKernelGGL(k_flag, dim3(1), dim3(1), 0, c->stream, c->dflag, c->hflag);
+  if (flags) hipLaunchKernelGGL(k_flag, dim3(1), dim3(1), 0, c->stream, c->dflag, c->hflag);
   for (int i = 0; i < slots && !rc; i++) rc = enqueue(i);
   // device-side errors are reported before anything reaches the caller's array
   if (!rc)
     rc = p.n == 1 ? hip_check(hipStreamSynchronize(c->stream), "stream synchronize")
                   : hip_check(hipEventSynchronize(io.ev[0]), "stream synchronize");
-  if (!rc) rc = flags_error(c);
+  if (!rc && flags) rc = flags_error(c);
   if (rc) {
     (void)hipStreamSynchronize(c->stream);
     return rc;
@@ -242,14 +242,15 @@ int io_read(emg_ctx *c, void *user, size_t bytes, size_t unit, const IoFn &fill)
   return rc;
 }
 
-int io_read_array(emg_ctx *c, void *user, const void *dev, size_t bytes) {
-  return io_read(c, user, bytes, 8, [c, dev](size_t off, size_t len, void *slot) {
+int io_read_array(emg_ctx *c, void *user, const void *dev, size_t bytes, bool flags) {
+  const IoFn fill = [c, dev](size_t off, size_t len, void *slot) {
     const int64_t n = (int64_t)(len / 8);
     hipLaunchKernelGGL(k_copy8, dim3((unsigned)((n + kBlock - 1) / kBlock)), dim3(kBlock), 0,
                        c->stream, (const unsigned long long *)((const char *)dev + off), n,
                        (unsigned long long *)slot);
     return hip_check(hipGetLastError(), "read-out");
-  });
+  };
+  return io_read(c, user, bytes, 8, fill, flags);
 }
 
 int io_ranges(emg_ctx *c, int64_t n, size_t bytes,

@@ -629,7 +629,8 @@ int solve_es(emg_ctx *c, double rhobk) {
 
 int read_potential(emg_ctx *c, double *phi) {
   if (!c->es) return set_error(EMG_ERR_STATE, "no field solve yet");
-  return io_read_array(c, phi, c->es->rho, sizeof(double) * c->ncell);
+  // (the particles' errors are left to the calls on them)
+  return io_read_array(c, phi, c->es->rho, sizeof(double) * c->ncell, false);
 }
 
 }  // namespace emg
