@@ -39,12 +39,13 @@ struct Tri {
 };
 
 // cell and weights of the reference's trilinear interpolation (int() cells,
-// psolve2.F90:154-183), positions in [0, L)
+// psolve2.F90:154-183), positions in [0, L]; the cell is held in the grid for one
+// beyond, which a push that reported it as moved too far may have left
 __device__ __forceinline__ Tri tri(double x, double y, double z, const Grid &g) {
   Tri t;
-  t.i = min((int)x, g.nx - 1);
-  t.j = min((int)y, g.ny - 1);
-  t.k = min((int)z, g.nz - 1);
+  t.i = min(max((int)x, 0), g.nx - 1);
+  t.j = min(max((int)y, 0), g.ny - 1);
+  t.k = min(max((int)z, 0), g.nz - 1);
   double x1 = x - t.i, y1 = y - t.j, z1 = z - t.k;
   t.wx[0] = 1.0 - x1;
   t.wx[1] = x1;
