@@ -463,7 +463,6 @@ int emg_destroy(emg_ctx *c) {
   dfree(c->runs[1]);
   dfree(c->run_base);
   dfree(c->sort_count);
-  dfree(c->sort_cursor);
   dfree(c->sort_start);
   dfree(c->scan_tmp);
   dfree(c->dflag);

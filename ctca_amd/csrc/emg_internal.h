@@ -17,8 +17,8 @@ constexpr int kFixShift = 24;  // rho fixed point: unit CIC weight = 2^24
 constexpr double kFixScale = 16777216.0;
 constexpr int kJShift = 24;  // current fixed point: 2^24 per unit flux (cell / unit time)
 constexpr double kJScale = 16777216.0;
-constexpr int kStateSlots = 64;
-constexpr int kUnsorted = 1 << 30;  // moves_after_sort of a state in no known order  // saved particle states of the adjoint window
+constexpr int kStateSlots = 64;     // saved particle states of the adjoint window
+constexpr int kUnsorted = 1 << 30;  // moves_after_sort of a state in no known order
 
 // device error flags
 constexpr int kFlagDomain = 1;    // particle outside [0, L] / non-finite
@@ -478,7 +478,6 @@ struct emg_ctx {
 
   // sort scratch
   int32_t *sort_count;   // nspec x ncell (or nb)
-  int32_t *sort_cursor;
   int64_t *sort_start;
   int64_t sort_len;
   void *sort_rec;        // cap_total x 64-byte records + cap_total int32 ranks (FP64 sort, lazy)
@@ -604,7 +603,7 @@ void launch_zero(void *p, size_t bytes, hipStream_t s);
 // last sort can ride on the next push instead: sort64_rank counts the
 // current cells (each key's start, each particle's rank in its key), the
 // push writes every particle to its sorted slot (SortDest), and sort64_commit
-// makes that the live state and builds the blocks' run tables of it.
+// makes that the live state.  A run table is built when a launch first needs it.
 int sort64(emg_ctx *c, bool patched);
 int sort64_runs(emg_ctx *c, int which);  // the run table of the charge (0) or the zigzag (1)
 bool sort64_fusable(const emg_ctx *c);

@@ -737,14 +737,11 @@ int sort64_alloc(emg_ctx *c) {
   int64_t len = nkey * c->sp.nspec;
   if (c->sort_len < len) {
     if (c->sort_count) (void)hipFree(c->sort_count);
-    if (c->sort_cursor) (void)hipFree(c->sort_cursor);
     if (c->sort_start) (void)hipFree(c->sort_start);
     c->sort_count = nullptr;
-    c->sort_cursor = nullptr;
     c->sort_start = nullptr;
     c->sort_len = 0;
     if (!dev_malloc(c, &c->sort_count, sizeof(int32_t) * len) ||
-        !dev_malloc(c, &c->sort_cursor, sizeof(int32_t) * len) ||
         !dev_malloc(c, &c->sort_start, sizeof(int64_t) * (len + 1)))
       return set_error(EMG_ERR_NOMEM, "sort scratch");
     c->sort_len = len;
