@@ -1948,9 +1948,9 @@ int fx_alloc(emg_ctx *c, int64_t ntotal) {
   for (int s = 0; s < c->sp.nspec; s++) maxs = c->cfg.capacity[s] > maxs ? c->cfg.capacity[s] : maxs;
   B.spill_cap = maxs / 16 + 4096;
   // 4^3 tiles in place of 8^3 ones keep what those would: evenly spread particles
-  // leave a tile of 4, or pass the cell beyond it, at most twice as often as one
-  // of 8, which has kObStride + kExtra places and its share of the spill for them
-  if (few) B.spill_cap = std::min(maxs, 2 * (B.spill_cap + (kObStride + kExtra) * nt8));
+  // leave a tile of 4, or pass the cell beyond it, at most twice as often as one of
+  // 8, whose eight times fewer buckets have as many outbox places each
+  if (few) B.spill_cap = std::min(maxs, 2 * (B.spill_cap + kExtra * nt8));
   B.spill_cap = align_up(B.spill_cap);
   if (B.spill_cap > (1 << 28)) B.spill_cap = 1 << 28;
   B.cap_total = B.area + B.spill_cap * c->sp.nspec;
