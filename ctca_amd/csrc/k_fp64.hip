@@ -629,7 +629,8 @@ __device__ __forceinline__ Relay relay_axis(double xnew, double lb, double cb, i
 constexpr double kEmFix = 281474976710656.0;          // 2^48
 
 // RESORT as in k_push_dep64.  Bound by latency and instruction issue (VALU about
-// 40%, LDS conflicts 30%, HBM 3 TB/s); four waves per SIMD (128 VGPRs).  On the
+// 40%, LDS bank conflicts 29% of the CUs' cycles and 81% of the LDS's active ones,
+// HBM 3 TB/s); four waves per SIMD (125 VGPRs, 128 with RESORT).  On the
 // 18.5M-particle two-stream (128 x 64 x 64), 1.42 ms before: one sum per node
 // for a particle that stays in its cell, the flush without divisions and the
 // short fixed-point conversion 1.12; four waves instead of three 1.02; the

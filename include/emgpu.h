@@ -227,7 +227,8 @@ int emg_field_energy(emg_ctx *ctx, double cs, double *engeb);
  * value); phi solves -lap7 phi = rho with the 7-point Laplacian's eigenvalues
  * sum_d (2 sin(pi k_d / n_d))^2 (inifft.F90:390-404), the zero mode dropped
  * (poissn.F90:398-410), through real-to-complex FFTs (the library's own, or
- * hipFFT's on large grids of small factors; not FFTW: the round-off differs); E = -grad phi on the staggered points (esfild.F90:
+ * hipFFT's on large grids of even nx and small factors; not FFTW: the
+ * round-off differs); E = -grad phi on the staggered points (esfild.F90:
  * 351-367) is written into the device eb (B kept; an eb(6, -1:n+1)^3 with
  * B = 0 is created if none was uploaded) and relocated to the nodes.
  * emg_get_potential reads phi(0:nx-1, 0:ny-1, 0:nz-1) of the last solve.
