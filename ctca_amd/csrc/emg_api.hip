@@ -852,11 +852,19 @@ static int sort_if_due(emg_ctx *c, int which, bool *carry = nullptr) {
   return rc;
 }
 
+// a call that moves the particles (and deposits their charge) is recorded
+static void note_recorded(emg_ctx *c, bool deposits) {
+  if (!capturing(c)) return;
+  c->push_recorded = true;
+  c->move_recorded = c->move_recorded || !deposits;
+}
+
 int emg_positn(emg_ctx *c, int32_t ustep) {
   CTX_CHECK(c);
   int rc = need_particles(c);
   if (rc) return rc;
   if (ustep < 0) return set_error(EMG_ERR_ARG, "ustep must be >= 0");
+  note_recorded(c, false);
   if ((rc = sort_if_due(c, 0))) return rc;
   if (c->cfg.precision == EMG_PLAIN_FP64) {
     launch_positn64(c, ustep);
@@ -876,6 +884,7 @@ int emg_push_es(emg_ctx *c, int32_t ustep) {
   if (!rc) rc = need_fields(c);
   if (rc) return rc;
   if (ustep < 0) return set_error(EMG_ERR_ARG, "ustep must be >= 0");
+  note_recorded(c, true);
   bool carry;
   if ((rc = sort_if_due(c, 0, &carry))) return rc;
   if (c->cfg.precision == EMG_PLAIN_FP64) {
@@ -902,7 +911,9 @@ int emg_deposit_rho(emg_ctx *c, int32_t func) {
   int rc = need_particles(c);
   if (rc) return rc;
   if (func < 0 || func > 2) return set_error(EMG_ERR_ARG, "func must be 0, 1 or 2");
-  if (!c->rho_valid) {  // a push deposits at its new positions itself
+  // a push deposits at its new positions itself (in a capture, the last call is
+  // the last one of a replay too)
+  if (!c->rho_valid || (c->move_recorded && !capturing(c))) {
     if (c->cfg.precision == EMG_PLAIN_FP64) {
       if ((rc = sort64_runs(c, 0))) return rc;
       launch_deposit64(c);
@@ -998,6 +1009,7 @@ int emg_push_em(emg_ctx *c, int32_t ustep) {
   if (!rc) rc = need_fields(c);
   if (rc) return rc;
   if (ustep < 1) return set_error(EMG_ERR_ARG, "ustep must be >= 1");
+  note_recorded(c, false);
   bool carry;
   if ((rc = sort_if_due(c, 1, &carry))) return rc;
   if (c->cfg.precision == EMG_PLAIN_FP64) {

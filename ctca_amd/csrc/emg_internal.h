@@ -469,6 +469,9 @@ struct emg_ctx {
   bool rho_valid;
   bool j_valid;
   void *face;       // nspec x face_len: upper-face charge (double, or fixed point in FP32_FIXED)
+  // a graph holds a push, and one that moves particles without depositing their
+  // charge: its replays move them unseen
+  bool push_recorded, move_recorded;
   bool faces_valid; // face holds the deposit of the current positions
 
   // energy

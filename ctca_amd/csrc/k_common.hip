@@ -687,7 +687,7 @@ bool prepare_read_rho(emg_ctx *c, const int lo[3], const int hi[3]) {
     const int nd = d == 0 ? c->g.nx : (d == 1 ? c->g.ny : c->g.nz);
     ghosts = ghosts || (lo[d] <= -1 && hi[d] >= -1) || (lo[d] <= nd + 1 && hi[d] >= nd + 1);
   }
-  if (ghosts && c->face && !c->faces_valid) {
+  if (ghosts && c->face && (!c->faces_valid || c->push_recorded)) {
     if (c->cfg.precision == EMG_PLAIN_FP64)
       launch_faces64(c);
     else

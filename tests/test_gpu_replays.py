@@ -173,3 +173,39 @@ def test_adjoint_steps_recorded_after_a_reset():
             got.append(program(ctx, recorded))
     for a, b in zip(*got):         # FP64 sums of some thousand terms in another order
         assert np.abs(a - b).max() <= 1e-11 * np.abs(a).max()
+
+
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+def test_ghost_planes_after_replays(precision):
+    need_torch()
+    from ctca_amd import emg
+    n, counts = (16, 20, 12), (9000, 4000)
+    rng = np.random.default_rng(6)
+    rec = np.zeros(sum(counts), dtype=emg.PARTICLE)
+    for c, m in zip("xyz", n):
+        rec[c] = rng.random(sum(counts)) * m
+        rec["v" + c] = rng.normal(size=sum(counts)) * 0.2
+    box = (-1,) * 3, tuple(m + 1 for m in n)
+
+    def program(ctx, recorded):
+        def steps():
+            ctx.push_es(2)
+            ctx.push_es(2)
+
+        out = []
+        ctx.upload(rec, counts)
+        ctx.set_fields(np.zeros((n[2] + 3, n[1] + 3, n[0] + 3, 6)))
+        steps()
+        two = Recorded(ctx, steps) if recorded else steps
+        for _ in range(3):
+            two()
+            out.append(ctx.rho(*box))
+        return out
+
+    got = []
+    for recorded in (False, True):
+        with emg.Context(n, [1.0, -0.5], [0.0, 0.0], [1.0, 1.0], counts,
+                         precision=emg.PLAIN_FP64 if precision == "fp64" else emg.FP32_FIXED) as c:
+            got.append(program(c, recorded))
+    for a, b in zip(*got):         # sums of some tens of weights in another order
+        assert np.abs(a - b).max() <= 1e-13 * np.abs(a).max()

@@ -68,3 +68,29 @@ def test_an_adjoint_step_allocates_nothing_after_the_window_has_begun(tmp_path):
                 fake.fake_capture(0)
                 assert fake.fake_mallocs() == before
     """)
+
+
+def test_charge_and_faces_are_computed_anew_where_a_replay_may_have_moved_particles(tmp_path):
+    fake_hip.run(tmp_path, """
+        n, counts = (16, 16, 16), (2000, 1000)
+        ghosts = ((-1,) * 3, (17,) * 3)
+        for precision in (emg.PLAIN_FP64, emg.FP32_FIXED):
+            for moves_alone in (False, True):
+                with emg.Context(n, [1.0, -1.0], [1.0, 1.0], [1.0, 1.0], counts,
+                                 precision=precision) as c:
+                    def faces():
+                        return any("faces" in k for k in launches(c.rho, *ghosts))
+
+                    c.upload(records(3000, n), counts)
+                    c.set_fields(np.zeros((19, 19, 19, 6)))
+                    c.push_es(2)
+                    assert launches(c.deposit_rho, 0) == []
+                    assert faces() and not faces()
+                    fake.fake_capture(1)
+                    c.positn(2) if moves_alone else c.push_es(2)
+                    deposit = launches(c.deposit_rho, 0)
+                    fake.fake_capture(0)
+                    assert (deposit != []) == moves_alone
+                    assert (launches(c.deposit_rho, 0) != []) == moves_alone
+                    assert faces() and faces()
+    """)
