@@ -4,11 +4,11 @@
 //
 // Element i of line l is buf[i * stride + l]: neighbouring threads take
 // neighbouring lines, so their accesses fall on different banks whatever the
-// radix.  A pass reads one buffer and writes the other (Stockham: no bit
-// reversal).  With ns the product of the radices done, pass r takes for
-// j = 0 .. n/r - 1, k = j mod ns, the inputs x[j + p n/r] times
-// w^(p k n / (ns r)), w = e^(-2 pi i / n), transforms those r values, and
-// writes result q to (j / ns) ns r + k + q ns.
+// radix.  A pass reads one buffer and writes the other (the self-sorting form that
+// Cochran et al. 1967 credit to Stockham: no bit reversal).  With ns the product of
+// the radices done, pass r takes for j = 0 .. n/r - 1, k = j mod ns, the inputs x[j
+// + p n/r] times w^(p k n / (ns r)), w = e^(-2 pi i / n), transforms those r
+// values, and writes result q to (j / ns) ns r + k + q ns.
 //
 // Radices 2, 3, 4, 5, 7, 8, 11 and 13 transform in registers; any other prime sums
 // its products straight from LDS, and comes first (ns = 1, no twiddles), where

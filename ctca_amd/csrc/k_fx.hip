@@ -1267,14 +1267,14 @@ __global__ __launch_bounds__(kBlock) void k_fx_prep(uint4 *acc, int64_t n16, boo
 //           neighbours' outboxes, its spill particles and kExtra direct slots;
 //   their exclusive scan (X's bucket starts) and that of the spill counts;
 //   the counters of the next step cleared.
-// The scan runs across blocks by look-back: a block publishes its two sums in
-// one 64-bit word (3 bits launch tag, 2 bits state, the capacities in units of
-// kAlign slots in 27 bits, the spill counts in 32), then its first wave adds
-// the words of the blocks before it, 64 at a time.  The word is the whole
-// message, so no other memory has to be made visible between blocks.  Blocks
-// take their place from a ticket, so every block waited for has started; the
-// ticket also numbers the launches (their tag), so a replayed graph's launches
-// differ like any others.
+// The scan runs across blocks by look-back (Merrill and Garland 2016): a block
+// publishes its two sums in one 64-bit word (3 bits launch tag, 2 bits state, the
+// capacities in units of kAlign slots in 27 bits, the spill counts in 32), then
+// its first wave adds the words of the blocks before it, 64 at a time.  The word
+// is the whole message, so no other memory has to be made visible between blocks.
+// Blocks take their place from a ticket, so every block waited for has started;
+// the ticket also numbers the launches (their tag), so a replayed graph's
+// launches differ like any others.
 // Seven launches (spill histogram, capacities, three scan kernels, spill
 // scatter, finish) and the clearing took 4-5 us each; this one and k_fx_prep
 // take 6.2 + 2.6 us on 32^3 cells (1,024 buckets).
